@@ -884,6 +884,7 @@ ColArgs<T> col_args(NsdContext* c) {
     a.m_inv_re = c->m_inv_re;
     a.src = c->closure ? (const cx<T>*)c->cl_src : nullptr;
     a.pairs = pairs_ok(c) ? 1 : 0;
+    a.jblocks = jblocks_ok(c) ? 1 : 0;  // J of the stage kernels; the transforms clear it
     a.prev = (cx<T>*)c->ec_prev;
     a.ymid = (cx<T>*)c->ec_ymid;
     a.errpart = c->ec_part;
@@ -902,6 +903,7 @@ RowArgs<T> row_args(NsdContext* c) {
     a.sc = c->sc;
     a.bm = M_of(c);
     a.pairs = pairs_ok(c) ? 1 : 0;
+    a.jblocks = jblocks_ok(c) ? 1 : 0;
     return a;
 }
 
@@ -1111,6 +1113,7 @@ void enqueue_closure(NsdContext* c) {
         ColArgs<T> f = col_args<T>(c);
         f.mode = COL_FWD;
         f.nbat = nb;
+        f.jblocks = 0;  // written by ROW_R2C
         f.nl = (const cx<T>*)c->cl_m;
         f.out_c = (cx<T>*)c->cl_src;
         f.fwd_scale = 1.0;
@@ -1295,6 +1298,7 @@ int op_forward(NsdContext* c, const double* in_phys, double* out_ref, double sca
     launch_row_t<T>(c, r, c->G.ny / 2);
     ColArgs<T> a = col_args<T>(c);
     a.mode = COL_FWD;
+    a.jblocks = 0;  // written by ROW_R2C
     a.out_ref = out_ref;
     a.fwd_scale = scale;
     launch_col_t<T>(c, a, c->G.nkx);
@@ -1319,7 +1323,6 @@ int op_nonlinear(NsdContext* c, const double* w_ref, const double* psi_ref, doub
     launch_row_t<T>(c, r, c->G.ny / 2);
     ColArgs<T> f = col_args<T>(c);
     f.mode = COL_FWD;
-    f.jblocks = jblocks_ok(c) ? 1 : 0;  // J of a pair-layout row stage
     f.out_ref = out_ref;
     f.fwd_scale = -1.0;  // spectral_core.c:108-111
     launch_col_t<T>(c, f, c->G.nkx);
@@ -1384,7 +1387,6 @@ int op_nl_member(NsdContext* c, int m, double* out_ref, int compute_rows) {
     ColArgs<T> f = col_args<T>(c);
     f.mode = COL_FWD;
     f.nl = (const cx<T>*)c->nl + (size_t)m * M_of(c);
-    f.jblocks = jblocks_ok(c) ? 1 : 0;  // J of a pair-layout row stage
     f.out_ref = out_ref;
     f.fwd_scale = -1.0;  // spectral_core.c:108-111
     launch_col_t<T>(c, f, c->G.nkx);

@@ -484,7 +484,7 @@ struct ColArgs {
     const cx<T>* nl;  // mixed input (COL_STAGE, COL_FWD)
     cx<T>* mixed[4];  // mixed outputs
     int pairs;        // COL_STAGE, COL_PRIME: write them in the stage layout (stage_layout)
-    int jblocks;      // COL_FWD: J in 2 x 2 blocks (written by a pair-layout row stage)
+    int jblocks;      // COL_STAGE, COL_FWD: J in 2 x 2 blocks (square pair-layout grids)
     cx<T>* state;     // compact state (read; written on the last stage)
     cx<T>* acc;       // compact RK accumulator
     cx<T>* stagebuf;  // compact stage state (classic scheme)
@@ -703,14 +703,19 @@ __global__ __launch_bounds__(NT, MW) void k_col(ColArgs<T> a) {
         std::conditional_t<WS, TwWs<T>, TwRegs<LC, T>> tw;
         if constexpr (WS) load_tw_ws(tw, j, a.tw);
         else load_tw_regs<LC, 0>(tw, j, a.tw);
-        if constexpr (pair_layout<T, LC, NT, PR>()) {  // J in 2 x 2 blocks
-            // jblock_elem(kxi, ny, y), y = j + s TPL (TPL even): a column base,
-            // the lane's offset j + (j & ~1), and 2 TPL per slot
-            const unsigned jb0 = __umul24((unsigned)(kxi & ~1), (unsigned)G.ny) +
-                                 2u * (unsigned)(kxi & 1) + (unsigned)(j + (j & ~1));
+        if constexpr (pair_layout<T, LC, NT, PR>()) {
+            // J in 2 x 2 blocks: jblock_elem(kxi, ny, y), y = j + s TPL (TPL
+            // even), is a column base, the lane's offset j + (j & ~1), and
+            // 2 TPL per slot; [kx][y] on rectangular grids, whose row stage
+            // has another length and writes that
+            const bool jb = a.jblocks != 0;
+            const unsigned jb0 = jb ? __umul24((unsigned)(kxi & ~1), (unsigned)G.ny) +
+                                          2u * (unsigned)(kxi & 1) + (unsigned)(j + (j & ~1))
+                                    : col_elem(kxi, G.ny, j);
+            const unsigned jbs = jb ? 2u * (unsigned)TPL : (unsigned)TPL;
 #pragma unroll
             for (int s = 0; s < P; ++s)
-                v[s] = has_data ? *at32(nl, jb0 + 2u * (unsigned)(s * TPL)) : zero;
+                v[s] = has_data ? *at32(nl, jb0 + (unsigned)s * jbs) : zero;
         } else if constexpr (rowpair_layout<T, LC, NT, PR>()) {
             // J's last reader, whole columns: non-temporal loads, which leave
             // the caches to the mixed fields written next (FP64 4096^2:
@@ -1171,6 +1176,7 @@ struct RowArgs {
     unsigned short* out_bf16;  // ROW_C2R: field 0 as bf16, times out_bf16_scale (if non-null)
     float out_bf16_scale;
     int pairs;                 // ROW_STAGE: mixed fields in the stage layout (stage_layout)
+    int jblocks;               // ROW_STAGE: write J in 2 x 2 blocks (square pair-layout grids)
     int skip_on_redo;          // ROW_STAGE, ERR: idle when the step restores a rejected one
 };
 
@@ -1279,7 +1285,7 @@ __device__ __forceinline__ void build_two_rows2(cx<T> (&v1)[P], cx<T> (&v2)[P], 
 template <int LC, typename T, typename TW, bool JB = false>
 __device__ __forceinline__ void fwd_rows_store(cx<T> (&v)[P], cx<T>* lds, int j, const Line& g,
                                                const Geo& G, const TW& tw, cx<T>* out, int y,
-                                               bool active) {
+                                               bool active, int jblocks = 0) {
     const int TPL = LC > 0 ? LC / P : g.TPL;
     const int Ll = LC > 0 ? LC : g.L;
     const int kxm = LC > 0 ? Band<LC>::kxm : G.kxmax;
@@ -1314,10 +1320,12 @@ __device__ __forceinline__ void fwd_rows_store(cx<T> (&v)[P], cx<T>* lds, int j,
             const cx<T> ja = mk(T(0.5) * (zk.x + zm.x), T(0.5) * (zk.y - zm.y));
             const cx<T> jb = mk(T(0.5) * (zk.y + zm.y), T(0.5) * (zm.x - zk.x));
             if constexpr (JB) {
-                // jblock_elem(k, ny, y) for even y: (k & ~1) ny + 2 (k & 1) + 2 y
+                // jblock_elem(k, ny, y) for even y: (k & ~1) ny + 2 (k & 1) + 2 y;
+                // [kx][y] where the column stage has another length
                 static_assert(sizeof(T) == 4, "J blocks are an FP32 layout");
-                const unsigned e = __umul24((unsigned)(k & ~1), (unsigned)G.ny) +
-                                   2u * (unsigned)((k & 1) + y);
+                const unsigned e = jblocks ? __umul24((unsigned)(k & ~1), (unsigned)G.ny) +
+                                                 2u * (unsigned)((k & 1) + y)
+                                           : col_elem(k, G.ny, y);
                 *reinterpret_cast<float4*>(at32(out, e)) = float4{ja.x, ja.y, jb.x, jb.y};
             } else {
                 cx<T>* dst = at32(out, col_elem(k, G.ny, y));
@@ -1630,7 +1638,8 @@ __global__ __launch_bounds__(NT, MW) void k_row(RowArgs<T> a) {
 #pragma unroll
             for (int s = 0; s < P; ++s)
                 v[s] = mk(X[s].x * v2[s].x - Jp[s].x * v[s].x, X[s].y * v2[s].y - Jp[s].y * v[s].y);
-            fwd_rows_store<LC, T, TwWs<T>, true>(v, lds, j, g, G, tw, a.nl + moff, y0, active);
+            fwd_rows_store<LC, T, TwWs<T>, true>(v, lds, j, g, G, tw, a.nl + moff, y0,
+                                                    active, a.jblocks);
         }
         if (a.track_umax) block_max_to(active ? double(um.value()) : 0.0, &a.sc[blockIdx.y].umax2_bits, red);
         return;
@@ -1689,7 +1698,7 @@ __global__ __launch_bounds__(NT, MW) void k_row(RowArgs<T> a) {
                 v[s] = mk(X[s].x * v2[s].x - Jp[s].x * v[s].x, X[s].y * v2[s].y - Jp[s].y * v[s].y);
             // a pair-layout row stage writes J in 2 x 2 blocks
             fwd_rows_store<LC, T, TwRegs<LC, T>, pair_layout<T, LC, NT, PR>()>(
-                v, lds, j, g, G, tw, a.nl + moff, y0, active);
+                v, lds, j, g, G, tw, a.nl + moff, y0, active, a.jblocks);
         }
         if (a.track_umax) block_max_to(active ? double(um.value()) : 0.0, &a.sc[blockIdx.y].umax2_bits, red);
         return;
