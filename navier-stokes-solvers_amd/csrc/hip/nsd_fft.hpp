@@ -586,12 +586,13 @@ __device__ __forceinline__ void line_fft2_c(cx<T> (&v1)[P], cx<T> (&v2)[P], cx<T
 }
 
 // ------------------------------------------------------------------------
-// 4096-point lines on 512 threads as 8 x 512 (wave-split transforms).
+// Lines of L = 512 W points on 64 W threads as W x 512 (wave-split
+// transforms), W = 4, 8 or 16 waves.
 //
 // Thread j = 64 w + l is lane l of wave w.  With n = n2 + 512 n1 and
-// k = k1 + 8 k2 the transform splits into 512 eight-point DFTs across the
-// waves and eight 512-point DFTs, one per wave:
-//   X[k1 + 8 k2] = sum_n2 W512^(n2 k2) W4096^(n2 k1) sum_n1 x[n2 + 512 n1] W8^(n1 k1).
+// k = k1 + W k2 the transform splits into 512 W-point DFTs across the waves
+// and W 512-point DFTs, one per wave:
+//   X[k1 + W k2] = sum_n2 W512^(n2 k2) W_L^(n2 k1) sum_n1 x[n2 + 512 n1] W_W^(n1 k1).
 // Only the step between the two crosses waves.  The 512-point transform of
 // wave w runs on row w of the line region (512 elements, padded one in
 // sixteen) in three radix-8 Stockham passes.  Its exchanges
@@ -600,12 +601,24 @@ __device__ __forceinline__ void line_fft2_c(cx<T> (&v1)[P], cx<T> (&v2)[P], cx<T
 // remain instead of seven, and the cross-wave step reads and writes rows and
 // columns at unit stride.
 //
-// ws_a: standard pattern in (thread j holds x[j + 512 s]), wave-strided
-//       pattern out (lane l of wave w holds X[w + 8 l + 512 s]).
+// ws_a: standard pattern in (thread j holds x[j + 64 W s]), wave-strided
+//       pattern out (lane l of wave w holds X[w + W (l + 64 s)]).
 // ws_b: wave-strided pattern in, standard pattern out: the 512-point DFTs of
-//       y[w + 8 m] first, then the cross-wave step with twiddle W4096^(j w).
+//       y[w + W m] first, then the cross-wave step with twiddle W_L^(j w).
 // A pointwise product between ws_a and ws_b transforms does not see the
 // pattern, which is how the row stage uses them.
+//
+// The cross-wave step on a thread's eight values:
+// - W <= 8: the thread's columns n2 = j + 64 W h, h < Q = 8 / W, each with all
+//   W members at slots h + Q n1; a W-point DFT and the powers of
+//   W_L^(n2) = W_L^j W8^h per column.
+// - W = 16: a column's sixteen members sit in two threads, j = n2 + 512 h with
+//   n1 = h + 2 s.  Each takes the 8-point DFT of its half, times W_L^(j k1),
+//   into row k1 + 8 h; the reader of row k = k1 + 8 q forms the last radix-2
+//   step, (row k1 +- row k1 + 8) W1024^(n2 q).  Two waves then read the same
+//   two rows before either may overwrite its own: one more barrier.  ws_b is
+//   the transpose of that: a thread reads all sixteen rows of its column and
+//   folds rows w and w + 8 (times W1024^j) before its 8-point DFT.
 
 // Row w of a line region starts at 576 w: 512 elements with the
 // one-in-sixteen padding take 544, and a stride of 576 elements (4608 bytes
@@ -614,22 +627,52 @@ __device__ __forceinline__ void line_fft2_c(cx<T> (&v1)[P], cx<T> (&v2)[P], cx<T
 // consecutive padded elements lose a cycle to a bank conflict wherever a
 // 32-lane phase crosses a padding gap; the paired forms do not.
 constexpr int WS_ROW = 576;
-constexpr int WS_REGION = 8 * WS_ROW;  // elements of a wave-split line region
+// waves, and elements of a wave-split line region
+constexpr int ws_waves(int L) { return L / 512; }
+constexpr int ws_region(int L) { return ws_waves(L) * WS_ROW; }
 
+template <int L, typename T>
+struct TwWsCross {};
 template <typename T>
-struct TwWs {
-    cx<T> wj;   // W4096^j: the cross-wave step
+struct TwWsCross<8192, T> {
+    cx<T> wl;                       // W1024^l: the radix-2 step of ws_a
+    const cx<T>* __restrict__ tab;  // the table: W1024^j for the one of ws_b
+};
+
+template <int L, typename T>
+struct TwWs : TwWsCross<L, T> {
+    cx<T> wj;   // W_L^j: the cross-wave step
     cx<T> w8;   // W64^(l mod 8): local pass of stride 8
     cx<T> w64;  // W512^l: local pass of stride 64
 };
 
-// tw is the 4096-point table W4096^m
-template <typename T>
-__device__ __forceinline__ void load_tw_ws(TwWs<T>& t, int j, const cx<T>* __restrict__ tw) {
+// tw is the L-point table W_L^m
+template <int L, typename T>
+__device__ __forceinline__ void load_tw_ws(TwWs<L, T>& t, int j, const cx<T>* __restrict__ tw) {
+    constexpr int W = ws_waves(L);
     const int l = j & 63;
     t.wj = tw[j];
-    t.w8 = tw[(l & 7) << 6];
-    t.w64 = tw[l << 3];
+    t.w8 = tw[(l & 7) * (8 * W)];
+    t.w64 = tw[l * W];
+    if constexpr (W == 16) {
+        t.wl = tw[8 * l];
+        t.tab = tw;
+    }
+}
+
+// Makes a twiddle's value new to the compiler, which otherwise keeps the powers
+// that a first transform formed in registers for the next one.
+template <typename T>
+__device__ __forceinline__ void renew(cx<T>& w) {
+    asm volatile("" : "+v"(w.x), "+v"(w.y));
+}
+template <int L, typename T>
+__device__ __forceinline__ void renew_tw(TwWs<L, T>& t) {
+    if constexpr (L == 8192) {
+        renew(t.wj);
+        renew(t.wl);
+        renew(t.w64);
+    }
 }
 
 // W^1 .. W^7 from W by squaring and products (as in cpass)
@@ -653,6 +696,36 @@ __device__ __forceinline__ void tw_apply8(cx<T> (&v)[P], const cx<T> (&w)[8]) {
 template <int DIR, typename T>
 __device__ __forceinline__ void dft8v(cx<T> (&v)[P]) {
     dft8<DIR>(v[0], v[1], v[2], v[3], v[4], v[5], v[6], v[7]);
+}
+
+// the cross-wave W-point DFTs of a thread's columns (slots h + Q n1), with
+// the twiddles W_L^(n2 k1) applied after (ws_a) or before (ws_b) them
+template <int DIR, int W, bool AFTER, typename T>
+__device__ __forceinline__ void ws_cross(cx<T> (&v)[P], cx<T> wj) {
+    static_assert(W == 4 || W == 8, "cross-wave steps held by one thread");
+    if constexpr (W == 8) {
+        cx<T> w[8];
+        tw_powers8(w, wj);
+        if (!AFTER) tw_apply8<DIR>(v, w);
+        dft8v<DIR>(v);
+        if (AFTER) tw_apply8<DIR>(v, w);
+    } else {
+        constexpr T r2 = Consts<T>::r2;
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            // W_L^(n2) of column n2 = j + 256 h: times W8 for the second one
+            const cx<T> b = h == 0 ? wj : mk(r2 * (wj.x + wj.y), r2 * (wj.y - wj.x));
+            const cx<T> b2 = cmul(b, b), b3 = cmul(b, b2);
+            auto tw = [&]() {
+                v[h + 2] = DIR < 0 ? cmul(v[h + 2], b) : cmulc(v[h + 2], b);
+                v[h + 4] = DIR < 0 ? cmul(v[h + 4], b2) : cmulc(v[h + 4], b2);
+                v[h + 6] = DIR < 0 ? cmul(v[h + 6], b3) : cmulc(v[h + 6], b3);
+            };
+            if (!AFTER) tw();
+            dft4<DIR>(v[h], v[h + 2], v[h + 4], v[h + 6]);
+            if (AFTER) tw();
+        }
+    }
 }
 
 // A wave's LDS operations complete in the order issued: between its writes
@@ -695,9 +768,9 @@ __device__ __forceinline__ int ws_swz(int c) { return c ^ ((c >> 3) & 7); }
 // NF rows (1 or 2) of the wave's 512-point transform, lane l holding elements
 // l + 64 s of each row in and out.  row[f] is this wave's row of field f; its
 // contents may be overwritten.
-template <int DIR, int NF, bool SWZ = false, typename T>
+template <int DIR, int NF, bool SWZ = false, int L, typename T>
 __device__ __forceinline__ void ws_local(cx<T> (*const (&v)[NF])[P], cx<T>* const (&row)[NF],
-                                         int l, const TwWs<T>& tw) {
+                                         int l, const TwWs<L, T>& tw) {
     static_assert(!SWZ || sizeof(T) == 8, "16-byte row layouts");
     // pass 0 (stride 1, no twiddles): butterfly l writes 8 l + r (padded: one
     // 16-element padding group; 16-byte rows: r ^ (l mod 8) inside the
@@ -753,48 +826,101 @@ __device__ __forceinline__ void ws_local(cx<T> (*const (&v)[NF])[P], cx<T>* cons
     }
 }
 
-// NF 4096-point transforms (regions lds[f]), standard pattern in,
+// W16^s times b (s < 8), b a twiddle W1024^l: the table value W1024^(l + 64 s)
+// to one rounding of the product
+template <int S, typename T>
+__device__ __forceinline__ cx<T> times_w16(cx<T> b) {
+    if constexpr (S == 5) return cmul(b, mk(-Consts<T>::s8, -Consts<T>::c8));
+    else if constexpr (S == 7) return cmul(b, mk(-Consts<T>::c8, -Consts<T>::s8));
+    else return w16<-1, S>(b);
+}
+
+// v[s] times W1024^(l + 64 s)
+template <int DIR, int S = 0, typename T>
+__device__ __forceinline__ void tw_apply1024(cx<T> (&v)[P], cx<T> wl) {
+    if constexpr (S < P) {
+        const cx<T> w = times_w16<S>(wl);
+        v[S] = DIR < 0 ? cmul(v[S], w) : cmulc(v[S], w);
+        tw_apply1024<DIR, S + 1>(v, wl);
+    }
+}
+
+// NF L-point transforms (regions lds[f]), standard pattern in,
 // wave-strided pattern out.  Every thread must be free to write the regions
 // on entry (the caller's barrier).  On return each wave still works in its
 // own rows: other waves may write the regions only after a workgroup barrier.
-template <int DIR, int NF, bool SWZ = false, typename T>
+template <int DIR, int NF, bool SWZ = false, int L, typename T>
 __device__ __forceinline__ void ws_a(cx<T> (*const (&v)[NF])[P], cx<T>* const (&lds)[NF], int j,
-                                     const TwWs<T>& tw) {
-    cx<T> w[8];
-    tw_powers8(w, tw.wj);
-#pragma unroll
-    for (int f = 0; f < NF; ++f) {
-        dft8v<DIR>(*v[f]);
-        tw_apply8<DIR>(*v[f], w);
-        cx<T>* o = lds[f] + ws_pos<SWZ>(j);  // u[k1] of column j to row k1
-#pragma unroll
-        for (int r = 0; r < 8; ++r) o[r * WS_ROW] = (*v[f])[r];
-    }
-    __syncthreads();
-    const int wv = j >> 6, l = j & 63;
-    cx<T>* row[NF];
-#pragma unroll
-    for (int f = 0; f < NF; ++f) {
-        row[f] = lds[f] + wv * WS_ROW;
-        const cx<T>* i = row[f] + ws_pos<SWZ>(l);
-#pragma unroll
-        for (int s = 0; s < 8; ++s) (*v[f])[s] = i[ws_off<SWZ>(s)];
-    }
-    wave_lds_fence();
-    ws_local<DIR, NF, SWZ>(v, row, l, tw);
-}
-
-// NF 4096-point transforms, wave-strided pattern in, standard pattern out.
-// On entry only the wave's own rows of the regions have to be free (as they
-// are right after ws_a on the same regions); on return other threads may
-// still be reading the regions.
-template <int DIR, int NF, bool SWZ = false, typename T>
-__device__ __forceinline__ void ws_b(cx<T> (*const (&v)[NF])[P], cx<T>* const (&lds)[NF], int j,
-                                     const TwWs<T>& tw) {
+                                     const TwWs<L, T>& tw) {
+    constexpr int W = ws_waves(L), Q = W <= 8 ? 8 / W : 1;
     const int wv = j >> 6, l = j & 63;
     cx<T>* row[NF];
 #pragma unroll
     for (int f = 0; f < NF; ++f) row[f] = lds[f] + wv * WS_ROW;
+    if constexpr (W == 16) {
+        cx<T> w[8];
+        tw_powers8(w, tw.wj);
+#pragma unroll
+        for (int f = 0; f < NF; ++f) {
+            dft8v<DIR>(*v[f]);
+            tw_apply8<DIR>(*v[f], w);
+            // u[k1] of column j mod 512 to row k1 + 8 (j / 512)
+            cx<T>* o = lds[f] + (j >> 9) * (8 * WS_ROW) + ws_pos<SWZ>(j & 511);
+#pragma unroll
+            for (int r = 0; r < 8; ++r) o[r * WS_ROW] = (*v[f])[r];
+        }
+        __syncthreads();
+        // row k1 +- row k1 + 8, the upper waves' times W1024^(n2)
+        const bool q = __builtin_amdgcn_readfirstlane(wv) >= 8;
+        const T sg = q ? T(-1) : T(1);
+#pragma unroll
+        for (int f = 0; f < NF; ++f) {
+            const cx<T>* i = lds[f] + (wv & 7) * WS_ROW + ws_pos<SWZ>(l);
+#pragma unroll
+            for (int s = 0; s < 8; ++s) {
+                const cx<T> e = i[ws_off<SWZ>(s)], o = i[8 * WS_ROW + ws_off<SWZ>(s)];
+                (*v[f])[s] = mk(fma(sg, o.x, e.x), fma(sg, o.y, e.y));
+            }
+            if (q) tw_apply1024<DIR>(*v[f], tw.wl);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        __syncthreads();  // wave w ^ 8 has read this wave's row
+    } else {
+#pragma unroll
+        for (int f = 0; f < NF; ++f) {
+            ws_cross<DIR, W, true>(*v[f], tw.wj);
+            cx<T>* o = lds[f] + ws_pos<SWZ>(j);  // u[k1] of column j + 64 W h to row k1
+#pragma unroll
+            for (int r = 0; r < W; ++r)
+#pragma unroll
+                for (int h = 0; h < Q; ++h) o[r * WS_ROW + ws_off<SWZ>(W * h)] = (*v[f])[h + Q * r];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int f = 0; f < NF; ++f) {
+            const cx<T>* i = row[f] + ws_pos<SWZ>(l);
+#pragma unroll
+            for (int s = 0; s < 8; ++s) (*v[f])[s] = i[ws_off<SWZ>(s)];
+        }
+        wave_lds_fence();
+    }
+    ws_local<DIR, NF, SWZ>(v, row, l, tw);
+}
+
+// NF L-point transforms, wave-strided pattern in, standard pattern out.
+// On entry only the wave's own rows of the regions have to be free (as they
+// are right after ws_a on the same regions); on return other threads may
+// still be reading the regions.
+template <int DIR, int NF, bool SWZ = false, int L, typename T>
+__device__ __forceinline__ void ws_b(cx<T> (*const (&v)[NF])[P], cx<T>* const (&lds)[NF], int j,
+                                     const TwWs<L, T>& tw) {
+    constexpr int W = ws_waves(L), Q = W <= 8 ? 8 / W : 1;
+    const int wv = j >> 6, l = j & 63;
+    cx<T>* row[NF];
+#pragma unroll
+    for (int f = 0; f < NF; ++f) row[f] = lds[f] + wv * WS_ROW;
+    cx<T> wq;
+    if constexpr (W == 16) wq = tw.tab[8 * j];  // W1024^j, arrives under the local passes
     ws_local<DIR, NF, SWZ>(v, row, l, tw);
 #pragma unroll
     for (int f = 0; f < NF; ++f) {
@@ -803,55 +929,71 @@ __device__ __forceinline__ void ws_b(cx<T> (*const (&v)[NF])[P], cx<T>* const (&
         for (int s = 0; s < 8; ++s) o[ws_off<SWZ>(s)] = (*v[f])[s];
     }
     __syncthreads();
-    cx<T> w[8];
-    tw_powers8(w, tw.wj);
+    if constexpr (W == 16) {
+        cx<T> w[8];
+        tw_powers8(w, tw.wj);
 #pragma unroll
-    for (int f = 0; f < NF; ++f) {
-        const cx<T>* i = lds[f] + ws_pos<SWZ>(j);  // column j of every row
+        for (int f = 0; f < NF; ++f) {
+            const cx<T>* i = lds[f] + ws_pos<SWZ>(j & 511);
 #pragma unroll
-        for (int r = 0; r < 8; ++r) (*v[f])[r] = i[r * WS_ROW];
-        tw_apply8<DIR>(*v[f], w);
-        dft8v<DIR>(*v[f]);
+            for (int r = 0; r < 8; ++r) {
+                const cx<T> y = i[(r + 8) * WS_ROW];
+                (*v[f])[r] = i[r * WS_ROW] + (DIR < 0 ? cmul(y, wq) : cmulc(y, wq));
+            }
+            tw_apply8<DIR>(*v[f], w);
+            dft8v<DIR>(*v[f]);
+        }
+    } else {
+#pragma unroll
+        for (int f = 0; f < NF; ++f) {
+            const cx<T>* i = lds[f] + ws_pos<SWZ>(j);  // columns j + 64 W h of every row
+#pragma unroll
+            for (int r = 0; r < W; ++r)
+#pragma unroll
+                for (int h = 0; h < Q; ++h) (*v[f])[h + Q * r] = i[r * WS_ROW + ws_off<SWZ>(W * h)];
+            ws_cross<DIR, W, false>(*v[f], tw.wj);
+        }
     }
 }
 
 // Wave-strided pattern to standard pattern through region tr.  Wave w writes
-// element c = l + 64 s of its transform at 544 w + (c + 4 w) mod 512 (its own
-// row: the skew by 4 w puts the eight rows of one column in different banks,
+// element c = l + 64 s of its transform at 576 w + (c + 32 w / W) mod 512 (its
+// own row: the skew puts the W rows of one column in different banks,
 // and each 16-lane write phase stays on 16 consecutive elements mod 512);
-// after a barrier thread j reads X[j + 512 s] from row j mod 8, column
-// j / 8 + 64 s, 32 lanes on 32 distinct banks pairs.  On entry the wave's own
+// after a barrier thread j reads X[j + 64 W s] from row j mod W, column
+// j / W + 64 s, 32 lanes on 32 distinct bank pairs.  On entry the wave's own
 // row of tr must be free; on return other threads may still read tr.
-template <int NF, typename T>
+template <int L, int NF, typename T>
 __device__ __forceinline__ void ws_transpose(cx<T> (*const (&v)[NF])[P], cx<T>* const (&tr)[NF],
                                              int j) {
+    constexpr int W = ws_waves(L), SK = 32 / W;
     const int wv = j >> 6, l = j & 63;
 #pragma unroll
     for (int f = 0; f < NF; ++f) {
         cx<T>* o = tr[f] + wv * WS_ROW;
 #pragma unroll
-        for (int s = 0; s < 8; ++s) o[(l + 4 * wv + 64 * s) & 511] = (*v[f])[s];
+        for (int s = 0; s < 8; ++s) o[(l + SK * wv + 64 * s) & 511] = (*v[f])[s];
     }
     __syncthreads();
-    const int rw = j & 7, c0 = j >> 3;
+    const int rw = j & (W - 1), c0 = j / W;
 #pragma unroll
     for (int f = 0; f < NF; ++f) {
         const cx<T>* i = tr[f] + rw * WS_ROW;
 #pragma unroll
-        for (int s = 0; s < 8; ++s) (*v[f])[s] = i[(c0 + 4 * rw + 64 * s) & 511];
+        for (int s = 0; s < 8; ++s) (*v[f])[s] = i[(c0 + SK * rw + 64 * s) & 511];
     }
 }
 
-// NF 4096-point transforms, standard pattern in and out: ws_a on regions
+// NF L-point transforms, standard pattern in and out: ws_a on regions
 // rows, then the transposing exchange through regions tr (which may be the
 // same regions: each wave writes only its own row there).  Entry condition
 // as for ws_a on rows and, when tr differs, every thread free to write tr;
 // on return other threads may still read tr and work in their rows.
-template <int DIR, int NF, bool SWZ = false, typename T>
+template <int DIR, int NF, bool SWZ = false, int L, typename T>
 __device__ __forceinline__ void ws_c(cx<T> (*const (&v)[NF])[P], cx<T>* const (&rows)[NF],
-                                     cx<T>* const (&tr)[NF], int j, const TwWs<T>& tw) {
+                                     cx<T>* const (&tr)[NF], int j, const TwWs<L, T>& tw) {
     ws_a<DIR, NF, SWZ>(v, rows, j, tw);
-    ws_transpose<NF>(v, tr, j);
+    ws_transpose<L, NF>(v, tr, j);
 }
 
 // XCD-aware block order: MI355X dispatches workgroup b to XCD b % 8; this

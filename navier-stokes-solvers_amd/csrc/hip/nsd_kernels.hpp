@@ -328,13 +328,12 @@ __device__ __forceinline__ void fft_any(cx<T> (&v)[P], cx<T>* lds, int j, const 
                                         const TwRegs<LC, T>& tw) {
     line_fft_c<DIR, LC>(v, lds, j, tw);
 }
-// wave-split 4096-point transform, wave-strided pattern in (a pointwise
+// wave-split transform, wave-strided pattern in (a pointwise
 // product of ws_a outputs), standard pattern out; the region is free again
 // only after a workgroup barrier
 template <int DIR, int LC, typename T>
 __device__ __forceinline__ void fft_any(cx<T> (&v)[P], cx<T>* lds, int j, const Line&,
-                                        const TwWs<T>& tw) {
-    static_assert(LC == 4096, "wave-split transforms are 4096-point");
+                                        const TwWs<LC, T>& tw) {
     cx<T>(*const vv[1])[P] = {&v};
     cx<T>* const ll[1] = {lds};
     ws_b<DIR, 1, (sizeof(T) == 8)>(vv, ll, j, tw);  // 16-byte rows at FP64
@@ -421,10 +420,15 @@ struct Band {
 // (needs two line regions per line in LDS).  PR < 0 decides automatically:
 // paired when the workgroup's two regions stay within 80 KB, so that two
 // workgroups share a CU; PR = 0 / 1 forces the choice (launch variants).
+// FP32 lines of 8192 are paired as well (147 KB, one workgroup of 16 waves per
+// CU): one region leaves room for no second workgroup either, and the
+// wave-split pairs took k_row at 8192^2 from 926 to 537 us and k_col from 527
+// to 450 us (per-pair layout).
 template <typename T, int LC, int NT = threads_for(LC), int PR = -1>
 constexpr bool paired_lines() {
     if (LC <= 0) return false;
     if (PR >= 0) return PR == 1;
+    if (sizeof(T) == 4 && LC == 8192) return true;
     return 2 * (LC + LC / 16) * (int)sizeof(cx<T>) * (NT * P / LC) <= 80 * 1024;
 }
 template <typename T, int LC, int NT = threads_for(LC), int PR = -1>
@@ -546,7 +550,7 @@ __device__ __forceinline__ cx<T> grow(cx<T> w, T em1) {
 // address path otherwise waits on the cache for about half of its cycles.
 // k_col still writes whole lines (one 16-byte store per lane and pair).
 // It is a property of the instantiation: the paired transforms of square
-// FP32 4096^2 grids (the gather-ahead k_row path reads it, the paired k_col
+// FP32 4096^2 and (in row-pair tiles, pairtile_layout) 8192^2 grids (the gather-ahead k_row path reads it, the paired k_col
 // path writes it).  The host selects it per launch (ColArgs/RowArgs::pairs)
 // when the row and column instantiations it launches both hold it
 // (stage_variant_pairs); the transform modes keep the per-field layout.  At
@@ -554,7 +558,7 @@ __device__ __forceinline__ cx<T> grow(cx<T> w, T em1) {
 // member-steps/s), so it stays at 4096.
 template <typename T, int LC, int NT, int PR>
 constexpr bool pair_layout() {
-    return sizeof(T) == 4 && LC == 4096 && paired_lines<T, LC, NT, PR>();
+    return sizeof(T) == 4 && (LC == 4096 || LC == 8192) && paired_lines<T, LC, NT, PR>();
 }
 
 // Row-pair tiles of the mixed fields (rowpair_elem): the FP64 stage kernels
@@ -570,6 +574,27 @@ constexpr bool pair_layout() {
 template <typename T, int LC, int NT, int PR>
 constexpr bool rowpair_layout() {
     return ws_lines64<T, LC, NT, PR>();
+}
+
+// Row-pair tiles of the pair buffers: FP32 lines of 8192.  Element (kx, y) of
+// member m of a pair at 4 ((y / 2) K + kx) + 2 (y mod 2) + m (pairtile_elem):
+// both rows of both fields are 32 bytes per column and a row pair's gather of
+// a pair buffer is one contiguous run, as in the FP64 tiles above; four
+// columns share a 128-byte line.  The 716 MB of mixed fields at 8192^2 lie
+// beyond the MALL and the reach of the address translation, as the FP64
+// 4096^2 ones do: against the pair layout k_row takes 423 us instead of 537
+// and k_col 499 instead of 450 (8192^2 step 3.93 -> 3.65 ms; at the start of
+// both, with Stockham lines in one region and the per-field layout, 5.81 ms).
+// What bounds them now: about 16 us of VALU issue in the 26 us of a row pair,
+// with one workgroup per CU whose waves wait at the same barriers.  A
+// persistent row stage that gathered the next row pair's psi fields under J's
+// transform took 477 us (96 bytes of scratch).
+template <typename T, int LC, int NT, int PR>
+constexpr bool pairtile_layout() {
+    return LC == 8192 && pair_layout<T, LC, NT, PR>();
+}
+__device__ __forceinline__ unsigned pairtile_elem(int k, int K, int y) {
+    return 4u * (__umul24((unsigned)y >> 1, (unsigned)K) + (unsigned)k) + 2u * ((unsigned)y & 1u);
 }
 
 // the stage kernels' own layout of the mixed fields, if any (RowArgs and
@@ -593,13 +618,27 @@ constexpr bool ws_stage() {
 // elements of one line region of a stage kernel (compile-time lengths)
 template <typename T, int LC, int NT = threads_for(LC), int PR = -1>
 constexpr int region_elems() {
-    return ws_stage<T, LC, NT, PR>() ? WS_REGION : LC + LC / 16;
+    return ws_stage<T, LC, NT, PR>() ? ws_region(LC) : LC + LC / 16;
 }
 
 // store (first, second) at pair element e of pair buffer B (one 16 bytes)
 __device__ __forceinline__ void store_pair(cx<float>* B, size_t e, cx<float> first,
                                            cx<float> second) {
     *reinterpret_cast<float4*>(B + 2 * e) = make_float4(first.x, first.y, second.x, second.y);
+}
+
+// a thread's slots (first, second) of column k into row-pair tiles of pair
+// buffer B: rows j + s LC / P
+template <int LC>
+__device__ __forceinline__ void store_pair_tiles(cx<float>* B, int k, int K, int j,
+                                                 const cx<float> (&first)[P],
+                                                 const cx<float> (&second)[P]) {
+    static_assert((LC / P) % 2 == 0, "slots step by whole tiles");
+    const unsigned e0 = pairtile_elem(k, K, j), es = 2u * (unsigned)(LC / P) * (unsigned)K;
+#pragma unroll
+    for (int s = 0; s < P; ++s)
+        *reinterpret_cast<float4*>(at32(B, e0 + (unsigned)s * es)) =
+            make_float4(first[s].x, first[s].y, second[s].x, second[s].y);
 }
 
 template <typename T>
@@ -663,9 +702,12 @@ __global__ __launch_bounds__(NT, MW) void k_col(ColArgs<T> a) {
     cx<T>* lds = smem + m * NB * RE;
     cx<T>* lds2 = lds + (NB - 1) * RE;
     constexpr bool WS = ws_lines64<T, LC, NT, PR>();
+    // forward transform through ws_c as well (two line regions free for it)
+    constexpr bool WSF = WS || pairtile_layout<T, LC, NT, PR>();
     // pair-layout kernels read J in 2 x 2 blocks: columns k and k ^ 1 share
     // lines; row-pair tiles put ROWPAIR_CPL columns in one line
-    constexpr int XG = pair_layout<T, LC, NT, PR>()      ? 2
+    constexpr int XG = pairtile_layout<T, LC, NT, PR>()   ? 4
+                       : pair_layout<T, LC, NT, PR>()    ? 2
                        : rowpair_layout<T, LC, NT, PR>() ? ROWPAIR_CPL
                                                          : 1;
     const int kxi = xcd_group_remap<XG>(blockIdx.x, gridDim.x) * lines + m;
@@ -700,8 +742,8 @@ __global__ __launch_bounds__(NT, MW) void k_col(ColArgs<T> a) {
 
     // ---- forward y-transform of the mixed nonlinear field
     if constexpr (PF) {
-        std::conditional_t<WS, TwWs<T>, TwRegs<LC, T>> tw;
-        if constexpr (WS) load_tw_ws(tw, j, a.tw);
+        std::conditional_t<WSF, TwWs<LC, T>, TwRegs<LC, T>> tw;
+        if constexpr (WSF) load_tw_ws(tw, j, a.tw);
         else load_tw_regs<LC, 0>(tw, j, a.tw);
         if constexpr (pair_layout<T, LC, NT, PR>()) {
             // J in 2 x 2 blocks: jblock_elem(kxi, ny, y), y = j + s TPL (TPL
@@ -747,11 +789,11 @@ __global__ __launch_bounds__(NT, MW) void k_col(ColArgs<T> a) {
             pacc[s] = zero;
             if (with_acc) pacc[s] = acc[ci];
         }
-        if constexpr (WS) {
+        if constexpr (WSF) {
             cx<T>(*const vv[1])[P] = {&v};
             cx<T>* const r1[1] = {lds};
             cx<T>* const t1[1] = {lds2};
-            ws_c<-1, 1, true>(vv, r1, t1, j, tw);
+            ws_c<-1, 1, WS>(vv, r1, t1, j, tw);
         } else {
             fft_any<-1, LC>(v, lds, j, g, tw);
         }
@@ -993,11 +1035,12 @@ __global__ __launch_bounds__(NT, MW) void k_col(ColArgs<T> a) {
             // FP32 4096 (pair layout): wave-split transforms, standard
             // pattern in and out (ws_c), transposing back in the same regions
             constexpr bool WSC = pair_layout<T, LC, NT, PR>();
-            std::conditional_t<WSC, TwWs<T>, TwRegs<LC, T>> tw;
+            std::conditional_t<WSC, TwWs<LC, T>, TwRegs<LC, T>> tw;
             cx<T>(*const vv[2])[P] = {&v, &v2};
             cx<T>* const rr[2] = {lds, lds2};
             if constexpr (WSC) {
                 load_tw_ws(tw, j, a.tw);
+                renew_tw(tw);
                 __syncthreads();  // the forward transform's last reads are done
                 ws_c<+1, 2>(vv, rr, rr, j, tw);  // omega_y, omega_x
             } else {
@@ -1008,8 +1051,13 @@ __global__ __launch_bounds__(NT, MW) void k_col(ColArgs<T> a) {
                 if constexpr (pair_layout<T, LC, NT, PR>()) {
                     if (a.pairs) {  // (omega_x, omega_y)
                         cx<T>* pb = a.mixed[2] + 2 * mixed_off;
+                        if constexpr (pairtile_layout<T, LC, NT, PR>()) {
+                            store_pair_tiles<LC>(pb, kxi, (G.nkx_keep + 1) & ~1, j, v2, v);
+                        } else {
 #pragma unroll
-                        for (int s = 0; s < P; ++s) store_pair(pb, mbase + j + s * TPL, v2[s], v[s]);
+                            for (int s = 0; s < P; ++s)
+                                store_pair(pb, mbase + j + s * TPL, v2[s], v[s]);
+                        }
                     }
                 }
                 if (!(pair_layout<T, LC, NT, PR>() && a.pairs)) {
@@ -1032,6 +1080,7 @@ __global__ __launch_bounds__(NT, MW) void k_col(ColArgs<T> a) {
             }
             if constexpr (WSC) {
                 __syncthreads();  // others may still read the transposed first pair
+                renew_tw(tw);
                 ws_c<+1, 2>(vv, rr, rr, j, tw);  // psi_y, psi_x
             } else {
                 line_fft2_c<+1, LC>(v, v2, lds, lds2, j, tw);  // psi_y, psi_x
@@ -1040,8 +1089,13 @@ __global__ __launch_bounds__(NT, MW) void k_col(ColArgs<T> a) {
                 if constexpr (pair_layout<T, LC, NT, PR>()) {
                     if (a.pairs) {  // (psi_x, psi_y)
                         cx<T>* pb = a.mixed[0] + 2 * mixed_off;
+                        if constexpr (pairtile_layout<T, LC, NT, PR>()) {
+                            store_pair_tiles<LC>(pb, kxi, (G.nkx_keep + 1) & ~1, j, v2, v);
+                        } else {
 #pragma unroll
-                        for (int s = 0; s < P; ++s) store_pair(pb, mbase + j + s * TPL, v2[s], v[s]);
+                            for (int s = 0; s < P; ++s)
+                                store_pair(pb, mbase + j + s * TPL, v2[s], v[s]);
+                        }
                     }
                 }
                 if (!(pair_layout<T, LC, NT, PR>() && a.pairs)) {
@@ -1087,7 +1141,7 @@ __global__ __launch_bounds__(NT, MW) void k_col(ColArgs<T> a) {
         // FP64 columns of 4096: the four outputs one at a time through ws_c
         // (spectral_core.c:62-99), swizzled rows in lds, the transposing
         // exchange in lds2: two barriers per transform
-        TwWs<T> tw;
+        TwWs<LC, T> tw;
         load_tw_ws(tw, j, a.tw);
         cx<T>(*const vv[1])[P] = {&v};
         cx<T>* const r1[1] = {lds};
@@ -1292,7 +1346,7 @@ __device__ __forceinline__ void fwd_rows_store(cx<T> (&v)[P], cx<T>* lds, int j,
     fft_any<-1, LC>(v, lds, j, g, tw);
     // after a wave-split transform the line goes unpadded (only unit-stride
     // accesses follow)
-    constexpr bool PADL = !std::is_same<TW, TwWs<T>>::value;
+    constexpr bool PADL = !std::is_same<TW, TwWs<(LC > 0 ? LC : 4096), T>>::value;
     auto at = [](int i) { return PADL ? pad(i) : i; };
     if constexpr (LC > 0) {
         // the separation below reads kept columns k and their partners
@@ -1445,6 +1499,29 @@ __device__ __forceinline__ void gather_pair_rows(RowPairRegs<float>& f0, RowPair
     }
 }
 
+// The same from row-pair tiles of the pair buffers: 32 contiguous bytes per
+// column, read by this row pair only (non-temporal, as in the FP64 tiles).
+template <int LC>
+__device__ __forceinline__ void gather_pair_tiles(RowPairRegs<float>& f0, RowPairRegs<float>& f1,
+                                                  int j, const cx<float>* B, int K, int y) {
+    typedef float f4 __attribute__((ext_vector_type(4)));
+    constexpr int kxm = Band<LC>::kxm;
+    const unsigned e0 = pairtile_elem(j, K, y);
+#pragma unroll
+    for (int s = 0; s < P; ++s) {
+        const int kind = slot_kind(s, LC, kxm);
+        const int k = j + s * (LC / P);
+        if (kind == 1 || (kind == 3 && k <= kxm)) {
+            const f4* src = reinterpret_cast<const f4*>(at32(B, e0 + (unsigned)(4 * s * (LC / P))));
+            const f4 r0 = __builtin_nontemporal_load(src), r1 = __builtin_nontemporal_load(src + 1);
+            f0.a[s] = mk(r0.x, r0.y);
+            f1.a[s] = mk(r0.z, r0.w);
+            f0.b[s] = mk(r1.x, r1.y);
+            f1.b[s] = mk(r1.z, r1.w);
+        }
+    }
+}
+
 // The LDS image of stage_two_rows, from gathered registers.  SKIP0: the
 // slots that lie inside the dealiased band for every thread (kind 0) are
 // left unwritten, for a reader that takes them as zero (lds_read_kept).
@@ -1477,6 +1554,14 @@ __device__ __forceinline__ void stage_two_rows_regs(cx<T>* lds, int j, const Row
             lds[at(k)] = zero;
         }
     }
+}
+
+// both fields of a pair buffer, in row-pair tiles (TILES) or pair by pair
+template <int LC, bool TILES>
+__device__ __forceinline__ void gather_pair(RowPairRegs<float>& f0, RowPairRegs<float>& f1, int j,
+                                            const Geo& G, const cx<float>* B, int y, bool active) {
+    if constexpr (TILES) gather_pair_tiles<LC>(f0, f1, j, B, (G.nkx_keep + 1) & ~1, y);
+    else gather_pair_rows<LC>(f0, f1, j, G, B, y, active);
 }
 
 // Paired row stages that issue the omega gathers ahead of the psi
@@ -1592,23 +1677,24 @@ __global__ __launch_bounds__(NT, MW) void k_row(RowArgs<T> a) {
         // outputs are in the wave-strided pattern, ws_b for J, which takes
         // that pattern back to the standard one): 11 workgroup barriers per
         // row pair instead of 27.
-        TwWs<T> tw;
+        TwWs<LC, T> tw;
         load_tw_ws(tw, j, a.tw);
         if (blk * lines < G.ny / 2) {
             // one line per workgroup: inside this branch its row pair exists,
             // and the gathers need no zero fill for an inactive one
             static_assert(NT * P / LC == 1, "one row pair per workgroup");
             constexpr bool live = true;
+            constexpr bool PT = pairtile_layout<T, LC, NT, PR>();
             RowPairRegs<T> r0, r1, q0, q1;
             const bool pl = a.pairs != 0;
-            if (pl) gather_pair_rows<LC>(r0, r1, j, G, a.mixed[0] + 2 * moff, y0, live);
+            if (pl) gather_pair<LC, PT>(r0, r1, j, G, a.mixed[0] + 2 * moff, y0, live);
             else {
                 gather_two_rows<LC>(r0, j, G, a.mixed[0] + moff, y0, live);
                 gather_two_rows<LC>(r1, j, G, a.mixed[1] + moff, y0, live);
             }
             stage_two_rows_regs<LC, true, false>(lds, j, r0);
             stage_two_rows_regs<LC, true, false>(lds2, j, r1);
-            if (pl) gather_pair_rows<LC>(q0, q1, j, G, a.mixed[2] + 2 * moff, y0, live);
+            if (pl) gather_pair<LC, PT>(q0, q1, j, G, a.mixed[2] + 2 * moff, y0, live);
             else {
                 gather_two_rows<LC>(q0, j, G, a.mixed[2] + moff, y0, live);
                 gather_two_rows<LC>(q1, j, G, a.mixed[3] + moff, y0, live);
@@ -1621,6 +1707,7 @@ __global__ __launch_bounds__(NT, MW) void k_row(RowArgs<T> a) {
             lds_read_kept<LC, false>(v2, lds2, j);
             __syncthreads();
             ws_a<+1, 2>(vv, ll, j, tw);  // psi_x, psi_y
+            renew_tw(tw);
             if (a.track_umax) add_speeds(um, v, v2);
 #pragma unroll
             for (int s = 0; s < P; ++s) {
@@ -1635,11 +1722,12 @@ __global__ __launch_bounds__(NT, MW) void k_row(RowArgs<T> a) {
             lds_read_kept<LC, false>(v2, lds2, j);
             __syncthreads();
             ws_a<+1, 2>(vv, ll, j, tw);  // omega_x, omega_y
+            renew_tw(tw);
 #pragma unroll
             for (int s = 0; s < P; ++s)
                 v[s] = mk(X[s].x * v2[s].x - Jp[s].x * v[s].x, X[s].y * v2[s].y - Jp[s].y * v[s].y);
-            fwd_rows_store<LC, T, TwWs<T>, true>(v, lds, j, g, G, tw, a.nl + moff, y0,
-                                                    active, a.jblocks);
+            fwd_rows_store<LC, T, TwWs<LC, T>, true>(v, lds, j, g, G, tw, a.nl + moff, y0, active,
+                                                     a.jblocks);
         }
         if (a.track_umax) block_max_to(active ? double(um.value()) : 0.0, &a.sc[blockIdx.y].umax2_bits, red);
         return;
@@ -1729,7 +1817,7 @@ __global__ __launch_bounds__(NT, MW) void k_row(RowArgs<T> a) {
         // transforms whose cross-wave rows live in lds2.  Every read of the
         // staged line in lds precedes the barrier inside ws_a, so the next
         // field is staged without one: 10 barriers per row pair instead of 45.
-        TwWs<T> tw;
+        TwWs<LC, T> tw;
         load_tw_ws(tw, j, a.tw);
         if (blk * lines < G.ny / 2) {
             cx<T>(*const vv[1])[P] = {&v};
@@ -1774,7 +1862,7 @@ __global__ __launch_bounds__(NT, MW) void k_row(RowArgs<T> a) {
             for (int s = 0; s < P; ++s)
                 v[s] = mk(Jp[s].x + X[s].x * v[s].x, Jp[s].y + X[s].y * v[s].y);
             // J: ws_b in lds, whose rows nobody reads any more
-            fwd_rows_store<LC, T, TwWs<T>>(v, lds, j, g, G, tw, a.nl + moff, y0, active);
+            fwd_rows_store<LC, T, TwWs<LC, T>>(v, lds, j, g, G, tw, a.nl + moff, y0, active);
         }
         if (a.track_umax) block_max_to(active ? double(um.value()) : 0.0, &a.sc[blockIdx.y].umax2_bits, red);
         return;

@@ -35,13 +35,25 @@ def two_steps(ns, nx, ny, fp32, integrating_factor):
     return w, t
 
 
-# a 4096-point side next to another length: the pair layout and J's 2 x 2
-# blocks are for square grids only
-@pytest.mark.parametrize("nx,ny", [(4096, 64), (64, 4096), (4096, 1024), (1024, 4096)])
+# a 4096- or 8192-point side next to another length: the layouts of the square
+# grids' stage kernels and J's 2 x 2 blocks are not for them
+@pytest.mark.parametrize("nx,ny", [(4096, 64), (64, 4096), (4096, 1024), (1024, 4096),
+                                   (8192, 128), (128, 8192), (8192, 4096)])
 def test_fp32_rectangles_match_fp64(ns, nx, ny):
     w32, t32 = two_steps(ns, nx, ny, True, True)
     w64, t64 = two_steps(ns, nx, ny, False, True)
     err = rel_l2(w32, w64)
     print(f"{nx} x {ny}: FP32 vs FP64 rel L2 {err:.2e}", flush=True)
+    assert err <= 1e-6
+    assert t32 == pytest.approx(t64, rel=1e-6)
+
+
+# 8192 points on sixteen waves, both schemes' column kernels
+@pytest.mark.parametrize("integrating_factor", [True, False])
+def test_fp32_8192_matches_fp64(ns, integrating_factor):
+    w32, t32 = two_steps(ns, 8192, 8192, True, integrating_factor)
+    w64, t64 = two_steps(ns, 8192, 8192, False, integrating_factor)
+    err = rel_l2(w32, w64)
+    print(f"8192^2: FP32 vs FP64 rel L2 {err:.2e}", flush=True)
     assert err <= 1e-6
     assert t32 == pytest.approx(t64, rel=1e-6)
