@@ -132,8 +132,10 @@ int nsd_batch_scalars(NsdContext *c, double *t, double *dt, int *status);
 int nsd_member_upload(NsdContext *c, int member, const double *omega_hat);
 int nsd_member_download(NsdContext *c, int member, double *omega_hat);
 
-/* Launch variants of the two time-step kernels (workgroup size and whether
- * inverse transforms run in lock-step pairs; lengths 64..1024 have several).
+/* Launch variants of the two time-step kernels (workgroup size, whether
+ * inverse transforms run in lock-step pairs, and field-parallel kernels whose
+ * four transforms run side by side; lengths 64..1024 have several; a context
+ * starts with the field-parallel ones where its launches are small).
  * nsd_autotune times every variant on this context's shape (reps launches
  * each) and keeps the fastest; results are cached per (length, precision,
  * batch members) for the process and, if the environment names a file in

@@ -862,6 +862,14 @@ bool pairs_ok(const NsdContext* c) {
 // J in 2 x 2 blocks: written by the FP32 pair-layout row stage
 bool jblocks_ok(const NsdContext* c) { return c->prec == NSD_FP32 && pairs_ok(c); }
 
+// launch variant that this context starts with (kind 0: rows, 1: columns)
+template <typename T>
+int default_variant(const NsdContext* c, int kind) {
+    const long lines = (long)c->nb * (kind == 0 ? c->G.ny / 2 : c->G.nkx_keep);
+    return stage_variant_default<T>(kind == 0 ? c->G.nx : c->G.ny, lines,
+                                    std::max(c->G.nx, c->G.ny), c->maxlds);
+}
+
 template <typename T>
 ColArgs<T> col_args(NsdContext* c) {
     ColArgs<T> a;
@@ -1476,10 +1484,19 @@ int op_autotune(NsdContext* c, int reps, int force) {
                 cached = true;
             }
         }
+        // a launch that starts with the field-parallel kernels keeps them, as a
+        // single context of its size does: nothing to time.  FP32 grids below
+        // 512^2 do without them (stage_variant_default has the reason)
+        const bool small32 = sizeof(T) == 4 && std::max(c->G.nx, c->G.ny) < 512;
+        if (!cached && default_variant<T>(c, kind) == kFieldsVariant) {
+            best = kFieldsVariant;
+            cached = true;
+        }
         if (!cached) {
             float best_ms = 1e30f;
             for (int v = 0; v < kStageVariants; ++v) {
                 if (!stage_variant_valid<T>(L, v, c->maxlds)) continue;
+                if (small32 && v == kFieldsVariant) continue;
                 auto launch = [&]() {
                     if (kind == 0) {
                         RowArgs<T> r = row_args<T>(c);
@@ -1744,6 +1761,8 @@ NsdContext* nsd_create_batch(int nx, int ny, double Lx, double Ly, int precision
     if (precision == NSD_FP32) set_lds_limits<float>(maxlds);
     else set_lds_limits<double>(maxlds);
     c->maxlds = maxlds;
+    c->vrow = precision == NSD_FP32 ? default_variant<float>(c, 0) : default_variant<double>(c, 0);
+    c->vcol = precision == NSD_FP32 ? default_variant<float>(c, 1) : default_variant<double>(c, 1);
     if (precision == NSD_FP32 && nx == 4096) c->stagger = dispatch_breadth_first(dev, c->ncu);
     nsd_set_params(c, &c->P);
     return c;
@@ -2144,11 +2163,14 @@ int nsd_autotune(NsdContext* c, int reps, int force, int* row_variant, int* col_
 
 int nsd_set_variants(NsdContext* c, int row_variant, int col_variant) {
     if (!c) return ST_PARAM;
-    const bool ok = c->prec == NSD_FP32
-                        ? stage_variant_valid<float>(c->G.nx, row_variant, c->maxlds) &&
-                              stage_variant_valid<float>(c->G.ny, col_variant, c->maxlds)
-                        : stage_variant_valid<double>(c->G.nx, row_variant, c->maxlds) &&
-                              stage_variant_valid<double>(c->G.ny, col_variant, c->maxlds);
+    const bool named = row_variant >= 0 && row_variant < kStageVariants && col_variant >= 0 &&
+                       col_variant < kStageVariants;
+    const bool ok =
+        named && (c->prec == NSD_FP32
+                      ? stage_variant_valid<float>(c->G.nx, row_variant, c->maxlds) &&
+                            stage_variant_valid<float>(c->G.ny, col_variant, c->maxlds)
+                      : stage_variant_valid<double>(c->G.nx, row_variant, c->maxlds) &&
+                            stage_variant_valid<double>(c->G.ny, col_variant, c->maxlds));
     if (!ok) {
         c->err = "launch variant not available for this size";
         return ST_PARAM;

@@ -1,0 +1,431 @@
+// nsd_fields.hpp -- field-parallel stage kernels for small launches.
+//
+// The stage kernels of nsd_kernels.hpp give a line to one group of L / 8
+// threads, which takes a row pair through its four inverse transforms and the
+// transform of J one after the other (two at a time in lock-step).  That is the
+// least work per launch, and where a launch has many lines the waves of other
+// lines fill the waits.  A launch with few lines has nothing to fill them with:
+// at 1024^2 the 512 row pairs are one wave per SIMD, and its time is the length
+// of that chain.  Here a row pair (or a column) is a unit of four groups of
+// L / 8 threads, one per derivative field: the four transforms of a unit run
+// side by side, the chain is one inverse and one forward transform, and the
+// launch has four times the waves.  The pointwise work (the per-mode update, the
+// separation of J's two rows) is spread over all four groups.  A line of up to
+// 512 points stays inside one wave, so its exchanges through LDS need no
+// workgroup barrier.
+//
+// Same layouts and the same formulas as the kernels of nsd_kernels.hpp:
+// per-field mixed fields and J, both [kx][y].
+#pragma once
+
+#include "nsd_kernels.hpp"
+
+namespace nsd {
+
+// ------------------------------------------------------------------ lines
+
+// All twiddles of a line's passes in registers: W^k of the full-radix passes
+// (powers by squaring, as TwRegs) and the table values of the closing radix-2
+// or radix-4 pass, so that no load sits inside a transform.
+template <int L, typename T>
+struct TwAll {
+    static constexpr int R = CLine<L>::rem;
+    static constexpr int QN = R > 1 ? P / R : 1, EN = R == 4 ? 2 : 1;
+    cx<T> w[CLine<L>::passes];
+    cx<T> tail[QN][EN];
+    template <int L2, int PASS>
+    __device__ __forceinline__ cx<T> get(int q, int e, int) const {
+        if constexpr (CLine<L>::radix(PASS) == P) {
+            cx<T> r = w[PASS];
+            for (int i = 0; i < e; ++i) r = cmul(r, r);
+            return r;
+        } else {
+            return tail[q][e];
+        }
+    }
+};
+
+template <int L, int PASS, typename T>
+__device__ __forceinline__ void load_tw_all(TwAll<L, T>& t, int j, const cx<T>* __restrict__ tw) {
+    if constexpr (PASS < CLine<L>::passes) {
+        using G = CLine<L>;
+        constexpr int Ns = G::stride(PASS), R = G::radix(PASS);
+        if constexpr (Ns > 1 && R == P) {
+            t.w[PASS] = tw[(j & (Ns - 1)) * (L / (Ns * P))];
+        } else if constexpr (Ns > 1) {
+#pragma unroll
+            for (int q = 0; q < P / R; ++q)
+#pragma unroll
+                for (int e = 0; e < (R == 4 ? 2 : 1); ++e)
+                    t.tail[q][e] = tw[(((j + q * G::TPL) & (Ns - 1)) << e) * (L / (Ns * R))];
+        }
+        load_tw_all<L, PASS + 1>(t, j, tw);
+    }
+}
+
+// the powers that one transform formed are not kept for the next (renew)
+template <int L, typename T>
+__device__ __forceinline__ void renew_tw_all(TwAll<L, T>& t) {
+#pragma unroll
+    for (int p = 1; p < CLine<L>::nP; ++p) renew(t.w[p]);
+}
+
+// threads of a unit (four lines side by side)
+template <int L>
+constexpr int unit_threads() { return L / 2; }
+
+// Exchanges between the threads of one line, and of one unit: inside a wave
+// only the compiler has to be held back.  NTH threads in aligned groups.
+template <int NTH>
+__device__ __forceinline__ void group_sync() {
+    if constexpr (NTH <= 64) wave_lds_fence();
+    else __syncthreads();
+}
+template <int L>
+__device__ __forceinline__ void line_sync() { group_sync<L / P>(); }
+template <int L>
+__device__ __forceinline__ void unit_sync() { group_sync<unit_threads<L>()>(); }
+
+// The transform of one line by its L / 8 threads, standard pattern in and out.
+// `act`: this line has one (uniform over its threads); every thread takes the
+// barriers.  The region must be free on entry; the line's threads may still
+// read it on return.
+template <int DIR, int L, int PASS = 0, typename T>
+__device__ __forceinline__ void line_fft_act(cx<T> (&v)[P], cx<T>* lds, int j,
+                                             const TwAll<L, T>& tw, bool act) {
+    if constexpr (PASS < CLine<L>::passes) {
+        if constexpr (PASS > 0) {
+            line_sync<L>();  // the previous pass is written
+            if (act) lds_read_c<L>(v, lds, j);
+            if constexpr (PASS + 1 < CLine<L>::passes) line_sync<L>();
+        }
+        if (act) cpass<DIR, L, PASS>(v, j, tw, lds);
+        line_fft_act<DIR, L, PASS + 1>(v, lds, j, tw, act);
+    }
+}
+
+// ------------------------------------------------------------ memory access
+
+// Fields that other workgroups of the same launch neither write nor read.
+struct MemLaunch {
+    template <typename T>
+    static __device__ __forceinline__ cx<T> load(const cx<T>* p) { return *p; }
+    template <typename T>
+    static __device__ __forceinline__ void load2(const cx<T>* p, cx<T>& a, cx<T>& b) {
+        a = p[0];
+        b = p[1];
+    }
+    template <typename T>
+    static __device__ __forceinline__ void store(cx<T>* p, cx<T> v) { *p = v; }
+};
+
+// ---------------------------------------------------------------- row stage
+
+// One row pair (rows y, y + 1) of the row stage: inverse x-transforms of the
+// four fields, J, the forward x-transform of J, kept columns stored.  r: this
+// thread of the unit; lds: the unit's four line regions.
+template <typename T, int L, typename MEM>
+__device__ __forceinline__ void row_unit(cx<T>* lds, int r, const Geo& G, const cx<T>* F, cx<T>* nl,
+                                         int y, bool active, TwAll<L, T>& tw, bool track,
+                                         SpeedMax<T>& um) {
+    constexpr int TPL = L / P, RE = L + L / 16, kxm = Band<L>::kxm;
+    constexpr bool KEPT = TPL % 16 == 0;
+    const int f = r / TPL, j = r - f * TPL;
+    cx<T>* const own = lds + f * RE;
+    cx<T> v[P];
+    {
+        RowPairRegs<T> q;
+#pragma unroll
+        for (int s = 0; s < P; ++s) {
+            const int kind = slot_kind(s, L, kxm), k = j + s * TPL;
+            if (kind == 1 || (kind == 3 && k <= kxm)) {
+                if (active) {
+                    MEM::load2(at32(F, col_elem(k, G.ny, y)), q.a[s], q.b[s]);
+                } else {
+                    q.a[s] = mk(T(0), T(0));
+                    q.b[s] = mk(T(0), T(0));
+                }
+            }
+        }
+        stage_two_rows_regs<L, KEPT>(own, j, q);
+    }
+    line_sync<L>();
+    lds_read_any<L, KEPT>(v, own, j);
+    line_sync<L>();
+    line_fft_act<+1, L>(v, own, j, tw, true);
+    // psi_y, omega_x, omega_y to the threads that hold psi_x
+    line_sync<L>();
+    if (f > 0) lds_write_c<L>(v, own, j);
+    unit_sync<L>();
+    const bool first = f == 0;
+    if (first) {
+        // J = psi_x omega_y - psi_y omega_x (spectral_core.c:101-104), in two
+        // sweeps so that few values are held at once
+        cx<T> b[P], c[P];
+        lds_read_c<L>(b, lds + RE, j);
+        lds_read_c<L>(c, lds + 2 * RE, j);
+        if (track) add_speeds(um, v, b);
+#pragma unroll
+        for (int s = 0; s < P; ++s) b[s] = mk(b[s].x * c[s].x, b[s].y * c[s].y);
+        __builtin_amdgcn_sched_barrier(0);
+        lds_read_c<L>(c, lds + 3 * RE, j);
+#pragma unroll
+        for (int s = 0; s < P; ++s)
+            v[s] = mk(v[s].x * c[s].x - b[s].x, v[s].y * c[s].y - b[s].y);
+    }
+    renew_tw_all(tw);
+    line_fft_act<-1, L>(v, lds, j, tw, first);
+    line_sync<L>();
+    if (first) {
+        // the slots that the separation reads (as fwd_rows_store)
+        if constexpr (KEPT) {
+            cx<T>* b = lds + pad(j);
+#pragma unroll
+            for (int s = 0; s < P; ++s)
+                if (slot_kind(s, L, kxm) != 0) b[padc(s * TPL)] = v[s];
+        } else {
+            lds_write_c<L>(v, lds, j);
+        }
+    }
+    unit_sync<L>();
+    // separation of the two rows, one kept column per thread
+    constexpr int UT = unit_threads<L>();
+#pragma unroll
+    for (int k0 = 0; k0 <= kxm; k0 += UT) {
+        const int k = k0 + r;
+        if (k <= kxm && active) {
+            const cx<T> zk = lds[pad(k)];
+            const cx<T> zm = lds[pad((L - k) & (L - 1))];
+            cx<T>* dst = at32(nl, col_elem(k, G.ny, y));
+            MEM::store(dst, mk(T(0.5) * (zk.x + zm.x), T(0.5) * (zk.y - zm.y)));
+            MEM::store(dst + 1, mk(T(0.5) * (zk.y + zm.y), T(0.5) * (zm.x - zk.x)));
+        }
+    }
+}
+
+// U row pairs per workgroup
+template <typename T, int L, int U, int MW>
+__global__ __launch_bounds__(U * L / 2, MW) void k_row_fields(RowArgs<T> a) {
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    __shared__ double red[U * L / 2 > 64 ? U * L / 128 : 1];
+    constexpr int UT = unit_threads<L>(), RE = L + L / 16;
+    const int u = threadIdx.x / UT, r = threadIdx.x - u * UT;
+    const int f = r / (L / P), j = r - f * (L / P);
+    const Geo& G = a.geo;
+    const int y = 2 * (xcd_remap(blockIdx.x, gridDim.x) * U + u);
+    const size_t moff = blockIdx.y * a.bm;
+    TwAll<L, T> tw;
+    load_tw_all<L, 0>(tw, j, a.tw);
+    const cx<T>* F = f < 2 ? (f == 0 ? a.mixed[0] : a.mixed[1]) : (f == 2 ? a.mixed[2] : a.mixed[3]);
+    SpeedMax<T> um;
+    row_unit<T, L, MemLaunch>(reinterpret_cast<cx<T>*>(smem_raw) + u * 4 * RE, r, G, F + moff,
+                              a.nl + moff, y, y < G.ny, tw, a.track_umax != 0, um);
+    if (a.track_umax) block_max_to(double(um.value()), &a.sc[blockIdx.y].umax2_bits, red);
+}
+
+// ------------------------------------------------------------- column stage
+
+// One mode's stage update: N (without the closure's source), the state at the
+// step's start w0, the accumulator av (from stage 1 on) and, in the classic
+// scheme, the stage field ws and the SFD state fs.  Returns the new stage field
+// and leaves the accumulator in av (stages 0..2) and the SFD state in fs.
+template <typename T, int SCHEME>
+__device__ __forceinline__ cx<T> mode_update(const Phys& ph, int stage, T h, double dt, T k2,
+                                             cx<T> N, cx<T> w0, cx<T>& av, cx<T> ws, cx<T>& fs) {
+    cx<T> wn;
+    if constexpr (SCHEME == 0) {
+        // classic RK4 (spectral_time_integration.c:50-100) with
+        // hyperviscosity_apply (hyperviscosity.c:104-150) and drag
+        const T lin = -(k2 * T(ph.inv_Re) + T(ph.drag) + hv_weight_t<T>(ph, k2));
+        cx<T> ks = N + lin * ws;
+        const T sw = sfd_weight_t<T>(ph, k2);
+        if (sw > T(0)) ks = ks - sw * (ws - fs);
+        if (stage == 0) {
+            av = w0 + (h / T(6)) * ks;
+            wn = w0 + (T(0.5) * h) * ks;
+        } else if (stage == 1) {
+            av = av + (h / T(3)) * ks;
+            wn = w0 + (T(0.5) * h) * ks;
+        } else if (stage == 2) {
+            av = av + (h / T(3)) * ks;
+            wn = w0 + h * ks;
+        } else {
+            wn = av + (h / T(6)) * ks;
+            if (ph.sfd_on && ph.sfd_tau > 0.0) {  // hyperviscosity.c:152-178
+                const T al = T(fmin(fmax(dt / ph.sfd_tau, 0.0), 1.0));
+                fs = (T(1) - al) * fs + al * wn;
+            }
+        }
+    } else {
+        // integrating factor through E - 1 (k_col has the reason)
+        const T lin = -(k2 * T(ph.inv_Re) + T(ph.drag) + hv_weight_t<T>(ph, k2));
+        const T e2 = expm1_t(lin * (T(0.5) * h));  // E2 - 1, E2 = exp(L h / 2)
+        const T e1 = e2 * (T(2) + e2);            // E - 1,  E = E2^2
+        if (stage == 0) {
+            av = grow(w0, e1) + (h / T(6)) * grow(N, e1);
+            wn = grow(w0 + (T(0.5) * h) * N, e2);
+        } else if (stage == 1) {
+            av = av + (h / T(3)) * grow(N, e2);
+            wn = grow(w0, e2) + (T(0.5) * h) * N;
+        } else if (stage == 2) {
+            av = av + (h / T(3)) * grow(N, e2);
+            wn = grow(w0, e1) + h * grow(N, e2);
+        } else {
+            wn = av + (h / T(6)) * N;
+        }
+    }
+    return wn;
+}
+
+// Kept modes of a column per thread of its unit (2 L / 3 over L / 2 threads)
+constexpr int kUnitModes = 2;
+
+// The step's scalars as the column stage needs them
+template <typename T>
+struct StageScalars {
+    double dt;
+    T h, norm, sqh;
+};
+
+// Inverse y-transforms of the derivative fields of one column's stage field,
+// whose kept modes lie in region 1 of the unit (padded, standard order): field
+// f of this thread's group into out.  Outputs 0 psi_x, 1 psi_y, 2 omega_x,
+// 3 omega_y (spectral_core.c:62-99).
+template <typename T, int L, typename MEM>
+__device__ __forceinline__ void col_unit_out(cx<T>* lds, int r, const Geo& G, int kxi, T kx,
+                                             cx<T>* out, bool active, const TwAll<L, T>& tw) {
+    constexpr int TPL = L / P, RE = L + L / 16, kym = Band<L>::kym;
+    const int f = r / TPL, j = r - f * TPL;
+    const T kys = T(2.0 * kPi / G.Ly);
+    cx<T> v[P];
+#pragma unroll
+    for (int s = 0; s < P; ++s) {
+        const int kind = slot_kind(s, L, kym), jy = j + s * TPL;
+        v[s] = mk(T(0), T(0));
+        if (kind == 0) continue;
+        const cx<T> w = lds[RE + pad(jy)];
+        if (kind != 3 || jy <= kym || jy >= L - kym) v[s] = w;
+    }
+    unit_sync<L>();  // region 1 is read: the transforms may use it
+    if (f < 2) {  // psi_hat = -omega_hat / k^2
+#pragma unroll
+        for (int s = 0; s < P; ++s) {
+            if (slot_kind(s, L, kym) == 0) continue;
+            const T ky = T(col_band<L>(G, j + s * TPL)) * kys;
+            const T k2 = kx * kx + ky * ky;
+            v[s] = k2 > T(1e-12) ? neg_inv_k2(k2) * v[s] : mk(T(0), T(0));
+        }
+    }
+#pragma unroll
+    for (int s = 0; s < P; ++s) {
+        const T ky = T(col_band<L>(G, j + s * TPL)) * kys;
+        v[s] = mul_i(v[s], (f & 1) ? ky : kx);
+    }
+    line_fft_act<+1, L>(v, lds + f * RE, j, tw, true);
+    if (active) {
+        cx<T>* o = out + (size_t)kxi * G.ny + j;
+#pragma unroll
+        for (int s = 0; s < P; ++s) MEM::store(o + s * TPL, v[s]);
+    }
+}
+
+// U columns per workgroup, one stage
+template <typename T, int L, int SCHEME, int U, int MW>
+__global__ __launch_bounds__(U * L / 2, MW) void k_col_fields(ColArgs<T> a) {
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    constexpr int UT = unit_threads<L>(), TPL = L / P, RE = L + L / 16;
+    constexpr int kym = Band<L>::kym, ncy = 2 * kym + 1;
+    static_assert(ncy <= kUnitModes * UT, "kept modes per thread");
+    const int u = threadIdx.x / UT, r = threadIdx.x - u * UT;
+    const int f = r / TPL, j = r - f * TPL;
+    cx<T>* const lds = reinterpret_cast<cx<T>*>(smem_raw) + u * 4 * RE;
+    const Geo& G = a.geo;
+    const size_t mb = blockIdx.y;
+    DevScalars* const sc = a.sc + mb;
+    Phys ph = a.phys;
+    if (a.m_inv_re) {
+        ph.inv_Re = a.m_inv_re[mb];
+        ph.Re = 1.0 / ph.inv_Re;
+    }
+    const int kxi = blockIdx.x * U + u;
+    const bool active = kxi < G.nkx_keep;
+    const T kx = T(kxi) * T(2.0 * kPi / G.Lx);
+    const cx<T> zero = mk(T(0), T(0));
+    TwAll<L, T> tw;
+    load_tw_all<L, 0>(tw, j, a.tw);
+    // J by the first group, whose transform runs while the modes' state arrives
+    cx<T> v[P];
+    const bool first = f == 0;
+    if (first) {
+        const cx<T>* nl = a.nl + mb * a.bm + (size_t)kxi * G.ny + j;
+#pragma unroll
+        for (int s = 0; s < P; ++s) v[s] = active ? nl[s * TPL] : zero;
+    }
+    const size_t c0 = mb * a.bc + (size_t)kxi * ncy;
+    cx<T> w0[kUnitModes], av[kUnitModes], ws[kUnitModes], fs[kUnitModes];
+#pragma unroll
+    for (int q = 0; q < kUnitModes; ++q) {
+        const int c = r + q * UT;
+        w0[q] = av[q] = ws[q] = fs[q] = zero;
+        if (c < ncy && active) {
+            w0[q] = a.state[c0 + c];
+            if (a.stage > 0) av[q] = a.acc[c0 + c];
+            if constexpr (SCHEME == 0) {
+                ws[q] = a.stage == 0 ? w0[q] : a.stagebuf[c0 + c];
+                if (ph.sfd_on) fs[q] = a.sfd[c0 + c];
+            }
+        }
+    }
+    line_fft_act<-1, L>(v, lds, j, tw, first);
+    double dt;
+    if (a.stage == 0 && ph.adaptive) {
+        const double u2 = __longlong_as_double((long long)sc->umax2_bits);
+        dt = cfl_dt(ph, sqrt(u2));
+        if (blockIdx.x == 0 && threadIdx.x == 0) {
+            sc->dt = dt;
+            if (!(u2 <= 1.0e300)) sc->status = 2;  // SOLVER_DIVERGED
+        }
+    } else {
+        dt = sc->dt;
+    }
+    const T h = T(dt), norm = T(1.0 / ((double)G.nx * (double)G.ny)), sqh = T(sqrt(dt));
+    line_sync<L>();
+    if (first) lds_write_c<L>(v, lds, j);
+    unit_sync<L>();
+#pragma unroll
+    for (int q = 0; q < kUnitModes; ++q) {
+        const int c = r + q * UT;
+        if (c >= ncy || !active) continue;
+        const int jy = c <= kym ? c : c + (L - ncy);
+        // N = -norm FFT(J) (spectral_core.c:106-111)
+        cx<T> N = (-norm) * lds[pad(jy)];
+        if (a.src) N = N + a.src[c0 + c];
+        const T ky = T(c <= kym ? jy : jy - L) * T(2.0 * kPi / G.Ly);
+        const T k2 = kx * kx + ky * ky;
+        cx<T> wn = mode_update<T, SCHEME>(ph, a.stage, h, dt, k2, N, w0[q], av[q], ws[q], fs[q]);
+        if (a.stage < 3) {
+            a.acc[c0 + c] = av[q];
+            if constexpr (SCHEME == 0) a.stagebuf[c0 + c] = wn;
+        } else {
+            if constexpr (SCHEME == 0) {
+                if (ph.sfd_on && ph.sfd_tau > 0.0) a.sfd[c0 + c] = fs[q];
+            }
+            if (ph.force_on && kxi < ph.fbx) {
+                const int b = c <= kym ? jy : jy - L;
+                if (b >= -ph.fby && b <= ph.fby)
+                    wn = wn + sqh * a.fbox[mb * a.bf + kxi * (2 * ph.fby + 1) + (b + ph.fby)];
+            }
+            a.state[c0 + c] = wn;
+        }
+        lds[RE + pad(jy)] = wn;
+    }
+    if (blockIdx.x == 0 && threadIdx.x == 0 && a.stage == 3) {
+        sc->t += dt;
+        sc->umax2_bits = 0ull;
+    }
+    unit_sync<L>();
+    cx<T>* out = f < 2 ? (f == 0 ? a.mixed[0] : a.mixed[1]) : (f == 2 ? a.mixed[2] : a.mixed[3]);
+    col_unit_out<T, L, MemLaunch>(lds, r, G, kxi, kx, out + mb * a.bm, active, tw);
+}
+
+}  // namespace nsd

@@ -3,8 +3,9 @@
 // constants.  Compiled once per precision with -DNSD_T=float / double.
 //
 // Lengths 64..1024 (the ensemble sizes) also get launch variants that the
-// autotuner chooses between: workgroup size (lines per workgroup) and whether
-// the inverse transforms run in lock-step pairs.
+// autotuner chooses between: workgroup size (lines per workgroup), whether
+// the inverse transforms run in lock-step pairs, and the field-parallel kernels
+// of nsd_fields.hpp.
 #include "nsd_stage.hpp"
 
 #ifndef NSD_T
@@ -23,16 +24,20 @@ constexpr int nt_for() {
 // variant V of length L: threads per workgroup and pairing (-1 automatic)
 template <int L, int V>
 constexpr int var_nt() {
-    return V <= 1 ? nt_for<L>() : (V <= 3 ? 2 * nt_for<L>() : nt_for<L>() / 2);
+    return V <= 1   ? nt_for<L>()
+           : V == 2 ? 2 * nt_for<L>()
+           : V == 4 ? nt_for<L>() / 2
+                    : (L / P > 64 ? L / P : 64);
 }
 template <int V>
 constexpr int var_pr() {
-    return (V == 1 || V == 3) ? 0 : -1;
+    return V == 1 ? 0 : -1;
 }
 template <int L, int V>
 constexpr bool var_ok() {
     constexpr int NT = var_nt<L, V>();
-    return V == 0 || (L >= 64 && L <= 1024 && NT <= 1024 && NT >= L / P && NT >= 64);
+    return V == 0 || (V == kSmallVariant && L <= 1024) ||
+           (V != kSmallVariant && L >= 64 && L <= 1024 && NT <= 1024 && NT >= L / P && NT >= 64);
 }
 
 // the stage kernels' LDS (FP64 lines of 4096 take a second line region)
@@ -49,7 +54,9 @@ size_t stage_lds() {
 template <typename T, int LOG, int V, bool ERR = false>
 void row_stage_LV(const RowArgs<T>& a, int items, int members, hipStream_t st) {
     constexpr int L = 1 << LOG;
-    if constexpr (var_ok<L, V>()) {
+    if constexpr (V == kFieldsVariant) {
+        if constexpr (L <= kFieldsMax) launch_row_fields<T>(a, L, items, members, st);
+    } else if constexpr (var_ok<L, V>()) {
         constexpr int NT = var_nt<L, V>();
         constexpr int PR = var_pr<V>();
         constexpr int lines = NT * P / L;
@@ -63,7 +70,12 @@ void row_stage_LV(const RowArgs<T>& a, int items, int members, hipStream_t st) {
 template <typename T, int LOG, int V, bool ERR = false>
 void col_fused_LV(const ColArgs<T>& a, int ncols, int members, hipStream_t st) {
     constexpr int L = 1 << LOG;
-    if constexpr (var_ok<L, V>()) {
+    if constexpr (V == kFieldsVariant) {
+        if constexpr (L <= kFieldsMax) {
+            if (a.mode == COL_PRIME) col_fused_LV<T, LOG, 0>(a, ncols, members, st);
+            else launch_col_fields<T>(a, L, ncols, members, st);
+        }
+    } else if constexpr (var_ok<L, V>()) {
         constexpr int NT = var_nt<L, V>();
         constexpr int PR = var_pr<V>();
         constexpr int lines = NT * P / L;
@@ -90,7 +102,7 @@ void lds_attr(K kernel, int bytes) {
 template <typename T, int LOG, int V>
 void limits_LV(int bytes) {
     constexpr int L = 1 << LOG;
-    if constexpr (var_ok<L, V>()) {
+    if constexpr (var_ok<L, V>() && V != kFieldsVariant) {
         constexpr int NT = var_nt<L, V>();
         constexpr int PR = var_pr<V>();
         lds_attr(k_row<T, NT, ROW_STAGE, L, PR>, bytes);
@@ -108,14 +120,15 @@ void limits_LV(int bytes) {
 template <typename T, int LOG, int V>
 int var_pairs() {
     constexpr int L = 1 << LOG;
-    if constexpr (var_ok<L, V>()) return stage_layout<T, L, var_nt<L, V>(), var_pr<V>()>() ? 1 : 0;
+    if constexpr (V != kFieldsVariant && var_ok<L, V>()) return stage_layout<T, L, var_nt<L, V>(), var_pr<V>()>() ? 1 : 0;
     return 0;
 }
 
 template <typename T, int LOG, int V>
 int var_valid(int maxlds) {
     constexpr int L = 1 << LOG;
-    if constexpr (var_ok<L, V>())
+    if constexpr (V == kFieldsVariant) return L >= 64 && fields_fits<T>(L, maxlds) ? 1 : 0;
+    else if constexpr (var_ok<L, V>())
         return stage_lds<T, L, V>() <= (size_t)maxlds ? 1 : 0;
     return 0;
 }
@@ -129,7 +142,7 @@ int log2i(int L) {
 }  // namespace
 
 #define NSD_FOR_LOGS(X) X(4) X(5) X(6) X(7) X(8) X(9) X(10) X(11) X(12) X(13)
-#define NSD_FOR_VARS(X, n) X(n, 0) X(n, 1) X(n, 2) X(n, 3) X(n, 4)
+#define NSD_FOR_VARS(X, n) X(n, 0) X(n, 1) X(n, 2) X(n, 3) X(n, 4) X(n, 5)
 
 template <typename T>
 void launch_row_stage(const RowArgs<T>& a, int L, int items, int members, int variant,
@@ -200,6 +213,7 @@ void stage_lds_limits(int bytes) {
     NSD_FOR_LOGS(X)
 #undef X
 #undef V_
+    fields_lds_limits<T>(bytes);
 }
 
 template void launch_row_stage<NSD_T>(const RowArgs<NSD_T>&, int, int, int, int, hipStream_t,
@@ -216,6 +230,28 @@ int col_fused_blocks(int L, int ncols) {
     return (ncols + lines - 1) / lines;
 }
 template int col_fused_blocks<NSD_T>(int, int);
+// Variant a context starts with, for `lines` lines (row pairs or kept columns,
+// times batch members) of length L on a grid whose longer side is `side`.
+// Launches that variant 0 would leave with at most one wave per SIMD (1024 on
+// this device) take the field-parallel kernels or, on FP32 grids below 512^2,
+// variant 0's own code in the smallest workgroups.  us per RK4 step of one field
+// as graph replays, variant 0 -> smallest workgroups -> field-parallel:
+//   64^2 FP64 72 -> 56 -> 49, 512^2 FP64 120 -> - -> 69, 1024^2 FP64 188 -> 172 -> 149,
+//   256^2 FP32 98 -> 81 -> 67, 512^2 FP32 103 -> 85 -> 71, 1024^2 FP32 140 -> 130 -> 124.
+// The small FP32 grids keep variant 0's code because its rounding is theirs: a
+// step's difference of one FP32 rounding grows to 2e-5 of the field within 400
+// forced steps at 256^2, and runs, batch members and restarts of these sizes are
+// compared with one another bit for bit.  Lines of 2048 stay with variant 0: a
+// unit is 1024 threads there, one to a compute unit at FP64, and 256 row pairs
+// take 22.0 us against 20.9 us.
+template <typename T>
+int stage_variant_default(int L, long lines, int side, int maxlds) {
+    const long waves = lines * (L / P) / 64;
+    if (waves > 1024 || L > kFieldsMax) return 0;
+    if (sizeof(T) == 4 && side < 512) return kSmallVariant;
+    return fields_fits<T>(L, maxlds) ? kFieldsVariant : 0;
+}
+template int stage_variant_default<NSD_T>(int, long, int, int);
 template int stage_variant_valid<NSD_T>(int, int, int);
 template int stage_variant_pairs<NSD_T>(int, int);
 template void stage_lds_limits<NSD_T>(int);

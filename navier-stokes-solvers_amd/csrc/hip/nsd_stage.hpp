@@ -8,6 +8,11 @@ namespace nsd {
 
 // number of launch variants per length (variant 0 is the default shape)
 constexpr int kStageVariants = 5;
+// the field-parallel kernels (nsd_fields.hpp), lines of up to kFieldsMax points
+constexpr int kFieldsVariant = 3;
+constexpr int kFieldsMax = 1024;
+// workgroups of one line's threads, or one wave
+constexpr int kSmallVariant = 5;
 
 // k_row in ROW_STAGE mode for rows of length L (power of two, 16..8192),
 // `members` batch members along grid y
@@ -22,6 +27,10 @@ void launch_col_fused(const ColArgs<T>& a, int L, int ncols, int members, int va
 // workgroups of the default (variant 0) column launch over ncols columns
 template <typename T>
 int col_fused_blocks(int L, int ncols);
+// variant that a context starts with for `lines` lines (members included) of a
+// grid whose longer side is `side`
+template <typename T>
+int stage_variant_default(int L, long lines, int side, int maxlds);
 // 1 if `variant` exists for length L and fits `maxlds` bytes of LDS
 template <typename T>
 int stage_variant_valid(int L, int variant, int maxlds);
@@ -29,6 +38,16 @@ int stage_variant_valid(int L, int variant, int maxlds);
 // (k_col) the mixed fields in a layout of their own (stage_layout)
 template <typename T>
 int stage_variant_pairs(int L, int variant);
+// the field-parallel launches (nsd_fields.hip): L <= kFieldsMax
+template <typename T>
+void launch_row_fields(const RowArgs<T>& a, int L, int items, int members, hipStream_t st);
+template <typename T>
+void launch_col_fields(const ColArgs<T>& a, int L, int ncols, int members, hipStream_t st);
+// whether they take lines of length L with `maxlds` bytes of LDS
+template <typename T>
+bool fields_fits(int L, int maxlds);
+template <typename T>
+void fields_lds_limits(int bytes);
 // raise the dynamic-LDS limit of every instantiation above
 template <typename T>
 void stage_lds_limits(int bytes);

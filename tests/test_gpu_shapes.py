@@ -57,3 +57,42 @@ def test_fp32_8192_matches_fp64(ns, integrating_factor):
     print(f"8192^2: FP32 vs FP64 rel L2 {err:.2e}", flush=True)
     assert err <= 1e-6
     assert t32 == pytest.approx(t64, rel=1e-6)
+
+
+# The field-parallel kernels, which small launches start with, against variant
+# 0: the shortest and longest lines they take, lines of one wave and of several,
+# closing passes of radix 2 and 4, workgroups with unused units.  The two
+# contract a few products differently (FP64 1e-13, FP32 1e-5 after 10 steps, as
+# the launch variants are held to).
+@pytest.mark.parametrize("nx,ny", [(16, 16), (32, 16), (64, 64), (128, 32), (256, 512), (512, 64),
+                                   (1024, 128), (2048, 256), (16, 1024), (1024, 1024)])
+@pytest.mark.parametrize("fp32", [False, True])
+@pytest.mark.parametrize("kind", ["forced", "sfd"])
+def test_field_parallel_kernels_match_variant_0(ns, nx, ny, fp32, kind):
+    runs = []
+    for variant in (None, 0):
+        s = ns.Spectral(nx, ny, TWO_PI, TWO_PI, 1e4 if kind == "forced" else 200.0)
+        s.init(taylor_green=False)
+        s.set_precision(fp32)
+        s.set_scheme(kind == "forced")
+        if kind == "forced" and min(nx, ny) >= 32:
+            s.set_forcing(4.0, 6.0, 1e-2, seed=3)
+        s.random_phase(5, k_peak=min(10.0, min(nx, ny) / 6.0), energy=1.0)
+        if kind == "sfd":
+            s.hv_set(enabled=1, coefficient=1.0, order=4, cutoff_ratio=0.4, sfd_enabled=1,
+                     sfd_strength=0.5, sfd_timescale=1.0)
+        if variant is not None:
+            assert s.L.nsd_set_variants(s.ctx, variant, variant) == 0
+        s.sync_device()
+        assert s.advance_n(10, True) == 0
+        assert s.sync_host() == 0
+        runs.append((s.spec("omega_hat").copy(), s.spec("sfd_hat").copy(), s.d.t))
+        s.close()
+    (w, f, t), (w0, f0, t0) = runs
+    err = rel_l2(w, w0)
+    print(f"{nx} x {ny} {'FP32' if fp32 else 'FP64'} {kind}: rel L2 {err:.1e}", flush=True)
+    tol = 1e-5 if fp32 else 1e-13
+    assert np.linalg.norm(w0) > 0 and err <= tol
+    if kind == "sfd":
+        assert rel_l2(f, f0) <= tol
+    assert t == pytest.approx(t0, rel=1e-6 if fp32 else 1e-13)
