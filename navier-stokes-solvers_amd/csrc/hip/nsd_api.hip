@@ -412,18 +412,6 @@ __global__ void k_sum_parts(const double* part, int nparts, DevScalars* sc) {
     }
 }
 
-__device__ __forceinline__ unsigned long long splitmix64_at(unsigned long long seed,
-                                                            unsigned long long k) {
-    // k-th output (k >= 1) of the SplitMix64 stream of forcing.c:11-16
-    unsigned long long z = seed + k * 0x9E3779B97F4A7C15ull;
-    z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
-    z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
-    return z ^ (z >> 31);
-}
-__device__ __forceinline__ double uniform_at(unsigned long long seed, unsigned long long k) {
-    return (double)(splitmix64_at(seed, k) >> 11) * (1.0 / 9007199254740992.0);
-}
-
 // Random-phase initial vorticity (build-defined, same definition as the oracle).
 template <typename T>
 __global__ void k_random_phase(Geo G, unsigned long long seed, const unsigned long long* seeds,
@@ -465,143 +453,12 @@ __global__ void k_scale_state(size_t n, cx<T>* st, const DevScalars* sc, double 
         st[q] = s * st[q];
 }
 
-// Forcing draws (forcing.c:117-184 semantics through the counter form of the
-// SplitMix64 stream: on call c with A active modes, mode rank a uses
-// uniforms 2(cA+a)+1 and 2(cA+a)+2), then the build-defined application:
-// Hermitian projection of the kx = 0 column, mask, and scaling to the
-// injection rate.  One workgroup.
-struct ForceArgs {
-    Geo geo;
-    int A;
-    const int* modes;    // reference index j*nkx + i per active mode (reference order)
-    const int* partner;  // rank of the (0, ny-j) partner for kx = 0 modes, else -1
-    unsigned long long seed;
-    int colored;
-    double tau, energy_target, rate;
-    double* ou;          // colored state per active rank (interleaved complex)
-    double* work;        // 2 * A doubles
-    int fbx, fby;
-    int box_T;           // 1: box in FP32, 0: FP64
-    void* fbox;
-    DevScalars* sc;
-    const unsigned long long* m_seed;  // per-member seeds of a batch (else seed)
-    int skip_on_redo;                  // error controller: no draw on a restoring step
-};
-
+// The draw as a kernel of its own: steps under the error controller, whose
+// restoring steps draw nothing
 __global__ void k_force(ForceArgs a) {
-    const Geo& G = a.geo;
     if (a.skip_on_redo && a.sc[blockIdx.y].redo) return;
-    {  // member blockIdx.y of a batch: its own generator, OU state, box and scalars
-        const int mb = blockIdx.y;
-        const size_t boxn = (size_t)a.fbx * (2 * a.fby + 1);
-        a.sc += mb;
-        a.ou += (size_t)mb * 2 * a.A;
-        a.work += (size_t)mb * 4 * a.A;
-        a.fbox = (char*)a.fbox + (size_t)mb * boxn * (a.box_T ? 2 * sizeof(float) : 2 * sizeof(double));
-        if (a.m_seed) a.seed = a.m_seed[mb];
-    }
-    const unsigned long long c = a.sc->fcount;
-    const double dt = a.sc->dt;
-    double alpha = 0.0, beta = 1.0;
-    if (a.colored) {
-        const double tau = fmax(a.tau, 1e-6);
-        alpha = exp(-dt / tau);
-        beta = sqrt(fmax(1.0 - alpha * alpha, 0.0));
-    }
-    __shared__ double red[16];
-    __shared__ double s_scale;
-    double part = 0.0;
-    for (int r = threadIdx.x; r < a.A; r += blockDim.x) {
-        const unsigned long long k = 2ull * (c * (unsigned long long)a.A + r) + 1ull;
-        double u1 = uniform_at(a.seed, k), u2 = uniform_at(a.seed, k + 1);
-        u1 = fmax(u1, 2.2250738585072014e-308);
-        const double rad = sqrt(-2.0 * log(u1));
-        const double th = 2.0 * kPi * u2;
-        double vr = rad * cos(th), vi = rad * sin(th);
-        if (a.colored) {
-            vr = alpha * a.ou[2 * r] + beta * vr;
-            vi = alpha * a.ou[2 * r + 1] + beta * vi;
-        }
-        a.work[2 * r] = vr;
-        a.work[2 * r + 1] = vi;
-        part += vr * vr + vi * vi;
-    }
-    part = wave_sum(part);
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = part;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        double t = 0.0;
-        for (int i = 0; i < (int)(blockDim.x >> 6); ++i) t += red[i];
-        t = fmax(t, 1e-16);
-        s_scale = sqrt(a.energy_target / t);
-    }
-    __syncthreads();
-    const double sc = s_scale;
-    for (int r = threadIdx.x; r < a.A; r += blockDim.x) {
-        a.work[2 * r] *= sc;
-        a.work[2 * r + 1] *= sc;
-        if (a.colored) {
-            a.ou[2 * r] = a.work[2 * r];
-            a.ou[2 * r + 1] = a.work[2 * r + 1];
-        }
-    }
-    __syncthreads();
-    // Hermitian projection + mask, rate of the projected field
-    double rate = 0.0;
-    double* pr = a.work + 2 * a.A;  // projected values
-    for (int r = threadIdx.x; r < a.A; r += blockDim.x) {
-        const int idx = a.modes[r];
-        const int jy = idx / G.nkx, i = idx % G.nkx;
-        double fr = a.work[2 * r], fi = a.work[2 * r + 1];
-        if (i == 0 || 2 * i == G.nx) {
-            const int p = a.partner[r];
-            if (p >= 0) {
-                fr = 0.5 * (fr + a.work[2 * p]);
-                fi = 0.5 * (fi - a.work[2 * p + 1]);
-            } else if (jy == 0 || 2 * jy == G.ny) {
-                fi = 0.0;
-            }
-        }
-        const double kx = kx_of(G, i), ky = ky_of(G, jy);
-        const double k2 = kx * kx + ky * ky;
-        if (!kept(G, i, jy) || k2 <= 1e-12) fr = fi = 0.0;
-        pr[2 * r] = fr;
-        pr[2 * r + 1] = fi;
-        const double wt = (i == 0 || 2 * i == G.nx) ? 1.0 : 2.0;
-        if (k2 > 1e-12) rate += 0.5 * wt * (fr * fr + fi * fi) / k2;
-    }
-    rate = wave_sum(rate);
-    __syncthreads();
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = rate;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        double t = 0.0;
-        for (int i = 0; i < (int)(blockDim.x >> 6); ++i) t += red[i];
-        s_scale = (t > 0.0 && a.rate > 0.0) ? sqrt(a.rate / t) : 0.0;
-    }
-    __syncthreads();
-    const double s2 = s_scale;
-    const int boxn = a.fbx * (2 * a.fby + 1);
-    for (int e = threadIdx.x; e < boxn; e += blockDim.x) {
-        if (a.box_T) reinterpret_cast<float*>(a.fbox)[2 * e] = 0.f, reinterpret_cast<float*>(a.fbox)[2 * e + 1] = 0.f;
-        else reinterpret_cast<double*>(a.fbox)[2 * e] = 0.0, reinterpret_cast<double*>(a.fbox)[2 * e + 1] = 0.0;
-    }
-    __syncthreads();
-    for (int r = threadIdx.x; r < a.A; r += blockDim.x) {
-        const int idx = a.modes[r];
-        const int jy = idx / G.nkx, i = idx % G.nkx;
-        const int b = band_of(G, jy);
-        if (i >= a.fbx || b < -a.fby || b > a.fby) continue;
-        const int e = i * (2 * a.fby + 1) + (b + a.fby);
-        if (a.box_T) {
-            reinterpret_cast<float*>(a.fbox)[2 * e] = float(s2 * pr[2 * r]);
-            reinterpret_cast<float*>(a.fbox)[2 * e + 1] = float(s2 * pr[2 * r + 1]);
-        } else {
-            reinterpret_cast<double*>(a.fbox)[2 * e] = s2 * pr[2 * r];
-            reinterpret_cast<double*>(a.fbox)[2 * e + 1] = s2 * pr[2 * r + 1];
-        }
-    }
-    if (threadIdx.x == 0) a.sc->fcount = c + 1;
+    __shared__ double red[17];
+    force_draw(a, blockIdx.y, red);
 }
 
 // forcing.c:117-184 on a full reference-layout output (compat entry point)
@@ -766,10 +623,6 @@ struct NsdContext {
     NsdParams P;
     Phys phys;
     hipStream_t stream = nullptr;
-    // the forcing draw runs beside stage 1 on its own stream (fork after
-    // stage 0, join before stage 2)
-    hipStream_t fstream = nullptr;
-    hipEvent_t fev[2] = {nullptr, nullptr};
     size_t esz;  // bytes per complex element at the working precision
     void* state = nullptr;
     void* acc = nullptr;
@@ -950,10 +803,11 @@ void launch_row_nt(NsdContext* c, const RowArgs<T>& a, int blocks, size_t lds) {
 }
 
 template <typename T>
-void launch_row_t(NsdContext* c, const RowArgs<T>& a, int items, bool errctl = false) {
+void launch_row_t(NsdContext* c, const RowArgs<T>& a, int items, bool errctl = false,
+                  bool force = false) {
     const int L = c->G.nx;
     if (a.mode == ROW_STAGE) {
-        launch_row_stage<T>(a, L, items, c->nb, c->vrow, c->stream, errctl);
+        launch_row_stage<T>(a, L, items, c->nb, c->vrow, c->stream, errctl, force);
         return;
     }
     const int NT = threads_for(L);
@@ -1005,6 +859,33 @@ int op_prime(NsdContext* c) {
     return lastk(c);
 }
 
+bool force_active(const NsdContext* c) { return c->phys.force_on && c->fA != 0; }
+
+template <typename T>
+ForceArgs force_args(const NsdContext* c) {
+    ForceArgs f;
+    memset(&f, 0, sizeof(f));
+    f.geo = c->G;
+    f.A = c->fA;
+    f.modes = c->fmodes;
+    f.partner = c->fpartner;
+    f.seed = c->P.force_seed ? c->P.force_seed : 0x123456789abcdefull;
+    f.colored = c->P.force_colored;
+    f.tau = c->P.force_tau;
+    f.energy_target = c->P.force_energy_target;
+    f.rate = c->P.force_rate;
+    f.ou = c->fou;
+    f.work = c->fwork;
+    f.fbx = c->fbx;
+    f.fby = c->fby;
+    f.box_T = (sizeof(T) == 4) ? 1 : 0;
+    f.fbox = c->fbox;
+    f.sc = c->sc;
+    f.m_seed = c->m_seed;
+    f.skip_on_redo = c->phys.errctl ? 1 : 0;
+    return f;
+}
+
 // the error controller runs with adaptive steps only
 bool errctl_on(const NsdContext* c, int adaptive) { return c->phys.errctl && adaptive; }
 
@@ -1023,11 +904,18 @@ void enqueue_stage(NsdContext* c, int s, int adaptive) {
     a.phys.adaptive = adaptive;
     // profiling: three events per stage bracket exactly the two kernels
     // (before k_row, between the kernels, after k_col), so neither bracket
-    // holds the forcing stream's join or another stage's event
+    // holds another stage's event
     const bool prof = c->prof != 0;
     const size_t e0 = (size_t)c->prof_steps * kEvPerStep + 3 * s;
+    // The forcing draw: one more workgroup of stage 1's row kernel, which neither
+    // reads nor writes what the draw touches (its box, OU state, work area and
+    // the forcing counter).  us per step against a kernel of its own on a side
+    // stream (whose fork and join cost more than its 5 us) and in line: 256^2
+    // FP32 81 / 68 / 63, 2048^2 FP32 206 / 200 / 194, 4096^2 FP32 568 / 579 / 556.
+    const bool draw = s == 1 && force_active(c) && !ec;
+    if (draw) r.force = force_args<T>(c);
     if (prof) (void)hipEventRecord(c->evs[e0], c->stream);
-    launch_row_t<T>(c, r, c->G.ny / 2, ec);
+    launch_row_t<T>(c, r, c->G.ny / 2, ec, draw);
     if (prof) (void)hipEventRecord(c->evs[e0 + 1], c->stream);
     launch_col_t<T>(c, a, c->G.nkx_keep, ec);
     if (prof) (void)hipEventRecord(c->evs[e0 + 2], c->stream);
@@ -1051,37 +939,6 @@ void enqueue_finalize(NsdContext* c) {
     a.finalize = 1;
     a.phys.adaptive = 1;
     launch_col_t<T>(c, a, c->G.nkx_keep, true);
-}
-
-template <typename T>
-bool force_active(const NsdContext* c) {
-    return c->phys.force_on && c->fA != 0;
-}
-
-template <typename T>
-void enqueue_force(NsdContext* c, hipStream_t st) {
-    if (!force_active<T>(c)) return;
-    ForceArgs f;
-    memset(&f, 0, sizeof(f));
-    f.geo = c->G;
-    f.A = c->fA;
-    f.modes = c->fmodes;
-    f.partner = c->fpartner;
-    f.seed = c->P.force_seed ? c->P.force_seed : 0x123456789abcdefull;
-    f.colored = c->P.force_colored;
-    f.tau = c->P.force_tau;
-    f.energy_target = c->P.force_energy_target;
-    f.rate = c->P.force_rate;
-    f.ou = c->fou;
-    f.work = c->fwork;
-    f.fbx = c->fbx;
-    f.fby = c->fby;
-    f.box_T = (sizeof(T) == 4) ? 1 : 0;
-    f.fbox = c->fbox;
-    f.sc = c->sc;
-    f.m_seed = c->m_seed;
-    f.skip_on_redo = c->phys.errctl ? 1 : 0;
-    hipLaunchKernelGGL(k_force, dim3(1, c->nb), dim3(256), 0, st, f);
 }
 
 // learned subgrid tendency of the state at the start of the step, into the
@@ -1129,25 +986,18 @@ void enqueue_closure(NsdContext* c) {
     }
 }
 
-// one RK4 step: stage 0 computes dt (adaptive) before the forcing draw,
-// which needs dt for the colored-noise decay and is consumed on stage 3.
-// The draw (one workgroup) runs on the side stream beside stage 1, which
-// neither reads nor writes what it touches (its box, OU state, work area
-// and the forcing counter).
+// one RK4 step: stage 0 computes dt (adaptive) before the forcing draw, which
+// needs dt for the colored-noise decay and is consumed on stage 3
 template <typename T>
 void enqueue_step(NsdContext* c, int adaptive) {
-    if (errctl_on(c, adaptive)) enqueue_judge(c);
+    const bool ec = errctl_on(c, adaptive);
+    if (ec) enqueue_judge(c);
     if (c->closure) enqueue_closure<T>(c);
-    const bool side = force_active<T>(c);
     for (int s = 0; s < 4; ++s) {
-        if (s == 2 && side) (void)hipStreamWaitEvent(c->stream, c->fev[1], 0);
         enqueue_stage<T>(c, s, adaptive);
-        if (s == 0 && side) {
-            (void)hipEventRecord(c->fev[0], c->stream);
-            (void)hipStreamWaitEvent(c->fstream, c->fev[0], 0);
-            enqueue_force<T>(c, c->fstream);
-            (void)hipEventRecord(c->fev[1], c->fstream);
-        }
+        if (s == 0 && ec && force_active(c))
+            hipLaunchKernelGGL(k_force, dim3(1, c->nb), dim3(256), 0, c->stream,
+                               force_args<T>(c));
     }
 }
 
@@ -1708,11 +1558,7 @@ NsdContext* nsd_create_batch(int nx, int ny, double Lx, double Ly, int precision
         }
         return false;
     };
-    if (bad(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking)) ||
-        bad(hipStreamCreateWithFlags(&c->fstream, hipStreamNonBlocking)) ||
-        bad(hipEventCreateWithFlags(&c->fev[0], hipEventDisableTiming)) ||
-        bad(hipEventCreateWithFlags(&c->fev[1], hipEventDisableTiming)))
-        return nullptr;
+    if (bad(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking))) return nullptr;
     const size_t C = C_of(c) * c->esz * members, M = M_of(c) * c->esz * members;
     const size_t S = sizeof(DevScalars) * members;
     if (bad(hipMalloc(&c->state, C)) || bad(hipMalloc(&c->acc, C)) ||
@@ -1781,10 +1627,6 @@ void nsd_destroy(NsdContext* c) {
                     c->cl_m, c->cl_y, c->cl_src, c->ec_prev, c->ec_ymid, c->ec_part};
     for (void* b : bufs)
         if (b) (void)hipFree(b);
-    if (c->fstream) (void)hipStreamSynchronize(c->fstream);
-    for (auto e : c->fev)
-        if (e) (void)hipEventDestroy(e);
-    if (c->fstream) (void)hipStreamDestroy(c->fstream);
     if (c->stream) (void)hipStreamDestroy(c->stream);
     delete c;
 }

@@ -25,12 +25,15 @@ constexpr size_t fields_lds() {
 }
 
 template <typename T, int L>
-void row_fields(const RowArgs<T>& a, int items, int members, hipStream_t st) {
+void row_fields(const RowArgs<T>& a, int items, int members, hipStream_t st, bool force) {
     constexpr int U = fields_units<L>();
     constexpr int MW = fields_mw<T, L>();
-    const dim3 grid((items + U - 1) / U, members);
+    const dim3 grid((items + U - 1) / U + (force ? 1 : 0), members);
     const size_t lds = fields_lds<T, L>();
-    hipLaunchKernelGGL((k_row_fields<T, L, U, MW>), grid, dim3(U * L / 2), lds, st, a);
+    if (force)
+        hipLaunchKernelGGL((k_row_fields<T, L, U, MW, true>), grid, dim3(U * L / 2), lds, st, a);
+    else
+        hipLaunchKernelGGL((k_row_fields<T, L, U, MW, false>), grid, dim3(U * L / 2), lds, st, a);
 }
 
 template <typename T, int L>
@@ -53,7 +56,8 @@ void lds_attr(K kernel, int bytes) {
 template <typename T, int L>
 void limits(int bytes) {
     constexpr int U = fields_units<L>(), MW = fields_mw<T, L>();
-    lds_attr(k_row_fields<T, L, U, MW>, bytes);
+    lds_attr(k_row_fields<T, L, U, MW, false>, bytes);
+    lds_attr(k_row_fields<T, L, U, MW, true>, bytes);
     lds_attr(k_col_fields<T, L, 0, U, MW>, bytes);
     lds_attr(k_col_fields<T, L, 1, U, MW>, bytes);
 }
@@ -64,9 +68,10 @@ void limits(int bytes) {
 static_assert(kFieldsMax == 1024, "the lengths above");
 
 template <typename T>
-void launch_row_fields(const RowArgs<T>& a, int L, int items, int members, hipStream_t st) {
+void launch_row_fields(const RowArgs<T>& a, int L, int items, int members, hipStream_t st,
+                       bool force) {
 #define X(n) \
-    if (L == n) return row_fields<T, n>(a, items, members, st);
+    if (L == n) return row_fields<T, n>(a, items, members, st, force);
     NSD_FOR_FIELDS(X)
 #undef X
 }
@@ -95,7 +100,7 @@ void fields_lds_limits(int bytes) {
 #undef X
 }
 
-template void launch_row_fields<NSD_T>(const RowArgs<NSD_T>&, int, int, int, hipStream_t);
+template void launch_row_fields<NSD_T>(const RowArgs<NSD_T>&, int, int, int, hipStream_t, bool);
 template void launch_col_fields<NSD_T>(const ColArgs<NSD_T>&, int, int, int, hipStream_t);
 template bool fields_fits<NSD_T>(int, int);
 template void fields_lds_limits<NSD_T>(int);

@@ -204,15 +204,22 @@ __device__ __forceinline__ void row_unit(cx<T>* lds, int r, const Geo& G, const 
 }
 
 // U row pairs per workgroup
-template <typename T, int L, int U, int MW>
+template <typename T, int L, int U, int MW, bool FORCE>
 __global__ __launch_bounds__(U * L / 2, MW) void k_row_fields(RowArgs<T> a) {
     extern __shared__ __align__(16) unsigned char smem_raw[];
+    if constexpr (FORCE) {  // workgroup 0 makes the step's forcing draw
+        if (blockIdx.x == 0) {
+            force_draw(a.force, blockIdx.y, reinterpret_cast<double*>(smem_raw));
+            return;
+        }
+    }
+    const int bx = (int)blockIdx.x - (FORCE ? 1 : 0);
     __shared__ double red[U * L / 2 > 64 ? U * L / 128 : 1];
     constexpr int UT = unit_threads<L>(), RE = L + L / 16;
     const int u = threadIdx.x / UT, r = threadIdx.x - u * UT;
     const int f = r / (L / P), j = r - f * (L / P);
     const Geo& G = a.geo;
-    const int y = 2 * (xcd_remap(blockIdx.x, gridDim.x) * U + u);
+    const int y = 2 * (xcd_remap(bx, gridDim.x - (FORCE ? 1 : 0)) * U + u);
     const size_t moff = blockIdx.y * a.bm;
     TwAll<L, T> tw;
     load_tw_all<L, 0>(tw, j, a.tw);

@@ -456,6 +456,158 @@ constexpr int slot_kind(int s, int L, int km) {
     return 3;
 }
 
+// ---------------------------------------------------------------- forcing
+
+__device__ __forceinline__ unsigned long long splitmix64_at(unsigned long long seed,
+                                                            unsigned long long k) {
+    // k-th output (k >= 1) of the SplitMix64 stream of forcing.c:11-16
+    unsigned long long z = seed + k * 0x9E3779B97F4A7C15ull;
+    z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
+    z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
+    return z ^ (z >> 31);
+}
+__device__ __forceinline__ double uniform_at(unsigned long long seed, unsigned long long k) {
+    return (double)(splitmix64_at(seed, k) >> 11) * (1.0 / 9007199254740992.0);
+}
+
+// Forcing draws (forcing.c:117-184 semantics through the counter form of the
+// SplitMix64 stream: on call c with A active modes, mode rank a uses
+// uniforms 2(cA+a)+1 and 2(cA+a)+2), then the build-defined application:
+// Hermitian projection of the kx = 0 column, mask, and scaling to the
+// injection rate.
+struct ForceArgs {
+    Geo geo;
+    int A;
+    const int* modes;    // reference index j*nkx + i per active mode (reference order)
+    const int* partner;  // rank of the (0, ny-j) partner for kx = 0 modes, else -1
+    unsigned long long seed;
+    int colored;
+    double tau, energy_target, rate;
+    double* ou;          // colored state per active rank (interleaved complex)
+    double* work;        // 2 * A doubles
+    int fbx, fby;
+    int box_T;           // 1: box in FP32, 0: FP64
+    void* fbox;
+    DevScalars* sc;
+    const unsigned long long* m_seed;  // per-member seeds of a batch (else seed)
+    int skip_on_redo;                  // error controller: no draw on a restoring step
+};
+
+// The draw for member mb, by one workgroup; red: 17 doubles of LDS.
+__device__ __forceinline__ void force_draw(const ForceArgs& a, int mb, double* red) {
+    const Geo& G = a.geo;
+    // member mb of a batch: its own generator, OU state, box and scalars
+    const size_t box0 = (size_t)a.fbx * (2 * a.fby + 1) * mb;
+    DevScalars* const dsc = a.sc + mb;
+    double* const ou = a.ou + (size_t)mb * 2 * a.A;
+    double* const work = a.work + (size_t)mb * 4 * a.A;
+    float* const box32 = reinterpret_cast<float*>(a.fbox) + 2 * box0;
+    double* const box64 = reinterpret_cast<double*>(a.fbox) + 2 * box0;
+    const unsigned long long seed = a.m_seed ? a.m_seed[mb] : a.seed;
+    const unsigned long long c = dsc->fcount;
+    const double dt = dsc->dt;
+    double& s_scale = red[16];
+    double alpha = 0.0, beta = 1.0;
+    if (a.colored) {
+        const double tau = fmax(a.tau, 1e-6);
+        alpha = exp(-dt / tau);
+        beta = sqrt(fmax(1.0 - alpha * alpha, 0.0));
+    }
+    double part = 0.0;
+    for (int r = threadIdx.x; r < a.A; r += blockDim.x) {
+        const unsigned long long k = 2ull * (c * (unsigned long long)a.A + r) + 1ull;
+        double u1 = uniform_at(seed, k), u2 = uniform_at(seed, k + 1);
+        u1 = fmax(u1, 2.2250738585072014e-308);
+        const double rad = sqrt(-2.0 * log(u1));
+        const double th = 2.0 * kPi * u2;
+        double vr = rad * cos(th), vi = rad * sin(th);
+        if (a.colored) {
+            vr = alpha * ou[2 * r] + beta * vr;
+            vi = alpha * ou[2 * r + 1] + beta * vi;
+        }
+        work[2 * r] = vr;
+        work[2 * r + 1] = vi;
+        part += vr * vr + vi * vi;
+    }
+    part = wave_sum(part);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = part;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        double t = 0.0;
+        for (int i = 0; i < (int)(blockDim.x >> 6); ++i) t += red[i];
+        t = fmax(t, 1e-16);
+        s_scale = sqrt(a.energy_target / t);
+    }
+    __syncthreads();
+    const double sc = s_scale;
+    for (int r = threadIdx.x; r < a.A; r += blockDim.x) {
+        work[2 * r] *= sc;
+        work[2 * r + 1] *= sc;
+        if (a.colored) {
+            ou[2 * r] = work[2 * r];
+            ou[2 * r + 1] = work[2 * r + 1];
+        }
+    }
+    __syncthreads();
+    // Hermitian projection + mask, rate of the projected field
+    double rate = 0.0;
+    double* pr = work + 2 * a.A;  // projected values
+    for (int r = threadIdx.x; r < a.A; r += blockDim.x) {
+        const int idx = a.modes[r];
+        const int jy = idx / G.nkx, i = idx % G.nkx;
+        double fr = work[2 * r], fi = work[2 * r + 1];
+        if (i == 0 || 2 * i == G.nx) {
+            const int p = a.partner[r];
+            if (p >= 0) {
+                fr = 0.5 * (fr + work[2 * p]);
+                fi = 0.5 * (fi - work[2 * p + 1]);
+            } else if (jy == 0 || 2 * jy == G.ny) {
+                fi = 0.0;
+            }
+        }
+        const double kx = kx_of(G, i), ky = ky_of(G, jy);
+        const double k2 = kx * kx + ky * ky;
+        if (!kept(G, i, jy) || k2 <= 1e-12) fr = fi = 0.0;
+        pr[2 * r] = fr;
+        pr[2 * r + 1] = fi;
+        const double wt = (i == 0 || 2 * i == G.nx) ? 1.0 : 2.0;
+        if (k2 > 1e-12) rate += 0.5 * wt * (fr * fr + fi * fi) / k2;
+    }
+    rate = wave_sum(rate);
+    __syncthreads();
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = rate;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        double t = 0.0;
+        for (int i = 0; i < (int)(blockDim.x >> 6); ++i) t += red[i];
+        s_scale = (t > 0.0 && a.rate > 0.0) ? sqrt(a.rate / t) : 0.0;
+    }
+    __syncthreads();
+    const double s2 = s_scale;
+    const int boxn = a.fbx * (2 * a.fby + 1);
+    for (int e = threadIdx.x; e < boxn; e += blockDim.x) {
+        if (a.box_T) box32[2 * e] = box32[2 * e + 1] = 0.f;
+        else box64[2 * e] = box64[2 * e + 1] = 0.0;
+    }
+    __syncthreads();
+    for (int r = threadIdx.x; r < a.A; r += blockDim.x) {
+        const int idx = a.modes[r];
+        const int jy = idx / G.nkx, i = idx % G.nkx;
+        const int b = band_of(G, jy);
+        if (i >= a.fbx || b < -a.fby || b > a.fby) continue;
+        const int e = i * (2 * a.fby + 1) + (b + a.fby);
+        if (a.box_T) {
+            box32[2 * e] = float(s2 * pr[2 * r]);
+            box32[2 * e + 1] = float(s2 * pr[2 * r + 1]);
+        } else {
+            box64[2 * e] = s2 * pr[2 * r];
+            box64[2 * e + 1] = s2 * pr[2 * r + 1];
+        }
+    }
+    if (threadIdx.x == 0) dsc->fcount = c + 1;
+}
+
+
 // ------------------------------------------------------------ column side
 
 enum ColMode { COL_STAGE = 0, COL_PRIME = 1, COL_FWD = 2, COL_INV = 3 };
@@ -1232,6 +1384,10 @@ struct RowArgs {
     int pairs;                 // ROW_STAGE: mixed fields in the stage layout (stage_layout)
     int jblocks;               // ROW_STAGE: write J in 2 x 2 blocks (square pair-layout grids)
     int skip_on_redo;          // ROW_STAGE, ERR: idle when the step restores a rejected one
+    // ROW_STAGE, FORCE: the step's forcing draw, made by workgroup 0 beside the
+    // row pairs of the others (stage 1: dt is known since stage 0, the box is
+    // read in stage 3)
+    ForceArgs force;
 };
 
 // Build the Hermitian extension of Z = A + iB in LDS for one row y from
@@ -1576,7 +1732,7 @@ constexpr bool row_prefetch() {
 }
 
 template <typename T, int NT, int MODE, int LC, int PR = -1, bool ERR = false,
-          int MW = min_waves<T>()>
+          int MW = min_waves<T>(), bool FORCE = false>
 __global__ __launch_bounds__(NT, MW) void k_row(RowArgs<T> a) {
     static_assert(!pair_layout<T, LC, NT, PR>() ||
                       (paired_lines<T, LC, NT, PR>() && row_prefetch<T, LC>()),
@@ -1599,7 +1755,14 @@ __global__ __launch_bounds__(NT, MW) void k_row(RowArgs<T> a) {
     const int RE = LC > 0 ? region_elems<T, LC, NT, PR>() : Ll + Ll / 16;
     cx<T>* lds = smem + m * NB * RE;
     cx<T>* lds2 = lds + (NB - 1) * RE;
-    const int blk = xcd_remap(blockIdx.x, gridDim.x);
+    if constexpr (FORCE) {
+        if (blockIdx.x == 0) {
+            force_draw(a.force, blockIdx.y, reinterpret_cast<double*>(smem_raw));
+            return;
+        }
+    }
+    const int bx = (int)blockIdx.x - (FORCE ? 1 : 0);
+    const int blk = xcd_remap(bx, gridDim.x - (FORCE ? 1 : 0));
     const int item = blk * lines + m;  // row pair (STAGE, R2C) or row (C2R)
     // Staggered start.  The dispatcher gives every compute unit one workgroup
     // before it gives any a second (the host checks this on the device when a
@@ -1613,7 +1776,7 @@ __global__ __launch_bounds__(NT, MW) void k_row(RowArgs<T> a) {
     // Stockham form, which waited at 27 barriers) measures 72.9 again and 24k
     // cycles 75.6.
     if constexpr (MODE == ROW_STAGE && LC == 4096 && sizeof(T) == 4) {
-        if (blockIdx.y == 0 && (int)blockIdx.x >= a.stagger_lo && (int)blockIdx.x < a.stagger_hi) {
+        if (blockIdx.y == 0 && bx >= a.stagger_lo && bx < a.stagger_hi) {
             __builtin_amdgcn_s_sleep(63);
             __builtin_amdgcn_s_sleep(63);
             __builtin_amdgcn_s_sleep(63);

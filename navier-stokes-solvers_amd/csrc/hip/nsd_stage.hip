@@ -52,16 +52,24 @@ size_t stage_lds() {
 
 // ERR: the error controller's instantiations (launch variant 0 only)
 template <typename T, int LOG, int V, bool ERR = false>
-void row_stage_LV(const RowArgs<T>& a, int items, int members, hipStream_t st) {
+void row_stage_LV(const RowArgs<T>& a, int items, int members, hipStream_t st,
+                  bool force = false) {
     constexpr int L = 1 << LOG;
     if constexpr (V == kFieldsVariant) {
-        if constexpr (L <= kFieldsMax) launch_row_fields<T>(a, L, items, members, st);
+        if constexpr (L <= kFieldsMax) launch_row_fields<T>(a, L, items, members, st, force);
     } else if constexpr (var_ok<L, V>()) {
         constexpr int NT = var_nt<L, V>();
         constexpr int PR = var_pr<V>();
         constexpr int lines = NT * P / L;
         const int blocks = (items + lines - 1) / lines;
         const size_t lds = stage_lds<T, L, V>();
+        if constexpr (!ERR) {
+            if (force) {
+                hipLaunchKernelGGL((k_row<T, NT, ROW_STAGE, L, PR, false, min_waves<T>(), true>),
+                                   dim3(blocks + 1, members), dim3(NT), lds, st, a);
+                return;
+            }
+        }
         hipLaunchKernelGGL((k_row<T, NT, ROW_STAGE, L, PR, ERR>), dim3(blocks, members), dim3(NT),
                            lds, st, a);
     }
@@ -106,6 +114,7 @@ void limits_LV(int bytes) {
         constexpr int NT = var_nt<L, V>();
         constexpr int PR = var_pr<V>();
         lds_attr(k_row<T, NT, ROW_STAGE, L, PR>, bytes);
+        lds_attr(k_row<T, NT, ROW_STAGE, L, PR, false, min_waves<T>(), true>, bytes);
         lds_attr(k_col<T, NT, COL_PRIME, 0, L, PR>, bytes);
         lds_attr(k_col<T, NT, COL_STAGE, 0, L, PR>, bytes);
         lds_attr(k_col<T, NT, COL_STAGE, 1, L, PR>, bytes);
@@ -146,7 +155,7 @@ int log2i(int L) {
 
 template <typename T>
 void launch_row_stage(const RowArgs<T>& a, int L, int items, int members, int variant,
-                      hipStream_t st, bool errctl) {
+                      hipStream_t st, bool errctl, bool force) {
     const int lg = log2i(L);
     if (errctl) {
 #define E_(n) \
@@ -156,7 +165,7 @@ void launch_row_stage(const RowArgs<T>& a, int L, int items, int members, int va
         return;
     }
 #define V_(n, v) \
-    if (lg == n && variant == v) return row_stage_LV<T, n, v>(a, items, members, st);
+    if (lg == n && variant == v) return row_stage_LV<T, n, v>(a, items, members, st, force);
 #define X(n) NSD_FOR_VARS(V_, n)
     NSD_FOR_LOGS(X)
 #undef X
@@ -217,7 +226,7 @@ void stage_lds_limits(int bytes) {
 }
 
 template void launch_row_stage<NSD_T>(const RowArgs<NSD_T>&, int, int, int, int, hipStream_t,
-                                      bool);
+                                      bool, bool);
 template void launch_col_fused<NSD_T>(const ColArgs<NSD_T>&, int, int, int, int, hipStream_t,
                                       bool);
 

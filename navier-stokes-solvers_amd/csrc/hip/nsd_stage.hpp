@@ -16,10 +16,11 @@ constexpr int kSmallVariant = 5;
 
 // k_row in ROW_STAGE mode for rows of length L (power of two, 16..8192),
 // `members` batch members along grid y
-// (errctl: the error controller's instantiation, launch variant 0)
+// (errctl: the error controller's instantiation, launch variant 0; force: one
+// more workgroup per member makes the forcing draw a.force, not with errctl)
 template <typename T>
 void launch_row_stage(const RowArgs<T>& a, int L, int items, int members, int variant,
-                      hipStream_t st, bool errctl = false);
+                      hipStream_t st, bool errctl = false, bool force = false);
 // k_col in COL_STAGE (scheme from a.phys.scheme) or COL_PRIME mode, length L
 template <typename T>
 void launch_col_fused(const ColArgs<T>& a, int L, int ncols, int members, int variant,
@@ -40,7 +41,8 @@ template <typename T>
 int stage_variant_pairs(int L, int variant);
 // the field-parallel launches (nsd_fields.hip): L <= kFieldsMax
 template <typename T>
-void launch_row_fields(const RowArgs<T>& a, int L, int items, int members, hipStream_t st);
+void launch_row_fields(const RowArgs<T>& a, int L, int items, int members, hipStream_t st,
+                       bool force);
 template <typename T>
 void launch_col_fields(const ColArgs<T>& a, int L, int ncols, int members, hipStream_t st);
 // whether they take lines of length L with `maxlds` bytes of LDS
