@@ -730,6 +730,9 @@ ColArgs<T> col_args(NsdContext* c) {
     a.geo = c->G;
     a.phys = c->phys;
     a.fwd_scale = 1.0;
+    a.kxs = 2.0 * kPi / c->G.Lx;
+    a.kys = 2.0 * kPi / c->G.Ly;
+    a.norm = 1.0 / ((double)c->G.nx * (double)c->G.ny);
     a.tw = (const cx<T>*)c->twy;
     a.nl = (const cx<T>*)c->nl;
     for (int i = 0; i < 4; ++i) a.mixed[i] = (cx<T>*)c->mixed[i];

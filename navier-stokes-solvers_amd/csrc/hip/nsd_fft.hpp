@@ -587,7 +587,7 @@ __device__ __forceinline__ void line_fft2_c(cx<T> (&v1)[P], cx<T> (&v2)[P], cx<T
 
 // ------------------------------------------------------------------------
 // Lines of L = 512 W points on 64 W threads as W x 512 (wave-split
-// transforms), W = 4, 8 or 16 waves.
+// transforms), W = 2, 4, 8 or 16 waves.
 //
 // Thread j = 64 w + l is lane l of wave w.  With n = n2 + 512 n1 and
 // k = k1 + W k2 the transform splits into 512 W-point DFTs across the waves
@@ -702,8 +702,19 @@ __device__ __forceinline__ void dft8v(cx<T> (&v)[P]) {
 // the twiddles W_L^(n2 k1) applied after (ws_a) or before (ws_b) them
 template <int DIR, int W, bool AFTER, typename T>
 __device__ __forceinline__ void ws_cross(cx<T> (&v)[P], cx<T> wj) {
-    static_assert(W == 4 || W == 8, "cross-wave steps held by one thread");
-    if constexpr (W == 8) {
+    static_assert(W == 2 || W == 4 || W == 8, "cross-wave steps held by one thread");
+    if constexpr (W == 2) {
+        constexpr T r2 = Consts<T>::r2;
+        // W_L^(n2) of columns n2 = j + 128 h: W_L^j W8^h
+        const cx<T> b[4] = {wj, mk(r2 * (wj.x + wj.y), r2 * (wj.y - wj.x)), mk(wj.y, -wj.x),
+                            mk(r2 * (wj.y - wj.x), -r2 * (wj.x + wj.y))};
+#pragma unroll
+        for (int h = 0; h < 4; ++h) {
+            if (!AFTER) v[h + 4] = DIR < 0 ? cmul(v[h + 4], b[h]) : cmulc(v[h + 4], b[h]);
+            dft2<DIR>(v[h], v[h + 4]);
+            if (AFTER) v[h + 4] = DIR < 0 ? cmul(v[h + 4], b[h]) : cmulc(v[h + 4], b[h]);
+        }
+    } else if constexpr (W == 8) {
         cx<T> w[8];
         tw_powers8(w, wj);
         if (!AFTER) tw_apply8<DIR>(v, w);

@@ -21,7 +21,7 @@ template <typename T, int L>
 constexpr int fields_mw() { return sizeof(T) == 8 && L <= 512 ? 3 : 4; }
 template <typename T, int L>
 constexpr size_t fields_lds() {
-    return (size_t)fields_units<L>() * 4 * (L + L / 16) * sizeof(cx<T>);
+    return (size_t)fields_units<L>() * 4 * unit_region<L>() * sizeof(cx<T>);
 }
 
 template <typename T, int L>

@@ -104,32 +104,89 @@ __device__ __forceinline__ void line_fft_act(cx<T> (&v)[P], cx<T>* lds, int j,
     }
 }
 
-// ------------------------------------------------------------ memory access
+// Lines of 1024 points (two waves): wave-split transforms (ws_a, ws_b), one
+// barrier each where the Stockham passes take six.
+template <int L>
+constexpr bool ws_unit() { return L > 512; }
+// elements of a line region
+template <int L>
+constexpr int unit_region() { return ws_unit<L>() ? ws_region(L) : L + L / 16; }
+template <int L, typename T>
+using UnitTw = std::conditional_t<ws_unit<L>(), TwWs<(L > 512 ? L : 1024), T>, TwAll<L, T>>;
 
-// Fields that other workgroups of the same launch neither write nor read.
-struct MemLaunch {
-    template <typename T>
-    static __device__ __forceinline__ cx<T> load(const cx<T>* p) { return *p; }
-    template <typename T>
-    static __device__ __forceinline__ void load2(const cx<T>* p, cx<T>& a, cx<T>& b) {
-        a = p[0];
-        b = p[1];
+template <int L, typename T>
+__device__ __forceinline__ void load_unit_tw(UnitTw<L, T>& t, int j, const cx<T>* __restrict__ tw) {
+    if constexpr (ws_unit<L>()) load_tw_ws(t, j, tw);
+    else load_tw_all<L, 0>(t, j, tw);
+}
+
+// ws_a and ws_b of one line, for the lines that have one (`act`)
+template <int DIR, int L, typename T>
+__device__ __forceinline__ void ws_a_act(cx<T> (&v)[P], cx<T>* lds, int j, const TwWs<L, T>& tw,
+                                         bool act) {
+    constexpr int W = ws_waves(L), Q = 8 / W;
+    constexpr bool SWZ = sizeof(T) == 8;
+    const int l = j & 63;
+    cx<T>* const row[1] = {lds + (j >> 6) * WS_ROW};
+    if (act) {
+        ws_cross<DIR, W, true>(v, tw.wj);
+        cx<T>* o = lds + ws_pos<SWZ>(j);
+#pragma unroll
+        for (int r = 0; r < W; ++r)
+#pragma unroll
+            for (int h = 0; h < Q; ++h) o[r * WS_ROW + ws_off<SWZ>(W * h)] = v[h + Q * r];
     }
-    template <typename T>
-    static __device__ __forceinline__ void store(cx<T>* p, cx<T> v) { *p = v; }
-};
+    __syncthreads();
+    if (act) {
+        const cx<T>* i = row[0] + ws_pos<SWZ>(l);
+#pragma unroll
+        for (int s = 0; s < 8; ++s) v[s] = i[ws_off<SWZ>(s)];
+        wave_lds_fence();
+        cx<T>(*const vv[1])[P] = {&v};
+        ws_local<DIR, 1, SWZ>(vv, row, l, tw);
+    }
+}
+template <int DIR, int L, typename T>
+__device__ __forceinline__ void ws_b_act(cx<T> (&v)[P], cx<T>* lds, int j, const TwWs<L, T>& tw,
+                                         bool act) {
+    constexpr int W = ws_waves(L), Q = 8 / W;
+    constexpr bool SWZ = sizeof(T) == 8;
+    const int l = j & 63;
+    cx<T>* const row[1] = {lds + (j >> 6) * WS_ROW};
+    if (act) {
+        cx<T>(*const vv[1])[P] = {&v};
+        ws_local<DIR, 1, SWZ>(vv, row, l, tw);
+        cx<T>* o = row[0] + ws_pos<SWZ>(l);
+#pragma unroll
+        for (int s = 0; s < 8; ++s) o[ws_off<SWZ>(s)] = v[s];
+    }
+    __syncthreads();
+    if (act) {
+        const cx<T>* i = lds + ws_pos<SWZ>(j);
+#pragma unroll
+        for (int r = 0; r < W; ++r)
+#pragma unroll
+            for (int h = 0; h < Q; ++h) v[h + Q * r] = i[r * WS_ROW + ws_off<SWZ>(W * h)];
+        ws_cross<DIR, W, false>(v, tw.wj);
+    }
+}
+// the wave-strided pattern's element of slot s is ws_index(j) + s L / 8, as the
+// standard pattern's is j + s L / 8
+template <int L>
+__device__ __forceinline__ int ws_index(int j) { return ws_waves(L) * (j & 63) + (j >> 6); }
 
 // ---------------------------------------------------------------- row stage
 
 // One row pair (rows y, y + 1) of the row stage: inverse x-transforms of the
 // four fields, J, the forward x-transform of J, kept columns stored.  r: this
 // thread of the unit; lds: the unit's four line regions.
-template <typename T, int L, typename MEM>
+template <typename T, int L>
 __device__ __forceinline__ void row_unit(cx<T>* lds, int r, const Geo& G, const cx<T>* F, cx<T>* nl,
-                                         int y, bool active, TwAll<L, T>& tw, bool track,
+                                         int y, bool active, UnitTw<L, T>& tw, bool track,
                                          SpeedMax<T>& um) {
-    constexpr int TPL = L / P, RE = L + L / 16, kxm = Band<L>::kxm;
-    constexpr bool KEPT = TPL % 16 == 0;
+    constexpr int TPL = L / P, RE = unit_region<L>(), kxm = Band<L>::kxm;
+    constexpr bool KEPT = TPL % 16 == 0, WS = ws_unit<L>();
+    auto at = [](int i) { return WS ? i : pad(i); };
     const int f = r / TPL, j = r - f * TPL;
     cx<T>* const own = lds + f * RE;
     cx<T> v[P];
@@ -140,49 +197,83 @@ __device__ __forceinline__ void row_unit(cx<T>* lds, int r, const Geo& G, const 
             const int kind = slot_kind(s, L, kxm), k = j + s * TPL;
             if (kind == 1 || (kind == 3 && k <= kxm)) {
                 if (active) {
-                    MEM::load2(at32(F, col_elem(k, G.ny, y)), q.a[s], q.b[s]);
+                    const cx<T>* src = at32(F, col_elem(k, G.ny, y));
+                    q.a[s] = src[0];
+                    q.b[s] = src[1];
                 } else {
                     q.a[s] = mk(T(0), T(0));
                     q.b[s] = mk(T(0), T(0));
                 }
             }
         }
-        stage_two_rows_regs<L, KEPT>(own, j, q);
+        stage_two_rows_regs<L, KEPT, !WS>(own, j, q);
     }
     line_sync<L>();
-    lds_read_any<L, KEPT>(v, own, j);
+    if constexpr (WS) lds_read_kept<L, false>(v, own, j);
+    else lds_read_any<L, KEPT>(v, own, j);
     line_sync<L>();
-    line_fft_act<+1, L>(v, own, j, tw, true);
+    // the exchange area of a thread: its slots of the line, or (wave-split) of
+    // its wave's own row
+    const int x0 = WS ? (j >> 6) * WS_ROW + (j & 63) : pad(j);
+    auto xo = [](int s) { return WS ? 64 * s : TPL % 16 == 0 ? padc(s * TPL) : 0; };
+    auto put = [&](cx<T>* o) {
+        if constexpr (WS || TPL % 16 == 0) {
+#pragma unroll
+            for (int s = 0; s < P; ++s) o[x0 + xo(s)] = v[s];
+        } else {
+            lds_write_c<L>(v, o, j);
+        }
+    };
+    auto get = [&](cx<T> (&d)[P], const cx<T>* o) {
+        if constexpr (WS || TPL % 16 == 0) {
+#pragma unroll
+            for (int s = 0; s < P; ++s) d[s] = o[x0 + xo(s)];
+        } else {
+            lds_read_c<L>(d, o, j);
+        }
+    };
+    if constexpr (WS) {
+        ws_a_act<+1, L>(v, own, j, tw, true);
+    } else {
+        line_fft_act<+1, L>(v, own, j, tw, true);
+        line_sync<L>();
+    }
     // psi_y, omega_x, omega_y to the threads that hold psi_x
-    line_sync<L>();
-    if (f > 0) lds_write_c<L>(v, own, j);
+    if (f > 0) put(own);
     unit_sync<L>();
     const bool first = f == 0;
     if (first) {
         // J = psi_x omega_y - psi_y omega_x (spectral_core.c:101-104), in two
         // sweeps so that few values are held at once
         cx<T> b[P], c[P];
-        lds_read_c<L>(b, lds + RE, j);
-        lds_read_c<L>(c, lds + 2 * RE, j);
+        get(b, lds + RE);
+        get(c, lds + 2 * RE);
         if (track) add_speeds(um, v, b);
 #pragma unroll
         for (int s = 0; s < P; ++s) b[s] = mk(b[s].x * c[s].x, b[s].y * c[s].y);
         __builtin_amdgcn_sched_barrier(0);
-        lds_read_c<L>(c, lds + 3 * RE, j);
+        get(c, lds + 3 * RE);
 #pragma unroll
         for (int s = 0; s < P; ++s)
             v[s] = mk(v[s].x * c[s].x - b[s].x, v[s].y * c[s].y - b[s].y);
     }
-    renew_tw_all(tw);
-    line_fft_act<-1, L>(v, lds, j, tw, first);
+    if constexpr (WS) {
+        renew(tw.wj);
+        renew(tw.w8);
+        renew(tw.w64);
+        ws_b_act<-1, L>(v, lds, j, tw, first);
+    } else {
+        renew_tw_all(tw);
+        line_fft_act<-1, L>(v, lds, j, tw, first);
+    }
     line_sync<L>();
     if (first) {
         // the slots that the separation reads (as fwd_rows_store)
         if constexpr (KEPT) {
-            cx<T>* b = lds + pad(j);
+            cx<T>* b = lds + at(j);
 #pragma unroll
             for (int s = 0; s < P; ++s)
-                if (slot_kind(s, L, kxm) != 0) b[padc(s * TPL)] = v[s];
+                if (slot_kind(s, L, kxm) != 0) b[WS ? s * TPL : padc(s * TPL)] = v[s];
         } else {
             lds_write_c<L>(v, lds, j);
         }
@@ -194,11 +285,11 @@ __device__ __forceinline__ void row_unit(cx<T>* lds, int r, const Geo& G, const 
     for (int k0 = 0; k0 <= kxm; k0 += UT) {
         const int k = k0 + r;
         if (k <= kxm && active) {
-            const cx<T> zk = lds[pad(k)];
-            const cx<T> zm = lds[pad((L - k) & (L - 1))];
+            const cx<T> zk = lds[at(k)];
+            const cx<T> zm = lds[at((L - k) & (L - 1))];
             cx<T>* dst = at32(nl, col_elem(k, G.ny, y));
-            MEM::store(dst, mk(T(0.5) * (zk.x + zm.x), T(0.5) * (zk.y - zm.y)));
-            MEM::store(dst + 1, mk(T(0.5) * (zk.y + zm.y), T(0.5) * (zm.x - zk.x)));
+            dst[0] = mk(T(0.5) * (zk.x + zm.x), T(0.5) * (zk.y - zm.y));
+            dst[1] = mk(T(0.5) * (zk.y + zm.y), T(0.5) * (zm.x - zk.x));
         }
     }
 }
@@ -215,17 +306,17 @@ __global__ __launch_bounds__(U * L / 2, MW) void k_row_fields(RowArgs<T> a) {
     }
     const int bx = (int)blockIdx.x - (FORCE ? 1 : 0);
     __shared__ double red[U * L / 2 > 64 ? U * L / 128 : 1];
-    constexpr int UT = unit_threads<L>(), RE = L + L / 16;
+    constexpr int UT = unit_threads<L>(), RE = unit_region<L>();
     const int u = threadIdx.x / UT, r = threadIdx.x - u * UT;
     const int f = r / (L / P), j = r - f * (L / P);
     const Geo& G = a.geo;
     const int y = 2 * (xcd_remap(bx, gridDim.x - (FORCE ? 1 : 0)) * U + u);
     const size_t moff = blockIdx.y * a.bm;
-    TwAll<L, T> tw;
-    load_tw_all<L, 0>(tw, j, a.tw);
+    UnitTw<L, T> tw;
+    load_unit_tw<L>(tw, j, a.tw);
     const cx<T>* F = f < 2 ? (f == 0 ? a.mixed[0] : a.mixed[1]) : (f == 2 ? a.mixed[2] : a.mixed[3]);
     SpeedMax<T> um;
-    row_unit<T, L, MemLaunch>(reinterpret_cast<cx<T>*>(smem_raw) + u * 4 * RE, r, G, F + moff,
+    row_unit<T, L>(reinterpret_cast<cx<T>*>(smem_raw) + u * 4 * RE, r, G, F + moff,
                               a.nl + moff, y, y < G.ny, tw, a.track_umax != 0, um);
     if (a.track_umax) block_max_to(double(um.value()), &a.sc[blockIdx.y].umax2_bits, red);
 }
@@ -287,52 +378,48 @@ __device__ __forceinline__ cx<T> mode_update(const Phys& ph, int stage, T h, dou
 // Kept modes of a column per thread of its unit (2 L / 3 over L / 2 threads)
 constexpr int kUnitModes = 2;
 
-// The step's scalars as the column stage needs them
-template <typename T>
-struct StageScalars {
-    double dt;
-    T h, norm, sqh;
-};
-
 // Inverse y-transforms of the derivative fields of one column's stage field,
-// whose kept modes lie in region 1 of the unit (padded, standard order): field
-// f of this thread's group into out.  Outputs 0 psi_x, 1 psi_y, 2 omega_x,
+// whose kept modes lie in region w of the unit (in order; padded unless
+// wave-split): field f of this thread's group into out.  Outputs 0 psi_x, 1 psi_y, 2 omega_x,
 // 3 omega_y (spectral_core.c:62-99).
-template <typename T, int L, typename MEM>
-__device__ __forceinline__ void col_unit_out(cx<T>* lds, int r, const Geo& G, int kxi, T kx,
-                                             cx<T>* out, bool active, const TwAll<L, T>& tw) {
-    constexpr int TPL = L / P, RE = L + L / 16, kym = Band<L>::kym;
+template <typename T, int L>
+__device__ __forceinline__ void col_unit_out(cx<T>* lds, const cx<T>* w, int r, const Geo& G,
+                                             int kxi, T kx, T kys, cx<T>* out, bool active,
+                                             const UnitTw<L, T>& tw) {
+    constexpr int TPL = L / P, RE = unit_region<L>(), kym = Band<L>::kym;
     const int f = r / TPL, j = r - f * TPL;
-    const T kys = T(2.0 * kPi / G.Ly);
+    constexpr bool WS = ws_unit<L>();
+    const int ji = WS ? ws_index<(L > 512 ? L : 1024)>(j) : j;  // input pattern
     cx<T> v[P];
 #pragma unroll
     for (int s = 0; s < P; ++s) {
-        const int kind = slot_kind(s, L, kym), jy = j + s * TPL;
+        const int kind = slot_kind(s, L, kym), jy = ji + s * TPL;
         v[s] = mk(T(0), T(0));
         if (kind == 0) continue;
-        const cx<T> w = lds[RE + pad(jy)];
-        if (kind != 3 || jy <= kym || jy >= L - kym) v[s] = w;
+        const cx<T> m = w[WS ? jy : pad(jy)];
+        if (kind != 3 || jy <= kym || jy >= L - kym) v[s] = m;
     }
-    unit_sync<L>();  // region 1 is read: the transforms may use it
+    unit_sync<L>();  // the modes are read: the transforms may use their region
     if (f < 2) {  // psi_hat = -omega_hat / k^2
 #pragma unroll
         for (int s = 0; s < P; ++s) {
             if (slot_kind(s, L, kym) == 0) continue;
-            const T ky = T(col_band<L>(G, j + s * TPL)) * kys;
+            const T ky = T(col_band<L>(G, ji + s * TPL)) * kys;
             const T k2 = kx * kx + ky * ky;
             v[s] = k2 > T(1e-12) ? neg_inv_k2(k2) * v[s] : mk(T(0), T(0));
         }
     }
 #pragma unroll
     for (int s = 0; s < P; ++s) {
-        const T ky = T(col_band<L>(G, j + s * TPL)) * kys;
+        const T ky = T(col_band<L>(G, ji + s * TPL)) * kys;
         v[s] = mul_i(v[s], (f & 1) ? ky : kx);
     }
-    line_fft_act<+1, L>(v, lds + f * RE, j, tw, true);
+    if constexpr (WS) ws_b_act<+1, L>(v, lds + f * RE, j, tw, true);
+    else line_fft_act<+1, L>(v, lds + f * RE, j, tw, true);
     if (active) {
         cx<T>* o = out + (size_t)kxi * G.ny + j;
 #pragma unroll
-        for (int s = 0; s < P; ++s) MEM::store(o + s * TPL, v[s]);
+        for (int s = 0; s < P; ++s) o[s * TPL] = v[s];
     }
 }
 
@@ -340,7 +427,7 @@ __device__ __forceinline__ void col_unit_out(cx<T>* lds, int r, const Geo& G, in
 template <typename T, int L, int SCHEME, int U, int MW>
 __global__ __launch_bounds__(U * L / 2, MW) void k_col_fields(ColArgs<T> a) {
     extern __shared__ __align__(16) unsigned char smem_raw[];
-    constexpr int UT = unit_threads<L>(), TPL = L / P, RE = L + L / 16;
+    constexpr int UT = unit_threads<L>(), TPL = L / P, RE = unit_region<L>();
     constexpr int kym = Band<L>::kym, ncy = 2 * kym + 1;
     static_assert(ncy <= kUnitModes * UT, "kept modes per thread");
     const int u = threadIdx.x / UT, r = threadIdx.x - u * UT;
@@ -356,10 +443,11 @@ __global__ __launch_bounds__(U * L / 2, MW) void k_col_fields(ColArgs<T> a) {
     }
     const int kxi = blockIdx.x * U + u;
     const bool active = kxi < G.nkx_keep;
-    const T kx = T(kxi) * T(2.0 * kPi / G.Lx);
+    // wavenumber steps and 1 / (nx ny) from the host: no division on the way
+    const T kx = T(kxi) * T(a.kxs), kys = T(a.kys);
     const cx<T> zero = mk(T(0), T(0));
-    TwAll<L, T> tw;
-    load_tw_all<L, 0>(tw, j, a.tw);
+    UnitTw<L, T> tw;
+    load_unit_tw<L>(tw, j, a.tw);
     // J by the first group, whose transform runs while the modes' state arrives
     cx<T> v[P];
     const bool first = f == 0;
@@ -383,7 +471,10 @@ __global__ __launch_bounds__(U * L / 2, MW) void k_col_fields(ColArgs<T> a) {
             }
         }
     }
-    line_fft_act<-1, L>(v, lds, j, tw, first);
+    constexpr bool WS = ws_unit<L>();
+    auto at = [](int i) { return WS ? i : pad(i); };
+    if constexpr (WS) ws_a_act<-1, L>(v, lds, j, tw, first);
+    else line_fft_act<-1, L>(v, lds, j, tw, first);
     double dt;
     if (a.stage == 0 && ph.adaptive) {
         const double u2 = __longlong_as_double((long long)sc->umax2_bits);
@@ -395,9 +486,21 @@ __global__ __launch_bounds__(U * L / 2, MW) void k_col_fields(ColArgs<T> a) {
     } else {
         dt = sc->dt;
     }
-    const T h = T(dt), norm = T(1.0 / ((double)G.nx * (double)G.ny)), sqh = T(sqrt(dt));
-    line_sync<L>();
-    if (first) lds_write_c<L>(v, lds, j);
+    const T h = T(dt), norm = T(a.norm), sqh = T(sqrt(dt));
+    // J's spectrum in order: region 0, or (wave-split, whose rows other waves may
+    // still read there) region 1; the updated modes go to the next region
+    cx<T>* const jh = lds + (WS ? RE : 0);
+    cx<T>* const wh = jh + RE;
+    if constexpr (WS) {
+        if (first) {
+            cx<T>* o = jh + ws_index<(L > 512 ? L : 1024)>(j);
+#pragma unroll
+            for (int s = 0; s < P; ++s) o[s * TPL] = v[s];
+        }
+    } else {
+        line_sync<L>();
+        if (first) lds_write_c<L>(v, jh, j);
+    }
     unit_sync<L>();
 #pragma unroll
     for (int q = 0; q < kUnitModes; ++q) {
@@ -405,9 +508,9 @@ __global__ __launch_bounds__(U * L / 2, MW) void k_col_fields(ColArgs<T> a) {
         if (c >= ncy || !active) continue;
         const int jy = c <= kym ? c : c + (L - ncy);
         // N = -norm FFT(J) (spectral_core.c:106-111)
-        cx<T> N = (-norm) * lds[pad(jy)];
+        cx<T> N = (-norm) * jh[at(jy)];
         if (a.src) N = N + a.src[c0 + c];
-        const T ky = T(c <= kym ? jy : jy - L) * T(2.0 * kPi / G.Ly);
+        const T ky = T(c <= kym ? jy : jy - L) * kys;
         const T k2 = kx * kx + ky * ky;
         cx<T> wn = mode_update<T, SCHEME>(ph, a.stage, h, dt, k2, N, w0[q], av[q], ws[q], fs[q]);
         if (a.stage < 3) {
@@ -424,7 +527,7 @@ __global__ __launch_bounds__(U * L / 2, MW) void k_col_fields(ColArgs<T> a) {
             }
             a.state[c0 + c] = wn;
         }
-        lds[RE + pad(jy)] = wn;
+        wh[at(jy)] = wn;
     }
     if (blockIdx.x == 0 && threadIdx.x == 0 && a.stage == 3) {
         sc->t += dt;
@@ -432,7 +535,7 @@ __global__ __launch_bounds__(U * L / 2, MW) void k_col_fields(ColArgs<T> a) {
     }
     unit_sync<L>();
     cx<T>* out = f < 2 ? (f == 0 ? a.mixed[0] : a.mixed[1]) : (f == 2 ? a.mixed[2] : a.mixed[3]);
-    col_unit_out<T, L, MemLaunch>(lds, r, G, kxi, kx, out + mb * a.bm, active, tw);
+    col_unit_out<T, L>(lds, wh, r, G, kxi, kx, kys, out + mb * a.bm, active, tw);
 }
 
 }  // namespace nsd

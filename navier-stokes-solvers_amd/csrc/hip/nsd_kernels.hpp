@@ -423,12 +423,15 @@ struct Band {
 // FP32 lines of 8192 are paired as well (147 KB, one workgroup of 16 waves per
 // CU): one region leaves room for no second workgroup either, and the
 // wave-split pairs took k_row at 8192^2 from 926 to 537 us and k_col from 527
-// to 450 us (per-pair layout).
+// to 450 us (per-pair layout).  FP64 lines of 2048 are not, though two regions
+// would fit: they run wave-split in a field at a time like those of 4096
+// (ws_lines64; 2048^2 FP64 step 351 -> 311 us).
 template <typename T, int LC, int NT = threads_for(LC), int PR = -1>
 constexpr bool paired_lines() {
     if (LC <= 0) return false;
     if (PR >= 0) return PR == 1;
     if (sizeof(T) == 4 && LC == 8192) return true;
+    if (sizeof(T) == 8 && LC == 2048) return false;
     return 2 * (LC + LC / 16) * (int)sizeof(cx<T>) * (NT * P / LC) <= 80 * 1024;
 }
 template <typename T, int LC, int NT = threads_for(LC), int PR = -1>
@@ -436,7 +439,7 @@ constexpr int line_regions() {
     return paired_lines<T, LC, NT, PR>() ? 2 : 1;
 }
 
-// FP64 lines of 4096 on 512 threads (one workgroup per CU): wave-split
+// FP64 lines of 2048 and 4096 (two workgroups or one per CU): wave-split
 // transforms with a second line region.  The row stage stages each field in
 // one region and runs the cross-wave rows in the other, so staging the next
 // field needs no barrier of its own; the column stage transposes back to the
@@ -444,7 +447,8 @@ constexpr int line_regions() {
 // none between them.
 template <typename T, int LC, int NT = threads_for(LC), int PR = -1>
 constexpr bool ws_lines64() {
-    return sizeof(T) == 8 && LC == 4096 && NT == 512 && !paired_lines<T, LC, NT, PR>();
+    return sizeof(T) == 8 && (LC == 2048 || LC == 4096) && NT * P == LC &&
+           !paired_lines<T, LC, NT, PR>();
 }
 
 
@@ -666,6 +670,7 @@ struct ColArgs {
     double* errpart;
     size_t bp;
     int finalize;
+    double kxs, kys, norm;  // 2 pi / Lx, 2 pi / Ly, 1 / (nx ny) (field-parallel kernels)
 };
 
 template <typename T>
@@ -692,7 +697,7 @@ __device__ __forceinline__ cx<T> grow(cx<T> w, T em1) {
 }
 
 // occupancy floor handed to the register allocator: waves per SIMD
-// Pair layout of the stage kernels' mixed fields (FP32, 4096-point lines):
+// Pair layout of the stage kernels' mixed fields (FP32, 2048- and 4096-point lines):
 // (psi_x, psi_y) interleaved per (kx, y) in the buffer of psi_x and psi_y,
 // (omega_x, omega_y) likewise in that of omega_x and omega_y; pair element e
 // = kx ny + y of member m sits at 2 (m M + e) of the pair's buffer (M = kept
@@ -701,20 +706,23 @@ __device__ __forceinline__ cx<T> grow(cx<T> w, T em1) {
 // line of its own: half the L1 misses of the row kernel's gathers, whose
 // address path otherwise waits on the cache for about half of its cycles.
 // k_col still writes whole lines (one 16-byte store per lane and pair).
-// It is a property of the instantiation: the paired transforms of square
-// FP32 4096^2 and (in row-pair tiles, pairtile_layout) 8192^2 grids (the gather-ahead k_row path reads it, the paired k_col
-// path writes it).  The host selects it per launch (ColArgs/RowArgs::pairs)
-// when the row and column instantiations it launches both hold it
-// (stage_variant_pairs); the transform modes keep the per-field layout.  At
-// 64..2048 it measured slower (256-member ensemble 92k -> 86k
-// member-steps/s), so it stays at 4096.
+// It is a property of the instantiation: the paired wave-split transforms of
+// square FP32 2048^2, 4096^2 and (in row-pair tiles, pairtile_layout) 8192^2
+// grids (the gather-ahead k_row path reads it, the paired k_col path writes
+// it).  The host selects it per launch (ColArgs/RowArgs::pairs) when the row and
+// column instantiations it launches both hold it (stage_variant_pairs); the
+// transform modes keep the per-field layout.  At 2048 it came with the
+// wave-split transforms (2048^2 FP32: k_row 29.2 -> 24.7 us, k_col 23.5 -> 24.1,
+// step 194 -> 180 us); at 64..1024, with Stockham lines, it measured slower
+// (256-member ensemble 92k -> 86k member-steps/s).
 template <typename T, int LC, int NT, int PR>
 constexpr bool pair_layout() {
-    return sizeof(T) == 4 && (LC == 4096 || LC == 8192) && paired_lines<T, LC, NT, PR>();
+    return sizeof(T) == 4 && (LC == 2048 || LC == 4096 || LC == 8192) && NT * P == LC &&
+           paired_lines<T, LC, NT, PR>();
 }
 
 // Row-pair tiles of the mixed fields (rowpair_elem): the FP64 stage kernels
-// of 4096 (ws_lines64), selected per launch like the pair layout.  A row
+// of 2048 and 4096 (ws_lines64), selected per launch like the pair layout.  A row
 // pair's gathers of one field then read one contiguous run of 32 bytes per
 // kept column, neighbouring columns adjacent (2 KB per wave instruction),
 // where the per-field layout puts every lane in a 64 KB column of its own and

@@ -35,10 +35,11 @@ def two_steps(ns, nx, ny, fp32, integrating_factor):
     return w, t
 
 
-# a 4096- or 8192-point side next to another length: the layouts of the square
+# a 2048-, 4096- or 8192-point side next to another length: the layouts of the square
 # grids' stage kernels and J's 2 x 2 blocks are not for them
 @pytest.mark.parametrize("nx,ny", [(4096, 64), (64, 4096), (4096, 1024), (1024, 4096),
-                                   (8192, 128), (128, 8192), (8192, 4096)])
+                                   (8192, 128), (128, 8192), (8192, 4096), (2048, 256),
+                                   (256, 2048), (2048, 4096)])
 def test_fp32_rectangles_match_fp64(ns, nx, ny):
     w32, t32 = two_steps(ns, nx, ny, True, True)
     w64, t64 = two_steps(ns, nx, ny, False, True)
@@ -96,3 +97,32 @@ def test_field_parallel_kernels_match_variant_0(ns, nx, ny, fp32, kind):
     if kind == "sfd":
         assert rel_l2(f, f0) <= tol
     assert t == pytest.approx(t0, rel=1e-6 if fp32 else 1e-13)
+
+
+# 2048^2 holds the mixed fields in the stage kernels' own layouts (FP32 pairs and J
+# in 2 x 2 blocks, FP64 row-pair tiles); the compat transforms, and the nonlinear
+# term whose row stage they feed, use the per-field one in the same buffers.
+@pytest.mark.parametrize("fp32", [True, False])
+def test_layout_transitions_2048(ns, fp32):
+    made = []
+    for single, compat in ((not fp32, True), (fp32, True), (fp32, False)):
+        s = ns.Spectral(2048, 2048, TWO_PI, TWO_PI, 1e4)
+        s.init(taylor_green=False)
+        s.set_precision(single)
+        s.random_phase(3, k_peak=10.0)
+        if compat:
+            s.L.ns_spectral_compute_velocity_from_vorticity(s.p)
+            s.L.ns_spectral_compute_nonlinear_terms(s.p)
+            s.check()
+        made.append(s)
+    other, mine, plain = made
+    err = rel_l2(mine.spec("nonlinear_hat"), other.spec("nonlinear_hat"))
+    print(f"nonlinear term at 2048^2, FP32 against FP64: rel L2 {err:.2e}", flush=True)
+    assert err < 1e-5
+    for s in (mine, plain):
+        assert s.advance_n(2, True) == 0
+        assert s.sync_host() == 0
+    assert mine.d.t == plain.d.t
+    assert np.array_equal(mine.spec("omega_hat"), plain.spec("omega_hat"))
+    for s in made:
+        s.close()
