@@ -17,6 +17,7 @@
 #include "ns_closure.h"
 #include "ns_device.h"
 #include "nsd_closure_link.hpp"
+#include "nsd_host.h"
 #include "nsd_stage.hpp"
 
 using namespace nsd;
@@ -116,6 +117,62 @@ __global__ void k_velocity_ref(Geo G, const double* __restrict__ w, double* __re
     }
 }
 
+// Host arrays read through pinned memory: kept modes of omega_hat (and of the SFD
+// state) and the scalars of nsd_set_time, the start of a step on host arrays.
+template <typename T>
+__global__ void k_host_in(Geo G, const double* __restrict__ w, const double* __restrict__ f,
+                          cx<T>* __restrict__ st, cx<T>* __restrict__ sfd, DevScalars* sc, double t,
+                          double dt, double dt_err) {
+    const size_t n = (size_t)G.nkx_keep * G.nky_keep;
+    for (size_t e = blockIdx.x * (size_t)blockDim.x + threadIdx.x; e < n;
+         e += (size_t)gridDim.x * blockDim.x) {
+        const int cy = (int)(e / G.nkx_keep), kx = (int)(e % G.nkx_keep);
+        const int jy = cy <= G.kymax ? cy : cy + (G.ny - G.nky_keep);
+        const size_t r = (size_t)jy * G.nkx + kx, o = (size_t)kx * G.nky_keep + cy;
+        st[o] = ld_ref<T>(w, r);
+        if (f) sfd[o] = ld_ref<T>(f, r);
+    }
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        sc->t = t;
+        sc->dt = dt;
+        sc->dt_err = dt_err;
+        sc->err = 0.0;
+        sc->n_acc = sc->n_rej = 0ull;
+        sc->pending = sc->redo = 0;
+    }
+}
+
+// ... and its end: the state's spectra as k_scatter_state and k_velocity_ref have
+// them, and the scalars, written straight to pinned memory.
+template <typename T>
+__global__ void k_host_out(Geo G, const cx<T>* __restrict__ st, const cx<T>* __restrict__ sfd,
+                           const DevScalars* sc, double* __restrict__ w, double* __restrict__ psi,
+                           double* __restrict__ u, double* __restrict__ v, double* __restrict__ f,
+                           double* __restrict__ head) {
+    const size_t n = (size_t)G.nkx * G.ny;
+    for (size_t e = blockIdx.x * (size_t)blockDim.x + threadIdx.x; e < n;
+         e += (size_t)gridDim.x * blockDim.x) {
+        const int jy = (int)(e / G.nkx), i = (int)(e % G.nkx);
+        const double kx = kx_of(G, i), ky = ky_of(G, jy);
+        const double k2 = kx * kx + ky * ky;
+        const bool k = kept(G, i, jy);
+        const size_t o = (size_t)i * G.nky_keep + compact_y(G, jy);
+        const cx<T> s = k ? st[o] : mk(T(0), T(0));
+        const cx<double> om = mk(double(s.x), double(s.y));
+        const cx<double> ps = k2 > 1e-12 ? (-1.0 / k2) * om : mk(0.0, 0.0);
+        st_ref(w, e, om);
+        st_ref(psi, e, ps);
+        st_ref(u, e, mul_i(ps, ky));
+        st_ref(v, e, mul_i(ps, -kx));
+        if (f) st_ref(f, e, k ? sfd[o] : mk(T(0), T(0)));
+    }
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        head[0] = sc->t;
+        head[1] = sc->dt;
+        head[2] = double(sc->status);
+    }
+}
+
 // spectral_transforms.c:35-43
 __global__ void k_dealias_ref(Geo G, double* f) {
     const size_t n = (size_t)G.nkx * G.ny;
@@ -190,6 +247,42 @@ __global__ void k_phys_reduce(size_t n, const double* u, const double* v, const 
     block_max_to(m, &sc->redmax[0], red);
     block_sum_to(e, &sc->red[0], red);
     block_sum_to(z, &sc->red[1], red);
+}
+
+// The same over pinned host arrays, each workgroup's {maximum as ordered bits,
+// energy, enstrophy} to pinned memory, added up by the host in index order.
+__global__ void k_phys_parts(size_t n, const double* u, const double* v, const double* w,
+                             double* part) {
+    double m = 0.0, e = 0.0, z = 0.0;
+    for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n;
+         i += (size_t)gridDim.x * blockDim.x) {
+        if (u && v) {
+            const double a = u[i], b = v[i];
+            const double s = a * a + b * b;
+            m = fmax(m, s);
+            e += 0.5 * s;
+        }
+        if (w) {
+            const double a = w[i];
+            z += 0.5 * a * a;
+        }
+    }
+    __shared__ double red[4];
+    __shared__ unsigned long long mx;
+    __shared__ double sum[2];
+    if (threadIdx.x == 0) {
+        mx = 0ull;
+        sum[0] = sum[1] = 0.0;
+    }
+    block_max_to(m, &mx, red);
+    block_sum_to(e, &sum[0], red);
+    block_sum_to(z, &sum[1], red);
+    if (threadIdx.x == 0) {
+        double* o = part + 3 * blockIdx.x;
+        o[0] = __longlong_as_double((long long)mx);
+        o[1] = sum[0];
+        o[2] = sum[1];
+    }
 }
 
 // spectral_analysis.c:36-66 and :69-96 (max_k from k2[last]: quirk Q7)
@@ -635,6 +728,8 @@ struct NsdContext {
     DevScalars* sc = nullptr;
     double* stH[4] = {nullptr, nullptr, nullptr, nullptr};
     double* stR[4] = {nullptr, nullptr, nullptr, nullptr};
+    double* pin = nullptr;                  // pinned staging of small grids' host arrays
+    bool pin_failed = false;
     int* fmodes = nullptr;
     int* fpartner = nullptr;
     double* fou = nullptr;
@@ -695,6 +790,31 @@ int sync(NsdContext* c) {
     CK(hipStreamSynchronize(c->stream));
     return ST_OK;
 }
+// Host arrays of small grids go through a pinned buffer of the context, which
+// kernels read and write in place: a header, five spectra, three physical fields.
+// The copies of pageable arrays that it replaces are 10 to 20 us each, whatever
+// their size, and there are nine in a step on host arrays.  ns_spectral_advance_rk4
+// at FP64, us: 64^2 293 -> 101, 128^2 360 -> 143, 256^2 495 -> 261, 512^2 1271 -> 954;
+// the CFL step before it 49 -> 23 at 128^2.  At 1024^2 (4.0 ms) the host's own copies
+// out of the buffer would take what the pageable ones do: kPinMost ends at 512^2.
+constexpr size_t kPinHead = 1024;              // doubles
+constexpr size_t kPinMost = (size_t)24 << 20;  // bytes
+bool pinned(NsdContext* c) {
+    const size_t n = kPinHead + 5 * 2 * H_of(c) + 3 * R_of(c);
+    if (c->pin) return true;
+    if (c->pin_failed || c->nb != 1 || n * sizeof(double) > kPinMost) return false;
+    if (hipHostMalloc(&c->pin, n * sizeof(double), hipHostMallocDefault) != hipSuccess) {
+        (void)hipGetLastError();
+        c->pin = nullptr;
+        c->pin_failed = true;
+    }
+    return c->pin != nullptr;
+}
+double* pinH(NsdContext* c, int i) { return c->pin + kPinHead + (size_t)i * 2 * H_of(c); }
+double* pinR(NsdContext* c, int i) {
+    return c->pin + kPinHead + 5 * 2 * H_of(c) + (size_t)i * R_of(c);
+}
+
 int lastk(NsdContext* c) {
     CK(hipGetLastError());
     return ST_OK;
@@ -1212,6 +1332,56 @@ int op_state_derived(NsdContext* c, double* psi_hat, double* u_hat, double* v_ha
     return sync(c);
 }
 
+// One step on host arrays (nsd_host.h).
+template <typename T>
+int op_host_step(NsdContext* c, NsdHostFields* f) {
+    const size_t hb = 2 * sizeof(double) * H_of(c), rb = sizeof(double) * R_of(c);
+    memcpy(pinH(c, 0), f->omega_hat, hb);
+    if (f->sfd_hat) memcpy(pinH(c, 4), f->sfd_hat, hb);
+    hipLaunchKernelGGL(k_host_in<T>, dim3(grid_for(C_of(c))), dim3(256), 0, c->stream, c->G,
+                       pinH(c, 0), f->sfd_hat ? pinH(c, 4) : nullptr, (cx<T>*)c->state,
+                       (cx<T>*)c->sfd, c->sc, f->t, f->dt, c->phys.dt_hi);
+    int rc = op_prime<T>(c);
+    if (!rc) rc = op_advance_graph<T>(c, 1, 0);
+    if (!rc) {
+        hipLaunchKernelGGL(k_host_out<T>, dim3(grid_for(H_of(c))), dim3(256), 0, c->stream, c->G,
+                           (const cx<T>*)c->state, (const cx<T>*)c->sfd, c->sc, pinH(c, 0),
+                           pinH(c, 1), pinH(c, 2), pinH(c, 3), f->sfd_hat ? pinH(c, 4) : nullptr,
+                           c->pin);
+        // psi_y = u and psi_x = -v lie transformed along y in the mixed buffers;
+        // omega joins them in the J buffer, which holds nothing between steps
+        ColArgs<T> a = col_args<T>(c);
+        a.mode = COL_INV;
+        a.in0 = (const cx<T>*)c->state;
+        a.nout = 1;
+        a.ops[0] = OP_ID0;
+        a.mixed[0] = (cx<T>*)c->nl;
+        launch_col_t<T>(c, a, c->G.nkx_keep);
+        RowArgs<T> r = row_args<T>(c);
+        r.mode = ROW_C2R;
+        r.nfields = 3;
+        r.mixed[0] = (const cx<T>*)c->mixed[1];
+        r.mixed[1] = (const cx<T>*)c->mixed[0];
+        r.mixed[2] = (const cx<T>*)c->nl;
+        r.minus1 = 1;
+        for (int i = 0; i < 3; ++i) r.out_ref[i] = pinR(c, i);
+        launch_row_t<T>(c, r, c->G.ny);
+        rc = lastk(c);
+    }
+    if (sync(c) || rc) return rc ? rc : ST_MEM;
+    f->t = c->pin[0];
+    f->dt = c->pin[1];
+    f->status = (int)c->pin[2];
+    if (f->status) return ST_OK;
+    double* const spec[5] = {f->omega_hat, f->psi_hat, f->u_hat, f->v_hat, f->sfd_hat};
+    for (int i = 0; i < 5; ++i)
+        if (spec[i]) memcpy(spec[i], pinH(c, i), hb);
+    double* const phys[3] = {f->u, f->v, f->omega};
+    for (int i = 0; i < 3; ++i)
+        if (phys[i]) memcpy(phys[i], pinR(c, i), rb);
+    return ST_OK;
+}
+
 // E and Z of every member: out[2 m], out[2 m + 1]
 template <typename T>
 int op_state_energy(NsdContext* c, double* out) {
@@ -1630,6 +1800,7 @@ void nsd_destroy(NsdContext* c) {
                     c->cl_m, c->cl_y, c->cl_src, c->ec_prev, c->ec_ymid, c->ec_part};
     for (void* b : bufs)
         if (b) (void)hipFree(b);
+    if (c->pin) (void)hipHostFree(c->pin);
     if (c->stream) (void)hipStreamDestroy(c->stream);
     delete c;
 }
@@ -1880,6 +2051,15 @@ int nsd_advance_graph(NsdContext* c, int nsteps, int adaptive) {
     if (!c || nsteps < 0) return ST_PARAM;
     if (nsteps == 0) return ST_OK;
     return TYPED(op_advance_graph, c, nsteps, adaptive ? 1 : 0);
+}
+
+int nsd_host_step_fits(NsdContext* c) {
+    return c && !pairs_ok(c) && pinned(c) ? 1 : 0;
+}
+
+int nsd_host_step(NsdContext* c, NsdHostFields* f) {
+    if (!c || !f || !f->omega_hat || !nsd_host_step_fits(c)) return ST_PARAM;
+    return TYPED(op_host_step, c, f);
 }
 
 int nsd_state_derived(NsdContext* c, double* psi_hat, double* u_hat, double* v_hat, double* u,
@@ -2323,6 +2503,30 @@ int nsd_phys_reduce(NsdContext* c, const double* u, const double* v, const doubl
                     double out[3]) {
     if (!c || !out) return ST_PARAM;
     const size_t rb = sizeof(double) * R_of(c);
+    if (pinned(c)) {
+        const double* in[3] = {u, v, w};
+        const double* at[3] = {nullptr, nullptr, nullptr};
+        for (int i = 0; i < 3; ++i)
+            if (in[i]) {
+                memcpy(pinR(c, i), in[i], rb);
+                at[i] = pinR(c, i);
+            }
+        const unsigned parts = std::min(grid_for(R_of(c)), (unsigned)(kPinHead / 3));
+        hipLaunchKernelGGL(k_phys_parts, dim3(parts), dim3(256), 0, c->stream, R_of(c), at[0], at[1],
+                           at[2], c->pin);
+        if (lastk(c) || sync(c)) return ST_MEM;
+        unsigned long long m = 0;
+        out[1] = out[2] = 0.0;
+        for (unsigned i = 0; i < parts; ++i) {
+            unsigned long long b;
+            memcpy(&b, &c->pin[3 * i], sizeof(b));
+            m = std::max(m, b);
+            out[1] += c->pin[3 * i + 1];
+            out[2] += c->pin[3 * i + 2];
+        }
+        memcpy(&out[0], &m, sizeof(double));
+        return ST_OK;
+    }
     if (ensure_staging(c) || up(c, c->stR[0], u, rb) || up(c, c->stR[1], v, rb) ||
         up(c, c->stR[2], w, rb))
         return ST_MEM;

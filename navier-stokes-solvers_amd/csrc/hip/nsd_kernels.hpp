@@ -1379,6 +1379,7 @@ struct RowArgs {
     cx<T>* nl;             // ROW_STAGE / ROW_R2C output (mixed)
     double* out_ref[4];    // ROW_C2R outputs (FP64 [ny][nx]) if non-null
     T* out[4];             // ROW_C2R outputs (T [ny][nx]) otherwise
+    int minus1;            // ROW_C2R: out_ref[1] negated
     const double* in_ref;  // ROW_R2C input (FP64 [ny][nx])
     const T* in_t;         // ROW_R2C input at the working precision (instead of in_ref)
     DevScalars* sc;
@@ -1812,7 +1813,8 @@ __global__ __launch_bounds__(NT, MW) void k_row(RowArgs<T> a) {
                             unsigned short, (__bf16)(a.out_bf16_scale * v[s].x));
                     else a.out[f][roff + o] = v[s].x;
                     if (B) {
-                        if (a.out_ref[f + 1]) a.out_ref[f + 1][o] = double(v[s].y);
+                        if (a.out_ref[f + 1])
+                            a.out_ref[f + 1][o] = double(f == 0 && a.minus1 ? -v[s].y : v[s].y);
                         else a.out[f + 1][roff + o] = v[s].y;
                     }
                 }

@@ -11,6 +11,7 @@
 #include <stdint.h>
 
 #include "ns_device.h"
+#include "nsd_host.h"
 #include "spectral_internal.h"
 
 static struct ns_fft_plan_s { int unused; } ns_plan_token;
@@ -223,7 +224,29 @@ void ns_spectral_compute_nonlinear_terms(NSSpectralData *d) {
 
 void ns_spectral_advance_rk4(NSSpectralData *d) {
     if (!ready(d)) return;
-    int rc = ns_spectral_sync_device(d);
+    int rc = sync_params(d);
+    if (rc == 0 && nsd_host_step_fits(d->device->ctx)) {
+        NsdHostFields f = {(double *)d->omega_hat,
+                           d->hyperviscosity.sfd_enabled ? (double *)d->sfd_hat : NULL,
+                           (double *)d->psi_hat,
+                           (double *)d->u_hat,
+                           (double *)d->v_hat,
+                           d->u,
+                           d->v,
+                           d->omega,
+                           d->t,
+                           d->dt,
+                           0};
+        rc = nsd_host_step(d->device->ctx, &f);
+        if (rc == 0) {
+            d->t = f.t;
+            d->dt = f.dt;
+            rc = f.status;
+        }
+        set_status(d, rc);
+        return;
+    }
+    if (rc == 0) rc = ns_spectral_sync_device(d);
     if (rc == 0) rc = ns_spectral_advance_n(d, 1, 0);
     if (rc == 0) rc = ns_spectral_sync_host(d);
     set_status(d, rc);
