@@ -78,6 +78,8 @@ enum ConvMode { CONV_FWD_GELU = 0, CONV_FWD_LAST = 1, CONV_BWD_DATA = 2 };
 struct ConvArgs {
     int n, lg, npix;
     const bf16* in;     // A source: [batch][npix][KC]
+    const float* in32;  // input layer: FP32 source times in32_scale instead (k_conv_tile)
+    float in32_scale;
     const bf16* w;      // layer weights, bf16 [cout][9][cin]
     const float* bias;  // [NN] (forward)
     bf16* z;            // forward: pre-activations [batch][npix][NN] (null: not kept)
@@ -188,146 +190,125 @@ void launch_conv(const ConvArgs& a, int batch, hipStream_t st) {
                            a);
 }
 
-// Layers from an LDS-staged input patch (forward, and the input gradient,
-// whose A operand is dZ shifted the other way).  A workgroup of 512
-// threads computes a tile of 8 rows x 64 pixels of one member: it stages the
-// tile's input with its one-pixel periodic halo (10 x 66 pixels, all KC
-// channels) in LDS with coalesced 16-byte loads issued together, holds its
-// part of the transposed weights in registers, and then each wave (one tile
-// row, four blocks of 16 pixels) reads every tap's A operand from LDS.
-// k_conv reloads each pixel's neighbourhood from global memory for each tap,
-// a chain of dependent loads per 16-pixel tile.  Same GEMM, lane layouts and
-// epilogue as k_conv; n must be a multiple of 64.
+// The tiled kernels compute D[channel][pixel] (weights as the A operand).  Row
+// 4 q + i of 16-channel block nb is channel 8 q + 4 nb + i: lane (m, kq) then ends
+// with channels 8 kq .. 8 kq + 7 of pixel m, 16 contiguous bytes, and a wave's
+// 16 pixels are 1 KB that leaves (or, for the input gradient's pre-activations,
+// arrives) as one coalesced access.  Weight row m of block nb is this channel:
+__device__ __forceinline__ int tile_channel(int nb, int m) { return 8 * (m >> 2) + 4 * nb + (m & 3); }
+
+__device__ __forceinline__ unsigned pack2(float x0, float x1) {
+    return (unsigned)f2bf(x0) | ((unsigned)f2bf(x1) << 16);
+}
+__device__ __forceinline__ uint4 pack8(const float (&x)[8]) {
+    return uint4{pack2(x[0], x[1]), pack2(x[2], x[3]), pack2(x[4], x[5]), pack2(x[6], x[7])};
+}
+// acc times gelu'(z), z: the eight pre-activations of one pixel
+__device__ __forceinline__ uint4 dgelu8(const f4 (&acc)[2], uint4 z) {
+    const unsigned zw[4] = {z.x, z.y, z.z, z.w};
+    float d[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+        d[i] = acc[i >> 2][i & 3] * gelu_d(bf2f((bf16)(zw[i >> 1] >> (16 * (i & 1)))));
+    return pack8(d);
+}
+
+// Layers with one input channel from an LDS-staged patch: the input layer
+// (forward) and the output layer's input gradient, whose A operand is dZ shifted
+// the other way.  A workgroup of 512 threads computes a tile of 8 rows x 64 pixels
+// of one member: it stages the tile's input with its one-pixel periodic halo
+// (10 x 66 pixels) in LDS, holds the weights in registers, and each wave (one tile
+// row, four blocks of 16 pixels) picks every tap from LDS.  n must be a multiple
+// of 64.  Bound by the 32-channel arrays that it writes (and reads).
 constexpr int kTileRows = 8, kTileCols = 64;
 
-template <int KC, int NN, int MODE>
+template <int MODE>
 __global__ __launch_bounds__(512) void k_conv_tile(ConvArgs a) {
     static_assert(kTileRows * 64 == 512, "one wave per tile row");
     constexpr int S = MODE == CONV_BWD_DATA ? -1 : 1;  // tap offsets applied to the input
-    constexpr int KP = (9 * KC + 31) / 32 * 32;
-    constexpr int NP = (NN + 15) / 16 * 16;
-    constexpr int PR = kTileRows + 2, PC = kTileCols + 2;
-    __shared__ __align__(16) bf16 Bt[NP * KP];
-    __shared__ __align__(16) bf16 Xs[PR * PC * KC];
-    const int tid = threadIdx.x;
+    constexpr int NN = 32;
+    constexpr int PR = kTileRows + 2, PC = kTileCols + 2, NBLK = kTileCols / 16;
+    __shared__ bf16 Xs[PR * PC];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int m = lane & 15, kq = lane >> 4;
     const int tiles_x = a.n / kTileCols;
     const int r0 = (blockIdx.x / tiles_x) * kTileRows, c0 = (blockIdx.x % tiles_x) * kTileCols;
     const size_t boff = (size_t)blockIdx.y * a.npix;
     const int nm = a.n - 1;
-    // input patch: Xs[(r PC + c) KC + ch] = in[(r0 + r - 1, c0 + c - 1) mod n][ch]
-    if constexpr (KC % 8 == 0) {
-        constexpr int CH = KC / 8;  // 16-byte pieces per pixel
-#pragma unroll 4
-        for (int e = tid; e < PR * PC * CH; e += 512) {
-            const int pix = e / CH, q = e - pix * CH;
-            const int r = pix / PC, c = pix - r * PC;
-            const int gy = (r0 + r - 1) & nm, gx = (c0 + c - 1) & nm;
-            const s8 v = *reinterpret_cast<const s8*>(
-                a.in + (boff + ((size_t)gy << a.lg) + gx) * KC + 8 * q);
-            *reinterpret_cast<s8*>(&Xs[pix * KC + 8 * q]) = v;
-        }
-    } else {
-        for (int e = tid; e < PR * PC * KC; e += 512) {
-            const int pix = e / KC, q = e - pix * KC;
-            const int r = pix / PC, c = pix - r * PC;
-            const int gy = (r0 + r - 1) & nm, gx = (c0 + c - 1) & nm;
-            Xs[e] = a.in[(boff + ((size_t)gy << a.lg) + gx) * KC + q];
-        }
+    // this lane's pixel in block 0 of its wave's row
+    const size_t q0 = boff + ((size_t)(r0 + wave) << a.lg) + c0 + m;
+    uint4 zp[NBLK];
+    if constexpr (MODE == CONV_BWD_DATA) {
+#pragma unroll
+        for (int b = 0; b < NBLK; ++b)
+            zp[b] = *reinterpret_cast<const uint4*>(&a.zprev[(q0 + 16 * b) * NN + 8 * kq]);
     }
-    for (int e = tid; e < NP * KP; e += 512) {
-        const int nn = e / KP, k = e % KP;
-        bf16 v = 0;
-        if (nn < NN && k < 9 * KC) {
-            const int tap = k / KC, kc = k % KC;
-            v = MODE == CONV_BWD_DATA ? a.w[(kc * 9 + tap) * NN + nn] : a.w[(nn * 9 + tap) * KC + kc];
+    // input patch: Xs[r PC + c] = in[(r0 + r - 1, c0 + c - 1) mod n]
+    for (int e = tid; e < PR * PC; e += 512) {
+        const int r = e / PC, c = e - r * PC;
+        const int gy = (r0 + r - 1) & nm, gx = (c0 + c - 1) & nm;
+        const size_t q = boff + ((size_t)gy << a.lg) + gx;
+        if (MODE == CONV_FWD_GELU && a.in32) Xs[e] = f2bf(a.in32_scale * a.in32[q]);
+        else Xs[e] = a.in[q];
+    }
+    s8 bv[2];
+    f4 bias4[2];
+#pragma unroll
+    for (int nb = 0; nb < 2; ++nb) {
+        const int nn = tile_channel(nb, m);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const int tap = 8 * kq + i;
+            bv[nb][i] = tap >= 9 ? 0 : (short)(MODE == CONV_BWD_DATA ? a.w[tap * NN + nn] : a.w[nn * 9 + tap]);
         }
-        Bt[e] = v;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            bias4[nb][i] = MODE == CONV_BWD_DATA ? 0.f : a.bias[8 * kq + 4 * nb + i];
     }
     __syncthreads();
-    const int lane = tid & 63, wave = tid >> 6;
-    const int m = lane & 15, kq = lane >> 4;
-    // this lane's B operands for the whole tile
-    s8 bv[KP / 32][NP / 16];
 #pragma unroll
-    for (int c = 0; c < KP / 32; ++c)
+    for (int b = 0; b < NBLK; ++b) {
+        s8 av;
 #pragma unroll
-        for (int nb = 0; nb < NP / 16; ++nb)
-            bv[c][nb] = *reinterpret_cast<const s8*>(&Bt[(nb * 16 + m) * KP + c * 32 + 8 * kq]);
-    const int lr = wave;  // tile row of this wave
-#pragma unroll 1
-    for (int blk = 0; blk < kTileCols / 16; ++blk) {
-        const int lc = blk * 16;
-        f4 acc[NP / 16];
-#pragma unroll
-        for (int nb = 0; nb < NP / 16; ++nb) acc[nb] = f4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int c = 0; c < KP / 32; ++c) {
-            const int k0 = c * 32 + 8 * kq;  // A lane l: row l % 16, k = 8 (l / 16) + i
-            s8 av;
-            if constexpr (KC % 32 == 0) {
-                const int tap = k0 / KC, kc = k0 % KC;
-                const int pr = lr + 1 + S * (tap / 3 - 1), pc = lc + m + 1 + S * (tap % 3 - 1);
-                av = *reinterpret_cast<const s8*>(&Xs[(pr * PC + pc) * KC + kc]);
-            } else {
-#pragma unroll
-                for (int i = 0; i < 8; ++i) {
-                    const int k = k0 + i;
-                    short v = 0;
-                    if (k < 9 * KC) {
-                        const int tap = k / KC, kc = k % KC;
-                        const int pr = lr + 1 + S * (tap / 3 - 1),
-                                  pc = lc + m + 1 + S * (tap % 3 - 1);
-                        v = (short)Xs[(pr * PC + pc) * KC + kc];
-                    }
-                    av[i] = v;
-                }
-            }
-#pragma unroll
-            for (int nb = 0; nb < NP / 16; ++nb) {
-                if constexpr (MODE == CONV_FWD_LAST)  // D[channel][pixel]
-                    acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                        __builtin_bit_cast(bf8, bv[c][nb]), __builtin_bit_cast(bf8, av), acc[nb], 0,
-                        0, 0);
-                else  // D[pixel][channel]
-                    acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                        __builtin_bit_cast(bf8, av), __builtin_bit_cast(bf8, bv[c][nb]), acc[nb], 0,
-                        0, 0);
-            }
+        for (int i = 0; i < 8; ++i) {  // lane: pixel m, taps 8 kq + i
+            const int tap = 8 * kq + i;
+            short v = 0;
+            if (tap < 9)
+                v = (short)Xs[(wave + 1 + S * (tap / 3 - 1)) * PC + 16 * b + m + 1 + S * (tap % 3 - 1)];
+            av[i] = v;
         }
-        const size_t q0 = boff + ((size_t)(r0 + lr) << a.lg) + c0 + lc;  // pixel of block column 0
-        if constexpr (MODE == CONV_FWD_LAST) {
-            if (kq == 0) a.y[q0 + m] = (acc[0][0] + a.bias[0]) * a.yscale;
+        f4 acc[2];
+#pragma unroll
+        for (int nb = 0; nb < 2; ++nb)
+            acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                __builtin_bit_cast(bf8, bv[nb]), __builtin_bit_cast(bf8, av), f4{0.f, 0.f, 0.f, 0.f},
+                0, 0, 0);
+        const size_t o = (q0 + 16 * b) * NN + 8 * kq;
+        if constexpr (MODE == CONV_BWD_DATA) {
+            *reinterpret_cast<uint4*>(&a.dzprev[o]) = dgelu8(acc, zp[b]);
         } else {
+            float zz[8], g[8];
 #pragma unroll
-            for (int nb = 0; nb < NP / 16; ++nb) {
-                const int nn = nb * 16 + m;
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const size_t q = q0 + 4 * kq + i;
-                    if (nn < NN) {
-                        if constexpr (MODE == CONV_BWD_DATA) {
-                            a.dzprev[q * NN + nn] =
-                                f2bf(acc[nb][i] * gelu_d(bf2f(a.zprev[q * NN + nn])));
-                        } else {
-                            const float zz = acc[nb][i] + a.bias[nn];
-                            if (a.z) a.z[q * NN + nn] = f2bf(zz);
-                            a.act[q * NN + nn] = f2bf(gelu(zz));
-                        }
-                    }
-                }
+            for (int i = 0; i < 8; ++i) {
+                zz[i] = acc[i >> 2][i & 3] + bias4[i >> 2][i & 3];
+                g[i] = gelu(zz[i]);
             }
+            if (a.z) *reinterpret_cast<uint4*>(&a.z[o]) = pack8(zz);
+            *reinterpret_cast<uint4*>(&a.act[o]) = pack8(g);
         }
     }
 }
 
 // 32-channel layers, persistent: two workgroups per CU walk the 8 x 32-pixel
-// tiles of all members.  A workgroup stages the layer's weights once (held
-// in registers, as in k_conv_tile) and keeps two LDS patches of 10 x 34
-// pixels: while it computes one tile from one patch, the next tile's patch
-// streams into the other with global_load_lds_dwordx4 (each lane's 16 bytes
-// land at the wave's LDS base + 16 x lane, which is the patch's own order of
-// 16-byte pieces), so no register holds it and one barrier per tile serves
-// both the reads of the old patch and the arrival of the new one.
+// tiles of all members.  A workgroup loads the layer's weights into registers
+// once and keeps two LDS patches of 10 x 34 pixels: while it computes one tile
+// from one patch, the next tile's patch streams into the other with
+// global_load_lds_dwordx4 (each lane's 16 bytes land at the wave's LDS base +
+// 16 x lane, which is the patch's own order of 16-byte pieces), so no register
+// holds it and one barrier per tile serves both the reads of the old patch and
+// the arrival of the new one.  The input gradient's pre-activations of the next
+// tile travel with its patch.  The wait before the barrier leaves the tile's own
+// stores in flight.
 constexpr int kT2Cols = 32;
 
 __device__ __forceinline__ void g2lds16(const void* g, bf16* lds_wave_base) {
@@ -335,8 +316,23 @@ __device__ __forceinline__ void g2lds16(const void* g, bf16* lds_wave_base) {
                                      0, 0);
 }
 
+// s_waitcnt until at most N vector-memory operations are in flight
+template <int N>
+__device__ __forceinline__ void wait_vm() {
+    static_assert(N < 16, "low four bits of the count");
+    __builtin_amdgcn_s_waitcnt(0x0f70 | N);
+}
+
+// workgroup barrier alone: __syncthreads() would also wait for every store, which
+// nobody in the workgroup reads (its LDS accesses before here have all returned)
+__device__ __forceinline__ void barrier_only() {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+
 template <int NN, int MODE>
-__global__ __launch_bounds__(512) void k_conv_tile2(ConvArgs a, int ntiles) {
+__global__ __launch_bounds__(512, 4) void k_conv_tile2(ConvArgs a, int ntiles) {
     constexpr int KC = 32;
     constexpr int S = MODE == CONV_BWD_DATA ? -1 : 1;
     constexpr int KP = 9 * KC;
@@ -344,33 +340,32 @@ __global__ __launch_bounds__(512) void k_conv_tile2(ConvArgs a, int ntiles) {
     constexpr int PR = kTileRows + 2, PC = kT2Cols + 2;
     constexpr int NPC = PR * PC * (KC / 8);  // 16-byte pieces per patch
     constexpr int PER = (NPC + 511) / 512;
-    __shared__ __align__(16) bf16 Bt[NP * KP];
+    constexpr int NBLK = kT2Cols / 16;
+    static_assert(MODE == CONV_FWD_LAST ? NN == 1 : NN == 32, "layers of this network");
     // two distinct arrays (not one of two rows): the compiler's wait for the
     // patch loads in flight then covers reads of the patch being loaded only
     __shared__ __align__(16) bf16 X0[PR * PC * KC];
     __shared__ __align__(16) bf16 X1[PR * PC * KC];
+    // pre-activations of a tile: each lane's own 16 bytes per block
+    constexpr int ZN = MODE == CONV_BWD_DATA ? 8 * NBLK * 64 * 8 : 8;
+    __shared__ __align__(16) bf16 Z0[ZN];
+    __shared__ __align__(16) bf16 Z1[ZN];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int m = lane & 15, kq = lane >> 4;
     const int tiles_x = a.n / kT2Cols, per_mem = tiles_x * (a.n / kTileRows);
     const int nm = a.n - 1;
-    for (int e = tid; e < NP * KP; e += 512) {
-        const int nn = e / KP, k = e % KP;
-        bf16 v = 0;
-        if (nn < NN) {
-            const int tap = k / KC, kc = k % KC;
-            v = MODE == CONV_BWD_DATA ? a.w[(kc * 9 + tap) * NN + nn] : a.w[(nn * 9 + tap) * KC + kc];
-        }
-        Bt[e] = v;
-    }
     // patch of tile t into buffer b: piece e = pixel (r PC + c), channel group e % 4
     auto issue = [&](int t, bf16* Xd) {
         const int mem = t / per_mem, rem = t - mem * per_mem;
         const int r0 = (rem / tiles_x) * kTileRows, c0 = (rem % tiles_x) * kT2Cols;
         const size_t boff = (size_t)mem * a.npix;
+        int l = lane;  // opaque: the pieces' rows and columns again per tile, not held
+        asm volatile("" : "+v"(l));
 #pragma unroll
         for (int i = 0; i < PER; ++i) {
             const int e0 = 512 * i + 64 * wave;  // this wave's first piece
             if (e0 < NPC) {
-                const int e = e0 + lane;
+                const int e = e0 + l;
                 if (e < NPC) {
                     const int pix = e >> 2, q = e & 3;
                     const int r = pix / PC, c = pix - r * PC;
@@ -380,39 +375,70 @@ __global__ __launch_bounds__(512) void k_conv_tile2(ConvArgs a, int ntiles) {
             }
         }
     };
+    // this lane's pixel in block 0 of its wave's row of tile t
+    auto pixel = [&](int t) {
+        const int mem = t / per_mem, rem = t - mem * per_mem;
+        const int r0 = (rem / tiles_x) * kTileRows, c0 = (rem % tiles_x) * kT2Cols;
+        return (size_t)mem * a.npix + ((size_t)(r0 + wave) << a.lg) + c0 + m;
+    };
     int t = blockIdx.x;
-    if (t < ntiles) issue(t, X0);
-    __builtin_amdgcn_s_waitcnt(0);
-    __syncthreads();
-    const int m = lane & 15, kq = lane >> 4;
+    if (t >= ntiles) return;
+    // weights: row m of block nb, 8 input channels 8 kq .. of each tap
     s8 bv[KP / 32][NP / 16];
+    if constexpr (MODE == CONV_BWD_DATA) {
+        // w[kc][tap][nn] transposed through the patch buffers
+        static_assert(NP * KP <= PR * PC * KC, "the weights fit a patch buffer");
+        for (int e = tid; e < KP * NN / 8; e += 512) {
+            const int row = e >> 2, tap = row % 9, kc = row / 9, n0 = 8 * (e & 3);
+            const s8 v = *reinterpret_cast<const s8*>(&a.w[row * NN + n0]);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) X0[(n0 + i) * KP + tap * KC + kc] = (bf16)v[i];
+        }
+        __syncthreads();
+    }
 #pragma unroll
     for (int c = 0; c < KP / 32; ++c)
 #pragma unroll
-        for (int nb = 0; nb < NP / 16; ++nb)
-            bv[c][nb] = *reinterpret_cast<const s8*>(&Bt[(nb * 16 + m) * KP + c * 32 + 8 * kq]);
-    const int lr = wave;
+        for (int nb = 0; nb < NP / 16; ++nb) {
+            const int nn = NN == 32 ? tile_channel(nb, m) : m;
+            bv[c][nb] = s8{0, 0, 0, 0, 0, 0, 0, 0};
+            if (nn < NN)
+                bv[c][nb] = *reinterpret_cast<const s8*>(
+                    (MODE == CONV_BWD_DATA ? X0 : a.w) + nn * KP + c * 32 + 8 * kq);
+        }
     // biases in registers: a global load in the loop would wait for the
     // patch loads in flight (the vector memory counter retires in order)
-    // Both forward modes compute D[channel][pixel] (weights as the A
-    // operand): a lane then holds channels 4 kq .. 4 kq + 3 of one pixel, which
-    // leave as one 8-byte store.
     f4 bias4[NP / 16];
 #pragma unroll
     for (int nb = 0; nb < NP / 16; ++nb)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            const int nn = nb * 16 + 4 * kq + i;
+            const int nn = NN == 32 ? 8 * kq + 4 * nb + i : 4 * kq + i;
             bias4[nb][i] = MODE == CONV_BWD_DATA || nn >= NN ? 0.f : a.bias[nn];
         }
+    if constexpr (MODE == CONV_BWD_DATA) __syncthreads();
+    issue(t, X0);
+    auto zissue = [&](int t, bf16* Zd) {
+        const bf16* z = a.zprev + pixel(t) * NN + 8 * kq;
+#pragma unroll
+        for (int b = 0; b < NBLK; ++b) g2lds16(z + 16 * b * NN, Zd + (wave * NBLK + b) * 64 * 8);
+    };
+    if constexpr (MODE == CONV_BWD_DATA) zissue(t, Z0);
+    wait_vm<0>();
+    __syncthreads();
     // one tile from patch X while the next tile's patch streams into Xn
-    auto step = [&](int t, const bf16* X, bf16* Xn) {
-        if (t + (int)gridDim.x < ntiles) issue(t + gridDim.x, Xn);
-        const int mem = t / per_mem, rem = t - mem * per_mem;
-        const int r0 = (rem / tiles_x) * kTileRows, c0 = (rem % tiles_x) * kT2Cols;
-        const size_t boff = (size_t)mem * a.npix;
-#pragma unroll 1
-        for (int blk = 0; blk < kT2Cols / 16; ++blk) {
+    auto step = [&](int t, const bf16* X, bf16* Xn, const bf16* Z, bf16* Zn) {
+        if (t + (int)gridDim.x < ntiles) {
+            issue(t + gridDim.x, Xn);
+            if constexpr (MODE == CONV_BWD_DATA) zissue(t + gridDim.x, Zn);
+        }
+        const size_t q0 = pixel(t);
+        float yv = 0.f;
+        // unrolled, so that the compiler can count the stores behind the patch loads;
+        // one block at a time, for its registers
+#pragma unroll
+        for (int blk = 0; blk < NBLK; ++blk) {
+            __builtin_amdgcn_sched_barrier(0);
             const int lc = blk * 16;
             f4 acc[NP / 16];
 #pragma unroll
@@ -420,72 +446,50 @@ __global__ __launch_bounds__(512) void k_conv_tile2(ConvArgs a, int ntiles) {
 #pragma unroll
             for (int c = 0; c < KP / 32; ++c) {  // one tap of 32 channels per MFMA
                 const int tap = c, kc = 8 * kq;
-                const int pr = lr + 1 + S * (tap / 3 - 1), pc = lc + m + 1 + S * (tap % 3 - 1);
+                const int pr = wave + 1 + S * (tap / 3 - 1), pc = lc + m + 1 + S * (tap % 3 - 1);
                 const s8 av = *reinterpret_cast<const s8*>(&X[(pr * PC + pc) * KC + kc]);
 #pragma unroll
-                for (int nb = 0; nb < NP / 16; ++nb) {
-                    if constexpr (MODE != CONV_BWD_DATA)  // D[channel][pixel]
-                        acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                            __builtin_bit_cast(bf8, bv[c][nb]), __builtin_bit_cast(bf8, av),
-                            acc[nb], 0, 0, 0);
-                    else  // D[pixel][channel]
-                        acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                            __builtin_bit_cast(bf8, av), __builtin_bit_cast(bf8, bv[c][nb]),
-                            acc[nb], 0, 0, 0);
-                }
+                for (int nb = 0; nb < NP / 16; ++nb)
+                    acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                        __builtin_bit_cast(bf8, bv[c][nb]), __builtin_bit_cast(bf8, av), acc[nb], 0,
+                        0, 0);
             }
-            const size_t q0 = boff + ((size_t)(r0 + lr) << a.lg) + c0 + lc;
             if constexpr (MODE == CONV_FWD_LAST) {
-                // D[row = channel 4 kq + i][col = pixel m]: channel 0 in lanes 0..15
-                if (kq == 0) a.y[q0 + m] = (acc[0][0] + bias4[0][0]) * a.yscale;
-            } else if constexpr (MODE == CONV_FWD_GELU) {
-                const size_t q = q0 + m;  // this lane's pixel
-#pragma unroll
-                for (int nb = 0; nb < NP / 16; ++nb) {
-                    const int cb = nb * 16 + 4 * kq;  // its first channel
-                    if (cb < NN) {
-                        float zz[4], g[4];
-#pragma unroll
-                        for (int i = 0; i < 4; ++i) {
-                            zz[i] = acc[nb][i] + bias4[nb][i];
-                            g[i] = gelu(zz[i]);
-                        }
-                        auto pack = [](float x0, float x1) {
-                            return (unsigned)f2bf(x0) | ((unsigned)f2bf(x1) << 16);
-                        };
-                        if (a.z)
-                            *reinterpret_cast<uint2*>(&a.z[q * NN + cb]) =
-                                uint2{pack(zz[0], zz[1]), pack(zz[2], zz[3])};
-                        *reinterpret_cast<uint2*>(&a.act[q * NN + cb]) =
-                            uint2{pack(g[0], g[1]), pack(g[2], g[3])};
-                    }
-                }
+                // channel 0 in lanes 0..15: block blk's pixels to the lanes of kq = blk
+                const float v = __shfl((acc[0][0] + bias4[0][0]) * a.yscale, m);
+                if (blk == (kq & 1)) yv = v;
             } else {
+                const size_t o = (q0 + lc) * NN + 8 * kq;
+                if constexpr (MODE == CONV_BWD_DATA) {
+                    *reinterpret_cast<uint4*>(&a.dzprev[o]) = dgelu8(
+                        acc, *reinterpret_cast<const uint4*>(&Z[((wave * NBLK + blk) * 64 + lane) * 8]));
+                } else {
+                    float zz[8], g[8];
 #pragma unroll
-                for (int nb = 0; nb < NP / 16; ++nb) {
-                    const int nn = nb * 16 + m;
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        const size_t q = q0 + 4 * kq + i;
-                        if (nn < NN) {
-                            if constexpr (MODE == CONV_BWD_DATA) {
-                                a.dzprev[q * NN + nn] =
-                                    f2bf(acc[nb][i] * gelu_d(bf2f(a.zprev[q * NN + nn])));
-                            }
-                        }
+                    for (int i = 0; i < 8; ++i) {
+                        zz[i] = acc[i >> 2][i & 3] + bias4[i >> 2][i & 3];
+                        g[i] = gelu(zz[i]);
                     }
+                    if (a.z) *reinterpret_cast<uint4*>(&a.z[o]) = pack8(zz);
+                    *reinterpret_cast<uint4*>(&a.act[o]) = pack8(g);
                 }
             }
         }
-        // the next patch has arrived and every read of this one is done
-        __builtin_amdgcn_s_waitcnt(0);
-        __syncthreads();
+        // one store of every lane (lanes 32.. repeat lanes 0..31)
+        if constexpr (MODE == CONV_FWD_LAST) {
+            static_assert(NBLK == 2, "two blocks in a tile row");
+            a.y[q0 + 16 * (kq & 1)] = yv;
+        }
+        // the next patch has arrived (this tile's stores are younger than it) and
+        // every read of this one is done
+        wait_vm<MODE == CONV_FWD_LAST ? 1 : NBLK>();
+        barrier_only();
     };
     while (t < ntiles) {
-        step(t, X0, X1);
+        step(t, X0, X1, Z0, Z1);
         t += gridDim.x;
         if (t >= ntiles) break;
-        step(t, X1, X0);
+        step(t, X1, X0, Z1, Z0);
         t += gridDim.x;
     }
 }
@@ -502,12 +506,10 @@ int conv_tile2_workgroups() {
     return wg;
 }
 
-// the tiled kernels where the grid is a multiple of their tiles (the input
-// gradient stays on k_conv_tile: its epilogue loads the layer below's
-// pre-activations, which would wait behind the patch in flight)
+// the tiled kernels where the grid is a multiple of their tiles
 template <int KC, int NN, int MODE>
 void launch_conv_lds(const ConvArgs& a, int batch, hipStream_t st) {
-    if constexpr (KC == 32 && MODE != CONV_BWD_DATA) {
+    if constexpr (KC == 32) {
         if (a.n % kT2Cols == 0 && a.n % kTileRows == 0) {
             const int ntiles = (a.n / kT2Cols) * (a.n / kTileRows) * batch;
             hipLaunchKernelGGL((k_conv_tile2<NN, MODE>),
@@ -515,12 +517,15 @@ void launch_conv_lds(const ConvArgs& a, int batch, hipStream_t st) {
                                a, ntiles);
             return;
         }
+    } else {
+        if (a.n % kTileCols == 0) {
+            hipLaunchKernelGGL((k_conv_tile<MODE>),
+                               dim3((a.n / kTileCols) * (a.n / kTileRows), batch), dim3(512), 0, st,
+                               a);
+            return;
+        }
     }
-    if (a.n % kTileCols == 0)
-        hipLaunchKernelGGL((k_conv_tile<KC, NN, MODE>),
-                           dim3((a.n / kTileCols) * (a.n / kTileRows), batch), dim3(512), 0, st, a);
-    else
-        launch_conv<KC, NN, MODE>(a, batch, st);
+    launch_conv<KC, NN, MODE>(a, batch, st);
 }
 
 // dW[co][(tap, ci)] += sum_q dZ[q][co] X[q + off(tap)][ci] over this
@@ -1011,15 +1016,25 @@ unsigned long long splitmix(unsigned long long& s) {
 }
 
 // the layers on `st`, output (times yscale) into y; keep_z keeps the
-// pre-activations for a backward pass
+// pre-activations for a backward pass; x: FP32 input (times in_scale) instead of
+// x0, which is used as workspace where the tiled kernel does not read it itself
 int launch_forward_to(NsdClosure* c, int batch, float* y, float yscale, hipStream_t st,
-                      bool keep_z) {
+                      bool keep_z, const float* x = nullptr) {
     ConvArgs a;
     memset(&a, 0, sizeof(a));
     a.n = c->n;
     a.lg = c->lg;
     a.npix = c->npix;
     a.yscale = yscale;
+    if (x) {
+        if (c->n % kTileCols == 0) {
+            a.in32 = x;
+            a.in32_scale = c->in_scale;
+        } else {
+            hipLaunchKernelGGL(k_to_bf16, dim3(256), dim3(256), 0, st, (size_t)batch * c->npix, x,
+                               c->in_scale, c->x0);
+        }
+    }
     for (int l = 0; l < kLayers; ++l) {
         a.in = l == 0 ? c->x0 : c->act[l - 1];
         a.w = c->wb + c->bwoff[l];
@@ -1407,9 +1422,7 @@ int nsd_closure_train(NsdClosure* c, int count, int epochs, int batch, double lr
 int nsd_closure_eval_batch(NsdClosure* c, const float* x, float* y, int batch, void* stream) {
     if (!c || !x || !y || batch < 1 || batch > c->max_batch) return 4;
     hipStream_t st = (hipStream_t)stream;
-    hipLaunchKernelGGL(k_to_bf16, dim3(256), dim3(256), 0, st, (size_t)batch * c->npix, x,
-                       c->in_scale, c->x0);
-    return launch_forward_to(c, batch, y, c->out_scale, st, false);
+    return launch_forward_to(c, batch, y, c->out_scale, st, false, x);
 }
 
 int nsd_closure_eval_device(NsdClosure* c, const float* x, float* y, void* stream) {
