@@ -57,7 +57,8 @@ __device__ __forceinline__ bf16 f2bf(float f) { return __builtin_bit_cast(bf16, 
 // 2 c (1 + 3 a z^2) with s = sigma(2u).
 __device__ __forceinline__ float sig2u(float z) {
     const float u = 0.7978845608028654f * (z + 0.044715f * z * z * z);
-    return __builtin_amdgcn_rcpf(1.f + __expf(-2.f * u));
+    // e^(-2u) as 2^(u (-2 log2 e)): the factor 2 is exact, so this is __expf(-2u)
+    return __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(u * (-2.f * 1.44269504f)));
 }
 __device__ __forceinline__ float gelu(float z) { return z * sig2u(z); }
 __device__ __forceinline__ float gelu_d(float z) {
@@ -197,8 +198,10 @@ void launch_conv(const ConvArgs& a, int batch, hipStream_t st) {
 // arrives) as one coalesced access.  Weight row m of block nb is this channel:
 __device__ __forceinline__ int tile_channel(int nb, int m) { return 8 * (m >> 2) + 4 * nb + (m & 3); }
 
-__device__ __forceinline__ unsigned pack2(float x0, float x1) {
-    return (unsigned)f2bf(x0) | ((unsigned)f2bf(x1) << 16);
+__device__ __forceinline__ unsigned pack2(float x0, float x1) {  // one v_cvt_pk_bf16_f32
+    typedef float f2 __attribute__((ext_vector_type(2)));
+    typedef __bf16 b2 __attribute__((ext_vector_type(2)));
+    return __builtin_bit_cast(unsigned, __builtin_convertvector((f2{x0, x1}), b2));
 }
 __device__ __forceinline__ uint4 pack8(const float (&x)[8]) {
     return uint4{pack2(x[0], x[1]), pack2(x[2], x[3]), pack2(x[4], x[5]), pack2(x[6], x[7])};
@@ -308,7 +311,10 @@ __global__ __launch_bounds__(512) void k_conv_tile(ConvArgs a) {
 // holds it and one barrier per tile serves both the reads of the old patch and
 // the arrival of the new one.  The input gradient's pre-activations of the next
 // tile travel with its patch.  The wait before the barrier leaves the tile's own
-// stores in flight.
+// stores in flight.  At 256^2 x 16 (67 MB per 32-channel array): forward 36 us,
+// bound by its vector instructions (GELU: two transcendental and eight others per
+// value) beside 134 MB; input gradient 41 us for 201 MB (106 us as one patch per
+// workgroup with 2-byte accesses).
 constexpr int kT2Cols = 32;
 
 __device__ __forceinline__ void g2lds16(const void* g, bf16* lds_wave_base) {
@@ -350,36 +356,40 @@ __global__ __launch_bounds__(512, 4) void k_conv_tile2(ConvArgs a, int ntiles) {
     constexpr int ZN = MODE == CONV_BWD_DATA ? 8 * NBLK * 64 * 8 : 8;
     __shared__ __align__(16) bf16 Z0[ZN];
     __shared__ __align__(16) bf16 Z1[ZN];
+    __shared__ __align__(16) float Bs[32];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int m = lane & 15, kq = lane >> 4;
     const int tiles_x = a.n / kT2Cols, per_mem = tiles_x * (a.n / kTileRows);
     const int nm = a.n - 1;
-    // patch of tile t into buffer b: piece e = pixel (r PC + c), channel group e % 4
+    // member, first row and column of tile t (uniform)
+    auto corner = [&](int t, int& r0, int& c0) {
+        const int mem = t / per_mem, rem = t - mem * per_mem, ty = rem / tiles_x;
+        r0 = ty * kTileRows;
+        c0 = (rem - ty * tiles_x) * kT2Cols;
+        return (size_t)mem * a.npix;
+    };
+    // patch of tile t into a buffer: piece e = pixel r PC + c, channel group e % 4; 32-bit byte offsets within a member (npix 64 <= 2^30)
     auto issue = [&](int t, bf16* Xd) {
-        const int mem = t / per_mem, rem = t - mem * per_mem;
-        const int r0 = (rem / tiles_x) * kTileRows, c0 = (rem % tiles_x) * kT2Cols;
-        const size_t boff = (size_t)mem * a.npix;
-        int l = lane;  // opaque: the pieces' rows and columns again per tile, not held
-        asm volatile("" : "+v"(l));
+        int r0, c0;
+        const char* in = reinterpret_cast<const char*>(a.in + corner(t, r0, c0) * KC);
 #pragma unroll
         for (int i = 0; i < PER; ++i) {
-            const int e0 = 512 * i + 64 * wave;  // this wave's first piece
-            if (e0 < NPC) {
-                const int e = e0 + l;
-                if (e < NPC) {
-                    const int pix = e >> 2, q = e & 3;
-                    const int r = pix / PC, c = pix - r * PC;
-                    const int gy = (r0 + r - 1) & nm, gx = (c0 + c - 1) & nm;
-                    g2lds16(a.in + (boff + ((size_t)gy << a.lg) + gx) * KC + 8 * q, Xd + 8 * e0);
-                }
+            int e = 512 * i + tid;  // opaque: rows and columns again per tile, not held
+            asm volatile("" : "+v"(e));
+            if (e < NPC) {
+                const unsigned pix = (unsigned)e >> 2, r = (pix * 1928u) >> 16, c = pix - r * PC;
+                static_assert(PC == 34 && NPC / 4 <= 340, "pix / 34 as a multiplication");
+                const int gy = (r0 - 1 + (int)r) & nm, gx = (c0 - 1 + (int)c) & nm;
+                const unsigned off = (((unsigned)(gy << a.lg) + (unsigned)gx) << 6) + 16u * (e & 3);
+                g2lds16(in + off, Xd + 8 * (512 * i + 64 * wave));
             }
         }
     };
     // this lane's pixel in block 0 of its wave's row of tile t
     auto pixel = [&](int t) {
-        const int mem = t / per_mem, rem = t - mem * per_mem;
-        const int r0 = (rem / tiles_x) * kTileRows, c0 = (rem % tiles_x) * kT2Cols;
-        return (size_t)mem * a.npix + ((size_t)(r0 + wave) << a.lg) + c0 + m;
+        int r0, c0;
+        const size_t b = corner(t, r0, c0);
+        return b + (unsigned)(((r0 + wave) << a.lg) + c0 + m);
     };
     int t = blockIdx.x;
     if (t >= ntiles) return;
@@ -406,16 +416,10 @@ __global__ __launch_bounds__(512, 4) void k_conv_tile2(ConvArgs a, int ntiles) {
                 bv[c][nb] = *reinterpret_cast<const s8*>(
                     (MODE == CONV_BWD_DATA ? X0 : a.w) + nn * KP + c * 32 + 8 * kq);
         }
-    // biases in registers: a global load in the loop would wait for the
-    // patch loads in flight (the vector memory counter retires in order)
-    f4 bias4[NP / 16];
-#pragma unroll
-    for (int nb = 0; nb < NP / 16; ++nb)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int nn = NN == 32 ? 8 * kq + 4 * nb + i : 4 * kq + i;
-            bias4[nb][i] = MODE == CONV_BWD_DATA || nn >= NN ? 0.f : a.bias[nn];
-        }
+    // biases in LDS: a global load in the loop would wait for the patch loads in
+    // flight (the vector memory counter retires in order), and the registers are
+    // the weights'
+    if (MODE != CONV_BWD_DATA && tid < 32) Bs[tid] = tid < NN ? a.bias[tid] : 0.f;
     if constexpr (MODE == CONV_BWD_DATA) __syncthreads();
     issue(t, X0);
     auto zissue = [&](int t, bf16* Zd) {
@@ -456,7 +460,7 @@ __global__ __launch_bounds__(512, 4) void k_conv_tile2(ConvArgs a, int ntiles) {
             }
             if constexpr (MODE == CONV_FWD_LAST) {
                 // channel 0 in lanes 0..15: block blk's pixels to the lanes of kq = blk
-                const float v = __shfl((acc[0][0] + bias4[0][0]) * a.yscale, m);
+                const float v = __shfl((acc[0][0] + Bs[0]) * a.yscale, m);
                 if (blk == (kq & 1)) yv = v;
             } else {
                 const size_t o = (q0 + lc) * NN + 8 * kq;
@@ -467,7 +471,7 @@ __global__ __launch_bounds__(512, 4) void k_conv_tile2(ConvArgs a, int ntiles) {
                     float zz[8], g[8];
 #pragma unroll
                     for (int i = 0; i < 8; ++i) {
-                        zz[i] = acc[i >> 2][i & 3] + bias4[i >> 2][i & 3];
+                        zz[i] = acc[i >> 2][i & 3] + Bs[8 * kq + i];
                         g[i] = gelu(zz[i]);
                     }
                     if (a.z) *reinterpret_cast<uint4*>(&a.z[o]) = pack8(zz);
@@ -619,12 +623,18 @@ __global__ __launch_bounds__(256) void k_conv_dw(DwArgs a) {
 // (ky, h) owns the three taps (ky, kx = 0..2) of channels 16 h .. 16 h + 15:
 // per 32 pixels a lane reads one 16-byte chunk of its row (plus one dword on
 // each side), forms the three column shifts with byte-align operations, and
-// issues 3 x NT MFMAs (v_mfma_f32_16x16x32_bf16).  Partial sums, and the
+// issues 3 x NT MFMAs (v_mfma_f32_16x16x32_bf16).  The next tile's input and dZ
+// are fetched into registers while a tile is multiplied.  At 256^2 x 16 43 us for
+// 134 MB (77 us without the fetch ahead and with channel strides of 960 and 512
+// bytes, where the reads of Dl met 16 at a time in one bank).  Partial sums, and the
 // bias gradient, go to part[workgroup][...]; k_dw_reduce adds them up in a
 // fixed order.
 constexpr int kDwRows = 4, kDwCols = 64;
 constexpr int kDwXs = 80;                     // LDS row stride of Xl (elements)
-constexpr int kDwXc = (kDwRows + 2) * kDwXs;  // LDS channel stride of Xl
+// LDS channel strides of Xl and Dl: eight elements past the rows, so that the 16
+// channels that a wave reads together lie in different banks
+constexpr int kDwXc = (kDwRows + 2) * kDwXs + 8;
+constexpr int kDwDc = kDwRows * kDwCols + 8;
 constexpr int kDwMaxWg = 1024;                // workgroups of one launch, at most
 
 struct DwTileArgs {
@@ -641,13 +651,14 @@ __device__ __forceinline__ unsigned align2(unsigned hi, unsigned lo) {
 }
 
 template <int COUT>
-__global__ __launch_bounds__(384) void k_conv_dw_tile(DwTileArgs a) {
+__global__ __launch_bounds__(384, 3) void k_conv_dw_tile(DwTileArgs a) {
+    static_assert(COUT == 32 || COUT == 1, "weight-gradient tiles for 32 or 1 output channels");
     constexpr int CIN = 32;
     constexpr int NT = (COUT + 15) / 16;
     constexpr int DC = NT * 16;
     constexpr int NW = 9 * CIN * COUT;
     __shared__ __align__(16) bf16 Xl[CIN * kDwXc];
-    __shared__ __align__(16) bf16 Dl[DC * kDwRows * kDwCols];
+    __shared__ __align__(16) bf16 Dl[DC * kDwDc];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int ky = wave >> 1, h = wave & 1;
     const int r = lane & 15, g = lane >> 4;
@@ -658,66 +669,64 @@ __global__ __launch_bounds__(384) void k_conv_dw_tile(DwTileArgs a) {
         for (int nb = 0; nb < NT; ++nb) acc[kx][nb] = f4{0.f, 0.f, 0.f, 0.f};
     float dbs = 0.f;  // bias gradient: thread 8 co + seg sums a quarter row of Dl[co]
     if constexpr (COUT < DC) {
-        for (int e = COUT * kDwRows * kDwCols + tid; e < DC * kDwRows * kDwCols; e += 384)
-            Dl[e] = 0;
+        for (int e = COUT * kDwDc + tid; e < DC * kDwDc; e += 384) Dl[e] = 0;
     }
     const int tx_n = a.n / kDwCols, ty_n = a.n / kDwRows;
     const int t_begin = blockIdx.x * a.per_wg;
     const int t_end = min(t_begin + a.per_wg, a.tiles);
-    for (int t = t_begin; t < t_end; ++t) {
+    // interior: 6 rows x 16 quads of pixels x 4 groups of 8 channels; dZ: the same
+    // of its 4 rows (one channel: rows of 64 contiguous values)
+    const int cg = tid & 3, qd = (tid >> 2) & 15, yy = tid >> 6;
+    // halo columns x = -1 and x = 64: 6 rows x 2 sides x 32 channels
+    const int side = tid & 1, ci = (tid >> 1) & 31;
+    const bool has_d = tid < (COUT == 32 ? 256 : 32);
+    s8 xv[4], dv[COUT == 32 ? 4 : 1];
+    bf16 xh = 0;
+    auto fetch = [&](int t) {
         const int mem = t / (tx_n * ty_n), rem = t - mem * (tx_n * ty_n);
         const int y0 = (rem / tx_n) * kDwRows, x0 = (rem % tx_n) * kDwCols;
         const bf16* xb = a.x + (size_t)mem * a.npix * CIN;
         const bf16* db = a.dz + (size_t)mem * a.npix * COUT;
+        const int gy = (y0 + yy - 1) & (a.n - 1);
+        const bf16* src = xb + ((size_t)(gy << a.lg) + x0 + 4 * qd) * CIN + 8 * cg;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) xv[i] = *reinterpret_cast<const s8*>(src + i * CIN);
+        const int gx = (side ? x0 + kDwCols : x0 - 1) & (a.n - 1);
+        xh = xb[((size_t)(gy << a.lg) + gx) * CIN + ci];
+        if (!has_d) return;
+        if constexpr (COUT == 32) {
+            const bf16* d = db + ((size_t)((y0 + yy) << a.lg) + x0 + 4 * qd) * COUT + 8 * cg;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) dv[i] = *reinterpret_cast<const s8*>(d + i * COUT);
+        } else {
+            dv[0] = *reinterpret_cast<const s8*>(db + ((size_t)((y0 + (tid >> 3)) << a.lg) + x0 +
+                                                       8 * (tid & 7)));
+        }
+    };
+    auto stage = [&]() {
+#pragma unroll
+        for (int c = 0; c < 8; ++c)
+            *reinterpret_cast<s4*>(&Xl[(8 * cg + c) * kDwXc + yy * kDwXs + 8 + 4 * qd]) =
+                s4{xv[0][c], xv[1][c], xv[2][c], xv[3][c]};
+        Xl[ci * kDwXc + yy * kDwXs + (side ? 8 + kDwCols : 7)] = xh;
+        if (!has_d) return;
+        if constexpr (COUT == 32) {
+#pragma unroll
+            for (int c = 0; c < 8; ++c)
+                *reinterpret_cast<s4*>(&Dl[(8 * cg + c) * kDwDc + yy * kDwCols + 4 * qd]) =
+                    s4{dv[0][c], dv[1][c], dv[2][c], dv[3][c]};
+        } else {
+            *reinterpret_cast<s8*>(&Dl[(tid >> 3) * kDwCols + 8 * (tid & 7)]) = dv[0];
+        }
+    };
+    if (t_begin < t_end) fetch(t_begin);
+    for (int t = t_begin; t < t_end; ++t) {
         __syncthreads();  // the previous tile's reads are done
-        {   // interior: 6 rows x 16 quads of pixels x 4 groups of 8 channels
-            const int cg = tid & 3, qd = (tid >> 2) & 15, yy = tid >> 6;
-            const int gy = (y0 + yy - 1) & (a.n - 1);
-            const bf16* src = xb + ((size_t)(gy << a.lg) + x0 + 4 * qd) * CIN + 8 * cg;
-            const s8 v0 = *reinterpret_cast<const s8*>(src);
-            const s8 v1 = *reinterpret_cast<const s8*>(src + CIN);
-            const s8 v2 = *reinterpret_cast<const s8*>(src + 2 * CIN);
-            const s8 v3 = *reinterpret_cast<const s8*>(src + 3 * CIN);
-#pragma unroll
-            for (int c = 0; c < 8; ++c) {
-                const s4 q = {v0[c], v1[c], v2[c], v3[c]};
-                *reinterpret_cast<s4*>(&Xl[(8 * cg + c) * kDwXc + yy * kDwXs + 8 + 4 * qd]) = q;
-            }
-        }
-        {   // halo columns x = -1 and x = 64: 6 rows x 2 sides x 32 channels
-            const int side = tid & 1, ci = (tid >> 1) & 31, yy = tid >> 6;
-            const int gy = (y0 + yy - 1) & (a.n - 1);
-            const int gx = (side ? x0 + kDwCols : x0 - 1) & (a.n - 1);
-            Xl[ci * kDwXc + yy * kDwXs + (side ? 8 + kDwCols : 7)] =
-                xb[((size_t)(gy << a.lg) + gx) * CIN + ci];
-        }
-        if constexpr (COUT == 32) {  // 4 rows x 16 quads x 4 groups of 8 channels
-            if (tid < 256) {
-                const int cg = tid & 3, qd = (tid >> 2) & 15, yr = tid >> 6;
-                const bf16* src =
-                    db + ((size_t)((y0 + yr) << a.lg) + x0 + 4 * qd) * COUT + 8 * cg;
-                const s8 v0 = *reinterpret_cast<const s8*>(src);
-                const s8 v1 = *reinterpret_cast<const s8*>(src + COUT);
-                const s8 v2 = *reinterpret_cast<const s8*>(src + 2 * COUT);
-                const s8 v3 = *reinterpret_cast<const s8*>(src + 3 * COUT);
-#pragma unroll
-                for (int c = 0; c < 8; ++c) {
-                    const s4 q = {v0[c], v1[c], v2[c], v3[c]};
-                    *reinterpret_cast<s4*>(
-                        &Dl[(8 * cg + c) * (kDwRows * kDwCols) + yr * kDwCols + 4 * qd]) = q;
-                }
-            }
-        } else {  // one channel: rows of 64 contiguous values
-            static_assert(COUT == 1, "weight-gradient tiles for 32 or 1 output channels");
-            if (tid < 32) {
-                const int yr = tid >> 3, seg = tid & 7;
-                *reinterpret_cast<s8*>(&Dl[yr * kDwCols + 8 * seg]) = *reinterpret_cast<const s8*>(
-                    db + ((size_t)((y0 + yr) << a.lg) + x0 + 8 * seg));
-            }
-        }
+        stage();
         __syncthreads();
+        if (t + 1 < t_end) fetch(t + 1);
         if (tid < 8 * COUT) {  // bias: channel tid / 8, pixels 32 (tid % 8) .. + 31
-            const bf16* d = &Dl[(tid >> 3) * (kDwRows * kDwCols) + 32 * (tid & 7)];
+            const bf16* d = &Dl[(tid >> 3) * kDwDc + 32 * (tid & 7)];
 #pragma unroll
             for (int e = 0; e < 32; ++e) dbs += bf2f(d[e]);
         }
@@ -737,7 +746,7 @@ __global__ __launch_bounds__(384) void k_conv_dw_tile(DwTileArgs a) {
 #pragma unroll
                 for (int nb = 0; nb < NT; ++nb) {
                     const uint4 bv = *reinterpret_cast<const uint4*>(
-                        &Dl[(16 * nb + r) * (kDwRows * kDwCols) + yr * kDwCols + xs]);
+                        &Dl[(16 * nb + r) * kDwDc + yr * kDwCols + xs]);
 #pragma unroll
                     for (int kx = 0; kx < 3; ++kx)
                         acc[kx][nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
@@ -777,7 +786,7 @@ __global__ __launch_bounds__(256) void k_conv_dw_tile_in(DwTileArgs a) {
     constexpr int NT = COUT / 16;
     constexpr int NW = 9 * COUT;
     __shared__ __align__(16) bf16 Xl[kDwXc];
-    __shared__ __align__(16) bf16 Dl[COUT * kDwRows * kDwCols];
+    __shared__ __align__(16) bf16 Dl[COUT * kDwDc];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int r = lane & 15, g = lane >> 4;
     const int tky = r / 3, tkx = r - 3 * (r / 3);  // tap of this lane's A row (r < 9)
@@ -816,12 +825,12 @@ __global__ __launch_bounds__(256) void k_conv_dw_tile_in(DwTileArgs a) {
             for (int c = 0; c < 8; ++c) {
                 const s4 q = {v0[c], v1[c], v2[c], v3[c]};
                 *reinterpret_cast<s4*>(
-                    &Dl[(8 * cg + c) * (kDwRows * kDwCols) + yr * kDwCols + 4 * qd]) = q;
+                    &Dl[(8 * cg + c) * kDwDc + yr * kDwCols + 4 * qd]) = q;
             }
         }
         __syncthreads();
         {   // bias: channel tid / 8, pixels 32 (tid % 8) .. + 31
-            const bf16* d = &Dl[(tid >> 3) * (kDwRows * kDwCols) + 32 * (tid & 7)];
+            const bf16* d = &Dl[(tid >> 3) * kDwDc + 32 * (tid & 7)];
 #pragma unroll
             for (int e = 0; e < 32; ++e) dbs += bf2f(d[e]);
         }
@@ -844,7 +853,7 @@ __global__ __launch_bounds__(256) void k_conv_dw_tile_in(DwTileArgs a) {
 #pragma unroll
             for (int nb = 0; nb < NT; ++nb) {
                 const uint4 bv = *reinterpret_cast<const uint4*>(
-                    &Dl[(16 * nb + r) * (kDwRows * kDwCols) + yr * kDwCols + xs]);
+                    &Dl[(16 * nb + r) * kDwDc + yr * kDwCols + xs]);
                 acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
                     __builtin_bit_cast(bf8, av), __builtin_bit_cast(bf8, bv), acc[nb], 0, 0, 0);
             }
@@ -865,7 +874,7 @@ __global__ __launch_bounds__(256) void k_conv_dw_tile_in(DwTileArgs a) {
     if (lane < COUT && (lane >> 3) != wave) out[NW + lane] = 0.f;
 }
 
-// grad[i] += sum over workgroups w of part[w][i]: 64 outputs per block; wave
+// grad[i] = sum over workgroups w of part[w][i]: 64 outputs per block; wave
 // q sums the workgroups w = q mod 4 in order, and the four sums are added in
 // a fixed order (the result does not depend on timing)
 __global__ __launch_bounds__(256) void k_dw_reduce(int nwg, int stride, const float* part,
@@ -875,27 +884,41 @@ __global__ __launch_bounds__(256) void k_dw_reduce(int nwg, int stride, const fl
     const int i = blockIdx.x * 64 + o;
     float s = 0.f;
     if (i < stride) {
-#pragma unroll 8
-        for (int w = q; w < nwg; w += 4) s += part[(size_t)w * stride + i];
+        constexpr int N = 16;  // loads in flight
+        int w = q;
+        for (; w + 4 * (N - 1) < nwg; w += 4 * N) {
+            float v[N];
+#pragma unroll
+            for (int k = 0; k < N; ++k) v[k] = part[(size_t)(w + 4 * k) * stride + i];
+#pragma unroll
+            for (int k = 0; k < N; ++k) s += v[k];
+        }
+        for (; w < nwg; w += 4) s += part[(size_t)w * stride + i];
     }
     red[q][o] = s;
     __syncthreads();
     if (q == 0 && i < stride) {
         const float t = (red[0][o] + red[1][o]) + (red[2][o] + red[3][o]);
-        if (i < nw) dw[i] += t;
-        else db[i - nw] += t;
+        if (i < nw) dw[i] = t;
+        else db[i - nw] = t;
     }
 }
 
 // mean squared error and its gradient dL/dy = 2 (y - t) / total, in bf16
-__global__ void k_mse(int total, const float* y, const float* t, bf16* dy, double* loss) {
+// four values a thread at a time (total is a multiple of 4)
+__global__ __launch_bounds__(256) void k_mse(int total, const float4* __restrict__ y,
+                                             const float4* __restrict__ t, uint2* __restrict__ dy,
+                                             double* loss) {
     __shared__ double red[4];
     double s = 0.0;
     const float sc = 2.f / (float)total;
-    for (int q = blockIdx.x * blockDim.x + threadIdx.x; q < total; q += gridDim.x * blockDim.x) {
-        const float d = y[q] - t[q];
-        s += (double)d * d;
-        dy[q] = f2bf(sc * d);
+#pragma unroll 4
+    for (int q = blockIdx.x * blockDim.x + threadIdx.x; q < total / 4; q += gridDim.x * blockDim.x) {
+        const float4 a = y[q], b = t[q];
+        const float d[4] = {a.x - b.x, a.y - b.y, a.z - b.z, a.w - b.w};
+#pragma unroll
+        for (int i = 0; i < 4; ++i) s += (double)d[i] * d[i];
+        dy[q] = uint2{pack2(sc * d[0], sc * d[1]), pack2(sc * d[2], sc * d[3])};
     }
     for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
@@ -903,25 +926,38 @@ __global__ void k_mse(int total, const float* y, const float* t, bf16* dy, doubl
     if (threadIdx.x == 0) atomicAdd(loss, (red[0] + red[1] + red[2] + red[3]) / total);
 }
 
-// minibatch from the data set: x (scaled, bf16) and target (scaled, FP32)
-__global__ void k_gather_batch(int npix, const int* idx, const float* ds_x, const float* ds_t,
-                               float xs, float ts, bf16* x0, float* t) {
-    const int b = blockIdx.y;
-    const size_t src = (size_t)idx[b] * npix, dst = (size_t)b * npix;
-    for (int p = blockIdx.x * blockDim.x + threadIdx.x; p < npix; p += gridDim.x * blockDim.x) {
-        x0[dst + p] = f2bf(xs * ds_x[src + p]);
-        t[dst + p] = ts * ds_t[src + p];
+// minibatch from the data set: x (scaled, bf16) and target (scaled, FP32) of the
+// members ids.v; zeroes the loss that k_mse adds to
+constexpr int kIds = 64;
+struct Ids {
+    int v[kIds];
+};
+__global__ __launch_bounds__(256) void k_gather_batch(int npix, Ids ids, const float4* __restrict__ ds_x,
+                                                      const float4* __restrict__ ds_t, float xs,
+                                                      float ts, uint2* __restrict__ x0,
+                                                      float4* __restrict__ t, double* loss) {
+    const int b = blockIdx.y, n4 = npix / 4;
+    const size_t src = (size_t)ids.v[b] * n4, dst = (size_t)b * n4;
+    for (int p = blockIdx.x * blockDim.x + threadIdx.x; p < n4; p += gridDim.x * blockDim.x) {
+        const float4 x = ds_x[src + p], y = ds_t[src + p];
+        x0[dst + p] = uint2{pack2(xs * x.x, xs * x.y), pack2(xs * x.z, xs * x.w)};
+        t[dst + p] = float4{ts * y.x, ts * y.y, ts * y.z, ts * y.w};
     }
+    if (blockIdx.x == 0 && b == 0 && threadIdx.x == 0) *loss = 0.0;
 }
 
-// sums of squares of the data set's inputs and targets (for the scales)
-__global__ void k_sumsq(size_t count, const float* x, const float* t, double* out) {
+// sums of squares of the data set's inputs and targets (for the scales), count a
+// multiple of 4
+__global__ __launch_bounds__(256) void k_sumsq(size_t count, const float4* __restrict__ x,
+                                               const float4* __restrict__ t, double* out) {
     __shared__ double red[2][4];
     double sx = 0.0, st = 0.0;
-    for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < count;
+#pragma unroll 4
+    for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < count / 4;
          i += (size_t)gridDim.x * blockDim.x) {
-        sx += (double)x[i] * x[i];
-        st += (double)t[i] * t[i];
+        const float4 a = x[i], b = t[i];
+        sx += ((double)a.x * a.x + (double)a.y * a.y) + ((double)a.z * a.z + (double)a.w * a.w);
+        st += ((double)b.x * b.x + (double)b.y * b.y) + ((double)b.z * b.z + (double)b.w * b.w);
     }
     for (int o = 32; o > 0; o >>= 1) {
         sx += __shfl_xor(sx, o, 64);
@@ -964,6 +1000,9 @@ __global__ void k_adam(int count, float* w, const float* g, float* m, float* v, 
 
 // ----------------------------------------------------------------- closure
 
+// minibatches whose losses wait on the device for one copy to the host
+constexpr int kLossSlots = 256;
+
 struct NsdClosure {
     int n = 0, lg = 0, npix = 0, max_batch = 0;
     int cin[kLayers] = {1, kHidden, kHidden, kHidden, kHidden};
@@ -984,13 +1023,12 @@ struct NsdClosure {
     bf16* dy = nullptr;      // gradient of the output [B][npix]
     float* xin = nullptr;    // FP32 staging [B][npix]
     float* tin = nullptr;
-    double* loss = nullptr;
+    double* loss = nullptr;  // kLossSlots minibatch losses
     unsigned long long adam_t = 0;
     float in_scale = 1.f, out_scale = 1.f;  // net input = in_scale x; tendency = out_scale net
     float* ds_x = nullptr;   // data set: inputs [count][npix]
     float* ds_t = nullptr;   // data set: targets [count][npix]
     int ds_count = 0;
-    int* idx = nullptr;      // minibatch indices
     double* sums = nullptr;
     float* dwpart = nullptr;  // weight-gradient partial sums per workgroup
     int dw_wg = 0;            // their rows
@@ -1065,9 +1103,16 @@ int adam_step(NsdClosure* c, float lr) {
     return ck(c, hipGetLastError(), "adam") ? 3 : 0;
 }
 
+// output gradient of `total` pixels; adds their mean square error to *loss
+void launch_mse(NsdClosure* c, int total, double* loss) {
+    hipLaunchKernelGGL(k_mse, dim3(std::min((total + 1023) / 1024, 512)), dim3(256), 0, c->stream, total,
+                       (const float4*)c->y, (const float4*)c->tin, (uint2*)c->dy, loss);
+}
+
 int launch_backward(NsdClosure* c, int batch) {
     const int total = batch * c->npix;
-    CKC(hipMemsetAsync(c->grad, 0, sizeof(float) * c->nparam, c->stream));
+    // (the tiled kernels' sums are stored, k_conv_dw adds to zeros)
+    if (!c->dwpart) CKC(hipMemsetAsync(c->grad, 0, sizeof(float) * c->nparam, c->stream));
     // dW, db of layer l from its input and dz_l; then dz_{l-1} = (W_l^T dz_l) * gelu'(z_{l-1})
     DwArgs d;
     memset(&d, 0, sizeof(d));
@@ -1172,7 +1217,7 @@ void nsd_closure_destroy(NsdClosure* c) {
     if (!c) return;
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     void* bufs[] = {c->prm, c->grad, c->adm, c->adv, c->widx, c->wb, c->x0, c->y, c->dy,
-                    c->xin, c->tin, c->loss, c->ds_x, c->ds_t, c->idx, c->sums, c->dwpart};
+                    c->xin, c->tin, c->loss, c->ds_x, c->ds_t, c->sums, c->dwpart};
     for (void* b : bufs)
         if (b) (void)hipFree(b);
     for (int i = 0; i < kHiddenLayers; ++i)
@@ -1217,8 +1262,7 @@ NsdClosure* nsd_closure_create(int n, int max_batch, unsigned long long seed, ch
          al((void**)&c->widx, 4 * off) && al((void**)&c->wb, 2 * wo) &&
          al((void**)&c->x0, 2 * P) && al((void**)&c->y, 4 * P) && al((void**)&c->dy, 2 * P) &&
          al((void**)&c->xin, 4 * P) && al((void**)&c->tin, 4 * P) &&
-         al((void**)&c->loss, sizeof(double)) && al((void**)&c->idx, sizeof(int) * max_batch) &&
-         al((void**)&c->sums, 2 * sizeof(double));
+         al((void**)&c->loss, sizeof(double) * kLossSlots) && al((void**)&c->sums, 2 * sizeof(double));
     for (int i = 0; i < kHiddenLayers && ok; ++i)
         ok = al((void**)&c->z[i], 2 * P * kHidden) && al((void**)&c->act[i], 2 * P * kHidden) &&
              al((void**)&c->dz[i], 2 * P * kHidden);
@@ -1280,8 +1324,7 @@ int nsd_closure_gradient(NsdClosure* c, const float* x, const float* t, int batc
     if (stage_input(c, x, batch) || launch_forward(c, batch)) return 3;
     CKC(hipMemcpyAsync(c->tin, t, sizeof(float) * total, hipMemcpyHostToDevice, c->stream));
     CKC(hipMemsetAsync(c->loss, 0, sizeof(double), c->stream));
-    hipLaunchKernelGGL(k_mse, dim3(256), dim3(256), 0, c->stream, total, c->y, c->tin, c->dy,
-                       c->loss);
+    launch_mse(c, total, c->loss);
     if (launch_backward(c, batch)) return 3;
     if (loss) CKC(hipMemcpyAsync(loss, c->loss, sizeof(double), hipMemcpyDeviceToHost, c->stream));
     if (grad)
@@ -1350,7 +1393,8 @@ int nsd_closure_train(NsdClosure* c, int count, int epochs, int batch, double lr
     const size_t cnt = (size_t)count * c->npix;
     // scales: unit mean square for the network's input and output
     CKC(hipMemsetAsync(c->sums, 0, 2 * sizeof(double), c->stream));
-    hipLaunchKernelGGL(k_sumsq, dim3(1024), dim3(256), 0, c->stream, cnt, c->ds_x, c->ds_t, c->sums);
+    hipLaunchKernelGGL(k_sumsq, dim3(512), dim3(256), 0, c->stream, cnt, (const float4*)c->ds_x,
+                       (const float4*)c->ds_t, c->sums);
     double sums[2];
     CKC(hipMemcpyAsync(sums, c->sums, sizeof(sums), hipMemcpyDeviceToHost, c->stream));
     CKC(hipStreamSynchronize(c->stream));
@@ -1370,7 +1414,6 @@ int nsd_closure_train(NsdClosure* c, int count, int epochs, int batch, double lr
     }
     const int ntrain = (int)order.size();
     unsigned long long s = seed ? seed : 0xc105eull;
-    const dim3 ggrid((c->npix + 255) / 256 < 64 ? (c->npix + 255) / 256 : 64, batch);
     // learning rate: cosine decay from lr to lr / 20 over all training steps
     const long total_steps = (long)epochs * (ntrain / batch);
     long step = 0;
@@ -1378,21 +1421,34 @@ int nsd_closure_train(NsdClosure* c, int count, int epochs, int batch, double lr
         const double f = total_steps > 1 ? (double)step / (double)(total_steps - 1) : 0.0;
         return lr * (0.05 + 0.475 * (1.0 + std::cos(3.14159265358979323846 * f)));
     };
+    // losses stay on the device until the slots are full or a sum is asked for: no
+    // wait between minibatches
+    int sizes[kLossSlots], slots = 0;
+    auto flush = [&](double* loss_acc) -> int {
+        double l[kLossSlots];
+        CKC(hipMemcpyAsync(l, c->loss, sizeof(double) * slots, hipMemcpyDeviceToHost, c->stream));
+        CKC(hipStreamSynchronize(c->stream));
+        for (int i = 0; i < slots; ++i) *loss_acc += l[i] * sizes[i];
+        slots = 0;
+        return 0;
+    };
     auto run_batch = [&](const int* ids, int nb, bool learn, double* loss_acc) -> int {
-        CKC(hipMemcpyAsync(c->idx, ids, sizeof(int) * nb, hipMemcpyHostToDevice, c->stream));
-        hipLaunchKernelGGL(k_gather_batch, dim3(ggrid.x, nb), dim3(256), 0, c->stream, c->npix,
-                           c->idx, c->ds_x, c->ds_t, c->in_scale, ts, c->x0, c->tin);
+        const int n4 = c->npix / 4;
+        for (int i0 = 0; i0 < nb; i0 += kIds) {
+            Ids v;
+            const int n = std::min(nb - i0, kIds);
+            for (int i = 0; i < n; ++i) v.v[i] = ids[i0 + i];
+            hipLaunchKernelGGL(k_gather_batch, dim3(std::min((n4 + 255) / 256, 64), n), dim3(256), 0,
+                               c->stream, c->npix, v, (const float4*)c->ds_x, (const float4*)c->ds_t,
+                               c->in_scale, ts, (uint2*)(c->x0 + (size_t)i0 * c->npix),
+                               (float4*)(c->tin + (size_t)i0 * c->npix), c->loss + slots);
+        }
         if (launch_forward(c, nb)) return 3;
-        CKC(hipMemsetAsync(c->loss, 0, sizeof(double), c->stream));
-        hipLaunchKernelGGL(k_mse, dim3(256), dim3(256), 0, c->stream, nb * c->npix, c->y, c->tin,
-                           c->dy, c->loss);
+        launch_mse(c, nb * c->npix, c->loss + slots);
+        sizes[slots++] = nb;
         if (learn && (launch_backward(c, nb) || adam_step(c, (float)rate()))) return 3;
         if (learn) ++step;
-        double l = 0.0;
-        CKC(hipMemcpyAsync(&l, c->loss, sizeof(double), hipMemcpyDeviceToHost, c->stream));
-        CKC(hipStreamSynchronize(c->stream));
-        *loss_acc += l * nb;
-        return 0;
+        return slots == kLossSlots ? flush(loss_acc) : 0;
     };
     for (int e = 0; e < epochs; ++e) {
         for (int i = ntrain - 1; i > 0; --i) {  // Fisher-Yates with SplitMix64
@@ -1402,6 +1458,7 @@ int nsd_closure_train(NsdClosure* c, int count, int epochs, int batch, double lr
         double acc = 0.0;
         for (int b0 = 0; b0 + batch <= ntrain; b0 += batch)
             if (run_batch(&order[b0], batch, true, &acc)) return 3;
+        if (slots && flush(&acc)) return 3;
         const double mean = acc / (double)(ntrain / batch * batch);
         if (e == 0 && loss_first) *loss_first = mean;
         if (loss_last) *loss_last = mean;
@@ -1413,6 +1470,7 @@ int nsd_closure_train(NsdClosure* c, int count, int epochs, int batch, double lr
         if (run_batch(&valid[b0], nb, false, &vacc)) return 3;
         done += nb;
     }
+    if (slots && flush(&vacc)) return 3;
     if (loss_valid) *loss_valid = vacc / done;
     return 0;
 }
