@@ -261,25 +261,29 @@ __global__ __launch_bounds__(512) void k_conv_tile(ConvArgs a) {
         const int nn = tile_channel(nb, m);
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
-            const int tap = 8 * kq + i;
-            bv[nb][i] = tap >= 9 ? 0 : (short)(MODE == CONV_BWD_DATA ? a.w[tap * NN + nn] : a.w[nn * 9 + tap]);
+            const int tap = min(8 * kq + i, 8);
+            const short w = (short)(MODE == CONV_BWD_DATA ? a.w[tap * NN + nn] : a.w[nn * 9 + tap]);
+            bv[nb][i] = 8 * kq + i < 9 ? w : (short)0;
         }
 #pragma unroll
         for (int i = 0; i < 4; ++i)
             bias4[nb][i] = MODE == CONV_BWD_DATA ? 0.f : a.bias[8 * kq + 4 * nb + i];
     }
     __syncthreads();
+    const bf16* const xs = Xs + (wave + 1) * PC + m + 1;
+    const unsigned rest = kq == 0 ? ~0u : 0u, first = kq == 1 ? 0xffffu : rest;
 #pragma unroll
     for (int b = 0; b < NBLK; ++b) {
-        s8 av;
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {  // lane: pixel m, taps 8 kq + i
-            const int tap = 8 * kq + i;
-            short v = 0;
-            if (tap < 9)
-                v = (short)Xs[(wave + 1 + S * (tap / 3 - 1)) * PC + 16 * b + m + 1 + S * (tap % 3 - 1)];
-            av[i] = v;
-        }
+        // lane: pixel m, taps 8 kq + i, that is taps 0 .. 7 (kq = 0), 8 (kq = 1) and
+        // zeros; every lane reads, at constant offsets, and masks
+        auto at = [](int tap) { return S * ((tap / 3 - 1) * PC + tap % 3 - 1); };
+        const bf16* x = xs + 16 * b;
+        uint4 u;
+        u.x = ((unsigned)x[kq == 0 ? at(0) : at(8)] | ((unsigned)x[at(1)] << 16)) & first;
+        u.y = ((unsigned)x[at(2)] | ((unsigned)x[at(3)] << 16)) & rest;
+        u.z = ((unsigned)x[at(4)] | ((unsigned)x[at(5)] << 16)) & rest;
+        u.w = ((unsigned)x[at(6)] | ((unsigned)x[at(7)] << 16)) & rest;
+        const s8 av = __builtin_bit_cast(s8, u);
         f4 acc[2];
 #pragma unroll
         for (int nb = 0; nb < 2; ++nb)
