@@ -126,3 +126,36 @@ def test_layout_transitions_2048(ns, fp32):
     assert np.array_equal(mine.spec("omega_hat"), plain.spec("omega_hat"))
     for s in made:
         s.close()
+
+
+# a long call replays several steps at a time; the counts cross that length and its
+# multiples, before and after the kernels' arguments changed
+@pytest.mark.parametrize("n,fp32,forced", [(64, False, False), (128, True, True), (512, False, True)])
+def test_long_calls_are_single_steps(ns, n, fp32, forced):
+    def solver():
+        s = ns.Spectral(n, n, 2 * np.pi, 2 * np.pi, 1e3)
+        s.init(taylor_green=False)
+        s.set_precision(fp32)
+        s.set_scheme(True)
+        s.d.cfl_factor = 0.5
+        if forced:
+            s.set_forcing(4.0, 6.0, 1e-3, seed=5)
+        s.random_phase(9, k_peak=6.0, energy=0.5)
+        s.sync_device()
+        return s
+
+    def state(s):
+        out = np.zeros((s.ny, s.nkx), np.complex128)
+        s.check(s.L.nsd_state_download(s.ctx, out.ctypes.data_as(ns.c_double_p)))
+        return out
+
+    a, b = solver(), solver()
+    for drag, counts in ((0.0, (37, 7, 8, 33)), (0.2, (9, 40))):
+        for s in (a, b):
+            s.set_drag(drag)
+        for k in counts:
+            a.check(a.advance_n(k, True))
+            for _ in range(k):
+                b.check(b.advance_n(1, True))
+            assert a.d.t == b.d.t
+            assert np.array_equal(state(a), state(b))
