@@ -899,6 +899,25 @@ __global__ __launch_bounds__(NT, MW) void k_col(ColArgs<T> a) {
     constexpr bool PF = MODE == COL_STAGE && LC >= 64 &&
                         (paired_lines<T, LC, NT, PR>() || (sizeof(T) == 8 && NT <= 512));
     cx<T> pw0[P], pacc[P];
+    // The smallest FP32 workgroups (launches with few waves): dt and the modes'
+    // factors before the transform of J, which waits a memory latency anyway.
+    // 256^2 step @@
+    constexpr bool EARLY = PF && sizeof(T) == 4 && NT == 64 && !ERR;
+    T el[P], es[P];  // el: L or E - 1, es: the SFD weight or E2 - 1
+    double dt = 0.0, u2 = 0.0;
+    auto pick_dt = [&]() {
+        dt = cfl_dt(ph, sqrt(u2));
+        // the error controller's step limit, within [dt_min, dt_max]
+        if constexpr (ERR) dt = fmin(fmax(fmin(dt, sc->dt_err), ph.dt_lo), ph.dt_hi);
+        if (blockIdx.x == 0 && threadIdx.x == 0 && !redo) {
+            sc->dt = dt;
+            if (!(u2 <= 1.0e300)) sc->status = 2;  // SOLVER_DIVERGED
+        }
+    };
+    if constexpr (EARLY) {
+        if (a.stage == 0 && ph.adaptive) u2 = __longlong_as_double((long long)sc->umax2_bits);
+        else dt = sc->dt;
+    }
 
     // ---- forward y-transform of the mixed nonlinear field
     if constexpr (PF) {
@@ -949,6 +968,24 @@ __global__ __launch_bounds__(NT, MW) void k_col(ColArgs<T> a) {
             pacc[s] = zero;
             if (with_acc) pacc[s] = acc[ci];
         }
+        if constexpr (EARLY) {
+            if (a.stage == 0 && ph.adaptive) pick_dt();
+#pragma unroll
+            for (int s = 0; s < P; ++s) {
+                if (slot_kind(s, LC, Band<LC>::kym) == 0) continue;
+                const T ky = T(col_band<LC>(G, j + s * TPL)) * T(2.0 * kPi / G.Ly);
+                const T k2 = kx * kx + ky * ky;
+                const T L = -(k2 * T(ph.inv_Re) + T(ph.drag) + hv_weight_t<T>(ph, k2));
+                if constexpr (SCHEME == 0) {
+                    el[s] = L;
+                    es[s] = sfd_weight_t<T>(ph, k2);
+                } else {
+                    es[s] = expm1_t(L * (T(0.5) * T(dt)));
+                    el[s] = es[s] * (T(2) + es[s]);
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
         if constexpr (WSF) {
             cx<T>(*const vv[1])[P] = {&v};
             cx<T>* const r1[1] = {lds};
@@ -990,17 +1027,10 @@ __global__ __launch_bounds__(NT, MW) void k_col(ColArgs<T> a) {
     }
 
     // ---- spectral state of this column after the stage (or as is)
-    double dt = 0.0;
-    if constexpr (MODE == COL_STAGE) {
+    if constexpr (MODE == COL_STAGE && !EARLY) {
         if (a.stage == 0 && ph.adaptive) {
-            const double u2 = __longlong_as_double((long long)sc->umax2_bits);
-            dt = cfl_dt(ph, sqrt(u2));
-            // the error controller's step limit, within [dt_min, dt_max]
-            if constexpr (ERR) dt = fmin(fmax(fmin(dt, sc->dt_err), ph.dt_lo), ph.dt_hi);
-            if (blockIdx.x == 0 && threadIdx.x == 0 && !redo) {
-                sc->dt = dt;
-                if (!(u2 <= 1.0e300)) sc->status = 2;  // SOLVER_DIVERGED
-            }
+            u2 = __longlong_as_double((long long)sc->umax2_bits);
+            pick_dt();
         } else {
             dt = sc->dt;
         }
@@ -1051,9 +1081,9 @@ __global__ __launch_bounds__(NT, MW) void k_col(ColArgs<T> a) {
             // classic RK4 (spectral_time_integration.c:50-100) with
             // hyperviscosity_apply (hyperviscosity.c:104-150) and drag
             const cx<T> ws = (a.stage == 0) ? w0 : stagebuf[ci];
-            const T lin = -(k2 * T(ph.inv_Re) + T(ph.drag) + hv_weight_t<T>(ph, k2));
+            const T lin = EARLY ? el[s] : -(k2 * T(ph.inv_Re) + T(ph.drag) + hv_weight_t<T>(ph, k2));
             cx<T> ks = N + lin * ws;
-            const T sw = sfd_weight_t<T>(ph, k2);
+            const T sw = EARLY ? es[s] : sfd_weight_t<T>(ph, k2);
             if (sw > T(0)) ks = ks - sw * (ws - sfd[ci]);
             if (a.stage == 0) {
                 acc[ci] = w0 + (h / T(6)) * ks;
@@ -1079,8 +1109,9 @@ __global__ __launch_bounds__(NT, MW) void k_col(ColArgs<T> a) {
             // ~1e-5, which 1 + (E - 1) keeps to full relative precision while
             // E itself, rounded to FP32, would lose ~0.3 % of it every step.
             const T L = -(k2 * T(ph.inv_Re) + T(ph.drag) + hv_weight_t<T>(ph, k2));
-            const T e2 = expm1_t(L * (T(0.5) * h));  // E2 - 1, E2 = exp(L h / 2)
-            const T e1 = e2 * (T(2) + e2);          // E - 1,  E = E2^2
+            // E2 - 1, E2 = exp(L h / 2), and E - 1, E = E2^2
+            const T e2 = EARLY ? es[s] : expm1_t(L * (T(0.5) * h));
+            const T e1 = EARLY ? el[s] : e2 * (T(2) + e2);
             if (a.stage == 0) {
                 acc[ci] = grow(w0, e1) + (h / T(6)) * grow(N, e1);
                 wn = grow(w0 + (T(0.5) * h) * N, e2);
