@@ -744,6 +744,7 @@ struct NsdContext {
     double* stH[4] = {nullptr, nullptr, nullptr, nullptr};
     double* stR[4] = {nullptr, nullptr, nullptr, nullptr};
     double* pin = nullptr;                  // pinned staging of small grids' host arrays
+    hipEvent_t pin_ev = nullptr;
     bool pin_failed = false;
     int* fmodes = nullptr;
     int* fpartner = nullptr;
@@ -807,7 +808,7 @@ int sync(NsdContext* c) {
 // kernels read and write in place: a header, five spectra, three physical fields.
 // The copies of pageable arrays that it replaces are 10 to 20 us each, whatever
 // their size, and there are nine in a step on host arrays.  ns_spectral_advance_rk4
-// at FP64, us: 64^2 293 -> 101, 128^2 360 -> 143, 256^2 495 -> 261, 512^2 1271 -> 954;
+// at FP64, us: 64^2 293 -> 99, 128^2 360 -> 132, 256^2 495 -> 228, 512^2 1271 -> 808;
 // the CFL step before it 49 -> 23 at 128^2.  At 1024^2 (4.0 ms) the host's own copies
 // out of the buffer would take what the pageable ones do: kPinMost ends at 512^2.
 constexpr size_t kPinHead = 1024;              // doubles
@@ -816,7 +817,8 @@ bool pinned(NsdContext* c) {
     const size_t n = kPinHead + 5 * 2 * H_of(c) + 3 * R_of(c);
     if (c->pin) return true;
     if (c->pin_failed || c->nb != 1 || n * sizeof(double) > kPinMost) return false;
-    if (hipHostMalloc(&c->pin, n * sizeof(double), hipHostMallocDefault) != hipSuccess) {
+    if (hipEventCreateWithFlags(&c->pin_ev, hipEventDisableTiming) != hipSuccess ||
+        hipHostMalloc(&c->pin, n * sizeof(double), hipHostMallocDefault) != hipSuccess) {
         (void)hipGetLastError();
         c->pin = nullptr;
         c->pin_failed = true;
@@ -1378,6 +1380,7 @@ int op_host_step(NsdContext* c, NsdHostFields* f) {
                            (const cx<T>*)c->state, (const cx<T>*)c->sfd, c->sc, pinH(c, 0),
                            pinH(c, 1), pinH(c, 2), pinH(c, 3), f->sfd_hat ? pinH(c, 4) : nullptr,
                            c->pin);
+        CK(hipEventRecord(c->pin_ev, c->stream));
         // psi_y = u and psi_x = -v lie transformed along y in the mixed buffers;
         // omega joins them in the J buffer, which holds nothing between steps
         ColArgs<T> a = col_args<T>(c);
@@ -1398,14 +1401,20 @@ int op_host_step(NsdContext* c, NsdHostFields* f) {
         launch_row_t<T>(c, r, c->G.ny);
         rc = lastk(c);
     }
-    if (sync(c) || rc) return rc ? rc : ST_MEM;
+    if (rc) {
+        (void)sync(c);
+        return rc;
+    }
+    // the spectra are copied out while the physical fields are transformed
+    CK(hipEventSynchronize(c->pin_ev));
     f->t = c->pin[0];
     f->dt = c->pin[1];
     f->status = (int)c->pin[2];
-    if (f->status) return ST_OK;
+    if (f->status) return sync(c);
     double* const spec[5] = {f->omega_hat, f->psi_hat, f->u_hat, f->v_hat, f->sfd_hat};
     for (int i = 0; i < 5; ++i)
         if (spec[i]) memcpy(spec[i], pinH(c, i), hb);
+    if (sync(c)) return ST_MEM;
     double* const phys[3] = {f->u, f->v, f->omega};
     for (int i = 0; i < 3; ++i)
         if (phys[i]) memcpy(phys[i], pinR(c, i), rb);
@@ -1831,6 +1840,7 @@ void nsd_destroy(NsdContext* c) {
     for (void* b : bufs)
         if (b) (void)hipFree(b);
     if (c->pin) (void)hipHostFree(c->pin);
+    if (c->pin_ev) (void)hipEventDestroy(c->pin_ev);
     if (c->stream) (void)hipStreamDestroy(c->stream);
     delete c;
 }
