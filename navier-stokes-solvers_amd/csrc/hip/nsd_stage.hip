@@ -239,12 +239,13 @@ int col_fused_blocks(int L, int ncols) {
     return (ncols + lines - 1) / lines;
 }
 template int col_fused_blocks<NSD_T>(int, int);
-// Variant a context starts with, for `lines` lines (row pairs or kept columns,
-// times batch members) of length L on a grid whose longer side is `side`.
-// Launches that variant 0 would leave with at most one wave per SIMD (1024 on
-// this device) take the field-parallel kernels or, on FP32 grids below 512^2,
-// variant 0's own code in the smallest workgroups.  us per RK4 step of one field
-// as graph replays, variant 0 -> smallest workgroups -> field-parallel:
+// Variant a context starts with, for `lines` lines (row pairs, kind 0, or kept
+// columns, kind 1, times batch members) of length L on a grid whose longer side is
+// `side`.  `waves`: what variant 0 would launch (the device holds 1024 SIMDs).
+//
+// Launches that leave at most one wave per SIMD take the field-parallel kernels
+// or, on FP32 grids below 512^2, variant 0's own code in the smallest workgroups.
+// us per RK4 step of one field, variant 0 -> smallest workgroups -> field-parallel:
 //   64^2 FP64 72 -> 56 -> 49, 512^2 FP64 120 -> - -> 69, 1024^2 FP64 188 -> 172 -> 149,
 //   256^2 FP32 98 -> 81 -> 67, 512^2 FP32 103 -> 85 -> 71, 1024^2 FP32 140 -> 130 -> 124.
 // The small FP32 grids keep variant 0's code because its rounding is theirs: a
@@ -253,14 +254,33 @@ template int col_fused_blocks<NSD_T>(int, int);
 // compared with one another bit for bit.  Lines of 2048 stay with variant 0: a
 // unit is 1024 threads there, one to a compute unit at FP64, and 256 row pairs
 // take 22.0 us against 20.9 us.
+//
+// Larger launches (us per step; 0, fields, 4: variant 0, field-parallel, half-size
+// workgroups, of the rows or columns named, variant 0 for the others):
+//   FP64 rows: 512 x 16 members 0 310.5, fields 288.9, 4 303.2; 1024 x 24 2073, 1801,
+//     1985; 256 x 100 442.6, 439.3, 418.5; 128 x 300 318.0, 343.2, 308.7.
+//   FP64 columns: 128 x 300 318.0, 297.5, 320.2; 256 x 300 1249, 1185, 1210; 512 x 80
+//     1411, 1346, 1356; 1024 x 4 368.8, 341.0, 350.7; 1024 x 24 2073, 1984, 1962.
+//   FP32 rows: 1024 x 4 192.6, 189.7, 190.1; 1024 x 8 311.0, 321.9, 311.2; 512 x 8
+//     129.9, 133.2, 132.2.
+//   FP32 columns: 512 x 8 129.9, 116.0, 126.4; 512 x 24 217.6, 211.5, 209.2; 1024 x 2
+//     154.6, 149.1, 146.5; 1024 x 16 566.8, 632.5, 552.6.
+//   FP32 below 512^2, both with variant 4: 256 x 32 126.8 -> 121.0, 128 x 120 121.9 -> 114.7.
 template <typename T>
-int stage_variant_default(int L, long lines, int side, int maxlds) {
+int stage_variant_default(int kind, int L, long lines, int side, int maxlds) {
     const long waves = lines * (L / P) / 64;
-    if (waves > 1024 || L > kFieldsMax) return 0;
-    if (sizeof(T) == 4 && side < 512) return kSmallVariant;
-    return fields_fits<T>(L, maxlds) ? kFieldsVariant : 0;
+    if (L > kFieldsMax) return 0;
+    const bool many = waves > 1024;
+    if (L < 64 && many) return 0;
+    const int half = stage_variant_valid<T>(L, 4, maxlds) ? 4 : 0;
+    if (sizeof(T) == 4 && side < 512) return many ? half : kSmallVariant;
+    bool fields;
+    if (sizeof(T) == 8) fields = !many || (kind == 0 ? L >= 512 : L <= 512 || waves <= 4096);
+    else fields = waves <= (kind == 0 ? (L == 1024 ? 4096 : 1024) : (L == 512 ? 2048 : 1024));
+    if (fields) return fields_fits<T>(L, maxlds) ? kFieldsVariant : 0;
+    return sizeof(T) == 8 || kind == 1 ? half : 0;
 }
-template int stage_variant_default<NSD_T>(int, long, int, int);
+template int stage_variant_default<NSD_T>(int, int, long, int, int);
 template int stage_variant_valid<NSD_T>(int, int, int);
 template int stage_variant_pairs<NSD_T>(int, int);
 template void stage_lds_limits<NSD_T>(int);
