@@ -6,6 +6,9 @@ stage kernels, whose layouts of the mixed fields and of J have to meet.  The
 tolerance is FP32 round-off: one step at 4096^2 differs by 7.7e-8 relative L2,
 and a layout, a mode or a twiddle that is wrong differs by 1e-3 and more, so
 1e-6 bounds two steps."""
+import ctypes as C
+import importlib
+
 import numpy as np
 import pytest
 
@@ -159,3 +162,34 @@ def test_long_calls_are_single_steps(ns, n, fp32, forced):
                 b.check(b.advance_n(1, True))
             assert a.d.t == b.d.t
             assert np.array_equal(state(a), state(b))
+
+
+# starting variants of batches on either side of the rule's lines, against variant 0:
+# FP64 rows and columns of 512 and 1024 points at more than one and more than four
+# waves per SIMD, 64 to 256 past one; FP32 the same, with equal bits below 512^2
+@pytest.mark.parametrize("n,members,fp32", [
+    (1024, 2, False), (1024, 7, False), (512, 5, False), (256, 17, False), (128, 70, False),
+    (64, 260, False), (1024, 2, True), (1024, 7, True), (512, 7, True), (512, 13, True),
+    (256, 17, True), (128, 70, True), (64, 260, True), (32, 600, True)])
+def test_starting_variants_of_batches(ns, n, members, fp32):
+    closure = importlib.import_module("navier-stokes-solvers_amd.closure")
+    L = ns.load()
+    prec = ns.NSD_FP32 if fp32 else ns.NSD_FP64
+    picks = (0, members // 2, members - 1)
+    out = []
+    for general in (False, True):
+        h = closure.context(n, prec, members, seeds=range(1, members + 1))
+        seeds = (C.c_ulonglong * members)(*range(1, members + 1))
+        assert L.nsd_batch_random_phase(h, seeds, 5.0, 1.0) == 0
+        if general:
+            assert L.nsd_set_variants(h, 0, 0) == 0
+        assert L.nsd_advance_graph(h, 5, 1) == 0
+        got = np.zeros((len(picks), n, n // 2 + 1), np.complex128)
+        for i, m in enumerate(picks):
+            assert L.nsd_member_download(h, m, got[i].ctypes.data_as(ns.c_double_p)) == 0
+        L.nsd_destroy(h)
+        out.append(got)
+    if fp32 and n < 512:
+        assert np.array_equal(out[0], out[1])
+    # five steps of rounding on either side
+    assert rel_l2(out[0], out[1]) <= (2e-6 if fp32 else 1e-14)
