@@ -11,8 +11,8 @@ Workload (the 4096^2 forced-turbulence case the headline metric is quoted on):
 
 A step is one full RK4 step (4 x {row kernel, column kernel} + the forcing
 draw) over the whole grid, state resident in HBM.  The timed region runs K
-steps the way ns_spectral_advance_n does, one captured step graph replayed K
-times (eager launches with --no-graph), host clock, the solver's stream
+steps the way ns_spectral_advance_n does, captured step graphs replayed
+(eager launches with --no-graph), host clock, the solver's stream
 synchronized on both sides.  The same K steps are then launched eagerly, and
 K more with a HIP event around every stage kernel on the solver's stream:
 the per-kernel averages give the roofline of the dominant kernel.  Prints one
@@ -100,8 +100,8 @@ def time_gpu(ns, n, fp32, steps, warmup, probe=False, compat=0, graph=True, ramp
     if warmup:
         s.check(L.nsd_advance_graph(ctx, warmup, 1) if graph else L.nsd_advance(ctx, warmup, 1))
     s.check(L.nsd_synchronize(ctx))
-    # timed region: K steps through the path of ns_spectral_advance_n (one
-    # captured step graph replayed K times; eager launches with graph=False),
+    # timed region: K steps through the path of ns_spectral_advance_n
+    # (captured step graphs replayed; eager launches with graph=False),
     # the solver's stream synchronized on both sides, host clock (nothing else
     # on the stream)
     t0 = time.perf_counter()

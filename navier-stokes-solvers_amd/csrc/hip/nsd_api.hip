@@ -1185,6 +1185,7 @@ int op_advance(NsdContext* c, int nsteps, int adaptive) {
 template <typename T>
 int capture_steps(NsdContext* c, StepGraph* g, int steps, int adaptive) {
     if (g->exec && g->adaptive == adaptive && g->gen == c->gen) return ST_OK;
+    if (g->exec) CK(hipStreamSynchronize(c->stream));  // its last replay may still run
     g->reset();
     const int prof = c->prof;
     c->prof = 0;
