@@ -260,7 +260,8 @@ template int col_fused_blocks<NSD_T>(int, int);
 //   FP64 rows: 512 x 16 members 0 310.5, fields 288.9, 4 303.2; 1024 x 24 2073, 1801,
 //     1985; 256 x 100 442.6, 439.3, 418.5; 128 x 300 318.0, 343.2, 308.7.
 //   FP64 columns: 128 x 300 318.0, 297.5, 320.2; 256 x 300 1249, 1185, 1210; 512 x 80
-//     1411, 1346, 1356; 1024 x 4 368.8, 341.0, 350.7; 1024 x 24 2073, 1984, 1962.
+//     1411, 1346, 1356; 2048 x 1024 grid, classic scheme 233.0, 261.5, 219.0,
+//     integrating factor 226.5, 226.5, 212.2; 4096 x 1024 473.7, 511.3, 465.1.
 //   FP32 rows: 1024 x 4 192.6, 189.7, 190.1; 1024 x 8 311.0, 321.9, 311.2; 512 x 8
 //     129.9, 133.2, 132.2.
 //   FP32 columns: 512 x 8 129.9, 116.0, 126.4; 512 x 24 217.6, 211.5, 209.2; 1024 x 2
@@ -275,7 +276,7 @@ int stage_variant_default(int kind, int L, long lines, int side, int maxlds) {
     const int half = stage_variant_valid<T>(L, 4, maxlds) ? 4 : 0;
     if (sizeof(T) == 4 && side < 512) return many ? half : kSmallVariant;
     bool fields;
-    if (sizeof(T) == 8) fields = !many || (kind == 0 ? L >= 512 : L <= 512 || waves <= 4096);
+    if (sizeof(T) == 8) fields = !many || (kind == 0 ? L >= 512 : L <= 512);
     else fields = waves <= (kind == 0 ? (L == 1024 ? 4096 : 1024) : (L == 512 ? 2048 : 1024));
     if (fields) return fields_fits<T>(L, maxlds) ? kFieldsVariant : 0;
     return sizeof(T) == 8 || kind == 1 ? half : 0;
