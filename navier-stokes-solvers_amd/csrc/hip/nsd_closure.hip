@@ -397,16 +397,23 @@ __global__ __launch_bounds__(512, 4) void k_conv_tile2(ConvArgs a, int ntiles) {
     };
     int t = blockIdx.x;
     if (t >= ntiles) return;
-    // weights: row m of block nb, 8 input channels 8 kq .. of each tap
+    // weights: row m of block nb, 8 input channels 8 kq .. of each tap; the layers with
+    // 32 outputs pass them once through a patch buffer (each wave needs all 18 KB),
+    // transposed from w[kc][tap][nn] for the input gradient.  Straight from memory
+    // into each wave's registers cost a workgroup with one tile about 0.8 us (15
+    // members of 32^2: evaluation 32.6 -> 29.4 us)
     s8 bv[KP / 32][NP / 16];
-    if constexpr (MODE == CONV_BWD_DATA) {
-        // w[kc][tap][nn] transposed through the patch buffers
-        static_assert(NP * KP <= PR * PC * KC, "the weights fit a patch buffer");
+    if constexpr (NN == 32) {
+        static_assert(NN * KP <= PR * PC * KC, "the weights fit a patch buffer");
         for (int e = tid; e < KP * NN / 8; e += 512) {
-            const int row = e >> 2, tap = row % 9, kc = row / 9, n0 = 8 * (e & 3);
-            const s8 v = *reinterpret_cast<const s8*>(&a.w[row * NN + n0]);
+            const s8 v = *reinterpret_cast<const s8*>(&a.w[8 * e]);
+            if constexpr (MODE == CONV_BWD_DATA) {
+                const int row = e >> 2, tap = row % 9, kc = row / 9, n0 = 8 * (e & 3);
 #pragma unroll
-            for (int i = 0; i < 8; ++i) X0[(n0 + i) * KP + tap * KC + kc] = (bf16)v[i];
+                for (int i = 0; i < 8; ++i) X0[(n0 + i) * KP + tap * KC + kc] = (bf16)v[i];
+            } else {
+                *reinterpret_cast<s8*>(&X1[8 * e]) = v;
+            }
         }
         __syncthreads();
     }
@@ -417,8 +424,8 @@ __global__ __launch_bounds__(512, 4) void k_conv_tile2(ConvArgs a, int ntiles) {
             const int nn = NN == 32 ? tile_channel(nb, m) : m;
             bv[c][nb] = s8{0, 0, 0, 0, 0, 0, 0, 0};
             if (nn < NN)
-                bv[c][nb] = *reinterpret_cast<const s8*>(
-                    (MODE == CONV_BWD_DATA ? X0 : a.w) + nn * KP + c * 32 + 8 * kq);
+                bv[c][nb] = *reinterpret_cast<const s8*>((NN == 1 ? a.w : MODE == CONV_BWD_DATA ? X0 : X1) + nn * KP + c * 32 +
+                                                         8 * kq);
         }
     // biases in LDS: a global load in the loop would wait for the patch loads in
     // flight (the vector memory counter retires in order), and the registers are
