@@ -137,9 +137,9 @@ int nsd_member_download(NsdContext *c, int member, double *omega_hat);
  * four transforms run side by side; lengths 64..1024 have several; a context
  * starts with the field-parallel ones where its launches are small).
  * nsd_autotune times every variant on this context's shape (reps launches
- * each) and keeps the fastest; results are cached per (length, precision,
+ * each) and keeps the fastest; results are cached per (grid, precision,
  * batch members) for the process and, if the environment names a file in
- * NSD_TUNE_FILE (lines "row|col L precision members variant"),
+ * NSD_TUNE_FILE (lines "row|col NXxNY precision members variant"),
  * across processes (force != 0 re-times).  It zeroes the state: call it
  * before setting the initial field.  Every variant gives identical results. */
 int nsd_autotune(NsdContext *c, int reps, int force, int *row_variant, int *col_variant);

@@ -1480,12 +1480,13 @@ int op_gather_prime(NsdContext* c, const double* in_ref) {
 
 // ----------------------------------------------------------------- autotuner
 
-// Tuned launch variants per (kernel, transform length, precision, batch
-// members): the best launch shape depends on how many workgroups the batch
-// gives the device.  Timed once per process, optionally persisted in the text
-// file named by NSD_TUNE_FILE (lines "row|col L precision members variant";
-// lines of another form are skipped).
-using TuneKey = std::tuple<int, int, int, int>;
+// Tuned launch variants per (kernel, nx, ny, precision, batch members): the best
+// launch shape depends on how many workgroups the batch gives the device, which
+// the length of the transforms alone does not tell.  Timed once per process,
+// optionally persisted in the text file named by NSD_TUNE_FILE (lines "row|col
+// NXxNY precision members variant"; lines of another form are skipped, and an
+// entry whose variant this launch cannot take is timed again).
+using TuneKey = std::tuple<int, int, int, int, int>;
 std::mutex g_tune_mu;
 std::map<TuneKey, int> g_tune;
 bool g_tune_loaded = false;
@@ -1498,21 +1499,34 @@ void tune_load() {
     FILE* fp = fopen(f, "r");
     if (!fp) return;
     char line[128], kind[8];
-    int L, prec, nb, v;
+    int nx, ny, prec, nb, v;
     while (fgets(line, sizeof(line), fp))
-        if (sscanf(line, "%7s %d %d %d %d", kind, &L, &prec, &nb, &v) == 5)
-            g_tune[TuneKey(strcmp(kind, "col") == 0 ? 1 : 0, L, prec, nb)] = v;
+        if (sscanf(line, "%7s %dx%d %d %d %d", kind, &nx, &ny, &prec, &nb, &v) == 6)
+            g_tune[TuneKey(strcmp(kind, "col") == 0 ? 1 : 0, nx, ny, prec, nb)] = v;
     fclose(fp);
 }
 
-void tune_store(int kind, int L, int prec, int nb, int v) {
-    g_tune[TuneKey(kind, L, prec, nb)] = v;
+TuneKey tune_key(const NsdContext* c, int kind) {
+    return TuneKey(kind, c->G.nx, c->G.ny, c->prec, c->nb);
+}
+
+void tune_store(const NsdContext* c, int kind, int v) {
+    g_tune[tune_key(c, kind)] = v;
     const char* f = getenv("NSD_TUNE_FILE");
     if (!f) return;
     FILE* fp = fopen(f, "a");
     if (!fp) return;
-    fprintf(fp, "%s %d %d %d %d\n", kind ? "col" : "row", L, prec, nb, v);
+    fprintf(fp, "%s %dx%d %d %d %d\n", kind ? "col" : "row", c->G.nx, c->G.ny, c->prec, c->nb, v);
     fclose(fp);
+}
+
+// whether the tuner may give variant v to this context's kernel (FP32 grids below
+// 512^2 do without the field-parallel ones: stage_variant_default has the reason)
+template <typename T>
+bool tunable(const NsdContext* c, int kind, int v) {
+    const bool small32 = sizeof(T) == 4 && std::max(c->G.nx, c->G.ny) < 512;
+    return v >= 0 && v < kStageVariants && !(small32 && v == kFieldsVariant) &&
+           stage_variant_valid<T>(kind == 0 ? c->G.nx : c->G.ny, v, c->maxlds);
 }
 
 // zero every field and scalar the step reads, so that timing runs leave a
@@ -1533,7 +1547,6 @@ int op_autotune(NsdContext* c, int reps, int force) {
     hipEvent_t e0, e1;
     CK(hipEventCreate(&e0));
     CK(hipEventCreate(&e1));
-    const int prec = c->prec;
     for (int kind = 0; kind < 2; ++kind) {
         const int L = kind == 0 ? c->G.nx : c->G.ny;
         int best = 0;
@@ -1541,16 +1554,14 @@ int op_autotune(NsdContext* c, int reps, int force) {
         {
             std::lock_guard<std::mutex> lk(g_tune_mu);
             tune_load();
-            auto it = g_tune.find(TuneKey(kind, L, prec, c->nb));
-            if (it != g_tune.end() && !force) {
+            auto it = g_tune.find(tune_key(c, kind));
+            if (it != g_tune.end() && !force && tunable<T>(c, kind, it->second)) {
                 best = it->second;
                 cached = true;
             }
         }
         // a launch that starts with the field-parallel kernels keeps them, as a
-        // single context of its size does: nothing to time.  FP32 grids below
-        // 512^2 do without them (stage_variant_default has the reason)
-        const bool small32 = sizeof(T) == 4 && std::max(c->G.nx, c->G.ny) < 512;
+        // single context of its size does: nothing to time
         if (!cached && default_variant<T>(c, kind) == kFieldsVariant) {
             best = kFieldsVariant;
             cached = true;
@@ -1558,8 +1569,7 @@ int op_autotune(NsdContext* c, int reps, int force) {
         if (!cached) {
             float best_ms = 1e30f;
             for (int v = 0; v < kStageVariants; ++v) {
-                if (!stage_variant_valid<T>(L, v, c->maxlds)) continue;
-                if (small32 && v == kFieldsVariant) continue;
+                if (!tunable<T>(c, kind, v)) continue;
                 auto launch = [&]() {
                     if (kind == 0) {
                         RowArgs<T> r = row_args<T>(c);
@@ -1588,7 +1598,7 @@ int op_autotune(NsdContext* c, int reps, int force) {
                 }
             }
             std::lock_guard<std::mutex> lk(g_tune_mu);
-            tune_store(kind, L, prec, c->nb, best);
+            tune_store(c, kind, best);
         }
         if (kind == 0) c->vrow = best;
         else c->vcol = best;
