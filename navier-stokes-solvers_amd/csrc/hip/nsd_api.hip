@@ -1635,7 +1635,13 @@ namespace {
 
 int multi_capture(NsdMulti* mh, int adaptive) {
     NsdContext* c0 = mh->cs[0];
-    if (mh->gexec) (void)hipGraphExecDestroy(mh->gexec);
+    if (mh->gexec) {  // its last replay may still run
+        if (hipStreamSynchronize(c0->stream) != hipSuccess) {
+            mh->err = "hipStreamSynchronize failed";
+            return ST_MEM;
+        }
+        (void)hipGraphExecDestroy(mh->gexec);
+    }
     if (mh->graph) (void)hipGraphDestroy(mh->graph);
     mh->gexec = nullptr;
     mh->graph = nullptr;
