@@ -550,7 +550,7 @@ __global__ void k_scale_state(size_t n, cx<T>* st, const DevScalars* sc, double 
 // restoring steps draw nothing
 __global__ void k_force(ForceArgs a) {
     if (a.skip_on_redo && a.sc[blockIdx.y].redo) return;
-    __shared__ double red[17];
+    __shared__ double red[kForceRed];
     force_draw(a, blockIdx.y, red);
 }
 

@@ -497,7 +497,33 @@ struct ForceArgs {
     int skip_on_redo;                  // error controller: no draw on a restoring step
 };
 
-// The draw for member mb, by one workgroup; red: 17 doubles of LDS.
+// Sums over the modes are formed over 256 lanes, whatever the workgroup, so that a
+// draw's bits do not depend on the launch that makes it: lane v adds the modes v,
+// v + 256, ..., and the four waves' sums are added in order.
+constexpr int kForceLanes = 256;
+
+// term(r) over the modes r < A, the waves' sums in red[0 .. 3]; every thread of a
+// workgroup of whole waves calls it
+template <typename F>
+__device__ __forceinline__ void force_sum(int A, double* red, F&& term) {
+    for (int v = threadIdx.x; v < kForceLanes; v += blockDim.x) {
+        double part = 0.0;
+        if ((v & ~63) < A) {
+            for (int r = v; r < A; r += kForceLanes) part += term(r);
+            part = wave_sum(part);
+        }
+        if ((v & 63) == 0) red[v >> 6] = part;
+    }
+    __syncthreads();
+}
+__device__ __forceinline__ double force_total(const double* red) {
+    double t = 0.0;
+    for (int i = 0; i < kForceLanes / 64; ++i) t += red[i];
+    return t;
+}
+
+// The draw for member mb, by one workgroup; red: kForceRed doubles of LDS.
+constexpr int kForceRed = kForceLanes / 64 + 1;
 __device__ __forceinline__ void force_draw(const ForceArgs& a, int mb, double* red) {
     const Geo& G = a.geo;
     // member mb of a batch: its own generator, OU state, box and scalars
@@ -510,15 +536,14 @@ __device__ __forceinline__ void force_draw(const ForceArgs& a, int mb, double* r
     const unsigned long long seed = a.m_seed ? a.m_seed[mb] : a.seed;
     const unsigned long long c = dsc->fcount;
     const double dt = dsc->dt;
-    double& s_scale = red[16];
+    double& s_scale = red[kForceLanes / 64];
     double alpha = 0.0, beta = 1.0;
     if (a.colored) {
         const double tau = fmax(a.tau, 1e-6);
         alpha = exp(-dt / tau);
         beta = sqrt(fmax(1.0 - alpha * alpha, 0.0));
     }
-    double part = 0.0;
-    for (int r = threadIdx.x; r < a.A; r += blockDim.x) {
+    force_sum(a.A, red, [&](int r) {
         const unsigned long long k = 2ull * (c * (unsigned long long)a.A + r) + 1ull;
         double u1 = uniform_at(seed, k), u2 = uniform_at(seed, k + 1);
         u1 = fmax(u1, 2.2250738585072014e-308);
@@ -531,17 +556,9 @@ __device__ __forceinline__ void force_draw(const ForceArgs& a, int mb, double* r
         }
         work[2 * r] = vr;
         work[2 * r + 1] = vi;
-        part += vr * vr + vi * vi;
-    }
-    part = wave_sum(part);
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = part;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        double t = 0.0;
-        for (int i = 0; i < (int)(blockDim.x >> 6); ++i) t += red[i];
-        t = fmax(t, 1e-16);
-        s_scale = sqrt(a.energy_target / t);
-    }
+        return vr * vr + vi * vi;
+    });
+    if (threadIdx.x == 0) s_scale = sqrt(a.energy_target / fmax(force_total(red), 1e-16));
     __syncthreads();
     const double sc = s_scale;
     for (int r = threadIdx.x; r < a.A; r += blockDim.x) {
@@ -554,9 +571,8 @@ __device__ __forceinline__ void force_draw(const ForceArgs& a, int mb, double* r
     }
     __syncthreads();
     // Hermitian projection + mask, rate of the projected field
-    double rate = 0.0;
     double* pr = work + 2 * a.A;  // projected values
-    for (int r = threadIdx.x; r < a.A; r += blockDim.x) {
+    force_sum(a.A, red, [&](int r) {
         const int idx = a.modes[r];
         const int jy = idx / G.nkx, i = idx % G.nkx;
         double fr = work[2 * r], fi = work[2 * r + 1];
@@ -575,15 +591,10 @@ __device__ __forceinline__ void force_draw(const ForceArgs& a, int mb, double* r
         pr[2 * r] = fr;
         pr[2 * r + 1] = fi;
         const double wt = (i == 0 || 2 * i == G.nx) ? 1.0 : 2.0;
-        if (k2 > 1e-12) rate += 0.5 * wt * (fr * fr + fi * fi) / k2;
-    }
-    rate = wave_sum(rate);
-    __syncthreads();
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = rate;
-    __syncthreads();
+        return k2 > 1e-12 ? 0.5 * wt * (fr * fr + fi * fi) / k2 : 0.0;
+    });
     if (threadIdx.x == 0) {
-        double t = 0.0;
-        for (int i = 0; i < (int)(blockDim.x >> 6); ++i) t += red[i];
+        const double t = force_total(red);
         s_scale = (t > 0.0 && a.rate > 0.0) ? sqrt(a.rate / t) : 0.0;
     }
     __syncthreads();
