@@ -546,8 +546,8 @@ __global__ void k_scale_state(size_t n, cx<T>* st, const DevScalars* sc, double 
         st[q] = s * st[q];
 }
 
-// The draw as a kernel of its own: steps under the error controller, whose
-// restoring steps draw nothing
+// The draw as a kernel of its own: wide shells, and steps under the error
+// controller, whose restoring steps draw nothing
 __global__ void k_force(ForceArgs a) {
     if (a.skip_on_redo && a.sc[blockIdx.y].redo) return;
     __shared__ double red[kForceRed];
@@ -999,8 +999,21 @@ int op_prime(NsdContext* c) {
 
 bool force_active(const NsdContext* c) { return c->phys.force_on && c->fA != 0; }
 
+// Whether the row kernel's extra workgroup makes the draw in about the time that
+// the others take: it has one pass (1.7 us) over the modes per workgroup's worth of
+// them.  us per step, in the row kernel -> a kernel of up to 1024 threads in line:
+//   64 threads: 256^2 FP32 130 modes 62.9 -> 64.1, 270 67.8 -> 65.2, 1400 106 -> 71
+//   256: 512^2 FP64 1400 modes 74.9 -> 74.9, 2500 85.6 -> 81.6; 2048^2 FP32 2500 192 -> 197,
+//     5600 229 -> 220
+//   512: 1024^2 FP32 2500 modes 110 -> 116, 5600 136 -> 137; 4096^2 FP32 5600 584 -> 612
 template <typename T>
-ForceArgs force_args(const NsdContext* c) {
+bool draw_in_rows(const NsdContext* c) {
+    const int passes = std::max(3, std::max(c->G.nx, c->G.ny) / 128);
+    return c->fA <= passes * row_stage_threads<T>(c->G.nx, c->vrow);
+}
+
+template <typename T>
+ForceArgs force_args(const NsdContext* c, bool ec) {
     ForceArgs f;
     memset(&f, 0, sizeof(f));
     f.geo = c->G;
@@ -1020,7 +1033,7 @@ ForceArgs force_args(const NsdContext* c) {
     f.fbox = c->fbox;
     f.sc = c->sc;
     f.m_seed = c->m_seed;
-    f.skip_on_redo = c->phys.errctl ? 1 : 0;
+    f.skip_on_redo = ec ? 1 : 0;
     return f;
 }
 
@@ -1050,8 +1063,8 @@ void enqueue_stage(NsdContext* c, int s, int adaptive) {
     // the forcing counter).  us per step against a kernel of its own on a side
     // stream (whose fork and join cost more than its 5 us) and in line: 256^2
     // FP32 81 / 68 / 63, 2048^2 FP32 206 / 200 / 194, 4096^2 FP32 568 / 579 / 556.
-    const bool draw = s == 1 && force_active(c) && !ec;
-    if (draw) r.force = force_args<T>(c);
+    const bool draw = s == 1 && force_active(c) && !ec && draw_in_rows<T>(c);
+    if (draw) r.force = force_args<T>(c, ec);
     if (prof) (void)hipEventRecord(c->evs[e0], c->stream);
     launch_row_t<T>(c, r, c->G.ny / 2, ec, draw);
     if (prof) (void)hipEventRecord(c->evs[e0 + 1], c->stream);
@@ -1133,9 +1146,9 @@ void enqueue_step(NsdContext* c, int adaptive) {
     if (c->closure) enqueue_closure<T>(c);
     for (int s = 0; s < 4; ++s) {
         enqueue_stage<T>(c, s, adaptive);
-        if (s == 0 && ec && force_active(c))
-            hipLaunchKernelGGL(k_force, dim3(1, c->nb), dim3(256), 0, c->stream,
-                               force_args<T>(c));
+        if (s == 0 && force_active(c) && (ec || !draw_in_rows<T>(c)))
+            hipLaunchKernelGGL(k_force, dim3(1, c->nb), dim3(c->fA > 256 ? 1024 : 256), 0,
+                               c->stream, force_args<T>(c, ec));
     }
 }
 

@@ -14,7 +14,7 @@ namespace {
 
 // whole units of L / 2 threads in workgroups of 256 where they fit
 template <int L>
-constexpr int fields_units() { return L <= 512 ? 512 / L : 1; }
+constexpr int fields_units() { return row_fields_threads(L) / (L / 2); }
 // occupancy floor (waves per SIMD): what the lines' LDS leaves room for, and at
 // FP64 the register budget that the rows of up to 512 points need
 template <typename T, int L>

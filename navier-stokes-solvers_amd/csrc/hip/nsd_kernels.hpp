@@ -497,19 +497,20 @@ struct ForceArgs {
     int skip_on_redo;                  // error controller: no draw on a restoring step
 };
 
-// Sums over the modes are formed over 256 lanes, whatever the workgroup, so that a
-// draw's bits do not depend on the launch that makes it: lane v adds the modes v,
-// v + 256, ..., and the four waves' sums are added in order.
+// Sums over the modes are formed over 256 lanes, whatever the workgroup, with the
+// products' roundings written out, so that a draw's bits do not depend on the launch
+// that makes it: lane v adds the modes v, v + 256, ..., and the four waves' sums are
+// added in order.
 constexpr int kForceLanes = 256;
 
-// term(r) over the modes r < A, the waves' sums in red[0 .. 3]; every thread of a
+// add(sum, r) over the modes r < A, the waves' sums in red[0 .. 3]; every thread of a
 // workgroup of whole waves calls it
 template <typename F>
-__device__ __forceinline__ void force_sum(int A, double* red, F&& term) {
+__device__ __forceinline__ void force_sum(int A, double* red, F&& add) {
     for (int v = threadIdx.x; v < kForceLanes; v += blockDim.x) {
         double part = 0.0;
         if ((v & ~63) < A) {
-            for (int r = v; r < A; r += kForceLanes) part += term(r);
+            for (int r = v; r < A; r += kForceLanes) part = add(part, r);
             part = wave_sum(part);
         }
         if ((v & 63) == 0) red[v >> 6] = part;
@@ -543,7 +544,7 @@ __device__ __forceinline__ void force_draw(const ForceArgs& a, int mb, double* r
         alpha = exp(-dt / tau);
         beta = sqrt(fmax(1.0 - alpha * alpha, 0.0));
     }
-    force_sum(a.A, red, [&](int r) {
+    for (int r = threadIdx.x; r < a.A; r += blockDim.x) {
         const unsigned long long k = 2ull * (c * (unsigned long long)a.A + r) + 1ull;
         double u1 = uniform_at(seed, k), u2 = uniform_at(seed, k + 1);
         u1 = fmax(u1, 2.2250738585072014e-308);
@@ -556,7 +557,11 @@ __device__ __forceinline__ void force_draw(const ForceArgs& a, int mb, double* r
         }
         work[2 * r] = vr;
         work[2 * r + 1] = vi;
-        return vr * vr + vi * vi;
+    }
+    __syncthreads();
+    force_sum(a.A, red, [&](double t, int r) {
+        const double vr = work[2 * r], vi = work[2 * r + 1];
+        return fma(vr, vr, fma(vi, vi, t));
     });
     if (threadIdx.x == 0) s_scale = sqrt(a.energy_target / fmax(force_total(red), 1e-16));
     __syncthreads();
@@ -572,7 +577,7 @@ __device__ __forceinline__ void force_draw(const ForceArgs& a, int mb, double* r
     __syncthreads();
     // Hermitian projection + mask, rate of the projected field
     double* pr = work + 2 * a.A;  // projected values
-    force_sum(a.A, red, [&](int r) {
+    for (int r = threadIdx.x; r < a.A; r += blockDim.x) {
         const int idx = a.modes[r];
         const int jy = idx / G.nkx, i = idx % G.nkx;
         double fr = work[2 * r], fi = work[2 * r + 1];
@@ -590,8 +595,16 @@ __device__ __forceinline__ void force_draw(const ForceArgs& a, int mb, double* r
         if (!kept(G, i, jy) || k2 <= 1e-12) fr = fi = 0.0;
         pr[2 * r] = fr;
         pr[2 * r + 1] = fi;
+    }
+    __syncthreads();
+    force_sum(a.A, red, [&](double t, int r) {
+        const int idx = a.modes[r];
+        const int jy = idx / G.nkx, i = idx % G.nkx;
+        const double fr = pr[2 * r], fi = pr[2 * r + 1];
+        const double kx = kx_of(G, i), ky = ky_of(G, jy);
+        const double k2 = kx * kx + ky * ky;
         const double wt = (i == 0 || 2 * i == G.nx) ? 1.0 : 2.0;
-        return k2 > 1e-12 ? 0.5 * wt * (fr * fr + fi * fi) / k2 : 0.0;
+        return k2 > 1e-12 ? t + 0.5 * wt * fma(fr, fr, fi * fi) / k2 : t;
     });
     if (threadIdx.x == 0) {
         const double t = force_total(red);

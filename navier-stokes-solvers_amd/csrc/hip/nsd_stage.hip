@@ -142,6 +142,14 @@ int var_valid(int maxlds) {
     return 0;
 }
 
+template <typename T, int LOG, int V>
+int row_threads() {
+    constexpr int L = 1 << LOG;
+    if constexpr (V == kFieldsVariant) return row_fields_threads(L);
+    else if constexpr (var_ok<L, V>()) return var_nt<L, V>();
+    return 0;
+}
+
 int log2i(int L) {
     int l = 0;
     while ((1 << l) < L) ++l;
@@ -214,6 +222,19 @@ int stage_variant_pairs(int L, int variant) {
 #undef V_
     return 0;
 }
+
+template <typename T>
+int row_stage_threads(int L, int variant) {
+    const int lg = log2i(L);
+#define V_(n, v) \
+    if (lg == n && variant == v) return row_threads<T, n, v>();
+#define X(n) NSD_FOR_VARS(V_, n)
+    NSD_FOR_LOGS(X)
+#undef X
+#undef V_
+    return 0;
+}
+template int row_stage_threads<NSD_T>(int, int);
 
 template <typename T>
 void stage_lds_limits(int bytes) {

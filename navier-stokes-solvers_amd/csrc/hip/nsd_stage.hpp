@@ -32,6 +32,9 @@ int col_fused_blocks(int L, int ncols);
 // row pairs, 1: columns) of a grid whose longer side is `side`
 template <typename T>
 int stage_variant_default(int kind, int L, long lines, int side, int maxlds);
+// threads of a workgroup of that row launch
+template <typename T>
+int row_stage_threads(int L, int variant);
 // 1 if `variant` exists for length L and fits `maxlds` bytes of LDS
 template <typename T>
 int stage_variant_valid(int L, int variant, int maxlds);
@@ -45,6 +48,8 @@ void launch_row_fields(const RowArgs<T>& a, int L, int items, int members, hipSt
                        bool force);
 template <typename T>
 void launch_col_fields(const ColArgs<T>& a, int L, int ncols, int members, hipStream_t st);
+// threads of a workgroup of theirs
+constexpr int row_fields_threads(int L) { return L <= 512 ? 256 : L / 2; }
 // whether they take lines of length L with `maxlds` bytes of LDS
 template <typename T>
 bool fields_fits(int L, int maxlds);
