@@ -1,0 +1,54 @@
+"""Plain steps behind a call of the error controller whose last candidate was rejected:
+the state is the accepted one again, and a plain step makes its own forcing draw."""
+import numpy as np
+import pytest
+
+from conftest import rel_l2
+
+pytestmark = pytest.mark.gpu
+TWO_PI = 2 * np.pi
+
+
+# 37 modes, drawn in the row kernel, and 623, by a kernel of their own
+@pytest.mark.parametrize("kmax", [6.0, 20.0])
+def test_plain_steps_after_a_rejected_candidate(ns, oc, kmax):
+    n, steps, rate = 64, 3, 1e-3
+    hv = dict(enabled=1, coefficient=1e-16 * (np.sqrt(2) * n / 2) ** 8, order=8, cutoff_ratio=0.0)
+    o = oc.Oracle(n, n, TWO_PI, TWO_PI, 1e4)
+    o.init_grids()
+    o.hv_set(**hv)
+    o.d.drag = 0.1
+    o.d.cfl_factor = 0.5
+    o.init_random_phase(42, 10.0, 1.0)
+    gen = oc.OracleForcing(o.k2, n // 2 + 1, n, 4.0, kmax, energy_target=1.0, seed=42)
+    ctl = oc.OracleErrorControl(o, 1e-6, 0.0, 0.9, 1e-8, 0.1, integrating_factor=True,
+                                forcing=gen, rate=rate)
+    ctl.attempt()
+    ctl.finish()
+    assert ctl.rejected == 1  # the restored state is the initial field
+    w0 = o.spec("omega_hat").copy()
+    for _ in range(steps):
+        o.advance_if(o.project_forcing(gen.generate(o.d.dt), rate))
+
+    s = ns.Spectral(n, n, TWO_PI, TWO_PI, 1e4)
+    s.init(taylor_green=False)
+    s.hv_set(**hv)
+    s.set_scheme(True)
+    s.set_drag(0.1)
+    s.set_forcing(4.0, kmax, rate, seed=42)
+    s.d.cfl_factor = 0.5
+    s.set_error_control(1e-6, 0.0, 0.9, 1e-8, 0.1)
+    s.random_phase(42, k_peak=10.0, energy=1.0)
+    s.sync_device()
+    assert s.advance_n(1, True) == 0
+    assert s.error_control_stats()[:2] == (0, 1)
+    assert s.advance_n(steps, False) == 0
+    assert s.sync_host() == 0
+    w, ref = s.spec("omega_hat").copy(), o.spec("omega_hat")
+    s.close()
+    assert rel_l2(w0, ref) > 1e-3  # the steps did something
+    # the draws of three steps enter at 1e-3 of the field and more; FP64 round-off is
+    # what the members of an ensemble are held to against the oracle
+    err = rel_l2(w, ref)
+    print(f"kmax {kmax:g}: rel L2 {err:.1e}", flush=True)
+    assert err <= 1e-11
