@@ -41,7 +41,9 @@ void col_fields(const ColArgs<T>& a, int ncols, int members, hipStream_t st) {
     constexpr int U = fields_units<L>(), MW = fields_mw<T, L>();
     const dim3 grid((ncols + U - 1) / U, members);
     const size_t lds = fields_lds<T, L>();
-    if (a.phys.scheme == 0)
+    if (a.mode == COL_PRIME)
+        hipLaunchKernelGGL((k_col_fields_prime<T, L, U, MW>), grid, dim3(U * L / 2), lds, st, a);
+    else if (a.phys.scheme == 0)
         hipLaunchKernelGGL((k_col_fields<T, L, 0, U, MW>), grid, dim3(U * L / 2), lds, st, a);
     else
         hipLaunchKernelGGL((k_col_fields<T, L, 1, U, MW>), grid, dim3(U * L / 2), lds, st, a);
@@ -58,6 +60,7 @@ void limits(int bytes) {
     constexpr int U = fields_units<L>(), MW = fields_mw<T, L>();
     lds_attr(k_row_fields<T, L, U, MW, false>, bytes);
     lds_attr(k_row_fields<T, L, U, MW, true>, bytes);
+    lds_attr(k_col_fields_prime<T, L, U, MW>, bytes);
     lds_attr(k_col_fields<T, L, 0, U, MW>, bytes);
     lds_attr(k_col_fields<T, L, 1, U, MW>, bytes);
 }

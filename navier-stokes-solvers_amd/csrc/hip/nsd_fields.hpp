@@ -568,4 +568,42 @@ __global__ __launch_bounds__(U * L / 2, MW) void k_col_fields(ColArgs<T> a) {
     col_unit_out<T, L>(lds, wh, r, G, kxi, kx, kys, out + mb * a.bm, active, tw);
 }
 
+// The derivative fields of the state as it is (COL_PRIME), through the output passes
+// of the stage kernel: a state that was uploaded, restored or primed again after
+// other transforms steps on with the bits of a run that kept its fields.
+template <typename T, int L, int U, int MW>
+__global__ __launch_bounds__(U * L / 2, MW) void k_col_fields_prime(ColArgs<T> a) {
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    constexpr int UT = unit_threads<L>(), TPL = L / P, RE = unit_region<L>();
+    constexpr int kym = Band<L>::kym, ncy = 2 * kym + 1;
+    constexpr bool WS = ws_unit<L>();
+    const int u = threadIdx.x / UT, r = threadIdx.x - u * UT;
+    const int f = r / TPL, j = r - f * TPL;
+    cx<T>* const lds = reinterpret_cast<cx<T>*>(smem_raw) + u * 4 * RE;
+    const Geo& G = a.geo;
+    const size_t mb = blockIdx.y;
+    const int kxi = blockIdx.x * U + u;
+    const bool active = kxi < G.nkx_keep;
+    UnitTw<L, T> tw;
+    load_unit_tw<L>(tw, j, a.tw);
+    cx<T>* const wh = lds + (WS ? 2 * RE : RE);
+#pragma unroll
+    for (int q = 0; q < kUnitModes; ++q) {
+        const int c = r + q * UT;
+        if (c >= ncy || !active) continue;
+        const int jy = c <= kym ? c : c + (L - ncy);
+        wh[WS ? jy : pad(jy)] = a.state[mb * a.bc + (size_t)kxi * ncy + c];
+    }
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        DevScalars* const sc = a.sc + mb;
+        sc->umax2_bits = 0ull;
+        sc->pending = 0;  // a new state: nothing waits to be judged
+        sc->redo = 0;
+    }
+    unit_sync<L>();
+    cx<T>* out = f < 2 ? (f == 0 ? a.mixed[0] : a.mixed[1]) : (f == 2 ? a.mixed[2] : a.mixed[3]);
+    col_unit_out<T, L>(lds, wh, r, G, kxi, T(kxi) * T(a.kxs), T(a.kys), out + mb * a.bm, active,
+                       tw);
+}
+
 }  // namespace nsd

@@ -79,10 +79,7 @@ template <typename T, int LOG, int V, bool ERR = false>
 void col_fused_LV(const ColArgs<T>& a, int ncols, int members, hipStream_t st) {
     constexpr int L = 1 << LOG;
     if constexpr (V == kFieldsVariant) {
-        if constexpr (L <= kFieldsMax) {
-            if (a.mode == COL_PRIME) col_fused_LV<T, LOG, 0>(a, ncols, members, st);
-            else launch_col_fields<T>(a, L, ncols, members, st);
-        }
+        if constexpr (L <= kFieldsMax) launch_col_fields<T>(a, L, ncols, members, st);
     } else if constexpr (var_ok<L, V>()) {
         constexpr int NT = var_nt<L, V>();
         constexpr int PR = var_pr<V>();
