@@ -132,16 +132,19 @@ int nsd_batch_scalars(NsdContext *c, double *t, double *dt, int *status);
 int nsd_member_upload(NsdContext *c, int member, const double *omega_hat);
 int nsd_member_download(NsdContext *c, int member, double *omega_hat);
 
-/* Launch variants of the two time-step kernels (workgroup size, whether
- * inverse transforms run in lock-step pairs, and field-parallel kernels whose
- * four transforms run side by side; lengths 64..1024 have several; a context
- * starts with the field-parallel ones where its launches are small).
- * nsd_autotune times every variant on this context's shape (reps launches
- * each) and keeps the fastest; results are cached per (grid, precision,
- * batch members) for the process and, if the environment names a file in
- * NSD_TUNE_FILE (lines "row|col NXxNY precision members variant"),
- * across processes (force != 0 re-times).  It zeroes the state: call it
- * before setting the initial field.  Every variant gives identical results. */
+/* Launch variants of the two time-step kernels, lengths of up to 1024: 0 the
+ * default shape, 1 workgroups of one wave (up to 512), 2 of twice and 4 of half the
+ * threads (from 64), 3 field-parallel kernels, whose four transforms run side by
+ * side.  A context starts with the ones that its launches are fastest with.  All
+ * agree to round-off; 0, 1 and 4 (at FP32 2 as well) give the same bits.
+ * nsd_autotune times the variants that give the bits of the starting ones on this
+ * context's shape (reps launches each) and keeps the fastest, so the choice does not
+ * show in the results; results are cached per (grid, precision, batch members) for
+ * the process and, if the environment names a file in NSD_TUNE_FILE (lines "row|col
+ * NXxNY precision members variant"), across processes (force != 0 re-times).  It
+ * zeroes the state: call it before setting the initial field.  nsd_set_variants
+ * takes any variant that the lengths have; nsd_get_variants returns the present
+ * ones. */
 int nsd_autotune(NsdContext *c, int reps, int force, int *row_variant, int *col_variant);
 /* Staggered start of the 4096-point FP32 row stage: the second resident
  * workgroup of each compute unit starts about 5 us late, so that the two
@@ -151,6 +154,7 @@ int nsd_autotune(NsdContext *c, int reps, int force, int *row_variant, int *col_
  * set = 0 turns it off, 1 turns it on if that check passed, -1 only queries;
  * returns the state (1 on, 0 off), -1 on error.  Results do not depend on it. */
 int nsd_row_stagger(NsdContext *c, int set);
+int nsd_get_variants(const NsdContext *c, int *row_variant, int *col_variant);
 int nsd_set_variants(NsdContext *c, int row_variant, int col_variant);
 
 /* One captured hipGraph that advances several batch contexts (different grid

@@ -70,7 +70,8 @@ EXPORTED = [
     "nsd_create_batch", "nsd_batch_members", "nsd_set_member_params", "nsd_batch_random_phase",
     "nsd_batch_energy", "nsd_batch_scalars", "nsd_member_upload", "nsd_member_download",
     "nsd_multi_create", "nsd_multi_destroy", "nsd_multi_error", "nsd_multi_advance",
-    "nsd_multi_synchronize", "nsd_autotune", "nsd_set_variants", "nsd_forcing_ou",
+    "nsd_multi_synchronize", "nsd_autotune", "nsd_get_variants", "nsd_set_variants",
+    "nsd_forcing_ou",
     "nsd_forcing_modes", "nsd_physical_to_spectral_noalloc", "nsd_errctl_stats",
     "nsd_row_stagger",
     # checkpoint.h
@@ -328,6 +329,7 @@ def load():
         "nsd_multi_advance": ([V, C.c_int, C.c_int], C.c_int),
         "nsd_multi_synchronize": ([V], C.c_int),
         "nsd_autotune": ([V, C.c_int, C.c_int, I, I], C.c_int),
+        "nsd_get_variants": ([V, I, I], C.c_int),
         "nsd_set_variants": ([V, C.c_int, C.c_int], C.c_int),
         "nsd_forcing_ou": ([V, D, C.c_int, C.c_int], C.c_int),
         "nsd_forcing_modes": ([V], C.c_int),

@@ -1533,13 +1533,14 @@ void tune_store(const NsdContext* c, int kind, int v) {
     fclose(fp);
 }
 
-// whether the tuner may give variant v to this context's kernel (FP32 grids below
-// 512^2 do without the field-parallel ones: stage_variant_default has the reason)
+// Whether the tuner may give variant v to this context's kernel: one with the bits
+// of the variant that it started with, so that no timing decides them.
 template <typename T>
 bool tunable(const NsdContext* c, int kind, int v) {
-    const bool small32 = sizeof(T) == 4 && std::max(c->G.nx, c->G.ny) < 512;
-    return v >= 0 && v < kStageVariants && !(small32 && v == kFieldsVariant) &&
-           stage_variant_valid<T>(kind == 0 ? c->G.nx : c->G.ny, v, c->maxlds);
+    const int L = kind == 0 ? c->G.nx : c->G.ny;
+    return v >= 0 && v < kStageVariants && stage_variant_valid<T>(L, v, c->maxlds) &&
+           stage_variant_rounding<T>(L, v) ==
+               stage_variant_rounding<T>(L, default_variant<T>(c, kind));
 }
 
 // zero every field and scalar the step reads, so that timing runs leave a
@@ -1573,10 +1574,10 @@ int op_autotune(NsdContext* c, int reps, int force) {
                 cached = true;
             }
         }
-        // a launch that starts with the field-parallel kernels keeps them, as a
-        // single context of its size does: nothing to time
-        if (!cached && default_variant<T>(c, kind) == kFieldsVariant) {
-            best = kFieldsVariant;
+        int choices = 0;
+        for (int v = 0; v < kStageVariants; ++v) choices += tunable<T>(c, kind, v) ? 1 : 0;
+        if (choices == 1) {  // nothing to time
+            best = default_variant<T>(c, kind);
             cached = true;
         }
         if (!cached) {
@@ -2254,6 +2255,13 @@ int nsd_autotune(NsdContext* c, int reps, int force, int* row_variant, int* col_
     if (row_variant) *row_variant = c->vrow;
     if (col_variant) *col_variant = c->vcol;
     return rc;
+}
+
+int nsd_get_variants(const NsdContext* c, int* row_variant, int* col_variant) {
+    if (!c) return ST_PARAM;
+    if (row_variant) *row_variant = c->vrow;
+    if (col_variant) *col_variant = c->vcol;
+    return ST_OK;
 }
 
 int nsd_set_variants(NsdContext* c, int row_variant, int col_variant) {

@@ -901,9 +901,11 @@ __global__ __launch_bounds__(NT, MW) void k_col(ColArgs<T> a) {
     // compiler drops the zero fills and masks of an idle column.  Taken for
     // the prime pass and the integrating-factor stage up to 4096 points: in
     // the classic scheme with the error controller, and at 8192, the freed
-    // schedule costs the compiler registers it then spills.
+    // schedule costs the compiler registers it then spills; up to 512 points
+    // one column per workgroup is a launch variant, which has to round as the
+    // others do.
     constexpr bool ALL_KEPT = (MODE == COL_PRIME || (MODE == COL_STAGE && SCHEME == 1)) &&
-                              LC > 0 && LC <= 4096 && NT * P / LC == 1;
+                              LC > 512 && LC <= 4096 && NT * P / LC == 1;
     const bool active = ALL_KEPT || kxi < ncols;
     const bool has_data = ALL_KEPT || (active && kxi < G.nkx_keep);
     const T kx = T(kxi) * T(2.0 * kPi / G.Lx);

@@ -2,10 +2,9 @@
 // transform length, so that all LDS addresses and strides are compile-time
 // constants.  Compiled once per precision with -DNSD_T=float / double.
 //
-// Lengths 64..1024 (the ensemble sizes) also get launch variants that the
-// autotuner chooses between: workgroup size (lines per workgroup), whether
-// the inverse transforms run in lock-step pairs, and the field-parallel kernels
-// of nsd_fields.hpp.
+// Lengths of up to 1024 (the ensemble sizes) also get launch variants: 1, 2 and 4
+// are variant 0's code in workgroups of one wave, of twice and of half the threads,
+// 3 the field-parallel kernels of nsd_fields.hpp.
 #include "nsd_stage.hpp"
 
 #ifndef NSD_T
@@ -21,23 +20,14 @@ constexpr int nt_for() {
     return L / P > 256 ? L / P : 256;
 }
 
-// variant V of length L: threads per workgroup and pairing (-1 automatic)
+// variant V of length L: threads per workgroup
 template <int L, int V>
 constexpr int var_nt() {
-    return V <= 1   ? nt_for<L>()
-           : V == 2 ? 2 * nt_for<L>()
-           : V == 4 ? nt_for<L>() / 2
-                    : (L / P > 64 ? L / P : 64);
-}
-template <int V>
-constexpr int var_pr() {
-    return V == 1 ? 0 : -1;
+    return V == kSmallVariant ? 64 : V == 2 ? 2 * nt_for<L>() : V == 4 ? nt_for<L>() / 2 : nt_for<L>();
 }
 template <int L, int V>
 constexpr bool var_ok() {
-    constexpr int NT = var_nt<L, V>();
-    return V == 0 || (V == kSmallVariant && L <= 1024) ||
-           (V != kSmallVariant && L >= 64 && L <= 1024 && NT <= 1024 && NT >= L / P && NT >= 64);
+    return V == 0 || (V == kSmallVariant ? L / P <= 64 : L >= 64 && L <= 1024);
 }
 
 // the stage kernels' LDS (FP64 lines of 4096 take a second line region)
@@ -45,7 +35,7 @@ template <typename T, int L, int V>
 size_t stage_lds() {
     constexpr int NT = var_nt<L, V>();
     constexpr int lines = NT * P / L;
-    constexpr int PR = var_pr<V>();
+    constexpr int PR = -1;
     return (size_t)lines * stage_regions<T, L, NT, PR>() * region_elems<T, L, NT, PR>() *
            sizeof(cx<T>);
 }
@@ -59,7 +49,7 @@ void row_stage_LV(const RowArgs<T>& a, int items, int members, hipStream_t st,
         if constexpr (L <= kFieldsMax) launch_row_fields<T>(a, L, items, members, st, force);
     } else if constexpr (var_ok<L, V>()) {
         constexpr int NT = var_nt<L, V>();
-        constexpr int PR = var_pr<V>();
+        constexpr int PR = -1;
         constexpr int lines = NT * P / L;
         const int blocks = (items + lines - 1) / lines;
         const size_t lds = stage_lds<T, L, V>();
@@ -82,7 +72,7 @@ void col_fused_LV(const ColArgs<T>& a, int ncols, int members, hipStream_t st) {
         if constexpr (L <= kFieldsMax) launch_col_fields<T>(a, L, ncols, members, st);
     } else if constexpr (var_ok<L, V>()) {
         constexpr int NT = var_nt<L, V>();
-        constexpr int PR = var_pr<V>();
+        constexpr int PR = -1;
         constexpr int lines = NT * P / L;
         const int blocks = (ncols + lines - 1) / lines;
         const dim3 grid(blocks, members);
@@ -109,7 +99,7 @@ void limits_LV(int bytes) {
     constexpr int L = 1 << LOG;
     if constexpr (var_ok<L, V>() && V != kFieldsVariant) {
         constexpr int NT = var_nt<L, V>();
-        constexpr int PR = var_pr<V>();
+        constexpr int PR = -1;
         lds_attr(k_row<T, NT, ROW_STAGE, L, PR>, bytes);
         lds_attr(k_row<T, NT, ROW_STAGE, L, PR, false, min_waves<T>(), true>, bytes);
         lds_attr(k_col<T, NT, COL_PRIME, 0, L, PR>, bytes);
@@ -126,14 +116,23 @@ void limits_LV(int bytes) {
 template <typename T, int LOG, int V>
 int var_pairs() {
     constexpr int L = 1 << LOG;
-    if constexpr (V != kFieldsVariant && var_ok<L, V>()) return stage_layout<T, L, var_nt<L, V>(), var_pr<V>()>() ? 1 : 0;
+    if constexpr (V != kFieldsVariant && var_ok<L, V>()) return stage_layout<T, L, var_nt<L, V>(), -1>() ? 1 : 0;
     return 0;
+}
+
+// -1: no such variant, 0: transforms one at a time, 1: in lock-step pairs, 2: field-parallel
+template <typename T, int LOG, int V>
+int var_rounding() {
+    constexpr int L = 1 << LOG;
+    if constexpr (V == kFieldsVariant) return L <= kFieldsMax ? 2 : -1;
+    else if constexpr (var_ok<L, V>()) return paired_lines<T, L, var_nt<L, V>(), -1>() ? 1 : 0;
+    return -1;
 }
 
 template <typename T, int LOG, int V>
 int var_valid(int maxlds) {
     constexpr int L = 1 << LOG;
-    if constexpr (V == kFieldsVariant) return L >= 64 && fields_fits<T>(L, maxlds) ? 1 : 0;
+    if constexpr (V == kFieldsVariant) return fields_fits<T>(L, maxlds) ? 1 : 0;
     else if constexpr (var_ok<L, V>())
         return stage_lds<T, L, V>() <= (size_t)maxlds ? 1 : 0;
     return 0;
@@ -156,7 +155,7 @@ int log2i(int L) {
 }  // namespace
 
 #define NSD_FOR_LOGS(X) X(4) X(5) X(6) X(7) X(8) X(9) X(10) X(11) X(12) X(13)
-#define NSD_FOR_VARS(X, n) X(n, 0) X(n, 1) X(n, 2) X(n, 3) X(n, 4) X(n, 5)
+#define NSD_FOR_VARS(X, n) X(n, 0) X(n, 1) X(n, 2) X(n, 3) X(n, 4)
 
 template <typename T>
 void launch_row_stage(const RowArgs<T>& a, int L, int items, int members, int variant,
@@ -219,6 +218,19 @@ int stage_variant_pairs(int L, int variant) {
 #undef V_
     return 0;
 }
+
+template <typename T>
+int stage_variant_rounding(int L, int variant) {
+    const int lg = log2i(L);
+#define V_(n, v) \
+    if (lg == n && variant == v) return var_rounding<T, n, v>();
+#define X(n) NSD_FOR_VARS(V_, n)
+    NSD_FOR_LOGS(X)
+#undef X
+#undef V_
+    return -1;
+}
+template int stage_variant_rounding<NSD_T>(int, int);
 
 template <typename T>
 int row_stage_threads(int L, int variant) {

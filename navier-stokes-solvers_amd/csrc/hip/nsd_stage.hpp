@@ -11,8 +11,8 @@ constexpr int kStageVariants = 5;
 // the field-parallel kernels (nsd_fields.hpp), lines of up to kFieldsMax points
 constexpr int kFieldsVariant = 3;
 constexpr int kFieldsMax = 1024;
-// workgroups of one line's threads, or one wave
-constexpr int kSmallVariant = 5;
+// workgroups of one wave, lines of up to 512 points
+constexpr int kSmallVariant = 1;
 
 // k_row in ROW_STAGE mode for rows of length L (power of two, 16..8192),
 // `members` batch members along grid y
@@ -38,6 +38,10 @@ int row_stage_threads(int L, int variant);
 // 1 if `variant` exists for length L and fits `maxlds` bytes of LDS
 template <typename T>
 int stage_variant_valid(int L, int variant, int maxlds);
+// Variants of one length with equal values here contract the same products and give
+// the same bits; -1: no such variant
+template <typename T>
+int stage_variant_rounding(int L, int variant);
 // 1 if the stage kernels of `variant` at length L read (k_row) and write
 // (k_col) the mixed fields in a layout of their own (stage_layout)
 template <typename T>
