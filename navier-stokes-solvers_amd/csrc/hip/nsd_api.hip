@@ -853,9 +853,8 @@ bool jblocks_ok(const NsdContext* c) { return c->prec == NSD_FP32 && pairs_ok(c)
 // launch variant that this context starts with (kind 0: rows, 1: columns)
 template <typename T>
 int default_variant(const NsdContext* c, int kind) {
-    const long lines = (long)c->nb * (kind == 0 ? c->G.ny / 2 : c->G.nkx_keep);
-    return stage_variant_default<T>(kind, kind == 0 ? c->G.nx : c->G.ny, lines,
-                                    std::max(c->G.nx, c->G.ny), c->maxlds);
+    return stage_variant_default<T>(kind, kind == 0 ? c->G.nx : c->G.ny,
+                                    kind == 0 ? c->G.ny / 2 : c->G.nkx_keep, c->nb, c->maxlds);
 }
 
 template <typename T>

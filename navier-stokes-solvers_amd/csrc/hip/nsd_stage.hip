@@ -269,47 +269,50 @@ int col_fused_blocks(int L, int ncols) {
     return (ncols + lines - 1) / lines;
 }
 template int col_fused_blocks<NSD_T>(int, int);
-// Variant a context starts with, for `lines` lines (row pairs, kind 0, or kept
-// columns, kind 1, times batch members) of length L on a grid whose longer side is
-// `side`.  `waves`: what variant 0 would launch (the device holds 1024 SIMDs).
+// Variant a context starts with, for `members` times `lines` lines (row pairs, kind 0,
+// or kept columns, kind 1) of length L.
 //
-// Launches that leave at most one wave per SIMD take the field-parallel kernels
-// or, on FP32 grids below 512^2, variant 0's own code in the smallest workgroups.
-// us per RK4 step of one field, variant 0 -> smallest workgroups -> field-parallel:
-//   64^2 FP64 72 -> 56 -> 49, 512^2 FP64 120 -> - -> 69, 1024^2 FP64 188 -> 172 -> 149,
-//   256^2 FP32 98 -> 81 -> 67, 512^2 FP32 103 -> 85 -> 71, 1024^2 FP32 140 -> 130 -> 124.
-// The small FP32 grids keep variant 0's code because its rounding is theirs: a
-// step's difference of one FP32 rounding grows to 2e-5 of the field within 400
-// forced steps at 256^2, and runs, batch members and restarts of these sizes are
-// compared with one another bit for bit.  Lines of 2048 stay with variant 0: a
-// unit is 1024 threads there, one to a compute unit at FP64, and 256 row pairs
-// take 22.0 us against 20.9 us.
+// Whether the field-parallel kernels or variant 0's code (in one workgroup size or
+// another) run a grid decides its rounding, so it follows the grid and the precision
+// alone: batch members have the bits of a single run.  FP64 takes the field-parallel
+// kernels where one field's launch leaves at most one wave per SIMD (`one`, the waves of
+// variant 0; the device holds 1024 SIMDs), and where they are the faster ones past that.
+// us per RK4 step, variant 0 / its fastest workgroups / field-parallel, FP64 members of
+//   64^2: 1 member 70 / 54 / 41, 64 76 / 67 / 55, 260 113 / 108 / 116
+//   128^2: 1 91 / 64 / 49, 60 125 / 119 / 121, 200 254 / 201 / 226
+//   256^2: 1 100 / 69 / 50, 64 290 / 260 / 262, 200 875 / 835 / 876
+//   512^2: 1 116 / 82 / 61, 8 190 / 172 / 165, 64 1171 / 1061 / 1026
+//   1024^2: 1 180 / 167 / 139, 8 664 / 603 / 555, 24 2078 / 1879 / 1709
+// and rows of one field: 1024 x 2048 209 / 209 / 193, 512 x 4096 201 / 201 / 196, 256 x 8192
+// 411 / 411 / 422; columns: 2048 x 1024 225 / 211 / 225, 4096 x 512 217 / 209 / 218.  Lines of
+// 2048 stay with variant 0: a unit is 1024 threads there, one to a compute unit, and 256
+// row pairs take 22.0 us against 20.9 us.
 //
-// Larger launches (us per step; 0, fields, 4: variant 0, field-parallel, half-size
-// workgroups, of the rows or columns named, variant 0 for the others):
-//   FP64 rows: 512 x 16 members 0 310.5, fields 288.9, 4 303.2; 1024 x 24 2073, 1801,
-//     1985; 256 x 100 442.6, 439.3, 418.5; 128 x 300 318.0, 343.2, 308.7.
-//   FP64 columns: 128 x 300 318.0, 297.5, 320.2; 256 x 300 1249, 1185, 1210; 512 x 80
-//     1411, 1346, 1356; 2048 x 1024 grid, classic scheme 233.0, 261.5, 219.0,
-//     integrating factor 226.5, 226.5, 212.2; 4096 x 1024 473.7, 511.3, 465.1.
-//   FP32 rows: 1024 x 4 192.6, 189.7, 190.1; 1024 x 8 311.0, 321.9, 311.2; 512 x 8
-//     129.9, 133.2, 132.2.
-//   FP32 columns: 512 x 8 129.9, 116.0, 126.4; 512 x 24 217.6, 211.5, 209.2; 1024 x 2
-//     154.6, 149.1, 146.5; 1024 x 16 566.8, 632.5, 552.6.
-//   FP32 below 512^2, both with variant 4: 256 x 32 126.8 -> 121.0, 128 x 120 121.9 -> 114.7.
+// FP32 does without them.  A single field would gain (512^2 82 / 63 / 49, 1024^2 118 / 110 /
+// 96), but batches lose against variant 0 (512^2 x 16 160 / 151 / 168, x 64 471 / 457 / 534;
+// 1024^2 x 16 544 / 531 / 659), and one rounding grows to 2e-5 of the field within 400
+// forced steps at 256^2.
+//
+// Workgroups of variant 0's code (us per step, one-wave ones, half-size from 1024 points):
+//   FP32 both kinds, 32^2 x 600 members 81 -> 61, 64^2 x 16 57 -> 47, x 260 76 -> 78, x 2000
+//     219 -> 199, 128^2 x 200 147 -> 128, 256^2 x 200 369 -> 337;
+//   columns of 512 512^2 x 24 214 -> 195, 4096 x 512 152 -> 144; of 1024 1024^2 x 64 2321 ->
+//     2245, 8192 x 1024 396 -> 385, FP64 2048 x 1024 225 -> 211;
+//   rows of 512 512^2 x 1 82 -> 76, x 8 128 -> 132, 512 x 4096 145 -> 162; of 1024 1024^2 x 1
+//     118 -> 116, x 64 2321 -> 2374, 1024 x 4096 213 -> 219: up to one wave per SIMD;
+//   shorter rows of tall grids 64 x 1024 74 -> 59 (with its columns), 128 x 8192 170 -> 175,
+//     256 x 8192 197 -> 212: up to half a wave per SIMD from one field.
 template <typename T>
-int stage_variant_default(int kind, int L, long lines, int side, int maxlds) {
-    const long waves = lines * (L / P) / 64;
+int stage_variant_default(int kind, int L, long lines, int members, int maxlds) {
+    const long one = lines * (L / P) / 64;
     if (L > kFieldsMax) return 0;
-    const bool many = waves > 1024;
-    if (L < 64 && many) return 0;
-    const int half = stage_variant_valid<T>(L, 4, maxlds) ? 4 : 0;
-    if (sizeof(T) == 4 && side < 512) return many ? half : kSmallVariant;
-    bool fields;
-    if (sizeof(T) == 8) fields = !many || (kind == 0 ? L >= 512 : L <= 512);
-    else fields = waves <= (kind == 0 ? (L == 1024 ? 4096 : 1024) : (L == 512 ? 2048 : 1024));
-    if (fields) return fields_fits<T>(L, maxlds) ? kFieldsVariant : 0;
-    return sizeof(T) == 8 || kind == 1 ? half : 0;
+    if (sizeof(T) == 8) {
+        if ((one <= 1024 || (kind == 0 ? L >= 512 : L <= 512)) && fields_fits<T>(L, maxlds))
+            return kFieldsVariant;
+        return kind == 1 && L == 1024 ? 4 : 0;
+    }
+    if (kind == 0 && (L >= 512 ? one * members > 1024 : one > 512)) return 0;
+    return L == 1024 ? 4 : kSmallVariant;
 }
 template int stage_variant_default<NSD_T>(int, int, long, int, int);
 template int stage_variant_valid<NSD_T>(int, int, int);

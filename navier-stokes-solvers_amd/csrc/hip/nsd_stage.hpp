@@ -28,10 +28,10 @@ void launch_col_fused(const ColArgs<T>& a, int L, int ncols, int members, int va
 // workgroups of the default (variant 0) column launch over ncols columns
 template <typename T>
 int col_fused_blocks(int L, int ncols);
-// variant that a context starts with for `lines` lines (members included; kind 0:
-// row pairs, 1: columns) of a grid whose longer side is `side`
+// variant that a context starts with for `lines` lines (kind 0: row pairs, 1: columns)
+// of each member
 template <typename T>
-int stage_variant_default(int kind, int L, long lines, int side, int maxlds);
+int stage_variant_default(int kind, int L, long lines, int members, int maxlds);
 // threads of a workgroup of that row launch
 template <typename T>
 int row_stage_threads(int L, int variant);
