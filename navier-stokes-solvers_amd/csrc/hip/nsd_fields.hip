@@ -25,28 +25,35 @@ constexpr size_t fields_lds() {
 }
 
 template <typename T, int L>
-void row_fields(const RowArgs<T>& a, int items, int members, hipStream_t st, bool force) {
+void row_fields(const RowArgs<T>& a, int items, int members, hipStream_t st, bool errctl,
+                bool force) {
     constexpr int U = fields_units<L>();
     constexpr int MW = fields_mw<T, L>();
-    const dim3 grid((items + U - 1) / U + (force ? 1 : 0), members);
+    const dim3 grid((items + U - 1) / U + (force ? 1 : 0), members), nt(U * L / 2);
     const size_t lds = fields_lds<T, L>();
-    if (force)
-        hipLaunchKernelGGL((k_row_fields<T, L, U, MW, true>), grid, dim3(U * L / 2), lds, st, a);
+    if (errctl)
+        hipLaunchKernelGGL((k_row_fields<T, L, U, MW, false, true>), grid, nt, lds, st, a);
+    else if (force)
+        hipLaunchKernelGGL((k_row_fields<T, L, U, MW, true, false>), grid, nt, lds, st, a);
     else
-        hipLaunchKernelGGL((k_row_fields<T, L, U, MW, false>), grid, dim3(U * L / 2), lds, st, a);
+        hipLaunchKernelGGL((k_row_fields<T, L, U, MW, false, false>), grid, nt, lds, st, a);
 }
 
 template <typename T, int L>
-void col_fields(const ColArgs<T>& a, int ncols, int members, hipStream_t st) {
+void col_fields(const ColArgs<T>& a, int ncols, int members, hipStream_t st, bool errctl) {
     constexpr int U = fields_units<L>(), MW = fields_mw<T, L>();
-    const dim3 grid((ncols + U - 1) / U, members);
+    const dim3 grid((ncols + U - 1) / U, members), nt(U * L / 2);
     const size_t lds = fields_lds<T, L>();
     if (a.mode == COL_PRIME)
-        hipLaunchKernelGGL((k_col_fields_prime<T, L, U, MW>), grid, dim3(U * L / 2), lds, st, a);
+        hipLaunchKernelGGL((k_col_fields_prime<T, L, U, MW>), grid, nt, lds, st, a);
+    else if (errctl && a.phys.scheme == 0)
+        hipLaunchKernelGGL((k_col_fields<T, L, 0, U, MW, true>), grid, nt, lds, st, a);
+    else if (errctl)
+        hipLaunchKernelGGL((k_col_fields<T, L, 1, U, MW, true>), grid, nt, lds, st, a);
     else if (a.phys.scheme == 0)
-        hipLaunchKernelGGL((k_col_fields<T, L, 0, U, MW>), grid, dim3(U * L / 2), lds, st, a);
+        hipLaunchKernelGGL((k_col_fields<T, L, 0, U, MW, false>), grid, nt, lds, st, a);
     else
-        hipLaunchKernelGGL((k_col_fields<T, L, 1, U, MW>), grid, dim3(U * L / 2), lds, st, a);
+        hipLaunchKernelGGL((k_col_fields<T, L, 1, U, MW, false>), grid, nt, lds, st, a);
 }
 
 template <typename K>
@@ -58,11 +65,14 @@ void lds_attr(K kernel, int bytes) {
 template <typename T, int L>
 void limits(int bytes) {
     constexpr int U = fields_units<L>(), MW = fields_mw<T, L>();
-    lds_attr(k_row_fields<T, L, U, MW, false>, bytes);
-    lds_attr(k_row_fields<T, L, U, MW, true>, bytes);
+    lds_attr(k_row_fields<T, L, U, MW, false, false>, bytes);
+    lds_attr(k_row_fields<T, L, U, MW, true, false>, bytes);
+    lds_attr(k_row_fields<T, L, U, MW, false, true>, bytes);
     lds_attr(k_col_fields_prime<T, L, U, MW>, bytes);
-    lds_attr(k_col_fields<T, L, 0, U, MW>, bytes);
-    lds_attr(k_col_fields<T, L, 1, U, MW>, bytes);
+    lds_attr(k_col_fields<T, L, 0, U, MW, false>, bytes);
+    lds_attr(k_col_fields<T, L, 1, U, MW, false>, bytes);
+    lds_attr(k_col_fields<T, L, 0, U, MW, true>, bytes);
+    lds_attr(k_col_fields<T, L, 1, U, MW, true>, bytes);
 }
 
 }  // namespace
@@ -72,17 +82,18 @@ static_assert(kFieldsMax == 1024, "the lengths above");
 
 template <typename T>
 void launch_row_fields(const RowArgs<T>& a, int L, int items, int members, hipStream_t st,
-                       bool force) {
+                       bool errctl, bool force) {
 #define X(n) \
-    if (L == n) return row_fields<T, n>(a, items, members, st, force);
+    if (L == n) return row_fields<T, n>(a, items, members, st, errctl, force);
     NSD_FOR_FIELDS(X)
 #undef X
 }
 
 template <typename T>
-void launch_col_fields(const ColArgs<T>& a, int L, int ncols, int members, hipStream_t st) {
+void launch_col_fields(const ColArgs<T>& a, int L, int ncols, int members, hipStream_t st,
+                       bool errctl) {
 #define X(n) \
-    if (L == n) return col_fields<T, n>(a, ncols, members, st);
+    if (L == n) return col_fields<T, n>(a, ncols, members, st, errctl);
     NSD_FOR_FIELDS(X)
 #undef X
 }
@@ -103,8 +114,9 @@ void fields_lds_limits(int bytes) {
 #undef X
 }
 
-template void launch_row_fields<NSD_T>(const RowArgs<NSD_T>&, int, int, int, hipStream_t, bool);
-template void launch_col_fields<NSD_T>(const ColArgs<NSD_T>&, int, int, int, hipStream_t);
+template void launch_row_fields<NSD_T>(const RowArgs<NSD_T>&, int, int, int, hipStream_t, bool,
+                                       bool);
+template void launch_col_fields<NSD_T>(const ColArgs<NSD_T>&, int, int, int, hipStream_t, bool);
 template bool fields_fits<NSD_T>(int, int);
 template void fields_lds_limits<NSD_T>(int);
 

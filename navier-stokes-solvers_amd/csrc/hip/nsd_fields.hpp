@@ -294,10 +294,15 @@ __device__ __forceinline__ void row_unit(cx<T>* lds, int r, const Geo& G, const 
     }
 }
 
-// U row pairs per workgroup
-template <typename T, int L, int U, int MW, bool FORCE>
+// U row pairs per workgroup (ERR: under the error controller, idle in the later stages
+// of a step that restores a rejected one)
+template <typename T, int L, int U, int MW, bool FORCE, bool ERR>
 __global__ __launch_bounds__(U * L / 2, MW) void k_row_fields(RowArgs<T> a) {
+    static_assert(!(FORCE && ERR), "the controller's draw is a kernel of its own");
     extern __shared__ __align__(16) unsigned char smem_raw[];
+    if constexpr (ERR) {
+        if (a.skip_on_redo && a.sc[blockIdx.y].redo) return;
+    }
     if constexpr (FORCE) {  // workgroup 0 makes the step's forcing draw
         if (blockIdx.x == 0) {
             force_draw(a.force, blockIdx.y, reinterpret_cast<double*>(smem_raw));
@@ -348,11 +353,11 @@ __device__ __forceinline__ ModeFactors<T> mode_factors(const Phys& ph, T h, T k2
 // step's start w0, the accumulator av (from stage 1 on) and, in the classic
 // scheme, the stage field ws and the SFD state fs; h6 = h / 6, h3 = h / 3.
 // Returns the new stage field and leaves the accumulator in av (stages 0..2) and
-// the SFD state in fs.
-template <typename T, int SCHEME>
+// the SFD state in fs; ERR: in stage 1 also the midpoint solution, in mid.
+template <typename T, int SCHEME, bool ERR>
 __device__ __forceinline__ cx<T> mode_update(const Phys& ph, int stage, T h, T h6, T h3, double dt,
                                              ModeFactors<T> m, cx<T> N, cx<T> w0, cx<T>& av,
-                                             cx<T> ws, cx<T>& fs) {
+                                             cx<T> ws, cx<T>& fs, cx<T>& mid) {
     cx<T> wn;
     if constexpr (SCHEME == 0) {
         // classic RK4 (spectral_time_integration.c:50-100) with
@@ -365,6 +370,7 @@ __device__ __forceinline__ cx<T> mode_update(const Phys& ph, int stage, T h, T h
         } else if (stage == 1) {
             av = av + h3 * ks;
             wn = w0 + (T(0.5) * h) * ks;
+            if constexpr (ERR) mid = w0 + h * ks;
         } else if (stage == 2) {
             av = av + h3 * ks;
             wn = w0 + h * ks;
@@ -383,6 +389,7 @@ __device__ __forceinline__ cx<T> mode_update(const Phys& ph, int stage, T h, T h
         } else if (stage == 1) {
             av = av + h3 * grow(N, e2);
             wn = grow(w0, e2) + (T(0.5) * h) * N;
+            if constexpr (ERR) mid = grow(w0, e1) + h * grow(N, e2);
         } else if (stage == 2) {
             av = av + h3 * grow(N, e2);
             wn = grow(w0, e1) + h * grow(N, e2);
@@ -441,8 +448,10 @@ __device__ __forceinline__ void col_unit_out(cx<T>* lds, const cx<T>* w, int r, 
     }
 }
 
-// U columns per workgroup, one stage
-template <typename T, int L, int SCHEME, int U, int MW>
+// U columns per workgroup, one stage (ERR: under the error controller, as k_col: the
+// state kept before a candidate, the midpoint solution, the sums of the estimate, and
+// the restoring pass of a rejected candidate)
+template <typename T, int L, int SCHEME, int U, int MW, bool ERR>
 __global__ __launch_bounds__(U * L / 2, MW) void k_col_fields(ColArgs<T> a) {
     extern __shared__ __align__(16) unsigned char smem_raw[];
     constexpr int UT = unit_threads<L>(), TPL = L / P, RE = unit_region<L>();
@@ -454,6 +463,11 @@ __global__ __launch_bounds__(U * L / 2, MW) void k_col_fields(ColArgs<T> a) {
     const Geo& G = a.geo;
     const size_t mb = blockIdx.y;
     DevScalars* const sc = a.sc + mb;
+    int redo = 0;  // uniform over the grid
+    if constexpr (ERR) {
+        redo = sc->redo;
+        if (redo ? a.stage > 0 : a.finalize != 0) return;
+    }
     Phys ph = a.phys;
     if (a.m_inv_re) {
         ph.inv_Re = a.m_inv_re[mb];
@@ -500,7 +514,8 @@ __global__ __launch_bounds__(U * L / 2, MW) void k_col_fields(ColArgs<T> a) {
     auto at = [](int i) { return WS ? i : pad(i); };
     if (pick) {
         dt = cfl_dt(ph, sqrt(u2));
-        if (blockIdx.x == 0 && threadIdx.x == 0) {
+        if constexpr (ERR) dt = fmin(fmax(fmin(dt, sc->dt_err), ph.dt_lo), ph.dt_hi);
+        if (blockIdx.x == 0 && threadIdx.x == 0 && !redo) {
             sc->dt = dt;
             if (!(u2 <= 1.0e300)) sc->status = 2;  // SOLVER_DIVERGED
         }
@@ -533,16 +548,36 @@ __global__ __launch_bounds__(U * L / 2, MW) void k_col_fields(ColArgs<T> a) {
         if (first) lds_write_c<L>(v, jh, j);
     }
     unit_sync<L>();
+    double esum = 0.0, ssum = 0.0;  // sums w |y4 - y2|^2 and w |y4|^2 of this thread
 #pragma unroll
     for (int q = 0; q < kUnitModes; ++q) {
         const int c = r + q * UT;
         if (c >= ncy || !active) continue;
         const int jy = c <= kym ? c : c + (L - ncy);
+        if constexpr (ERR) {
+            if (redo) {  // the state of the last accepted step comes back
+                const cx<T> back = a.prev[c0 + c];
+                a.state[c0 + c] = back;
+                wh[at(jy)] = back;
+                continue;
+            }
+            if (a.stage == 0) a.prev[c0 + c] = w0[q];
+        }
         // N = -norm FFT(J) (spectral_core.c:106-111)
         cx<T> N = (-norm) * jh[at(jy)];
         if (a.src) N = N + a.src[c0 + c];
-        cx<T> wn = mode_update<T, SCHEME>(ph, a.stage, h, h6, h3, dt, mf[q], N, w0[q], av[q], ws[q],
-                                          fs[q]);
+        cx<T> mid = zero;
+        cx<T> wn = mode_update<T, SCHEME, ERR>(ph, a.stage, h, h6, h3, dt, mf[q], N, w0[q], av[q],
+                                               ws[q], fs[q], mid);
+        if constexpr (ERR) {
+            if (a.stage == 1) a.ymid[c0 + c] = mid;
+            if (a.stage == 3) {  // embedded estimate, before the forcing kick
+                const cx<T> e = wn - a.ymid[c0 + c];
+                const double wt = kxi == 0 ? 1.0 : 2.0;
+                esum += wt * ((double)e.x * (double)e.x + (double)e.y * (double)e.y);
+                ssum += wt * ((double)wn.x * (double)wn.x + (double)wn.y * (double)wn.y);
+            }
+        }
         if (a.stage < 3) {
             a.acc[c0 + c] = av[q];
             if constexpr (SCHEME == 0) a.stagebuf[c0 + c] = wn;
@@ -562,6 +597,36 @@ __global__ __launch_bounds__(U * L / 2, MW) void k_col_fields(ColArgs<T> a) {
     if (blockIdx.x == 0 && threadIdx.x == 0 && a.stage == 3) {
         sc->t += dt;
         sc->umax2_bits = 0ull;
+    }
+    if constexpr (ERR) {
+        // stage 3 does not run on a restoring step
+        if (blockIdx.x == 0 && threadIdx.x == 0 && redo) sc->umax2_bits = 0ull;
+        if (a.stage == 3) {  // workgroup sums in a fixed order
+            constexpr int NW = U * L / 128;
+            __shared__ double ered[2 * NW];
+            esum = wave_sum(esum);
+            ssum = wave_sum(ssum);
+            const int wv = threadIdx.x >> 6;
+            if ((threadIdx.x & 63) == 0) {
+                ered[2 * wv] = esum;
+                ered[2 * wv + 1] = ssum;
+            }
+            __syncthreads();
+            if (threadIdx.x == 0) {
+                double e = 0.0, z = 0.0;
+                for (int i = 0; i < NW; ++i) {
+                    e += ered[2 * i];
+                    z += ered[2 * i + 1];
+                }
+                double* part = a.errpart + mb * a.bp + 2 * (size_t)blockIdx.x;
+                part[0] = e;
+                part[1] = z;
+                if (blockIdx.x == 0) {
+                    sc->pending = 1;
+                    sc->errparts = (int)gridDim.x;
+                }
+            }
+        }
     }
     unit_sync<L>();
     cx<T>* out = f < 2 ? (f == 0 ? a.mixed[0] : a.mixed[1]) : (f == 2 ? a.mixed[2] : a.mixed[3]);

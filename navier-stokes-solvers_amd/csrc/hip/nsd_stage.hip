@@ -40,13 +40,13 @@ size_t stage_lds() {
            sizeof(cx<T>);
 }
 
-// ERR: the error controller's instantiations (launch variant 0 only)
+// ERR: the error controller's instantiations (variants 0 and 3)
 template <typename T, int LOG, int V, bool ERR = false>
 void row_stage_LV(const RowArgs<T>& a, int items, int members, hipStream_t st,
                   bool force = false) {
     constexpr int L = 1 << LOG;
     if constexpr (V == kFieldsVariant) {
-        if constexpr (L <= kFieldsMax) launch_row_fields<T>(a, L, items, members, st, force);
+        if constexpr (L <= kFieldsMax) launch_row_fields<T>(a, L, items, members, st, ERR, force);
     } else if constexpr (var_ok<L, V>()) {
         constexpr int NT = var_nt<L, V>();
         constexpr int PR = -1;
@@ -69,7 +69,7 @@ template <typename T, int LOG, int V, bool ERR = false>
 void col_fused_LV(const ColArgs<T>& a, int ncols, int members, hipStream_t st) {
     constexpr int L = 1 << LOG;
     if constexpr (V == kFieldsVariant) {
-        if constexpr (L <= kFieldsMax) launch_col_fields<T>(a, L, ncols, members, st);
+        if constexpr (L <= kFieldsMax) launch_col_fields<T>(a, L, ncols, members, st, ERR);
     } else if constexpr (var_ok<L, V>()) {
         constexpr int NT = var_nt<L, V>();
         constexpr int PR = -1;
@@ -163,6 +163,8 @@ void launch_row_stage(const RowArgs<T>& a, int L, int items, int members, int va
     const int lg = log2i(L);
     if (errctl) {
 #define E_(n) \
+    if (lg == n && variant == kFieldsVariant) \
+        return row_stage_LV<T, n, kFieldsVariant, true>(a, items, members, st); \
     if (lg == n) return row_stage_LV<T, n, 0, true>(a, items, members, st);
         NSD_FOR_LOGS(E_)
 #undef E_
@@ -182,6 +184,8 @@ void launch_col_fused(const ColArgs<T>& a, int L, int ncols, int members, int va
     const int lg = log2i(L);
     if (errctl && a.mode == COL_STAGE) {
 #define E_(n) \
+    if (lg == n && variant == kFieldsVariant) \
+        return col_fused_LV<T, n, kFieldsVariant, true>(a, ncols, members, st); \
     if (lg == n) return col_fused_LV<T, n, 0, true>(a, ncols, members, st);
         NSD_FOR_LOGS(E_)
 #undef E_

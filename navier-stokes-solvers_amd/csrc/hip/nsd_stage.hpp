@@ -16,8 +16,9 @@ constexpr int kSmallVariant = 1;
 
 // k_row in ROW_STAGE mode for rows of length L (power of two, 16..8192),
 // `members` batch members along grid y
-// (errctl: the error controller's instantiation, launch variant 0; force: one
-// more workgroup per member makes the forcing draw a.force, not with errctl)
+// (errctl: the error controller's instantiation, of the field-parallel kernels and of
+// variant 0, which stands for its other workgroup sizes; force: one more workgroup
+// per member makes the forcing draw a.force, not with errctl)
 template <typename T>
 void launch_row_stage(const RowArgs<T>& a, int L, int items, int members, int variant,
                       hipStream_t st, bool errctl = false, bool force = false);
@@ -49,9 +50,10 @@ int stage_variant_pairs(int L, int variant);
 // the field-parallel launches (nsd_fields.hip): L <= kFieldsMax
 template <typename T>
 void launch_row_fields(const RowArgs<T>& a, int L, int items, int members, hipStream_t st,
-                       bool force);
+                       bool errctl, bool force);
 template <typename T>
-void launch_col_fields(const ColArgs<T>& a, int L, int ncols, int members, hipStream_t st);
+void launch_col_fields(const ColArgs<T>& a, int L, int ncols, int members, hipStream_t st,
+                       bool errctl);
 // threads of a workgroup of theirs
 constexpr int row_fields_threads(int L) { return L <= 512 ? 256 : L / 2; }
 // whether they take lines of length L with `maxlds` bytes of LDS
