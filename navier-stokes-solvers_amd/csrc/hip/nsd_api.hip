@@ -838,7 +838,7 @@ int lastk(NsdContext* c) {
 // The stage kernels' mixed fields use a layout of their own (stage_layout in
 // nsd_kernels.hpp: the pair layout at FP32, row-pair tiles at FP64) when the
 // row and the column instantiations this context launches both hold it
-// (square 4096^2 grids); the answer follows the launch variants.
+// (square 2048^2, 4096^2 and FP32 8192^2 grids); the answer follows the launch variants.
 bool pairs_ok(const NsdContext* c) {
     if (c->G.nx != c->G.ny) return false;
     if (c->prec == NSD_FP32)

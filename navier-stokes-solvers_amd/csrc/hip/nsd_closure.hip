@@ -12,15 +12,13 @@
 //   input gradient: A[p][(tap, co)] = dZ[p - off(tap)][co], B = W[co][tap][n]
 //   weight grad.:   dW[co][(tap, ci)] = sum_p dZ[p][co] X[p + off(tap)][ci]
 // A wave computes 16 pixels x 16 channels per MFMA (v_mfma_f32_16x16x32_bf16,
-// depth 32: one 3x3 tap of 32 channels); the B operand (at most 288 x 32
-// bf16) sits in LDS, transposed so each lane's 8 k-values are one 16-byte
-// read, and each lane's A values are one 16-byte load of 8 channels.  A workgroup stages B once and walks TILES tiles of 64
-// pixels, so the staging is paid once per 64 x TILES pixels.  Grids that are
-// multiples of 64 use the LDS-tiled kernels instead: k_conv_tile2 (forward
-// layers with 32 input channels: persistent, the next patch streamed into LDS
-// while the current one is computed), k_conv_tile (the input layer and the
-// input gradients) and k_conv_dw_tile / k_conv_dw_tile_in (weight
-// gradients); k_conv and k_conv_dw serve the smaller grids.
+// depth 32: one 3x3 tap of 32 channels); a lane's eight k-values of either operand
+// are one 16-byte read.  The layers with 32 input channels (and the 32-channel
+// input gradients) run on k_conv_tile2 on grids that are multiples of 32:
+// persistent, the next patch streamed into LDS while the current one is computed.
+// Those with one input channel run on k_conv_tile on multiples of 64, as do the
+// weight gradients on k_conv_dw_tile / k_conv_dw_tile_in.  k_conv (the weights in
+// LDS, TILES tiles of 64 pixels per workgroup) and k_conv_dw serve the smaller grids.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -180,15 +178,18 @@ __global__ __launch_bounds__(256) void k_conv(ConvArgs a) {
     }  // tiles
 }
 
-// grid and launch of k_conv: 8 tiles per workgroup when the grid allows it
+// grid and launch of k_conv: 8 tiles per workgroup at n = 32, which only the layers
+// with one input channel come here with
 template <int KC, int NN, int MODE>
 void launch_conv(const ConvArgs& a, int batch, hipStream_t st) {
-    if (a.npix % (64 * 8) == 0)
-        hipLaunchKernelGGL((k_conv<KC, NN, MODE, 8>), dim3(a.npix / (64 * 8), batch), dim3(256), 0,
-                           st, a);
-    else
-        hipLaunchKernelGGL((k_conv<KC, NN, MODE, 1>), dim3(a.npix / 64, batch), dim3(256), 0, st,
-                           a);
+    if constexpr (KC == 1) {
+        if (a.npix % (64 * 8) == 0) {
+            hipLaunchKernelGGL((k_conv<KC, NN, MODE, 8>), dim3(a.npix / (64 * 8), batch), dim3(256),
+                               0, st, a);
+            return;
+        }
+    }
+    hipLaunchKernelGGL((k_conv<KC, NN, MODE, 1>), dim3(a.npix / 64, batch), dim3(256), 0, st, a);
 }
 
 // The tiled kernels compute D[channel][pixel] (weights as the A operand).  Row

@@ -417,26 +417,24 @@ struct Band {
 };
 
 // Whether the time-step kernels run their inverse transforms two at a time
-// (needs two line regions per line in LDS).  PR < 0 decides automatically:
-// paired when the workgroup's two regions stay within 80 KB, so that two
-// workgroups share a CU; PR = 0 / 1 forces the choice (launch variants).
+// (needs two line regions per line in LDS): when the workgroup's two regions stay
+// within 80 KB, so that two workgroups share a CU.
 // FP32 lines of 8192 are paired as well (147 KB, one workgroup of 16 waves per
 // CU): one region leaves room for no second workgroup either, and the
 // wave-split pairs took k_row at 8192^2 from 926 to 537 us and k_col from 527
 // to 450 us (per-pair layout).  FP64 lines of 2048 are not, though two regions
 // would fit: they run wave-split in a field at a time like those of 4096
 // (ws_lines64; 2048^2 FP64 step 351 -> 311 us).
-template <typename T, int LC, int NT = threads_for(LC), int PR = -1>
+template <typename T, int LC, int NT = threads_for(LC)>
 constexpr bool paired_lines() {
     if (LC <= 0) return false;
-    if (PR >= 0) return PR == 1;
     if (sizeof(T) == 4 && LC == 8192) return true;
     if (sizeof(T) == 8 && LC == 2048) return false;
     return 2 * (LC + LC / 16) * (int)sizeof(cx<T>) * (NT * P / LC) <= 80 * 1024;
 }
-template <typename T, int LC, int NT = threads_for(LC), int PR = -1>
+template <typename T, int LC, int NT = threads_for(LC)>
 constexpr int line_regions() {
-    return paired_lines<T, LC, NT, PR>() ? 2 : 1;
+    return paired_lines<T, LC, NT>() ? 2 : 1;
 }
 
 // FP64 lines of 2048 and 4096 (two workgroups or one per CU): wave-split
@@ -445,10 +443,10 @@ constexpr int line_regions() {
 // field needs no barrier of its own; the column stage transposes back to the
 // standard pattern through the second region, so consecutive transforms need
 // none between them.
-template <typename T, int LC, int NT = threads_for(LC), int PR = -1>
+template <typename T, int LC, int NT = threads_for(LC)>
 constexpr bool ws_lines64() {
     return sizeof(T) == 8 && (LC == 2048 || LC == 4096) && NT * P == LC &&
-           !paired_lines<T, LC, NT, PR>();
+           !paired_lines<T, LC, NT>();
 }
 
 
@@ -739,10 +737,10 @@ __device__ __forceinline__ cx<T> grow(cx<T> w, T em1) {
 // wave-split transforms (2048^2 FP32: k_row 29.2 -> 24.7 us, k_col 23.5 -> 24.1,
 // step 194 -> 180 us); at 64..1024, with Stockham lines, it measured slower
 // (256-member ensemble 92k -> 86k member-steps/s).
-template <typename T, int LC, int NT, int PR>
+template <typename T, int LC, int NT>
 constexpr bool pair_layout() {
     return sizeof(T) == 4 && (LC == 2048 || LC == 4096 || LC == 8192) && NT * P == LC &&
-           paired_lines<T, LC, NT, PR>();
+           paired_lines<T, LC, NT>();
 }
 
 // Row-pair tiles of the mixed fields (rowpair_elem): the FP64 stage kernels
@@ -755,9 +753,9 @@ constexpr bool pair_layout() {
 // one XCD, one after the other).  J stays [kx][y]: in tiles of 2, 4 or 8
 // rows the column stage's reads of it cost more than the row stage's stores
 // gained.
-template <typename T, int LC, int NT, int PR>
+template <typename T, int LC, int NT>
 constexpr bool rowpair_layout() {
-    return ws_lines64<T, LC, NT, PR>();
+    return ws_lines64<T, LC, NT>();
 }
 
 // Row-pair tiles of the pair buffers: FP32 lines of 8192.  Element (kx, y) of
@@ -773,9 +771,9 @@ constexpr bool rowpair_layout() {
 // with one workgroup per CU whose waves wait at the same barriers.  A
 // persistent row stage that gathered the next row pair's psi fields under J's
 // transform took 477 us (96 bytes of scratch).
-template <typename T, int LC, int NT, int PR>
+template <typename T, int LC, int NT>
 constexpr bool pairtile_layout() {
-    return LC == 8192 && pair_layout<T, LC, NT, PR>();
+    return LC == 8192 && pair_layout<T, LC, NT>();
 }
 __device__ __forceinline__ unsigned pairtile_elem(int k, int K, int y) {
     return 4u * (__umul24((unsigned)y >> 1, (unsigned)K) + (unsigned)k) + 2u * ((unsigned)y & 1u);
@@ -783,26 +781,26 @@ __device__ __forceinline__ unsigned pairtile_elem(int k, int K, int y) {
 
 // the stage kernels' own layout of the mixed fields, if any (RowArgs and
 // ColArgs::pairs select it per launch)
-template <typename T, int LC, int NT, int PR>
+template <typename T, int LC, int NT>
 constexpr bool stage_layout() {
-    return pair_layout<T, LC, NT, PR>() || rowpair_layout<T, LC, NT, PR>();
+    return pair_layout<T, LC, NT>() || rowpair_layout<T, LC, NT>();
 }
 
 // line regions of the stage kernels
-template <typename T, int LC, int NT = threads_for(LC), int PR = -1>
+template <typename T, int LC, int NT = threads_for(LC)>
 constexpr int stage_regions() {
-    return ws_lines64<T, LC, NT, PR>() ? 2 : line_regions<T, LC, NT, PR>();
+    return ws_lines64<T, LC, NT>() ? 2 : line_regions<T, LC, NT>();
 }
 // stage kernels that run wave-split transforms (their line regions hold
 // WS_REGION elements; staged lines in them are unpadded)
-template <typename T, int LC, int NT = threads_for(LC), int PR = -1>
+template <typename T, int LC, int NT = threads_for(LC)>
 constexpr bool ws_stage() {
-    return pair_layout<T, LC, NT, PR>() || ws_lines64<T, LC, NT, PR>();
+    return pair_layout<T, LC, NT>() || ws_lines64<T, LC, NT>();
 }
 // elements of one line region of a stage kernel (compile-time lengths)
-template <typename T, int LC, int NT = threads_for(LC), int PR = -1>
+template <typename T, int LC, int NT = threads_for(LC)>
 constexpr int region_elems() {
-    return ws_stage<T, LC, NT, PR>() ? ws_region(LC) : LC + LC / 16;
+    return ws_stage<T, LC, NT>() ? ws_region(LC) : LC + LC / 16;
 }
 
 // store (first, second) at pair element e of pair buffer B (one 16 bytes)
@@ -840,10 +838,10 @@ struct TwSource<true, L, T> {
 };
 
 // MW: occupancy floor handed to the register allocator (waves per SIMD)
-template <typename T, int NT, int MODE, int SCHEME, int LC, int PR = -1, bool ERR = false,
+template <typename T, int NT, int MODE, int SCHEME, int LC, bool ERR = false,
           int MW = min_waves<T>()>
 __global__ __launch_bounds__(NT, MW) void k_col(ColArgs<T> a) {
-    static_assert(!pair_layout<T, LC, NT, PR>() || paired_lines<T, LC, NT, PR>(),
+    static_assert(!pair_layout<T, LC, NT>() || paired_lines<T, LC, NT>(),
                   "the pair layout is written by the paired k_col path");
     extern __shared__ __align__(16) unsigned char smem_raw[];
     cx<T>* smem = reinterpret_cast<cx<T>*>(smem_raw);
@@ -881,18 +879,18 @@ __global__ __launch_bounds__(NT, MW) void k_col(ColArgs<T> a) {
     const int Ll = LC > 0 ? LC : g.L;
     const int lines = NT / TPL;
     const int m = threadIdx.x / TPL, j = threadIdx.x - m * TPL;
-    constexpr int NB = stage_regions<T, LC, NT, PR>();
-    const int RE = LC > 0 ? region_elems<T, LC, NT, PR>() : Ll + Ll / 16;
+    constexpr int NB = stage_regions<T, LC, NT>();
+    const int RE = LC > 0 ? region_elems<T, LC, NT>() : Ll + Ll / 16;
     cx<T>* lds = smem + m * NB * RE;
     cx<T>* lds2 = lds + (NB - 1) * RE;
-    constexpr bool WS = ws_lines64<T, LC, NT, PR>();
+    constexpr bool WS = ws_lines64<T, LC, NT>();
     // forward transform through ws_c as well (two line regions free for it)
-    constexpr bool WSF = WS || pairtile_layout<T, LC, NT, PR>();
+    constexpr bool WSF = WS || pairtile_layout<T, LC, NT>();
     // pair-layout kernels read J in 2 x 2 blocks: columns k and k ^ 1 share
     // lines; row-pair tiles put ROWPAIR_CPL columns in one line
-    constexpr int XG = pairtile_layout<T, LC, NT, PR>()   ? 4
-                       : pair_layout<T, LC, NT, PR>()    ? 2
-                       : rowpair_layout<T, LC, NT, PR>() ? ROWPAIR_CPL
+    constexpr int XG = pairtile_layout<T, LC, NT>()   ? 4
+                       : pair_layout<T, LC, NT>()    ? 2
+                       : rowpair_layout<T, LC, NT>() ? ROWPAIR_CPL
                                                          : 1;
     const int kxi = xcd_group_remap<XG>(blockIdx.x, gridDim.x) * lines + m;
     const int ncols = (MODE == COL_FWD) ? G.nkx : G.nkx_keep;
@@ -923,7 +921,7 @@ __global__ __launch_bounds__(NT, MW) void k_col(ColArgs<T> a) {
     // runs while they arrive (its twiddles in registers, loaded first, so that
     // it has no global load of its own to wait behind them).
     constexpr bool PF = MODE == COL_STAGE && LC >= 64 &&
-                        (paired_lines<T, LC, NT, PR>() || (sizeof(T) == 8 && NT <= 512));
+                        (paired_lines<T, LC, NT>() || (sizeof(T) == 8 && NT <= 512));
     cx<T> pw0[P], pacc[P];
     // The smallest FP32 workgroups (launches with few waves): dt and the modes'
     // factors before the transform of J, which waits a memory latency anyway.
@@ -950,7 +948,7 @@ __global__ __launch_bounds__(NT, MW) void k_col(ColArgs<T> a) {
         std::conditional_t<WSF, TwWs<LC, T>, TwRegs<LC, T>> tw;
         if constexpr (WSF) load_tw_ws(tw, j, a.tw);
         else load_tw_regs<LC, 0>(tw, j, a.tw);
-        if constexpr (pair_layout<T, LC, NT, PR>()) {
+        if constexpr (pair_layout<T, LC, NT>()) {
             // J in 2 x 2 blocks: jblock_elem(kxi, ny, y), y = j + s TPL (TPL
             // even), is a column base, the lane's offset j + (j & ~1), and
             // 2 TPL per slot; [kx][y] on rectangular grids, whose row stage
@@ -963,7 +961,7 @@ __global__ __launch_bounds__(NT, MW) void k_col(ColArgs<T> a) {
 #pragma unroll
             for (int s = 0; s < P; ++s)
                 v[s] = has_data ? *at32(nl, jb0 + (unsigned)s * jbs) : zero;
-        } else if constexpr (rowpair_layout<T, LC, NT, PR>()) {
+        } else if constexpr (rowpair_layout<T, LC, NT>()) {
             // J's last reader, whole columns: non-temporal loads, which leave
             // the caches to the mixed fields written next (FP64 4096^2:
             // k_col 177.1 -> 174.0 us); every column of the grid is kept
@@ -1233,7 +1231,7 @@ __global__ __launch_bounds__(NT, MW) void k_col(ColArgs<T> a) {
                 for (int s = 0; s < P; ++s) out[mbase + j + s * TPL] = v[s];
             }
         }
-    } else if constexpr (paired_lines<T, LC, NT, PR>()) {
+    } else if constexpr (paired_lines<T, LC, NT>()) {
         // outputs 0 psi_x, 1 psi_y, 2 omega_x, 3 omega_y (spectral_core.c:62-99),
         // transformed two at a time: (omega_y, omega_x), then w becomes
         // psi_hat = -w/k^2 in place and (psi_y, psi_x)
@@ -1249,9 +1247,9 @@ __global__ __launch_bounds__(NT, MW) void k_col(ColArgs<T> a) {
                 v[s] = mul_i(w[s], ky);
                 v2[s] = mul_i(w[s], kx);
             }
-            // FP32 4096 (pair layout): wave-split transforms, standard
+            // FP32 2048 to 8192 (pair layout): wave-split transforms, standard
             // pattern in and out (ws_c), transposing back in the same regions
-            constexpr bool WSC = pair_layout<T, LC, NT, PR>();
+            constexpr bool WSC = pair_layout<T, LC, NT>();
             std::conditional_t<WSC, TwWs<LC, T>, TwRegs<LC, T>> tw;
             cx<T>(*const vv[2])[P] = {&v, &v2};
             cx<T>* const rr[2] = {lds, lds2};
@@ -1265,10 +1263,10 @@ __global__ __launch_bounds__(NT, MW) void k_col(ColArgs<T> a) {
                 load_tw_regs<LC, 0>(tw, j, a.tw);
             }
             if (has_data) {
-                if constexpr (pair_layout<T, LC, NT, PR>()) {
+                if constexpr (pair_layout<T, LC, NT>()) {
                     if (a.pairs) {  // (omega_x, omega_y)
                         cx<T>* pb = a.mixed[2] + 2 * mixed_off;
-                        if constexpr (pairtile_layout<T, LC, NT, PR>()) {
+                        if constexpr (pairtile_layout<T, LC, NT>()) {
                             store_pair_tiles<LC>(pb, kxi, (G.nkx_keep + 1) & ~1, j, v2, v);
                         } else {
 #pragma unroll
@@ -1277,7 +1275,7 @@ __global__ __launch_bounds__(NT, MW) void k_col(ColArgs<T> a) {
                         }
                     }
                 }
-                if (!(pair_layout<T, LC, NT, PR>() && a.pairs)) {
+                if (!(pair_layout<T, LC, NT>() && a.pairs)) {
                     cx<T>* o1 = a.mixed[3] + mixed_off;
                     cx<T>* o2 = a.mixed[2] + mixed_off;
 #pragma unroll
@@ -1303,10 +1301,10 @@ __global__ __launch_bounds__(NT, MW) void k_col(ColArgs<T> a) {
                 line_fft2_c<+1, LC>(v, v2, lds, lds2, j, tw);  // psi_y, psi_x
             }
             if (has_data) {
-                if constexpr (pair_layout<T, LC, NT, PR>()) {
+                if constexpr (pair_layout<T, LC, NT>()) {
                     if (a.pairs) {  // (psi_x, psi_y)
                         cx<T>* pb = a.mixed[0] + 2 * mixed_off;
-                        if constexpr (pairtile_layout<T, LC, NT, PR>()) {
+                        if constexpr (pairtile_layout<T, LC, NT>()) {
                             store_pair_tiles<LC>(pb, kxi, (G.nkx_keep + 1) & ~1, j, v2, v);
                         } else {
 #pragma unroll
@@ -1315,7 +1313,7 @@ __global__ __launch_bounds__(NT, MW) void k_col(ColArgs<T> a) {
                         }
                     }
                 }
-                if (!(pair_layout<T, LC, NT, PR>() && a.pairs)) {
+                if (!(pair_layout<T, LC, NT>() && a.pairs)) {
                     cx<T>* o1 = a.mixed[1] + mixed_off;
                     cx<T>* o2 = a.mixed[0] + mixed_off;
 #pragma unroll
@@ -1355,7 +1353,7 @@ __global__ __launch_bounds__(NT, MW) void k_col(ColArgs<T> a) {
             }
         }
     } else if constexpr (WS) {
-        // FP64 columns of 4096: the four outputs one at a time through ws_c
+        // FP64 columns of 2048 and 4096: the four outputs one at a time through ws_c
         // (spectral_core.c:62-99), swizzled rows in lds, the transposing
         // exchange in lds2: two barriers per transform
         TwWs<LC, T> tw;
@@ -1797,11 +1795,11 @@ constexpr bool row_prefetch() {
     return LC >= 64 && (LC != 1024 || sizeof(T) == 4);
 }
 
-template <typename T, int NT, int MODE, int LC, int PR = -1, bool ERR = false,
+template <typename T, int NT, int MODE, int LC, bool ERR = false,
           int MW = min_waves<T>(), bool FORCE = false>
 __global__ __launch_bounds__(NT, MW) void k_row(RowArgs<T> a) {
-    static_assert(!pair_layout<T, LC, NT, PR>() ||
-                      (paired_lines<T, LC, NT, PR>() && row_prefetch<T, LC>()),
+    static_assert(!pair_layout<T, LC, NT>() ||
+                      (paired_lines<T, LC, NT>() && row_prefetch<T, LC>()),
                   "the pair layout is read by the paired gather-ahead k_row path");
     // error controller: stages 1-3 of a step that restores a rejected
     // candidate have nothing to do (uniform over the grid)
@@ -1817,8 +1815,8 @@ __global__ __launch_bounds__(NT, MW) void k_row(RowArgs<T> a) {
     const int Ll = LC > 0 ? LC : g.L;
     const int lines = NT / TPL;
     const int m = threadIdx.x / TPL, j = threadIdx.x - m * TPL;
-    constexpr int NB = stage_regions<T, LC, NT, PR>();
-    const int RE = LC > 0 ? region_elems<T, LC, NT, PR>() : Ll + Ll / 16;
+    constexpr int NB = stage_regions<T, LC, NT>();
+    const int RE = LC > 0 ? region_elems<T, LC, NT>() : Ll + Ll / 16;
     cx<T>* lds = smem + m * NB * RE;
     cx<T>* lds2 = lds + (NB - 1) * RE;
     if constexpr (FORCE) {
@@ -1901,12 +1899,12 @@ __global__ __launch_bounds__(NT, MW) void k_row(RowArgs<T> a) {
     // accumulators live across transforms.
     cx<T> X[P], Jp[P];
     SpeedMax<T> um;
-    if constexpr (pair_layout<T, LC, NT, PR>()) {
-        // FP32 rows of 4096 on 512 threads: the paired gather-ahead schedule
+    if constexpr (pair_layout<T, LC, NT>()) {
+        // FP32 rows of 2048 to 8192, one to a workgroup: the paired gather-ahead schedule
         // below with wave-split transforms (ws_a for the four fields, whose
         // outputs are in the wave-strided pattern, ws_b for J, which takes
         // that pattern back to the standard one): 11 workgroup barriers per
-        // row pair instead of 27.
+        // row pair instead of 27 (at 4096).
         TwWs<LC, T> tw;
         load_tw_ws(tw, j, a.tw);
         if (blk * lines < G.ny / 2) {
@@ -1914,7 +1912,7 @@ __global__ __launch_bounds__(NT, MW) void k_row(RowArgs<T> a) {
             // and the gathers need no zero fill for an inactive one
             static_assert(NT * P / LC == 1, "one row pair per workgroup");
             constexpr bool live = true;
-            constexpr bool PT = pairtile_layout<T, LC, NT, PR>();
+            constexpr bool PT = pairtile_layout<T, LC, NT>();
             RowPairRegs<T> r0, r1, q0, q1;
             const bool pl = a.pairs != 0;
             if (pl) gather_pair<LC, PT>(r0, r1, j, G, a.mixed[0] + 2 * moff, y0, live);
@@ -1962,7 +1960,7 @@ __global__ __launch_bounds__(NT, MW) void k_row(RowArgs<T> a) {
         if (a.track_umax) block_max_to(active ? double(um.value()) : 0.0, &a.sc[blockIdx.y].umax2_bits, red);
         return;
     }
-    if constexpr (paired_lines<T, LC, NT, PR>() && row_prefetch<T, LC>()) {
+    if constexpr (paired_lines<T, LC, NT>() && row_prefetch<T, LC>()) {
         // Twiddles first, then the psi gathers, then the omega gathers,
         // which stay in flight while the psi fields are transformed: with
         // the twiddles in registers the transforms issue no global loads
@@ -1975,24 +1973,12 @@ __global__ __launch_bounds__(NT, MW) void k_row(RowArgs<T> a) {
         // the compiler's schedule of the loads above within 128 VGPRs)
         if (blk * lines < G.ny / 2) {
             RowPairRegs<T> r0, r1, q0, q1;
-            bool pl = false;
-            if constexpr (pair_layout<T, LC, NT, PR>()) pl = a.pairs != 0;
-            if constexpr (pair_layout<T, LC, NT, PR>()) {
-                if (pl) gather_pair_rows<LC>(r0, r1, j, G, a.mixed[0] + 2 * moff, y0, active);
-            }
-            if (!pl) {
-                gather_two_rows<LC>(r0, j, G, a.mixed[0] + moff, y0, active);
-                gather_two_rows<LC>(r1, j, G, a.mixed[1] + moff, y0, active);
-            }
+            gather_two_rows<LC>(r0, j, G, a.mixed[0] + moff, y0, active);
+            gather_two_rows<LC>(r1, j, G, a.mixed[1] + moff, y0, active);
             stage_two_rows_regs<LC, KEPT>(lds, j, r0);
             stage_two_rows_regs<LC, KEPT>(lds2, j, r1);
-            if constexpr (pair_layout<T, LC, NT, PR>()) {
-                if (pl) gather_pair_rows<LC>(q0, q1, j, G, a.mixed[2] + 2 * moff, y0, active);
-            }
-            if (!pl) {
-                gather_two_rows<LC>(q0, j, G, a.mixed[2] + moff, y0, active);
-                gather_two_rows<LC>(q1, j, G, a.mixed[3] + moff, y0, active);
-            }
+            gather_two_rows<LC>(q0, j, G, a.mixed[2] + moff, y0, active);
+            gather_two_rows<LC>(q1, j, G, a.mixed[3] + moff, y0, active);
             __syncthreads();
             cx<T> v2[P];
             lds_read_any<LC, KEPT>(v, lds, j);
@@ -2014,14 +2000,12 @@ __global__ __launch_bounds__(NT, MW) void k_row(RowArgs<T> a) {
 #pragma unroll
             for (int s = 0; s < P; ++s)
                 v[s] = mk(X[s].x * v2[s].x - Jp[s].x * v[s].x, X[s].y * v2[s].y - Jp[s].y * v[s].y);
-            // a pair-layout row stage writes J in 2 x 2 blocks
-            fwd_rows_store<LC, T, TwRegs<LC, T>, pair_layout<T, LC, NT, PR>()>(
-                v, lds, j, g, G, tw, a.nl + moff, y0, active, a.jblocks);
+            fwd_rows_store<LC, T, TwRegs<LC, T>>(v, lds, j, g, G, tw, a.nl + moff, y0, active);
         }
         if (a.track_umax) block_max_to(active ? double(um.value()) : 0.0, &a.sc[blockIdx.y].umax2_bits, red);
         return;
     }
-    if constexpr (paired_lines<T, LC, NT, PR>()) {
+    if constexpr (paired_lines<T, LC, NT>()) {
         // FP64 rows of 1024: gathers at their use
         cx<T> v2[P];
         build_two_rows2<LC>(v, v2, lds, lds2, j, g, G, a.mixed[0] + moff, a.mixed[1] + moff, y0, active);
@@ -2041,8 +2025,8 @@ __global__ __launch_bounds__(NT, MW) void k_row(RowArgs<T> a) {
         if (a.track_umax) block_max_to(active ? double(um.value()) : 0.0, &a.sc[blockIdx.y].umax2_bits, red);
         return;
     }
-    if constexpr (ws_lines64<T, LC, NT, PR>()) {
-        // FP64 rows of 4096: one field at a time, each gather in flight while
+    if constexpr (ws_lines64<T, LC, NT>()) {
+        // FP64 rows of 2048 and 4096: one field at a time, each gather in flight while
         // the previous field is transformed (as below), with wave-split
         // transforms whose cross-wave rows live in lds2.  Every read of the
         // staged line in lds precedes the barrier inside ws_a, so the next

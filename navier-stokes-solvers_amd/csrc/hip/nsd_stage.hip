@@ -30,13 +30,12 @@ constexpr bool var_ok() {
     return V == 0 || (V == kSmallVariant ? L / P <= 64 : L >= 64 && L <= 1024);
 }
 
-// the stage kernels' LDS (FP64 lines of 4096 take a second line region)
+// the stage kernels' LDS (FP64 lines of 2048 and 4096 take a second line region)
 template <typename T, int L, int V>
 size_t stage_lds() {
     constexpr int NT = var_nt<L, V>();
     constexpr int lines = NT * P / L;
-    constexpr int PR = -1;
-    return (size_t)lines * stage_regions<T, L, NT, PR>() * region_elems<T, L, NT, PR>() *
+    return (size_t)lines * stage_regions<T, L, NT>() * region_elems<T, L, NT>() *
            sizeof(cx<T>);
 }
 
@@ -49,18 +48,17 @@ void row_stage_LV(const RowArgs<T>& a, int items, int members, hipStream_t st,
         if constexpr (L <= kFieldsMax) launch_row_fields<T>(a, L, items, members, st, ERR, force);
     } else if constexpr (var_ok<L, V>()) {
         constexpr int NT = var_nt<L, V>();
-        constexpr int PR = -1;
         constexpr int lines = NT * P / L;
         const int blocks = (items + lines - 1) / lines;
         const size_t lds = stage_lds<T, L, V>();
         if constexpr (!ERR) {
             if (force) {
-                hipLaunchKernelGGL((k_row<T, NT, ROW_STAGE, L, PR, false, min_waves<T>(), true>),
+                hipLaunchKernelGGL((k_row<T, NT, ROW_STAGE, L, false, min_waves<T>(), true>),
                                    dim3(blocks + 1, members), dim3(NT), lds, st, a);
                 return;
             }
         }
-        hipLaunchKernelGGL((k_row<T, NT, ROW_STAGE, L, PR, ERR>), dim3(blocks, members), dim3(NT),
+        hipLaunchKernelGGL((k_row<T, NT, ROW_STAGE, L, ERR>), dim3(blocks, members), dim3(NT),
                            lds, st, a);
     }
 }
@@ -72,18 +70,17 @@ void col_fused_LV(const ColArgs<T>& a, int ncols, int members, hipStream_t st) {
         if constexpr (L <= kFieldsMax) launch_col_fields<T>(a, L, ncols, members, st, ERR);
     } else if constexpr (var_ok<L, V>()) {
         constexpr int NT = var_nt<L, V>();
-        constexpr int PR = -1;
         constexpr int lines = NT * P / L;
         const int blocks = (ncols + lines - 1) / lines;
         const dim3 grid(blocks, members);
         const size_t lds = stage_lds<T, L, V>();
         if (a.mode == COL_PRIME)
-            hipLaunchKernelGGL((k_col<T, NT, COL_PRIME, 0, L, PR>), grid, dim3(NT), lds, st, a);
+            hipLaunchKernelGGL((k_col<T, NT, COL_PRIME, 0, L>), grid, dim3(NT), lds, st, a);
         else if (a.phys.scheme == 0)
-            hipLaunchKernelGGL((k_col<T, NT, COL_STAGE, 0, L, PR, ERR>), grid, dim3(NT), lds, st,
+            hipLaunchKernelGGL((k_col<T, NT, COL_STAGE, 0, L, ERR>), grid, dim3(NT), lds, st,
                                a);
         else
-            hipLaunchKernelGGL((k_col<T, NT, COL_STAGE, 1, L, PR, ERR>), grid, dim3(NT), lds, st,
+            hipLaunchKernelGGL((k_col<T, NT, COL_STAGE, 1, L, ERR>), grid, dim3(NT), lds, st,
                                a);
     }
 }
@@ -99,16 +96,15 @@ void limits_LV(int bytes) {
     constexpr int L = 1 << LOG;
     if constexpr (var_ok<L, V>() && V != kFieldsVariant) {
         constexpr int NT = var_nt<L, V>();
-        constexpr int PR = -1;
-        lds_attr(k_row<T, NT, ROW_STAGE, L, PR>, bytes);
-        lds_attr(k_row<T, NT, ROW_STAGE, L, PR, false, min_waves<T>(), true>, bytes);
-        lds_attr(k_col<T, NT, COL_PRIME, 0, L, PR>, bytes);
-        lds_attr(k_col<T, NT, COL_STAGE, 0, L, PR>, bytes);
-        lds_attr(k_col<T, NT, COL_STAGE, 1, L, PR>, bytes);
+        lds_attr(k_row<T, NT, ROW_STAGE, L>, bytes);
+        lds_attr(k_row<T, NT, ROW_STAGE, L, false, min_waves<T>(), true>, bytes);
+        lds_attr(k_col<T, NT, COL_PRIME, 0, L>, bytes);
+        lds_attr(k_col<T, NT, COL_STAGE, 0, L>, bytes);
+        lds_attr(k_col<T, NT, COL_STAGE, 1, L>, bytes);
         if constexpr (V == 0) {
-            lds_attr(k_row<T, NT, ROW_STAGE, L, PR, true>, bytes);
-            lds_attr(k_col<T, NT, COL_STAGE, 0, L, PR, true>, bytes);
-            lds_attr(k_col<T, NT, COL_STAGE, 1, L, PR, true>, bytes);
+            lds_attr(k_row<T, NT, ROW_STAGE, L, true>, bytes);
+            lds_attr(k_col<T, NT, COL_STAGE, 0, L, true>, bytes);
+            lds_attr(k_col<T, NT, COL_STAGE, 1, L, true>, bytes);
         }
     }
 }
@@ -116,7 +112,7 @@ void limits_LV(int bytes) {
 template <typename T, int LOG, int V>
 int var_pairs() {
     constexpr int L = 1 << LOG;
-    if constexpr (V != kFieldsVariant && var_ok<L, V>()) return stage_layout<T, L, var_nt<L, V>(), -1>() ? 1 : 0;
+    if constexpr (V != kFieldsVariant && var_ok<L, V>()) return stage_layout<T, L, var_nt<L, V>()>() ? 1 : 0;
     return 0;
 }
 
@@ -125,7 +121,7 @@ template <typename T, int LOG, int V>
 int var_rounding() {
     constexpr int L = 1 << LOG;
     if constexpr (V == kFieldsVariant) return L <= kFieldsMax ? 2 : -1;
-    else if constexpr (var_ok<L, V>()) return paired_lines<T, L, var_nt<L, V>(), -1>() ? 1 : 0;
+    else if constexpr (var_ok<L, V>()) return paired_lines<T, L, var_nt<L, V>()>() ? 1 : 0;
     return -1;
 }
 
@@ -264,15 +260,6 @@ template void launch_row_stage<NSD_T>(const RowArgs<NSD_T>&, int, int, int, int,
 template void launch_col_fused<NSD_T>(const ColArgs<NSD_T>&, int, int, int, int, hipStream_t,
                                       bool);
 
-// workgroups of the default column launch over ncols columns of length L
-// (the number of partials the error controller's last stage leaves)
-template <typename T>
-int col_fused_blocks(int L, int ncols) {
-    const int NT = L / P > 256 ? L / P : 256;
-    const int lines = NT * P / L;
-    return (ncols + lines - 1) / lines;
-}
-template int col_fused_blocks<NSD_T>(int, int);
 // Variant a context starts with, for `members` times `lines` lines (row pairs, kind 0,
 // or kept columns, kind 1) of length L.
 //

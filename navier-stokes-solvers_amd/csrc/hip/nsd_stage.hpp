@@ -26,9 +26,6 @@ void launch_row_stage(const RowArgs<T>& a, int L, int items, int members, int va
 template <typename T>
 void launch_col_fused(const ColArgs<T>& a, int L, int ncols, int members, int variant,
                       hipStream_t st, bool errctl = false);
-// workgroups of the default (variant 0) column launch over ncols columns
-template <typename T>
-int col_fused_blocks(int L, int ncols);
 // variant that a context starts with for `lines` lines (kind 0: row pairs, 1: columns)
 // of each member
 template <typename T>
