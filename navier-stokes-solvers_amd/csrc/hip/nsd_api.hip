@@ -839,8 +839,13 @@ int lastk(NsdContext* c) {
 // nsd_kernels.hpp: the pair layout at FP32, row-pair tiles at FP64) when the
 // row and the column instantiations this context launches both hold it
 // (square 2048^2, 4096^2 and FP32 8192^2 grids); the answer follows the launch variants.
+// Larger FP64 batches of 2048^2 keep the per-field layout: past the MALL the column
+// stage's stores into tiles, 32 bytes a column, cost more than the row stage's gathers
+// gain (k_row + k_col, us, tiles against per field: 2 members 145 / 144, 5 378 / 380, 8
+// 613 / 577, 16 1272 / 1109; 4096^2 x 4 1306 / 1359).
 bool pairs_ok(const NsdContext* c) {
     if (c->G.nx != c->G.ny) return false;
+    if (c->prec == NSD_FP64 && c->G.nx == 2048 && c->nb > 5) return false;
     if (c->prec == NSD_FP32)
         return stage_variant_pairs<float>(c->G.nx, c->vrow) &&
                stage_variant_pairs<float>(c->G.ny, c->vcol);

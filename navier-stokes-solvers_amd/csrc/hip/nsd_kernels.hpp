@@ -1659,36 +1659,29 @@ __device__ __forceinline__ void gather_two_rows(RowPairRegs<T>& r, int j, const 
     }
 }
 
-// The same from slot elements (row_slots): the per-field layout or row-pair
-// tiles, rows y and y + 1 adjacent in both.  Non-temporal loads: in row-pair
-// tiles no other row pair reads these bytes, and the stage reads each field
-// once, so they need not displace from L2 and the MALL the J values and
-// compact fields that k_col reads next (FP64 4096^2 step 1.368 -> 1.346 ms:
-// k_row +3.7 us, k_col -9.7 us).  The per-field layout, which only the
-// nonlinear-term entry point hands this kernel, shares each line among four
-// row pairs and pays for the loads there; that call is not on the step's
-// path.  The FP32 pair layout keeps ordinary loads (gather_pair_rows): the
-// same loads there took k_row from 76 to 137 us.
-template <int LC, typename T>
+// The same from slot elements (row_slots), rows y and y + 1 adjacent: the per-field
+// layout, or row-pair tiles.  In tiles no other row pair reads these bytes, and the
+// stage reads each field once, so they need not displace from L2 and the MALL the J
+// values and compact fields that k_col reads next: non-temporal loads there (FP64
+// 4096^2 step 1.368 -> 1.346 ms: k_row +3.7 us, k_col -9.7 us).  The per-field layout
+// (rectangles, large batches) shares each line among four row pairs: ordinary loads
+// (non-temporal ones took k_row at 2048 x 4096 from 84 to 144 us).  The FP32 pair
+// layout keeps ordinary loads as well (gather_pair_rows): 76 against 137 us.
+template <int LC, bool TILES, typename T>
 __device__ __forceinline__ void gather_two_rows(RowPairRegs<T>& r, int j, const cx<T>* F,
-                                                SlotElems se, bool active) {
+                                                SlotElems se) {
     typedef T t2 __attribute__((ext_vector_type(2)));
     constexpr int kxm = Band<LC>::kxm;
+    auto load = [](const t2* p) { return TILES ? __builtin_nontemporal_load(p) : *p; };
 #pragma unroll
     for (int s = 0; s < P; ++s) {
         const int kind = slot_kind(s, LC, kxm);
         const int k = j + s * (LC / P);
         if (kind == 1 || (kind == 3 && k <= kxm)) {
-            if (active) {
-                const t2* src = reinterpret_cast<const t2*>(at32(F, se.e0 + (unsigned)s * se.es));
-                const t2 a = __builtin_nontemporal_load(src);
-                const t2 b = __builtin_nontemporal_load(src + 1);
-                r.a[s] = mk(a.x, a.y);
-                r.b[s] = mk(b.x, b.y);
-            } else {
-                r.a[s] = mk(T(0), T(0));
-                r.b[s] = mk(T(0), T(0));
-            }
+            const t2* src = reinterpret_cast<const t2*>(at32(F, se.e0 + (unsigned)s * se.es));
+            const t2 a = load(src), b = load(src + 1);
+            r.a[s] = mk(a.x, a.y);
+            r.b[s] = mk(b.x, b.y);
         }
     }
 }
@@ -1795,8 +1788,10 @@ constexpr bool row_prefetch() {
     return LC >= 64 && (LC != 1024 || sizeof(T) == 4);
 }
 
+// FORCE: workgroup 0 makes the forcing draw; TILES (ws_lines64): the inputs are in
+// row-pair tiles, else per field ([kx][y])
 template <typename T, int NT, int MODE, int LC, bool ERR = false,
-          int MW = min_waves<T>(), bool FORCE = false>
+          int MW = min_waves<T>(), bool FORCE = false, bool TILES = true>
 __global__ __launch_bounds__(NT, MW) void k_row(RowArgs<T> a) {
     static_assert(!pair_layout<T, LC, NT>() ||
                       (paired_lines<T, LC, NT>() && row_prefetch<T, LC>()),
@@ -2036,15 +2031,16 @@ __global__ __launch_bounds__(NT, MW) void k_row(RowArgs<T> a) {
         if (blk * lines < G.ny / 2) {
             cx<T>(*const vv[1])[P] = {&v};
             cx<T>* const rr[1] = {lds2};
-            // the inputs in row-pair tiles or per field ([kx][y]); one line
-            // per workgroup, whose row pair exists inside this branch
+            // one line per workgroup, whose row pair exists inside this branch
             static_assert(NT * P / LC == 1, "one row pair per workgroup");
-            constexpr bool live = true;
-            const SlotElems se = row_slots<LC>(j, G.ny, (G.nkx_keep + 1) & ~1, y0, a.pairs != 0);
+            // (pairs is set where TILES is; as a run-time value it keeps a schedule of the
+            // gathers that is 1.5 % faster: FP64 4096^2 162.5 -> 159.5 us)
+            const SlotElems se =
+                row_slots<LC>(j, G.ny, (G.nkx_keep + 1) & ~1, y0, TILES && a.pairs != 0);
             RowPairRegs<T> r;
-            gather_two_rows<LC>(r, j, a.mixed[0] + moff, se, live);
+            gather_two_rows<LC, TILES>(r, j, a.mixed[0] + moff, se);
             stage_two_rows_regs<LC, true, false>(lds, j, r);
-            gather_two_rows<LC>(r, j, a.mixed[1] + moff, se, live);
+            gather_two_rows<LC, TILES>(r, j, a.mixed[1] + moff, se);
             __syncthreads();
             lds_read_kept<LC, false>(v, lds, j);
             ws_a<+1, 1, true>(vv, rr, j, tw);  // psi_x
@@ -2052,7 +2048,7 @@ __global__ __launch_bounds__(NT, MW) void k_row(RowArgs<T> a) {
             for (int s = 0; s < P; ++s) X[s] = v[s];
             __builtin_amdgcn_sched_barrier(0);
             stage_two_rows_regs<LC, true, false>(lds, j, r);
-            gather_two_rows<LC>(r, j, a.mixed[2] + moff, se, live);
+            gather_two_rows<LC, TILES>(r, j, a.mixed[2] + moff, se);
             __syncthreads();
             lds_read_kept<LC, false>(v, lds, j);
             ws_a<+1, 1, true>(vv, rr, j, tw);  // psi_y
@@ -2061,7 +2057,7 @@ __global__ __launch_bounds__(NT, MW) void k_row(RowArgs<T> a) {
             for (int s = 0; s < P; ++s) Jp[s] = v[s];
             __builtin_amdgcn_sched_barrier(0);
             stage_two_rows_regs<LC, true, false>(lds, j, r);
-            gather_two_rows<LC>(r, j, a.mixed[3] + moff, se, live);
+            gather_two_rows<LC, TILES>(r, j, a.mixed[3] + moff, se);
             __syncthreads();
             lds_read_kept<LC, false>(v, lds, j);
             ws_a<+1, 1, true>(vv, rr, j, tw);  // omega_x

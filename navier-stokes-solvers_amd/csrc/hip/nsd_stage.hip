@@ -51,15 +51,26 @@ void row_stage_LV(const RowArgs<T>& a, int items, int members, hipStream_t st,
         constexpr int lines = NT * P / L;
         const int blocks = (items + lines - 1) / lines;
         const size_t lds = stage_lds<T, L, V>();
-        if constexpr (!ERR) {
-            if (force) {
-                hipLaunchKernelGGL((k_row<T, NT, ROW_STAGE, L, false, min_waves<T>(), true>),
-                                   dim3(blocks + 1, members), dim3(NT), lds, st, a);
-                return;
+        const dim3 grid(blocks + (force && !ERR ? 1 : 0), members), nt(NT);
+        auto go = [&](auto tiles) {
+            constexpr bool TI = decltype(tiles)::value;
+            constexpr int MW = min_waves<T>();
+            if constexpr (!ERR) {
+                if (force) {
+                    hipLaunchKernelGGL((k_row<T, NT, ROW_STAGE, L, false, MW, true, TI>), grid, nt,
+                                       lds, st, a);
+                    return;
+                }
             }
+            hipLaunchKernelGGL((k_row<T, NT, ROW_STAGE, L, ERR, MW, false, TI>), grid, nt, lds, st,
+                               a);
+        };
+        // kernels of their own: as branches of one the tiles' loads lose their hint, or
+        // the step 0.5 % (FP64 4096^2)
+        if constexpr (ws_lines64<T, L, NT>()) {
+            if (!a.pairs) return go(std::false_type{});
         }
-        hipLaunchKernelGGL((k_row<T, NT, ROW_STAGE, L, ERR>), dim3(blocks, members), dim3(NT),
-                           lds, st, a);
+        go(std::true_type{});
     }
 }
 
@@ -96,8 +107,14 @@ void limits_LV(int bytes) {
     constexpr int L = 1 << LOG;
     if constexpr (var_ok<L, V>() && V != kFieldsVariant) {
         constexpr int NT = var_nt<L, V>();
+        constexpr int MW = min_waves<T>();
         lds_attr(k_row<T, NT, ROW_STAGE, L>, bytes);
-        lds_attr(k_row<T, NT, ROW_STAGE, L, false, min_waves<T>(), true>, bytes);
+        lds_attr(k_row<T, NT, ROW_STAGE, L, false, MW, true>, bytes);
+        if constexpr (ws_lines64<T, L, NT>()) {
+            lds_attr(k_row<T, NT, ROW_STAGE, L, false, MW, false, false>, bytes);
+            lds_attr(k_row<T, NT, ROW_STAGE, L, false, MW, true, false>, bytes);
+            lds_attr(k_row<T, NT, ROW_STAGE, L, true, MW, false, false>, bytes);
+        }
         lds_attr(k_col<T, NT, COL_PRIME, 0, L>, bytes);
         lds_attr(k_col<T, NT, COL_STAGE, 0, L>, bytes);
         lds_attr(k_col<T, NT, COL_STAGE, 1, L>, bytes);

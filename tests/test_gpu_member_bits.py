@@ -13,7 +13,8 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("nx,ny,fp32,counts", [
     (16, 16, False, (2, 700)), (32, 32, False, (2, 600)), (64, 64, False, (20, 260)),
     (128, 128, False, (16, 70)), (256, 256, False, (8, 17, 40)), (512, 512, False, (2, 9)),
-    (1024, 1024, False, (2, 7)), (2048, 1024, False, (2,)), (512, 1024, False, (3,)),
+    (1024, 1024, False, (2, 7)), (2048, 1024, False, (2,)),
+    (2048, 2048, False, (2, 6)), (512, 1024, False, (3,)),
     (16, 16, True, (2, 700)), (32, 32, True, (2, 600)), (64, 64, True, (20, 260)),
     (128, 128, True, (16, 70)), (256, 256, True, (8, 17, 40)), (512, 512, True, (2, 5, 24)),
     (1024, 1024, True, (2, 4, 16)), (1024, 512, True, (3, 5)), (2048, 2048, True, (2,))])
