@@ -551,7 +551,7 @@ __global__ void k_scale_state(size_t n, cx<T>* st, const DevScalars* sc, double 
 __global__ void k_force(ForceArgs a) {
     if (a.skip_on_redo && a.sc[blockIdx.y].redo) return;
     __shared__ double red[kForceRed];
-    force_draw(a, blockIdx.y, red);
+    force_draw<true>(a, blockIdx.y, red);
 }
 
 // forcing.c:117-184 on a full reference-layout output (compat entry point)
@@ -1004,15 +1004,15 @@ int op_prime(NsdContext* c) {
 bool force_active(const NsdContext* c) { return c->phys.force_on && c->fA != 0; }
 
 // Whether the row kernel's extra workgroup makes the draw in about the time that
-// the others take: it has one pass (1.7 us) over the modes per workgroup's worth of
-// them.  us per step, in the row kernel -> a kernel of up to 1024 threads in line:
-//   64 threads: 256^2 FP32 130 modes 62.9 -> 64.1, 270 67.8 -> 65.2, 1400 106 -> 71
-//   256: 512^2 FP64 1400 modes 74.9 -> 74.9, 2500 85.6 -> 81.6; 2048^2 FP32 2500 192 -> 197,
-//     5600 229 -> 220
-//   512: 1024^2 FP32 2500 modes 110 -> 116, 5600 136 -> 137; 4096^2 FP32 5600 584 -> 612
+// the others take: one pass (1.7 us) over the modes per workgroup's worth of them.  us
+// per step, in the row kernel / by a kernel of up to 1024 threads in line: 256^2 FP32 (64
+// threads) 37 modes 58 / 64, 270 66 / 65, 1400 98 / 70, 5600 214 / 90; 512^2 FP64 (256) 1400
+// 72 / 73, 2500 80 / 78; 1024^2 FP64 (512) 2500 147 / 156, 5600 171 / 176, 15700 237 / 234; 2048^2
+// FP32 (256) 2500 188 / 198, 5600 220 / 216; 4096^2 FP32 (512) 15700 638 / 658.
 template <typename T>
 bool draw_in_rows(const NsdContext* c) {
-    const int passes = std::max(3, std::max(c->G.nx, c->G.ny) / 128);
+    const int side = std::max(c->G.nx, c->G.ny);
+    const int passes = std::max(3, side / 128);
     return c->fA <= passes * row_stage_threads<T>(c->G.nx, c->vrow);
 }
 
@@ -2002,7 +2002,7 @@ int nsd_set_params(NsdContext* c, const NsdParams* p) {
         CK(hipMalloc(&c->fpartner, sizeof(int) * A));
         const size_t nb = (size_t)c->nb;
         CK(hipMalloc(&c->fou, 2 * sizeof(double) * A * nb));
-        CK(hipMalloc(&c->fwork, 4 * sizeof(double) * A * nb));
+        CK(hipMalloc(&c->fwork, 5 * sizeof(double) * A * nb));
         CK(hipMalloc(&c->fbox, c->esz * box * nb));
         CK(hipMemcpy(c->fmodes, modes.data(), sizeof(int) * A, hipMemcpyHostToDevice));
         CK(hipMemcpy(c->fpartner, partner.data(), sizeof(int) * A, hipMemcpyHostToDevice));

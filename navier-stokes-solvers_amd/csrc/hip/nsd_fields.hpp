@@ -305,7 +305,7 @@ __global__ __launch_bounds__(U * L / 2, MW) void k_row_fields(RowArgs<T> a) {
     }
     if constexpr (FORCE) {  // workgroup 0 makes the step's forcing draw
         if (blockIdx.x == 0) {
-            force_draw(a.force, blockIdx.y, reinterpret_cast<double*>(smem_raw));
+            force_draw<(U * L / 2 > kForceLanes)>(a.force, blockIdx.y, reinterpret_cast<double*>(smem_raw));
             return;
         }
     }

@@ -486,7 +486,7 @@ struct ForceArgs {
     int colored;
     double tau, energy_target, rate;
     double* ou;          // colored state per active rank (interleaved complex)
-    double* work;        // 2 * A doubles
+    double* work;        // 5 A doubles
     int fbx, fby;
     int box_T;           // 1: box in FP32, 0: FP64
     void* fbox;
@@ -501,14 +501,33 @@ struct ForceArgs {
 // added in order.
 constexpr int kForceLanes = 256;
 
-// add(sum, r) over the modes r < A, the waves' sums in red[0 .. 3]; every thread of a
-// workgroup of whole waves calls it
-template <typename F>
-__device__ __forceinline__ void force_sum(int A, double* red, F&& add) {
+// value(r) for the modes r < A, which also stores it where load(r) finds it, and
+// add(sum, value) over them, the waves' sums in red[0 .. 3]; every thread of a workgroup
+// of whole waves calls it.  ALL: the values by all threads of a larger workgroup, then
+// summed from memory; else by the lanes of the sums.
+template <bool ALL, typename V, typename L, typename F>
+__device__ __forceinline__ void force_sum(int A, double* red, V&& value, L&& load, F&& add) {
+    if constexpr (ALL) {
+        for (int r = threadIdx.x; r < A; r += blockDim.x) (void)value(r);
+        __syncthreads();
+    }
     for (int v = threadIdx.x; v < kForceLanes; v += blockDim.x) {
         double part = 0.0;
         if ((v & ~63) < A) {
-            for (int r = v; r < A; r += kForceLanes) part = add(part, r);
+            int r = v;
+            if constexpr (ALL) {
+                constexpr int N = 8;  // loads in flight
+                for (; r + (N - 1) * kForceLanes < A; r += N * kForceLanes) {
+                    decltype(load(0)) x[N];
+#pragma unroll
+                    for (int i = 0; i < N; ++i) x[i] = load(r + i * kForceLanes);
+#pragma unroll
+                    for (int i = 0; i < N; ++i) part = add(part, x[i]);
+                }
+                for (; r < A; r += kForceLanes) part = add(part, load(r));
+            } else {
+                for (; r < A; r += kForceLanes) part = add(part, value(r));
+            }
             part = wave_sum(part);
         }
         if ((v & 63) == 0) red[v >> 6] = part;
@@ -523,13 +542,14 @@ __device__ __forceinline__ double force_total(const double* red) {
 
 // The draw for member mb, by one workgroup; red: kForceRed doubles of LDS.
 constexpr int kForceRed = kForceLanes / 64 + 1;
+template <bool ALL>
 __device__ __forceinline__ void force_draw(const ForceArgs& a, int mb, double* red) {
     const Geo& G = a.geo;
     // member mb of a batch: its own generator, OU state, box and scalars
     const size_t box0 = (size_t)a.fbx * (2 * a.fby + 1) * mb;
     DevScalars* const dsc = a.sc + mb;
     double* const ou = a.ou + (size_t)mb * 2 * a.A;
-    double* const work = a.work + (size_t)mb * 4 * a.A;
+    double* const work = a.work + (size_t)mb * 5 * a.A;
     float* const box32 = reinterpret_cast<float*>(a.fbox) + 2 * box0;
     double* const box64 = reinterpret_cast<double*>(a.fbox) + 2 * box0;
     const unsigned long long seed = a.m_seed ? a.m_seed[mb] : a.seed;
@@ -542,7 +562,7 @@ __device__ __forceinline__ void force_draw(const ForceArgs& a, int mb, double* r
         alpha = exp(-dt / tau);
         beta = sqrt(fmax(1.0 - alpha * alpha, 0.0));
     }
-    for (int r = threadIdx.x; r < a.A; r += blockDim.x) {
+    auto draw = [&](int r) {
         const unsigned long long k = 2ull * (c * (unsigned long long)a.A + r) + 1ull;
         double u1 = uniform_at(seed, k), u2 = uniform_at(seed, k + 1);
         u1 = fmax(u1, 2.2250738585072014e-308);
@@ -555,12 +575,11 @@ __device__ __forceinline__ void force_draw(const ForceArgs& a, int mb, double* r
         }
         work[2 * r] = vr;
         work[2 * r + 1] = vi;
-    }
-    __syncthreads();
-    force_sum(a.A, red, [&](double t, int r) {
-        const double vr = work[2 * r], vi = work[2 * r + 1];
-        return fma(vr, vr, fma(vi, vi, t));
-    });
+        return mk(vr, vi);
+    };
+    force_sum<ALL>(
+        a.A, red, draw, [&](int r) { return mk(work[2 * r], work[2 * r + 1]); },
+        [](double t, cx<double> f) { return fma(f.x, f.x, fma(f.y, f.y, t)); });
     if (threadIdx.x == 0) s_scale = sqrt(a.energy_target / fmax(force_total(red), 1e-16));
     __syncthreads();
     const double sc = s_scale;
@@ -574,8 +593,9 @@ __device__ __forceinline__ void force_draw(const ForceArgs& a, int mb, double* r
     }
     __syncthreads();
     // Hermitian projection + mask, rate of the projected field
-    double* pr = work + 2 * a.A;  // projected values
-    for (int r = threadIdx.x; r < a.A; r += blockDim.x) {
+    double* const pr = work + 2 * a.A;  // projected values
+    double* const er = work + 4 * a.A;  // and the rates that they inject
+    auto project = [&](int r) {
         const int idx = a.modes[r];
         const int jy = idx / G.nkx, i = idx % G.nkx;
         double fr = work[2 * r], fi = work[2 * r + 1];
@@ -593,17 +613,13 @@ __device__ __forceinline__ void force_draw(const ForceArgs& a, int mb, double* r
         if (!kept(G, i, jy) || k2 <= 1e-12) fr = fi = 0.0;
         pr[2 * r] = fr;
         pr[2 * r + 1] = fi;
-    }
-    __syncthreads();
-    force_sum(a.A, red, [&](double t, int r) {
-        const int idx = a.modes[r];
-        const int jy = idx / G.nkx, i = idx % G.nkx;
-        const double fr = pr[2 * r], fi = pr[2 * r + 1];
-        const double kx = kx_of(G, i), ky = ky_of(G, jy);
-        const double k2 = kx * kx + ky * ky;
         const double wt = (i == 0 || 2 * i == G.nx) ? 1.0 : 2.0;
-        return k2 > 1e-12 ? t + 0.5 * wt * fma(fr, fr, fi * fi) / k2 : t;
-    });
+        const double e = k2 > 1e-12 ? 0.5 * wt * fma(fr, fr, fi * fi) / k2 : 0.0;
+        if constexpr (ALL) er[r] = e;
+        return e;
+    };
+    force_sum<ALL>(
+        a.A, red, project, [&](int r) { return er[r]; }, [](double t, double e) { return t + e; });
     if (threadIdx.x == 0) {
         const double t = force_total(red);
         s_scale = (t > 0.0 && a.rate > 0.0) ? sqrt(a.rate / t) : 0.0;
@@ -632,7 +648,6 @@ __device__ __forceinline__ void force_draw(const ForceArgs& a, int mb, double* r
     }
     if (threadIdx.x == 0) dsc->fcount = c + 1;
 }
-
 
 // ------------------------------------------------------------ column side
 
@@ -1816,7 +1831,7 @@ __global__ __launch_bounds__(NT, MW) void k_row(RowArgs<T> a) {
     cx<T>* lds2 = lds + (NB - 1) * RE;
     if constexpr (FORCE) {
         if (blockIdx.x == 0) {
-            force_draw(a.force, blockIdx.y, reinterpret_cast<double*>(smem_raw));
+            force_draw<(NT > kForceLanes)>(a.force, blockIdx.y, reinterpret_cast<double*>(smem_raw));
             return;
         }
     }
