@@ -31,7 +31,8 @@ typedef struct {
     double injection_rate;      /* energy injection rate of the forcing               */
     double k_peak;              /* random-phase initial field: E(k) ~ k^4 e^-(k/k_peak)^2 */
     double energy;              /* ... normalised to this energy                       */
-    int autotune;               /* choose kernel launch variants per size, default 1  */
+    int autotune;               /* choose kernel launch variants per size (the choice
+                                   does not show in the results), default 1           */
 } NSEnsembleConfig;
 
 typedef struct NSEnsemble NSEnsemble;

@@ -56,7 +56,7 @@ def context(n, precision=NSD_FP32, members=1, phys=PHYSICS, seeds=None, force_se
         raise RuntimeError(err.value.decode())
     p = params(n, phys, force_seed)
     _check(L, L.nsd_set_params(h, C.byref(p)), h, "nsd_set_params")
-    # launch shapes timed on this batch (lengths 64..1024; the tuner clears
+    # launch shapes timed on this batch (lengths up to 1024; the tuner clears
     # the state, so it runs before the initial field), as ensembles do
     _check(L, L.nsd_autotune(h, 3, 0, None, None), h, "nsd_autotune")
     if seeds is not None:

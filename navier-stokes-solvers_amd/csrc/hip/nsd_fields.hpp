@@ -1,4 +1,5 @@
-// nsd_fields.hpp -- field-parallel stage kernels for small launches.
+// nsd_fields.hpp -- field-parallel stage kernels: small FP64 grids, and any grid of up
+// to 1024 points a side by name (stage_variant_default has the rule).
 //
 // The stage kernels of nsd_kernels.hpp give a line to one group of L / 8
 // threads, which takes a row pair through its four inverse transforms and the
