@@ -500,6 +500,8 @@ struct ForceArgs {
 // that makes it: lane v adds the modes v, v + 256, ..., and the four waves' sums are
 // added in order.
 constexpr int kForceLanes = 256;
+// those that have modes, in whole waves
+__device__ __forceinline__ int force_lanes(int A) { return min(kForceLanes, (A + 63) & ~63); }
 
 // value(r) for the modes r < A, which also stores it where load(r) finds it, and
 // add(sum, value) over them, the waves' sums in red[0 .. 3]; every thread of a workgroup
@@ -511,32 +513,30 @@ __device__ __forceinline__ void force_sum(int A, double* red, V&& value, L&& loa
         for (int r = threadIdx.x; r < A; r += blockDim.x) (void)value(r);
         __syncthreads();
     }
-    for (int v = threadIdx.x; v < kForceLanes; v += blockDim.x) {
+    for (int v = threadIdx.x; v < force_lanes(A); v += blockDim.x) {
         double part = 0.0;
-        if ((v & ~63) < A) {
-            int r = v;
-            if constexpr (ALL) {
-                constexpr int N = 8;  // loads in flight
-                for (; r + (N - 1) * kForceLanes < A; r += N * kForceLanes) {
-                    decltype(load(0)) x[N];
+        int r = v;
+        if constexpr (ALL) {
+            constexpr int N = 8;  // loads in flight
+            for (; r + (N - 1) * kForceLanes < A; r += N * kForceLanes) {
+                decltype(load(0)) x[N];
 #pragma unroll
-                    for (int i = 0; i < N; ++i) x[i] = load(r + i * kForceLanes);
+                for (int i = 0; i < N; ++i) x[i] = load(r + i * kForceLanes);
 #pragma unroll
-                    for (int i = 0; i < N; ++i) part = add(part, x[i]);
-                }
-                for (; r < A; r += kForceLanes) part = add(part, load(r));
-            } else {
-                for (; r < A; r += kForceLanes) part = add(part, value(r));
+                for (int i = 0; i < N; ++i) part = add(part, x[i]);
             }
-            part = wave_sum(part);
+            for (; r < A; r += kForceLanes) part = add(part, load(r));
+        } else {
+            for (; r < A; r += kForceLanes) part = add(part, value(r));
         }
+        part = wave_sum(part);
         if ((v & 63) == 0) red[v >> 6] = part;
     }
     __syncthreads();
 }
-__device__ __forceinline__ double force_total(const double* red) {
+__device__ __forceinline__ double force_total(int A, const double* red) {
     double t = 0.0;
-    for (int i = 0; i < kForceLanes / 64; ++i) t += red[i];
+    for (int i = 0; i < force_lanes(A) / 64; ++i) t += red[i];
     return t;
 }
 
@@ -580,7 +580,7 @@ __device__ __forceinline__ void force_draw(const ForceArgs& a, int mb, double* r
     force_sum<ALL>(
         a.A, red, draw, [&](int r) { return mk(work[2 * r], work[2 * r + 1]); },
         [](double t, cx<double> f) { return fma(f.x, f.x, fma(f.y, f.y, t)); });
-    if (threadIdx.x == 0) s_scale = sqrt(a.energy_target / fmax(force_total(red), 1e-16));
+    if (threadIdx.x == 0) s_scale = sqrt(a.energy_target / fmax(force_total(a.A, red), 1e-16));
     __syncthreads();
     const double sc = s_scale;
     for (int r = threadIdx.x; r < a.A; r += blockDim.x) {
@@ -621,7 +621,7 @@ __device__ __forceinline__ void force_draw(const ForceArgs& a, int mb, double* r
     force_sum<ALL>(
         a.A, red, project, [&](int r) { return er[r]; }, [](double t, double e) { return t + e; });
     if (threadIdx.x == 0) {
-        const double t = force_total(red);
+        const double t = force_total(a.A, red);
         s_scale = (t > 0.0 && a.rate > 0.0) ? sqrt(a.rate / t) : 0.0;
     }
     __syncthreads();
