@@ -9,10 +9,11 @@ pytestmark = pytest.mark.gpu
 TWO_PI = 2 * np.pi
 
 
-# 37 modes, drawn in the row kernel, and 623, by a kernel of their own
-@pytest.mark.parametrize("kmax", [6.0, 20.0])
-def test_plain_steps_after_a_rejected_candidate(ns, oc, kmax):
-    n, steps, rate = 64, 3, 1e-3
+# 37 modes, drawn in the row kernel, 623 and 2527, by a kernel of their own (more than
+# the lanes of its sums take at once)
+@pytest.mark.parametrize("n,kmax", [(64, 6.0), (64, 20.0), (128, 40.0)])
+def test_plain_steps_after_a_rejected_candidate(ns, oc, n, kmax):
+    steps, rate = 3, 1e-3
     hv = dict(enabled=1, coefficient=1e-16 * (np.sqrt(2) * n / 2) ** 8, order=8, cutoff_ratio=0.0)
     o = oc.Oracle(n, n, TWO_PI, TWO_PI, 1e4)
     o.init_grids()
